@@ -51,52 +51,32 @@ void launch_gemm(T* pool, const GemmTask* tasks, int count, int kind, const int*
 template <typename T>
 void launch_gemm_seg(T* pool, const GemmTask* tasks, const SegTask* segs, const int* seg_ptr, int groups,
                      const FixTask* fixes, int nfix, T* part, const int* lidx, hipStream_t st, int lowp = 0);
-void launch_fwd_init(double* zpool, const double* b, int ldb, int nrhs, const NodeDev* nodes, const int2* tasks,
-                     int count, hipStream_t st);
-void launch_fwd_add(double* zpool, int nrhs, const NodeDev* nodes, const int* lidx, const int2* tasks, int count,
-                    hipStream_t st);
-template <typename T>
-void launch_fwd_step(const T* pool, double* zpool, int nrhs, const NodeDev* nodes, const SolveTask* tasks, int count,
-                     hipStream_t st);
-// The chunk tasks of a forward step alone (row0 >= 0), several workgroups
-// per CU.
-template <typename T>
-void launch_fwd_chunk(const T* pool, double* zpool, int nrhs, const NodeDev* nodes, const SolveTask* tasks, int count,
-                      hipStream_t st);
-// The chunk tasks of a backward step alone (row0 >= 0).
-template <typename T>
-void launch_bwd_chunk(const T* pool, const double* zpool, double* part, int nrhs, const NodeDev* nodes,
-                      const SolveTask* tasks, int count, hipStream_t st);
 // 64 x 64 blocks of the superblock matrices: X by block distance (wv =
 // false), then the W and V blocks (wv = true, MFMA tile products)
 template <typename T>
 void launch_superinv(const T* pool, T* sinv, const NodeDev* nodes, const SuperInvTask* tasks, int count, bool wv,
                      hipStream_t st);
-// forward sweep step over 256-column superblocks
-template <typename T>
-void launch_fwd_super(const T* pool, const T* sinv, double* zpool, int nrhs, const NodeDev* nodes,
-                      const SuperTask* tasks, int count, hipStream_t st);
-// backward top tasks over 256-column superblocks (the partial sums of the
-// rows after superblock u+1 come from k_bwd_step chunk tasks)
-template <typename T>
-void launch_bwd_super(const T* pool, const T* sinv, double* zpool, const double* part, double* x, int ldx, int nrhs,
-                      const NodeDev* nodes, const SuperTask* tasks, int count, hipStream_t st);
-// One launch of a forward step's superblock tasks (xtasks, workgroups [0,
-// nx)) and its 64-column step tasks (the rest).
-template <typename T>
-void launch_fwd_pair(const T* pool, const T* sinv, double* zpool, int nrhs, const NodeDev* nodes,
-                     const SuperTask* xtasks, int nx, const SolveTask* tasks, int count, hipStream_t st);
-// One launch of a backward step's superblock top tasks (xtasks, workgroups
-// [0, nx)) and its step tasks (the rest).
-template <typename T>
-void launch_bwd_pair(const T* pool, const T* sinv, double* zpool, double* part, double* x, int ldx, int nrhs,
-                     const NodeDev* nodes, const SuperTask* xtasks, int nx, const SolveTask* tasks, int count,
-                     hipStream_t st);
-void launch_bwd_gather(double* zpool, int nrhs, const NodeDev* nodes, const int* lidx, const int2* tasks, int count,
-                       hipStream_t st);
-template <typename T>
-void launch_bwd_step(const T* pool, double* zpool, double* part, double* x, int ldx, int nrhs, const NodeDev* nodes,
-                     const SolveTask* tasks, int count, hipStream_t st);
+// The solves (mfd_solve.hip): tasks of bundles bundle0 .. bundle0 + nbundles
+// - 1 for every group of 16 right-hand sides, one ticket word per launch.
+// z: planes of zs entries, one per right-hand side; b, y, x: n x nrhs.
+// flags: kSolveCtl control words, then nflags counters per group, all zero
+// at the start (launch_solve_reset); err: set when a wait reached its bound.
+template <typename T> struct SolveArgs {
+    const T* pool;
+    const T* sinv;
+    double* z;
+    const double* b;
+    double *y, *x;
+    const int *grow, *gptr, *gsrc;
+    const SolveTask* tasks;
+    const SolveBundle* bundles;
+    int *flags, *err;
+    int64_t zs;
+    int n, nrhs, ngroups, nflags, bundle0, nbundles, ticket;
+};
+constexpr int kRhsGroup = 16;
+void launch_solve_reset(int* flags, int64_t n, hipStream_t st);
+template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st);
 void launch_set_int(int* p, int v, hipStream_t st);
 void launch_residual(double* r, const double* b, const double* x, int n, int nrhs, const int* ptr, const int* col,
                      const double* val, hipStream_t st);

@@ -16,8 +16,7 @@
 //   k_upd_diag      with its panel's DTRSM tiles      border_kernel_m.f90:9-30
 //   k_gemm          DTRSM (modes 1, 2), DSYRK / DGEMM factorize_kernel_m.f90:11-33, border_kernel_m.f90:21-30,
 //                   updates (modes 0, 3)              border_subroutines_m.f90:41-73
-//   k_fwd_*         seq_forward (scatter_add, TRSV, GEMV)   seq_solve/seq_forward_m.f90:14-81
-//   k_bwd_*         seq_backward (gather, GEMV, TRSV)       seq_solve/seq_backward_m.f90:14-131
+// The solves are in mfd_solve.hip.
 #include <hip/hip_runtime.h>
 
 #include "mfd_kernels.h"
@@ -1310,346 +1309,6 @@ __global__ __launch_bounds__(kThreads) void k_front_wg(T* pool, const NodeDev* n
     }
 }
 
-// ------------------------------------------------------------------ solve
-// Blocked supernodal sweeps, level by level (the level's fronts in one
-// launch).  Front s's solve slice (per right-hand side, ld n and ld c):
-// Z[0:n] is the right-hand side being reduced (pivot part, then the update
-// part passed to the parent), Y[0:c] the solved pivot values (forward: y,
-// backward: x).  Diagonal blocks are applied through their stored inverses,
-// so no kernel runs a sequential loop: forward one launch per 64-column
-// block, backward two (seq_forward_m.f90:14-81, seq_backward_m.f90:14-131).
-constexpr int kRhsGroup = 8;  // right-hand sides processed together
-
-// LDS of the solve tasks, named so that a launch holding two kinds of task
-// keeps them in one union.
-struct FwdStepLds {
-    union {
-        struct {
-            double LI[64][65];
-            double Lp[64][65];  // Lp[k][i] = L[k0 + i][k0 - 64 + k], block task
-        } b;
-        double red[4][64][kRhsGroup + 1];  // chunk task: partial sums per column quarter
-    } u;
-    double zt[64][kRhsGroup], yt[64][kRhsGroup];
-};
-struct SuperLds {
-    double zs[kSuper][kRhsGroup + 1], ys[kSuper][kRhsGroup + 1];  // the backward task's x_{u+1} in ys
-    double red[16][16][kRhsGroup + 1];
-};
-// block and chunk tasks of the backward step use disjoint layouts (two
-// workgroups per CU)
-struct BwdChunkLds {
-    double Ls[64][65];              // L columns, staged rows
-    double Xs[256][kRhsGroup + 1];  // x of the chunk's rows
-};
-union BwdStepLds {
-    struct {
-        double LI[64][65];             // the diagonal block's inverse
-        double Ln[64][65];             // Ln[k][i] = L[k0 + 64 + i][k0 + k]
-        double zt[64][kRhsGroup];
-        double Xn[64][kRhsGroup + 1];  // x of block t+1
-    } b;
-    BwdChunkLds c;
-};
-
-// Forward, first launch of a level, task (front, first row): 256 rows of
-// the front's Z, pivot part from b, update part zero.
-__global__ __launch_bounds__(kThreads) void k_fwd_init(double* zpool, const double* b, int ldb, int nrhs,
-                                                       const NodeDev* nodes, const int2* tasks)
-{
-    const int2 t = tasks[blockIdx.x];
-    const NodeDev nd = nodes[t.x];
-    const int i = t.y + threadIdx.x;
-    if (i >= nd.n) return;
-    double* Z = zpool + nd.z * nrhs;
-    for (int r = 0; r < nrhs; ++r)
-        Z[i + (int64_t)r * nd.n] = i < nd.c ? b[(int64_t)(nd.first + i) + (int64_t)r * ldb] : 0.0;
-}
-
-// Forward, one launch per child rank: task (child, first row) adds 256 rows
-// of the child's update part into its parent's Z (scatter_add,
-// sparse_add_subroutines_m.f90:13-30).  A launch holds at most one child of
-// each parent, and the ranks run in child order.
-__global__ __launch_bounds__(kThreads) void k_fwd_add(double* zpool, int nrhs, const NodeDev* nodes, const int* lidx,
-                                                      const int2* tasks)
-{
-    const int2 t = tasks[blockIdx.x];
-    const NodeDev ch = nodes[t.x];
-    const int i = t.y + threadIdx.x;
-    if (i >= ch.w) return;
-    const NodeDev pa = nodes[ch.parent];
-    double* Zp = zpool + pa.z * nrhs;
-    const double* Zc = zpool + ch.z * nrhs;
-    const int p = lidx[ch.lidx + i] - 1;
-    for (int r = 0; r < nrhs; ++r) Zp[p + (int64_t)r * pa.n] += Zc[(ch.c + i) + (int64_t)r * ch.n];
-}
-
-// Forward sweep, one launch per block step t (DTRSV "U","T" and DGEMV "T",
-// solve_kernel_m.f90:4-23), pipelined one block behind:
-//   - the block task (row0 < 0) solves block t: z = Z_t - L[B_t, B_{t-1}]
-//     y_{t-1} (pad = order of block t-1; 0 for the first block), y_t =
-//     inv(L_tt) z, written to Y_t;
-//   - a chunk task (row0 >= 0) applies block k0/64 (= t - 1) to its 64
-//     rows, all after block t: Z[rows] -= L[rows, B_{t-1}] y_{t-1} (four
-//     threads per row, 16 columns each, summed through LDS).
-// No task of a launch depends on another task of the same launch, and every
-// global read of a task is issued before its first wait.
-// Forward chunk task (row0 >= 0, pad0 != 1): block B = k0/64 applied to the
-// 64 rows from row0 (all after the block the step solves), Z[rows] -=
-// L[rows, B] y_B (yt: staging of y_B; red: the four column quarters' partial
-// sums).
-template <typename T>
-__device__ __forceinline__ void fwd_chunk_task(const T* pool, double* zpool, int nrhs, const NodeDev* nodes,
-                                               const SolveTask t, double (&yt)[64][kRhsGroup],
-                                               double (&red)[4][64][kRhsGroup + 1])
-{
-    const NodeDev nd = nodes[t.node];
-    const int n = nd.n, c = nd.c, kb = t.kb, tid = threadIdx.x, lane = tid & 63, ty = tid >> 6;
-    double* Z = zpool + nd.z * nrhs;
-    const double* Y = Z + (int64_t)n * nrhs;
-    const T* Lb = pool + nd.front + (int64_t)t.k0 * n;
-    // 64 rows; thread (row lane, quarter ty) takes columns 16 ty .. 16 ty + 15
-    const int row = t.row0 + lane;
-    const bool live = row < n;
-    // Unconditional loads from clamped (in-bounds) positions, kept in the
-    // raw element type (a conditional or converted load would wait for
-    // the previous one) and not masked: past column kb they multiply the
-    // zeros of yt, and rows past n are not stored, so the z and y loads
-    // below go out without waiting for these.
-    const int rowc = min(row, n - 1);
-    T l[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) l[j] = ld_off(Lb, (unsigned)(rowc + min(16 * ty + j, kb - 1) * n));
-    for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-        // this thread stores right-hand sides r0 + ty and r0 + ty + 4; the
-        // right-hand side of every load below is uniform over the wave (no
-        // load for the group's missing ones), its row clamped in bounds
-        const double z0 = ty < nr ? Z[rowc + (int64_t)(r0 + ty) * n] : 0.0;
-        const double z1 = ty + 4 < nr ? Z[rowc + (int64_t)(r0 + ty + 4) * n] : 0.0;
-        static_assert(64 * kRhsGroup == 2 * kThreads, "two staged entries per thread");
-        double yv[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = tid + kThreads * h, k = e & 63, r = e >> 6;
-            yv[h] = r < nr ? Y[t.k0 + min(k, kb - 1) + (int64_t)(r0 + r) * c] : 0.0;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = tid + kThreads * h, k = e & 63, r = e >> 6;
-            yt[k][r] = (k < kb && r < nr) ? yv[h] : 0.0;
-        }
-        __syncthreads();
-        double acc[kRhsGroup];
-#pragma unroll
-        for (int r = 0; r < kRhsGroup; ++r) acc[r] = 0.0;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const double lk = (double)l[j];
-#pragma unroll
-            for (int r = 0; r < kRhsGroup; ++r) acc[r] += lk * yt[16 * ty + j][r];
-        }
-#pragma unroll
-        for (int r = 0; r < kRhsGroup; ++r) red[ty][lane][r] = acc[r];
-        __syncthreads();
-        if (live) {
-            if (ty < nr)
-                Z[row + (int64_t)(r0 + ty) * n] =
-                    z0 - ((red[0][lane][ty] + red[1][lane][ty]) + (red[2][lane][ty] + red[3][lane][ty]));
-            if (ty + 4 < nr)
-                Z[row + (int64_t)(r0 + ty + 4) * n] =
-                    z1 - ((red[0][lane][ty + 4] + red[1][lane][ty + 4]) +
-                          (red[2][lane][ty + 4] + red[3][lane][ty + 4]));
-        }
-        __syncthreads();
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void fwd_step_task(const T* pool, double* zpool, int nrhs, const NodeDev* nodes,
-                                              const SolveTask t, FwdStepLds& S)
-{
-    const NodeDev nd = nodes[t.node];
-    auto& u = S.u;
-    auto& zt = S.zt;
-    auto& yt = S.yt;
-    double(*LI)[65] = u.b.LI;
-    double(*Lp)[65] = u.b.Lp;
-    const int n = nd.n, c = nd.c, kb = t.kb, tid = threadIdx.x, lane = tid & 63, ty = tid >> 6;
-    double* Z = zpool + nd.z * nrhs;
-    double* Y = Z + (int64_t)n * nrhs;
-    const T* Lb = pool + nd.front + (int64_t)t.k0 * n;
-    if (t.pad0 == 1) {
-        // a front of one pivot block (k0 = 0, kb = c): y = inv(L_00) z, then
-        // its update rows 64 at a time, Z[rows] -= L[rows, 0:c] y
-        const T* inv = pool + nd.inv;
-        T li[16];
-#pragma unroll
-        for (int p = 0; p < 16; ++p) {
-            const int e = tid + kThreads * p, i = e & 63, k = e >> 6;
-            li[p] = ld_off(inv, (unsigned)((i < kb && k < kb) ? e : 0));
-        }
-#pragma unroll
-        for (int p = 0; p < 16; ++p) {
-            const int e = tid + kThreads * p, i = e & 63, k = e >> 6;
-            li[p] = (i < kb && k < kb) ? li[p] : T(0);
-        }
-        for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-            const int nr = min(kRhsGroup, nrhs - r0);
-#pragma unroll
-            for (int p = 0; p < 16; ++p) {
-                const int e = tid + kThreads * p;
-                LI[e & 63][e >> 6] = (double)li[p];
-            }
-            double zv[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int e = tid + kThreads * h, k = e & 63, r = e >> 6;  // r: uniform over the wave
-                zv[h] = r < nr ? Z[min(k, kb - 1) + (int64_t)(r0 + r) * n] : 0.0;
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int e = tid + kThreads * h, k = e & 63, r = e >> 6;
-                zt[k][r] = (k < kb && r < nr) ? zv[h] : 0.0;
-            }
-            __syncthreads();
-            for (int r = ty; r < kRhsGroup; r += 4) {
-                double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int k = 0; k < 64; ++k) acc[k & 3] += LI[k][lane] * zt[k][r];
-                const double y = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-                if (lane < kb && r < nr) Y[lane + (int64_t)(r0 + r) * c] = y;
-                yt[lane][r] = (lane < kb && r < nr) ? y : 0.0;
-            }
-            __syncthreads();
-            for (int rr = c; rr < n; rr += 64) {
-                const int row = rr + lane;
-                const bool live = row < n;
-                const int rowc = min(row, n - 1);
-                T l[16];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) l[j] = ld_off(Lb, (unsigned)(rowc + min(16 * ty + j, kb - 1) * n));
-                // rows clamped in bounds (used only where in range); ty: the wave
-                const double z0 = ty < nr ? Z[rowc + (int64_t)(r0 + ty) * n] : 0.0;
-                const double z1 = ty + 4 < nr ? Z[rowc + (int64_t)(r0 + ty + 4) * n] : 0.0;
-                double acc[kRhsGroup];
-#pragma unroll
-                for (int r = 0; r < kRhsGroup; ++r) acc[r] = 0.0;
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const double lk = (double)l[j];
-#pragma unroll
-                    for (int r = 0; r < kRhsGroup; ++r) acc[r] += lk * yt[16 * ty + j][r];
-                }
-#pragma unroll
-                for (int r = 0; r < kRhsGroup; ++r) u.red[ty][lane][r] = acc[r];
-                __syncthreads();
-                if (live) {
-                    if (ty < nr)
-                        Z[row + (int64_t)(r0 + ty) * n] =
-                            z0 - ((u.red[0][lane][ty] + u.red[1][lane][ty]) + (u.red[2][lane][ty] + u.red[3][lane][ty]));
-                    if (ty + 4 < nr)
-                        Z[row + (int64_t)(r0 + ty + 4) * n] =
-                            z1 - ((u.red[0][lane][ty + 4] + u.red[1][lane][ty + 4]) +
-                                  (u.red[2][lane][ty + 4] + u.red[3][lane][ty + 4]));
-                }
-                __syncthreads();
-            }
-        }
-        return;
-    }
-    if (t.row0 >= 0) {
-        fwd_chunk_task<T>(pool, zpool, nrhs, nodes, t, yt, u.red);
-        return;
-    }
-    // block task
-    const int kp = t.pad;
-    const T* inv = pool + nd.inv + (int64_t)(t.k0 / 64) * 4096;
-    // block (B_t, B_{t-1}): rows k0.., columns k0 - 64.. (only read when kp > 0)
-    const T* Lq = kp > 0 ? pool + nd.front + t.k0 + (int64_t)(t.k0 - 64) * n : Lb;
-    // entries outside the kb x kb block read entry 0 (one line for all of
-    // them instead of the whole padded 64 x 64 block) and are zeroed below
-    T li[16], lp[16];
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p, i = e & 63, k = e >> 6;
-        li[p] = ld_off(inv, (unsigned)((i < kb && k < kb) ? e : 0));
-        lp[p] = ld_off(Lq, (unsigned)(min(i, kb - 1) + min(k, max(kp, 1) - 1) * n));
-    }
-    // the first right-hand-side group's z and y, in flight with the above
-    double zv[2], yv[2];
-    // from clamped in-bounds positions (y of block t-1 from entry 0 when
-    // there is none), masked as they are staged
-    auto load_zy = [&](int r0) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = tid + kThreads * h, k = e & 63, r = e >> 6;  // r: uniform over the wave
-            const int64_t rc = r0 + r;
-            zv[h] = r < nr ? Z[t.k0 + min(k, kb - 1) + rc * n] : 0.0;
-            yv[h] = (r < nr && kp > 0) ? Y[t.k0 - 64 + min(k, kp - 1) + rc * c] : 0.0;
-        }
-    };
-    load_zy(0);
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p, i = e & 63, k = e >> 6;
-        lp[p] = (i < kb && k < kp) ? lp[p] : T(0);
-        li[p] = (i < kb && k < kb) ? li[p] : T(0);
-    }
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p;
-        LI[e & 63][e >> 6] = li[p];
-        Lp[e >> 6][e & 63] = lp[p];
-    }
-    // Lp, LI, zt and yt are zero past kp / kb, so the products run over all
-    // 64 entries, unrolled, with four partial sums.
-    for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-        if (r0 > 0) load_zy(r0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = tid + kThreads * h, k = e & 63, r = e >> 6;
-            zt[k][r] = (k < kb && r < nr) ? zv[h] : 0.0;
-            yt[k][r] = (k < kp && r < nr) ? yv[h] : 0.0;
-        }
-        __syncthreads();
-        for (int r = ty; r < nr; r += 4) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int k = 0; k < 64; ++k) acc[k & 3] += Lp[k][lane] * yt[k][r];
-            zt[lane][r] -= (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        }
-        __syncthreads();
-        for (int r = ty; r < nr; r += 4) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int k = 0; k < 64; ++k) acc[k & 3] += LI[k][lane] * zt[k][r];
-            if (lane < kb) Y[t.k0 + lane + (int64_t)(r0 + r) * c] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        }
-        __syncthreads();
-    }
-}
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_fwd_step(const T* pool, double* zpool, int nrhs, const NodeDev* nodes,
-                                                       const SolveTask* tasks)
-{
-    __shared__ FwdStepLds S;
-    fwd_step_task<T>(pool, zpool, nrhs, nodes, tasks[blockIdx.x], S);
-}
-
-// A forward step's chunk tasks alone (steps with many of them): without the
-// block task's LDS and registers several workgroups share a CU.
-template <typename T>
-__global__ __launch_bounds__(kThreads, 6) void k_fwd_chunk(const T* pool, double* zpool, int nrhs, const NodeDev* nodes,
-                                                        const SolveTask* tasks)
-{
-    __shared__ double yt[64][kRhsGroup];
-    __shared__ double red[4][64][kRhsGroup + 1];
-    fwd_chunk_task<T>(pool, zpool, nrhs, nodes, tasks[blockIdx.x], yt, red);
-}
-
 // ------------------------------------------------------------ superblocks
 // The three 256 x 256 matrices of superblock u, column-major, X at xoff, W
 // at xoff + 256^2 (u >= 1), V at xoff + 2 256^2 (superblock u+1 not empty):
@@ -1760,517 +1419,6 @@ __global__ __launch_bounds__(kThreads) void k_superwv(const T* pool, T* sinv, co
     }
     const int row = threadIdx.x & 63;
     for (int col = threadIdx.x >> 6; col < 64; col += 4) dst[row + kSuper * col] = u.Cs[col][row];
-}
-
-// Forward sweep over superblocks, one launch per superblock step u, every
-// task 16 rows wide (thread: row tid % 16, columns 16 g .. 16 g + 15 of
-// each 256-column operand, g = tid / 16; the 16 partial sums per row summed
-// through LDS):
-//   - top task (kind 1, rows row0 .. row0 + 15 of superblock u):
-//     y_u = X z_u - W y_{u-1}, written to Y (z_u: Z at the superblock's
-//     rows, already holding every superblock before u - 1);
-//   - chunk task (kind 0, front rows row0 .. row0 + 15, all after
-//     superblock u): Z[rows] -= L[rows, B_{u-1}] y_{u-1}.
-// Every matrix load of a task is issued before its first wait.
-template <typename T>
-__device__ __forceinline__ void fwd_super_task(const T* pool, const T* sinv, double* zpool, int nrhs,
-                                               const NodeDev* nodes, const SuperTask t, SuperLds& S)
-{
-    const NodeDev nd = nodes[t.node];
-    const int n = nd.n, c = nd.c, c0 = kSuper * t.u, cp = c0 - kSuper, tid = threadIdx.x;
-    const int i = tid & 15, g = tid >> 4;
-    double* Z = zpool + nd.z * nrhs;
-    double* Y = Z + (int64_t)n * nrhs;
-    auto& zs = S.zs;
-    auto& ys = S.ys;
-    auto& red = S.red;
-    const int pb = t.pb, sb = t.sb;
-    const bool top = t.kind == 1;
-    T a[16], w[16];
-    if (top) {
-        const T* X = sinv + t.xoff;
-        const int r = t.row0 + i;
-        // all loads inside the superblock's X and W (W of the first
-        // superblock is unused storage), masked where used
-#pragma unroll
-        for (int q = 0; q < 16; ++q) a[q] = X[r + kSuper * (16 * g + q)];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) w[q] = X[kSuper * kSuper + r + kSuper * (16 * g + q)];
-    } else {
-        const T* Lr = pool + nd.front + min(t.row0 + i, n - 1) + (int64_t)cp * n;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) w[q] = Lr[(int64_t)min(16 * g + q, pb - 1) * n];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) a[q] = T(0);
-    }
-    const bool lower = 16 * g <= t.row0 + 15;  // X is lower triangular
-    for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-        // y of superblock u-1 and z of superblock u from clamped positions
-        // (entry 0 where there is none), all loads before the masked stores
-        static_assert(kSuper == kThreads, "one superblock entry per thread");
-        double yv[kRhsGroup], zv[kRhsGroup];
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) {
-            // rr < nr, pb > 0 and top are uniform
-            yv[rr] = (rr < nr && pb > 0) ? Y[cp + min(tid, pb - 1) + (int64_t)(r0 + rr) * c] : 0.0;
-            zv[rr] = (rr < nr && top) ? Z[c0 + min(tid, sb - 1) + (int64_t)(r0 + rr) * n] : 0.0;
-        }
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) {
-            ys[tid][rr] = (tid < pb && rr < nr) ? yv[rr] : 0.0;
-            if (top) zs[tid][rr] = (tid < sb && rr < nr) ? zv[rr] : 0.0;
-        }
-        __syncthreads();
-        double acc[kRhsGroup];
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) acc[rr] = 0.0;
-        if (top) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const double av = lower ? (double)a[q] : 0.0;
-#pragma unroll
-                for (int rr = 0; rr < kRhsGroup; ++rr) acc[rr] += av * zs[16 * g + q][rr];
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const double wv = 16 * g + q < pb ? (double)w[q] : 0.0;  // pb = 0: w unused
-#pragma unroll
-            for (int rr = 0; rr < kRhsGroup; ++rr) acc[rr] -= wv * ys[16 * g + q][rr];
-        }
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) red[g][i][rr] = acc[rr];
-        __syncthreads();
-        if (tid < 16 * kRhsGroup) {
-            const int i2 = tid & 15, rr = tid >> 4;
-            double v = 0.0;
-#pragma unroll
-            for (int gg = 0; gg < 16; ++gg) v += red[gg][i2][rr];
-            if (rr < nr) {
-                if (top) {
-                    if (t.row0 + i2 < sb) Y[c0 + t.row0 + i2 + (int64_t)(r0 + rr) * c] = v;
-                } else if (t.row0 + i2 < n) {
-                    Z[t.row0 + i2 + (int64_t)(r0 + rr) * n] += v;
-                }
-            }
-        }
-        __syncthreads();
-    }
-}
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_fwd_super(const T* pool, const T* sinv, double* zpool, int nrhs,
-                                                        const NodeDev* nodes, const SuperTask* tasks)
-{
-    __shared__ SuperLds S;
-    fwd_super_task<T>(pool, sinv, zpool, nrhs, nodes, tasks[blockIdx.x], S);
-}
-
-// A forward step's superblock tasks (workgroups [0, nx)) and 64-column step
-// tasks (the rest) in one launch: they touch different fronts.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_fwd_pair(const T* pool, const T* sinv, double* zpool, int nrhs,
-                                                       const NodeDev* nodes, const SuperTask* xtasks, int nx,
-                                                       const SolveTask* tasks)
-{
-    __shared__ union {
-        SuperLds x;
-        FwdStepLds s;
-    } u;
-    if ((int)blockIdx.x < nx)
-        fwd_super_task<T>(pool, sinv, zpool, nrhs, nodes, xtasks[blockIdx.x], u.x);
-    else
-        fwd_step_task<T>(pool, zpool, nrhs, nodes, tasks[blockIdx.x - nx], u.s);
-}
-
-// Backward sweep over superblocks, top tasks (kind 2), 16 rows of
-// superblock u each, in the launch of backward step u (thread: row
-// tid % 16, entries 16 g .. 16 g + 15 of each 256-long operand, g = tid /
-// 16; the 16 partial sums per row summed through LDS):
-//   x_u = X^T (y_u - q_u) - V^T x_{u+1},
-// y_u from Y, q_u summed in a fixed order from the partial-sum slots that
-// the previous launch's chunk tasks wrote (the rows after superblock u+1),
-// x_{u+1} from Z (the pivot part of x of these fronts lives in Z, so that
-// no task of a launch reads what another writes); x_u goes to Z and to x.
-template <typename T>
-__device__ __forceinline__ void bwd_super_task(const T* pool, const T* sinv, double* zpool, const double* part,
-                                               double* x, int ldx, int nrhs, const NodeDev* nodes, const SuperTask t,
-                                               SuperLds& S)
-{
-    const NodeDev nd = nodes[t.node];
-    const int n = nd.n, c = nd.c, c0 = kSuper * t.u, cn = c0 + kSuper, tid = threadIdx.x;
-    const int i = tid & 15, g = tid >> 4;
-    double* Z = zpool + nd.z * nrhs;
-    const double* Y = Z + (int64_t)n * nrhs;
-    auto& zs = S.zs;
-    auto& xs = S.ys;
-    auto& red = S.red;
-    const int pb = t.pb, sb = t.sb;
-    const T* X = sinv + t.xoff;
-    const T* V = X + 2 * kSuper * kSuper;
-    const int col = t.row0 + i;  // column of X and V: the row of x_u
-    T a[16], v[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) a[q] = X[(16 * g + q) + kSuper * col];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = V[(16 * g + q) + kSuper * col];  // unused storage when pb = 0
-    static_assert(kSuper == kThreads, "one superblock entry per thread");
-    const int m = tid;  // the entry of y_u, q_u and x_{u+1} this thread stages
-    // every load below from a clamped in-bounds position (x_{u+1} from entry
-    // 0 when there is none), masked as it is staged
-    const int mc = min(m, sb - 1);
-    const double* pp = part + (int64_t)(t.slot + t.nchunk * (mc >> 6)) * 64 * nrhs + (mc & 63);
-    const int64_t cs = (int64_t)64 * nrhs;  // stride between chunks
-    for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-        // the chunks' partial sums two at a time, every load of a pair (all
-        // right-hand sides of the group) issued before the subtractions
-        double zv[kRhsGroup], xv[kRhsGroup];
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) {
-            // rr < nr and pb > 0 are uniform
-            zv[rr] = rr < nr ? Y[c0 + mc + (int64_t)(r0 + rr) * c] : 0.0;
-            xv[rr] = (rr < nr && pb > 0) ? Z[cn + min(m, pb - 1) + (int64_t)(r0 + rr) * n] : 0.0;
-        }
-        for (int ch = 0; ch < t.nchunk; ch += 2) {
-            const int ch2 = min(ch + 1, t.nchunk - 1);  // the last chunk twice when odd
-            double p0[kRhsGroup], p1[kRhsGroup];
-#pragma unroll
-            for (int rr = 0; rr < kRhsGroup; ++rr) {
-                const double* q = pp + (int64_t)(r0 + rr) * 64;
-                p0[rr] = rr < nr ? q[ch * cs] : 0.0;
-                p1[rr] = rr < nr ? q[ch2 * cs] : 0.0;
-            }
-            const bool two = ch + 1 < t.nchunk;
-#pragma unroll
-            for (int rr = 0; rr < kRhsGroup; ++rr) zv[rr] = (zv[rr] - p0[rr]) - (two ? p1[rr] : 0.0);
-        }
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) {
-            zs[m][rr] = (rr < nr && m < sb) ? zv[rr] : 0.0;
-            xs[m][rr] = (rr < nr && m < pb) ? xv[rr] : 0.0;
-        }
-        __syncthreads();
-        double acc[kRhsGroup];
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) acc[rr] = 0.0;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const double av = (double)a[q], vv = pb > 0 ? (double)v[q] : 0.0;
-#pragma unroll
-            for (int rr = 0; rr < kRhsGroup; ++rr) acc[rr] += av * zs[16 * g + q][rr] - vv * xs[16 * g + q][rr];
-        }
-#pragma unroll
-        for (int rr = 0; rr < kRhsGroup; ++rr) red[g][i][rr] = acc[rr];
-        __syncthreads();
-        if (tid < 16 * kRhsGroup) {
-            const int i2 = tid & 15, rr = tid >> 4, row = t.row0 + i2;
-            double s = 0.0;
-#pragma unroll
-            for (int gg = 0; gg < 16; ++gg) s += red[gg][i2][rr];
-            if (rr < nr && row < sb) {
-                Z[c0 + row + (int64_t)(r0 + rr) * n] = s;
-                x[(int64_t)(nd.first + c0 + row) + (int64_t)(r0 + rr) * ldx] = s;
-            }
-        }
-        __syncthreads();
-    }
-}
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_bwd_super(const T* pool, const T* sinv, double* zpool, const double* part,
-                                                        double* x, int ldx, int nrhs, const NodeDev* nodes,
-                                                        const SuperTask* tasks)
-{
-    __shared__ SuperLds S;
-    bwd_super_task<T>(pool, sinv, zpool, part, x, ldx, nrhs, nodes, tasks[blockIdx.x], S);
-}
-
-// Backward, first launch of a level, task (front, first row): 256 rows of
-// the update part of Z take the parent's solution at the parent-front
-// positions -- pivot positions from the parent's Y, update positions from
-// the parent's Z (gather, sparse_add_subroutines_m.f90:32-49).
-__global__ __launch_bounds__(kThreads) void k_bwd_gather(double* zpool, int nrhs, const NodeDev* nodes, const int* lidx,
-                                                         const int2* tasks)
-{
-    const int2 t = tasks[blockIdx.x];
-    const NodeDev nd = nodes[t.x];
-    const int i = t.y + threadIdx.x;
-    if (nd.parent < 0 || i >= nd.w) return;
-    const NodeDev pa = nodes[nd.parent];
-    double* Z = zpool + nd.z * nrhs;
-    const double* Zp = zpool + pa.z * nrhs;
-    const double* Yp = Zp + (int64_t)pa.n * nrhs;
-    const int p = lidx[nd.lidx + i] - 1;
-    for (int r = 0; r < nrhs; ++r)
-        Z[(nd.c + i) + (int64_t)r * nd.n] = (p < pa.c && !pa.xz) ? Yp[p + (int64_t)r * pa.c] : Zp[p + (int64_t)r * pa.n];
-}
-
-// Backward sweep, one launch per block step t (DGEMV "N" + DTRSV "U","N",
-// solve_kernel_m.f90:11-16,25-30), pipelined one block ahead:
-//   - the block task (row0 < 0) solves block t:
-//       z = Y_t - sum of the nchunk partials at part[slot..] (rows after
-//           block t+1, formed by the previous launch) - L[B_{t+1}, B_t]^T x_{t+1}
-//       x_t = inv(L_tt)^T z, written to Y_t (and, for t = 0, the front's
-//       pivot part of x);  pad = kb of block t+1 (0: no such block);
-//   - a chunk task (row0 >= 0) forms, for block k0/64 (= t - 1), the partial
-//     products P[slot][k][r] = sum over its 256 rows of L[row][k0+k] x[row][r]
-//     for its 16 of the block's columns (pad0 = which 16; four tasks per
-//     chunk) or, with pad0 < 0, for all 64 (launches with many chunks) on
-//     MFMA (x from Y on pivot rows, from Z on update rows; every row lies
-//     after block t, so its x is final).
-// No task of a launch depends on another task of the same launch, and the
-// partials are summed in a fixed order.
-// Backward chunk task (row0 >= 0): the partial sums of block k0/64 (all 64
-// columns, pad0 < 0, or columns 16 pad0 .. 16 pad0 + 15) over the 256 rows
-// from row0, into slot `slot` of part.
-template <typename T>
-__device__ __forceinline__ void bwd_chunk_task(const T* pool, const double* zpool, double* part, int nrhs,
-                                               const NodeDev* nodes, const SolveTask t, BwdChunkLds& S)
-{
-    const NodeDev nd = nodes[t.node];
-    const int n = nd.n, c = nd.c, kb = t.kb, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const double* Z = zpool + nd.z * nrhs;
-    const double* Y = Z + (int64_t)n * nrhs;
-    const T* Lb = pool + nd.front + (int64_t)t.k0 * n;
-    if (t.row0 >= 0 && t.pad0 < 0) {
-        // all 64 columns in one task: wave w takes columns 16 w .. 16 w + 15,
-        // the 256 rows staged 64 at a time through LDS
-        typedef typename Mfma<double>::acc_t acc_t;
-        const int row = t.row0 + tid;
-        const bool live = row < n;
-        // Unconditional loads from clamped (in-bounds) positions, kept in the
-        // raw element type (a conditional or converted load would wait for
-        // the previous one) and not masked: rows past n meet the zero x of
-        // Xs, and partials past column kb are never read, so the x loads
-        // below go out without waiting for these.
-        const int rowc = min(row, n - 1);
-        T l[64];
-#pragma unroll
-        for (int k = 0; k < 64; ++k) l[k] = ld_off(Lb, (unsigned)(rowc + min(k, kb - 1) * n));
-        for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-            const int nr = min(kRhsGroup, nrhs - r0);
-#pragma unroll
-            for (int r = 0; r < kRhsGroup; ++r)
-                S.Xs[tid][r] = (live && r < nr) ? ((row < c && !nd.xz) ? Y[row + (int64_t)(r0 + r) * c]
-                                                                          : Z[row + (int64_t)(r0 + r) * n])
-                                              : 0.0;
-            acc_t acc = {0, 0, 0, 0};
-            const int rc = lane & 15;
-            for (int sb = 0; sb < 4; ++sb) {
-                __syncthreads();
-                if (wv == sb) {
-#pragma unroll
-                    for (int k = 0; k < 64; ++k) S.Ls[k][lane] = l[k];
-                }
-                __syncthreads();
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const int rr = 4 * q + (lane >> 4);
-                    const double a = S.Ls[16 * wv + rc][rr];
-                    const double b = rc < nr ? S.Xs[64 * sb + rr][rc] : 0.0;
-                    acc = Mfma<double>::mma(a, b, acc);
-                }
-            }
-            if (rc < nr) {
-                double* P = part + (int64_t)t.slot * 64 * nrhs + (int64_t)(r0 + rc) * 64;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) P[16 * wv + Mfma<double>::row(lane, v)] = acc[v];
-            }
-            __syncthreads();
-        }
-        return;
-    }
-    if (t.row0 >= 0) {
-        // columns 16 pad0 .. 16 pad0 + 15 of block k0/64 over the chunk's 256
-        // rows: one row per thread, a quarter of the rows per wave, the four
-        // waves' 16 x 16 products added through LDS
-        typedef typename Mfma<double>::acc_t acc_t;
-        const int col0 = 16 * t.pad0, row = t.row0 + tid;
-        const bool live = row < n;
-        // Unconditional loads from clamped (in-bounds) positions, kept in the
-        // raw element type (a conditional or converted load would wait for
-        // the previous one) and not masked: rows past n meet the zero x of
-        // Xs, and partials past column kb are never read, so the x loads
-        // below go out without waiting for these.
-        const int rowc = min(row, n - 1);
-        T l[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) l[j] = ld_off(Lb, (unsigned)(rowc + min(col0 + j, kb - 1) * n));
-        double(*Lc)[kThreads + 4] = reinterpret_cast<double(*)[kThreads + 4]>(&S.Ls[0][0]);   // 16 x 260
-        double(*red)[16][17] = reinterpret_cast<double(*)[16][17]>(&S.Ls[0][0]);              // 4 x 16 x 17
-        const int rc = lane & 15;
-        for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-            const int nr = min(kRhsGroup, nrhs - r0);
-#pragma unroll
-            for (int r = 0; r < kRhsGroup; ++r)
-                S.Xs[tid][r] = (live && r < nr) ? ((row < c && !nd.xz) ? Y[row + (int64_t)(r0 + r) * c]
-                                                                          : Z[row + (int64_t)(r0 + r) * n])
-                                              : 0.0;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) Lc[j][tid] = (double)l[j];
-            __syncthreads();
-            acc_t acc = {0, 0, 0, 0};
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int rr = 64 * wv + 4 * q + (lane >> 4);
-                const double a = Lc[rc][rr];
-                const double b = rc < nr ? S.Xs[rr][rc] : 0.0;
-                acc = Mfma<double>::mma(a, b, acc);
-            }
-            __syncthreads();
-#pragma unroll
-            for (int v = 0; v < 4; ++v) red[wv][Mfma<double>::row(lane, v)][rc] = acc[v];
-            __syncthreads();
-            if (tid < 16 * nr) {
-                const int m = tid & 15, r = tid >> 4;
-                part[(int64_t)t.slot * 64 * nrhs + (int64_t)(r0 + r) * 64 + col0 + m] =
-                    (red[0][m][r] + red[1][m][r]) + (red[2][m][r] + red[3][m][r]);
-            }
-            __syncthreads();
-        }
-        return;
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void bwd_step_task(const T* pool, double* zpool, double* part, double* x, int ldx, int nrhs,
-                                              const NodeDev* nodes, const SolveTask t, BwdStepLds& u)
-{
-    const NodeDev nd = nodes[t.node];
-    const int n = nd.n, c = nd.c, kb = t.kb, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    double* Z = zpool + nd.z * nrhs;
-    double* Y = Z + (int64_t)n * nrhs;
-    const T* Lb = pool + nd.front + (int64_t)t.k0 * n;
-    if (t.row0 >= 0) {
-        bwd_chunk_task<T>(pool, zpool, part, nrhs, nodes, t, u.c);
-        return;
-    }
-    // block task: every global read first
-    const int kn = t.pad;  // rows of block t+1 (0: none)
-    const T* inv = pool + nd.inv + (int64_t)(t.k0 / 64) * 4096;
-    // entries outside the kb x kb block read entry 0 and are zeroed below
-    T li[16], ln[16];
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p, i = e & 63, k = e >> 6;
-        li[p] = ld_off(inv, (unsigned)((i < kb && k < kb) ? e : 0));
-        // (row k0 itself when there is no next block: always inside the front)
-        ln[p] = ld_off(Lb, (unsigned)(t.k0 + (kn > 0 ? 64 + min(i, kn - 1) : 0) + min(k, kb - 1) * n));
-    }
-    // z = y_t - the partial sums, and x of block t+1, for one group of
-    // right-hand sides (two entries of each per thread); the first group's
-    // loads go out with the factor loads above
-    double zv[2], xv[2];
-    // (from clamped in-bounds positions, x of block t+1 from entry 0 when
-    // there is none; masked as they are staged)
-    auto load_zx = [&](int r0) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = tid + kThreads * h, k = e & 63, r = e >> 6, kc = min(k, kb - 1);  // r: uniform over the wave
-            const int64_t rc = r0 + r;
-            double z = 0.0;
-            if (r < nr) {
-                z = Y[t.k0 + kc + rc * c];
-                const double* pp = part + (int64_t)t.slot * 64 * nrhs + kc + rc * 64;
-#pragma unroll 4
-                for (int ch = 0; ch < t.nchunk; ++ch) z -= pp[(int64_t)ch * 64 * nrhs];
-            }
-            zv[h] = z;
-            xv[h] = (r < nr && kn > 0) ? Y[t.k0 + 64 + min(k, kn - 1) + rc * c] : 0.0;
-        }
-    };
-    load_zx(0);
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p, i = e & 63, k = e >> 6;
-        ln[p] = (i < kn && k < kb) ? ln[p] : T(0);
-        li[p] = (i < kb && k < kb) ? li[p] : T(0);
-    }
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p;
-        u.b.LI[e & 63][e >> 6] = li[p];
-        u.b.Ln[e >> 6][e & 63] = ln[p];
-    }
-    for (int r0 = 0; r0 < nrhs; r0 += kRhsGroup) {
-        const int nr = min(kRhsGroup, nrhs - r0);
-        if (r0 > 0) load_zx(r0);
-        // zt, and x of block t+1 staged in u.b.Xn[0..kn)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = tid + kThreads * h, k = e & 63, r = e >> 6;
-            u.b.zt[k][r] = (k < kb && r < nr) ? zv[h] : 0.0;
-            u.b.Xn[k][r] = (k < kn && r < nr) ? xv[h] : 0.0;
-        }
-        __syncthreads();
-        // z_k -= sum_i L[k0 + 64 + i][k0 + k] x_{t+1}[i]; Ln, LI, Xn and zt
-        // are zero past kn / kb, so the sums run over all 64 entries,
-        // unrolled, with four partial sums
-        for (int r = wv; r < nr; r += 4) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int i = 0; i < 64; ++i) acc[i & 3] += u.b.Ln[lane][i] * u.b.Xn[i][r];
-            if (lane < kb) u.b.zt[lane][r] -= (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        }
-        __syncthreads();
-        for (int r = wv; r < nr; r += 4) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int m = 0; m < 64; ++m) acc[m & 3] += u.b.LI[lane][m] * u.b.zt[m][r];
-            const double v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-            if (lane < kb) {
-                Y[t.k0 + lane + (int64_t)(r0 + r) * c] = v;
-                if (t.k0 == 0) x[(int64_t)(nd.first + lane) + (int64_t)(r0 + r) * ldx] = v;
-            }
-        }
-        __syncthreads();
-    }
-    // The front's first block is its last one solved: the other blocks'
-    // values were written to Y by earlier launches.
-    if (t.k0 == 0 && c > kb) {
-        const int rest = c - kb;
-        for (int e = tid; e < rest * nrhs; e += kThreads) {
-            int i = kb + e % rest, r = e / rest;
-            x[(int64_t)(nd.first + i) + (int64_t)r * ldx] = Y[i + (int64_t)r * c];
-        }
-    }
-}
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_bwd_step(const T* pool, double* zpool, double* part, double* x, int ldx,
-                                                       int nrhs, const NodeDev* nodes, const SolveTask* tasks)
-{
-    __shared__ BwdStepLds u;
-    bwd_step_task<T>(pool, zpool, part, x, ldx, nrhs, nodes, tasks[blockIdx.x], u);
-}
-
-// A backward step's chunk tasks alone (steps with many of them): without the
-// block task's LDS and registers more workgroups share a CU.
-template <typename T>
-__global__ __launch_bounds__(kThreads, 3) void k_bwd_chunk(const T* pool, const double* zpool, double* part, int nrhs,
-                                                        const NodeDev* nodes, const SolveTask* tasks)
-{
-    __shared__ BwdChunkLds S;
-    bwd_chunk_task<T>(pool, zpool, part, nrhs, nodes, tasks[blockIdx.x], S);
-}
-
-// A backward step's superblock top tasks (workgroups [0, nx)) and its step
-// tasks (the rest) in one launch: the top tasks of superblock t read the
-// partial sums of the bank the step tasks do not write and x of superblock
-// t + 1, and write x of superblock t, which no step task of the launch reads.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_bwd_pair(const T* pool, const T* sinv, double* zpool, double* part,
-                                                       double* x, int ldx, int nrhs, const NodeDev* nodes,
-                                                       const SuperTask* xtasks, int nx, const SolveTask* tasks)
-{
-    __shared__ union {
-        SuperLds x;
-        BwdStepLds s;
-    } u;
-    if ((int)blockIdx.x < nx)
-        bwd_super_task<T>(pool, sinv, zpool, part, x, ldx, nrhs, nodes, xtasks[blockIdx.x], u.x);
-    else
-        bwd_step_task<T>(pool, zpool, part, x, ldx, nrhs, nodes, tasks[blockIdx.x - nx], u.s);
 }
 
 // ----------------------------------------------- permutations and residual
@@ -2577,36 +1725,6 @@ void launch_gemm_seg(T* pool, const GemmTask* tasks, const SegTask* segs, const 
     if (nfix > 0)
         hipLaunchKernelGGL(k_gemm_fix<T>, dim3(nfix), dim3(kThreads), 0, st, pool, tasks, fixes, part, lidx);
 }
-void launch_fwd_init(double* zpool, const double* b, int ldb, int nrhs, const NodeDev* nodes, const int2* tasks,
-                     int count, hipStream_t st)
-{
-    if (count > 0) hipLaunchKernelGGL(k_fwd_init, dim3(count), dim3(kThreads), 0, st, zpool, b, ldb, nrhs, nodes, tasks);
-}
-void launch_fwd_add(double* zpool, int nrhs, const NodeDev* nodes, const int* lidx, const int2* tasks, int count,
-                    hipStream_t st)
-{
-    if (count > 0) hipLaunchKernelGGL(k_fwd_add, dim3(count), dim3(kThreads), 0, st, zpool, nrhs, nodes, lidx, tasks);
-}
-template <typename T>
-void launch_fwd_step(const T* pool, double* zpool, int nrhs, const NodeDev* nodes, const SolveTask* tasks, int count,
-                     hipStream_t st)
-{
-    if (count > 0) hipLaunchKernelGGL(k_fwd_step<T>, dim3(count), dim3(kThreads), 0, st, pool, zpool, nrhs, nodes, tasks);
-}
-template <typename T>
-void launch_fwd_chunk(const T* pool, double* zpool, int nrhs, const NodeDev* nodes, const SolveTask* tasks, int count,
-                      hipStream_t st)
-{
-    if (count > 0)
-        hipLaunchKernelGGL(k_fwd_chunk<T>, dim3(count), dim3(kThreads), 0, st, pool, zpool, nrhs, nodes, tasks);
-}
-template <typename T>
-void launch_bwd_chunk(const T* pool, const double* zpool, double* part, int nrhs, const NodeDev* nodes,
-                      const SolveTask* tasks, int count, hipStream_t st)
-{
-    if (count > 0)
-        hipLaunchKernelGGL(k_bwd_chunk<T>, dim3(count), dim3(kThreads), 0, st, pool, zpool, part, nrhs, nodes, tasks);
-}
 template <typename T>
 void launch_superinv(const T* pool, T* sinv, const NodeDev* nodes, const SuperInvTask* tasks, int count, bool wv,
                      hipStream_t st)
@@ -2616,51 +1734,6 @@ void launch_superinv(const T* pool, T* sinv, const NodeDev* nodes, const SuperIn
         hipLaunchKernelGGL(k_superwv<T>, dim3(count), dim3(kThreads), 0, st, pool, sinv, nodes, tasks);
     else
         hipLaunchKernelGGL(k_superinv<T>, dim3(count), dim3(kThreads), 0, st, pool, sinv, nodes, tasks);
-}
-template <typename T>
-void launch_fwd_super(const T* pool, const T* sinv, double* zpool, int nrhs, const NodeDev* nodes,
-                      const SuperTask* tasks, int count, hipStream_t st)
-{
-    if (count > 0)
-        hipLaunchKernelGGL(k_fwd_super<T>, dim3(count), dim3(kThreads), 0, st, pool, sinv, zpool, nrhs, nodes, tasks);
-}
-template <typename T>
-void launch_bwd_super(const T* pool, const T* sinv, double* zpool, const double* part, double* x, int ldx, int nrhs,
-                      const NodeDev* nodes, const SuperTask* tasks, int count, hipStream_t st)
-{
-    if (count > 0)
-        hipLaunchKernelGGL(k_bwd_super<T>, dim3(count), dim3(kThreads), 0, st, pool, sinv, zpool, part, x, ldx, nrhs,
-                           nodes, tasks);
-}
-template <typename T>
-void launch_fwd_pair(const T* pool, const T* sinv, double* zpool, int nrhs, const NodeDev* nodes,
-                     const SuperTask* xtasks, int nx, const SolveTask* tasks, int count, hipStream_t st)
-{
-    if (nx + count > 0)
-        hipLaunchKernelGGL(k_fwd_pair<T>, dim3(nx + count), dim3(kThreads), 0, st, pool, sinv, zpool, nrhs, nodes, xtasks,
-                           nx, tasks);
-}
-template <typename T>
-void launch_bwd_pair(const T* pool, const T* sinv, double* zpool, double* part, double* x, int ldx, int nrhs,
-                     const NodeDev* nodes, const SuperTask* xtasks, int nx, const SolveTask* tasks, int count,
-                     hipStream_t st)
-{
-    if (nx + count > 0)
-        hipLaunchKernelGGL(k_bwd_pair<T>, dim3(nx + count), dim3(kThreads), 0, st, pool, sinv, zpool, part, x, ldx, nrhs,
-                           nodes, xtasks, nx, tasks);
-}
-void launch_bwd_gather(double* zpool, int nrhs, const NodeDev* nodes, const int* lidx, const int2* tasks, int count,
-                       hipStream_t st)
-{
-    if (count > 0) hipLaunchKernelGGL(k_bwd_gather, dim3(count), dim3(kThreads), 0, st, zpool, nrhs, nodes, lidx, tasks);
-}
-template <typename T>
-void launch_bwd_step(const T* pool, double* zpool, double* part, double* x, int ldx, int nrhs, const NodeDev* nodes,
-                     const SolveTask* tasks, int count, hipStream_t st)
-{
-    if (count > 0)
-        hipLaunchKernelGGL(k_bwd_step<T>, dim3(count), dim3(kThreads), 0, st, pool, zpool, part, x, ldx, nrhs, nodes,
-                           tasks);
 }
 void launch_gather_rows(double* out, int ld_out, const double* in, int ld_in, const int* perm, int n, int nrhs,
                         hipStream_t st)
@@ -2691,23 +1764,9 @@ void launch_scatter_rows(double* out, int ld_out, const double* in, int ld_in, c
     template void launch_gemm<T>(T*, const GemmTask*, int, int, const int*, hipStream_t, int);                         \
     template void launch_scatter_a_scaled<T>(T*, const double*, const int64_t*, const int64_t*, const int2*,           \
                                              const double*, int64_t, hipStream_t);                                    \
-    template void launch_fwd_step<T>(const T*, double*, int, const NodeDev*, const SolveTask*, int, hipStream_t);       \
-    template void launch_fwd_chunk<T>(const T*, double*, int, const NodeDev*, const SolveTask*, int, hipStream_t);      \
-    template void launch_bwd_chunk<T>(const T*, const double*, double*, int, const NodeDev*, const SolveTask*, int,    \
-                                      hipStream_t);                                                                    \
     template void launch_superinv<T>(const T*, T*, const NodeDev*, const SuperInvTask*, int, bool, hipStream_t);      \
-    template void launch_fwd_super<T>(const T*, const T*, double*, int, const NodeDev*, const SuperTask*, int,         \
-                                      hipStream_t);                                                                    \
     template void launch_gemm_seg<T>(T*, const GemmTask*, const SegTask*, const int*, int, const FixTask*, int, T*,  \
-                                     const int*, hipStream_t, int);                                                    \
-    template void launch_bwd_super<T>(const T*, const T*, double*, const double*, double*, int, int, const NodeDev*,    \
-                                      const SuperTask*, int, hipStream_t);                                             \
-    template void launch_fwd_pair<T>(const T*, const T*, double*, int, const NodeDev*, const SuperTask*, int,          \
-                                     const SolveTask*, int, hipStream_t);                                              \
-    template void launch_bwd_pair<T>(const T*, const T*, double*, double*, double*, int, int, const NodeDev*,          \
-                                     const SuperTask*, int, const SolveTask*, int, hipStream_t);                       \
-    template void launch_bwd_step<T>(const T*, double*, double*, double*, int, int, const NodeDev*, const SolveTask*,  \
-                                     int, hipStream_t);
+                                     const int*, hipStream_t, int);
 MFD_INSTANTIATE(double)
 MFD_INSTANTIATE(float)
 

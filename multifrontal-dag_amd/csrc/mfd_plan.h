@@ -18,14 +18,11 @@ constexpr int kSmallFront = 64;  // fronts up to this order are factored whole i
 struct NodeDev {
     int64_t front;   // element offset of the front in the pool
     int64_t lidx;    // offset of this node's local_index (w entries) in the lidx array
-    int64_t z;       // per-rhs offset of the solve slice ((n + c) entries per rhs) in the z pool
     int64_t inv;     // element offset (in the pool) of the inverses of the 64 x 64 diagonal blocks
     int n, c, w;
     int parent;      // 0-based parent node, -1 for a root
     int first;       // 0-based first global (postordered) column
-    int xz;          // 1: the backward solve keeps the pivot part of x in Z
-                     // (fronts solved over superblocks), 0: in Y
-    int pad[2];
+    int pad;
 };
 
 // Extend-add of one 64 x 64 tile (ti >= tj) of child's update matrix.
@@ -48,43 +45,53 @@ struct DiagTask {
     int kpp, applied, pad1, pad2;
 };
 
-// One block step of the blocked supernodal solves: the pivot block
-// [k0, k0+kb) of a front and, for the row-chunk tasks, the rows from row0
-// (forward: 64 rows; backward: 256; row0 < 0: the block's own task).
-// Forward: a block task's pad is the order of the previous pivot block;
-// pad0 = 1 marks a front of one pivot block, whose task also applies it to
-// the front's update rows.
-// Backward: a chunk task writes columns 16 pad0 .. 16 pad0 + 15 of
-// partial-sum slot `slot` (64 x nrhs doubles); a block task reads the nchunk
-// slots from `slot` and pad is the order of the next pivot block (0 for the
-// front's last block).
-struct SolveTask {
-    int node, k0, kb, row0;
-    int slot, nchunk, pad0, pad;
-};
-
-// Superblocks: the solves of a front with many pivot columns step over
-// 256-column superblocks u (columns B_u) with three 256 x 256 matrices per
-// superblock (column-major, in a separate array at xoff): X, the inverse of
-// the superblock's diagonal block (zero past its width); at xoff + 256^2
-// W = X L[B_u, B_{u-1}] (u >= 1, forward); at xoff + 2 256^2
-// V = L[B_{u+1}, B_u] X (B_{u+1} not empty, backward).
+// Superblocks: the solves step over 256-column superblocks u (columns B_u) of
+// a front.  Fronts with many pivot columns ("super") do so through three 256
+// x 256 matrices per superblock (column-major, in a separate array at xoff):
+// X, the inverse of the superblock's diagonal block (zero past its width);
+// at xoff + 256^2 W = X L[B_u, B_{u-1}] (u >= 1, forward); at xoff + 2 256^2
+// V = L[B_{u+1}, B_u] X (B_{u+1} not empty, backward).  The others solve a
+// superblock by one workgroup through the stored inverses of its 64 x 64
+// diagonal blocks.
 constexpr int kSuper = 256;
 constexpr int64_t kSuperMats = 3 * (int64_t)kSuper * kSuper;  // entries per superblock
-// Forward task of superblock step u, 16 rows: kind 1, rows row0 .. row0 +
-// 15 of superblock u (width sb; pb the width of superblock u-1, 0 for
-// u = 0); kind 0, front rows row0 .. row0 + 15 after superblock u, to which
-// superblock u-1 (width pb) is applied.
-// Backward task (kind 2), rows row0 .. row0 + 15 of superblock u (width
-// sb; pb the width of superblock u+1, 0 if none): x_u = X^T (y_u - q) -
-// V^T x_{u+1}, with q summed from the partial-sum slots slot + nchunk j +
-// ch (64 columns of block j of the superblock, chunk ch < nchunk).
-struct SuperTask {
-    int node, u, row0, sb;
-    int pb, kind;
-    int slot, nchunk;
-    int64_t xoff;
+
+// A workgroup's turn in the solves (mfd_solve.hip; built by
+// mfd_solve_plan.cpp).  Forward: kFwdRows / kFwdRows64, nr (<= 16 / 64) front
+// rows from r0, superblocks v < nslot applied to them, sig raised; kFwdTop,
+// rows r0 .. r0 + 15 of superblock u (super fronts); kFwdPiv, superblock u
+// (other fronts) and then, nr > 0, the front's nr update rows, sig raised.
+// Backward: kBwdPart, partial sums of the 64 columns from column nslot over
+// nr (<= 256) rows from r0, to plane offset slot, sig raised; kBwdCols, nr
+// (<= 16) columns r0 .. of superblock u, superblocks v >= grow applied to
+// them, sig raised; kBwdTop, columns r0 .. r0 + 15 of superblock u; kBwdPiv,
+// superblock u, before it (nr > 0) the front's nr update rows.  In kBwdCols,
+// kBwdTop and kBwdPiv, nslot chunks of partial sums per 64 columns lie at
+// slot.  Every task waits for counter w0 to reach w0t (w0 < 0: for nothing)
+// and for the y_v (x_v) it takes up.
+enum SolveKind { kFwdRows, kFwdRows64, kFwdTop, kFwdPiv, kBwdPart, kBwdCols, kBwdTop, kBwdPiv };
+struct SolveTask {
+    int64_t front;  // element offset of the front in the pool
+    int64_t aux;    // kFwdTop, kBwdTop: superblock u's matrices; kFwdPiv, kBwdPiv: inverse of its first 64 x 64 block
+    int n, c, first;  // the front; its 0-based first global column
+    int z;            // front row i lies at z + i of a right-hand side's plane
+    int kind, u, r0, nr;
+    int goff;         // the front's gather list (gptr[goff + i], row i; < 0: no children)
+    int grow;         // its update rows' global rows (backward), or the first superblock of kBwdCols
+    int slot, nslot;
+    int w0, w0t, sig;
+    int flag, fstr;   // the front's counters: asm, then z, y, p, t, x of each superblock, fstr apart
+    int nsup, super;  // superblocks; 1: super front
+    int pad;
 };
+// A ticket: tasks [first, first + count) in order.
+struct SolveBundle {
+    int first, count;
+};
+// Words before the counters in the solve's control array: the two tickets
+// (whole solve or forward part; backward part), the stop word.
+constexpr int kSolveTicket = 0, kSolveTicketBwd = 16, kSolveStop = 32, kSolveCtl = 64;
+
 // One 64 x 64 block (i, j) of superblock u's matrices: j = i copies the
 // stored 64 x 64 inverse (and clears the row's blocks above the diagonal,
 // or the whole row past the superblock's width); j < i forms

@@ -29,6 +29,7 @@
 #include "mfd_host.h"
 #include "mfd_kernels.h"
 #include "mfd_layout.h"
+#include "mfd_solve_plan.h"
 #include "mfdag.h"
 
 using namespace mfd;
@@ -55,24 +56,16 @@ struct Launch {
     // side_id) beside the next step's launch; wait_id >= 0: this launch
     // first waits for side launch wait_id.  Serial when profiling.
     int side = 0, side_id = -1, wait_id = -1;
-    // solve launches: the step they belong to (a step's kFS and kFX
-    // launches, and its kBS and kBX launches, run as one launch)
-    int step = -1;
 };
 
 // A step's update tiles join the step's launch (k_upd_diag, one workgroup
 // per CU at its LDS) up to this many; more run as their own launch.
 constexpr int kFillGroups = 32;  // most level groups the front zeroing is split into
-constexpr int kWholeRows = 128;   // update rows of a one-block front solved by its block task
 constexpr int kFuseTiles = 1024;
 
 // Step launches with at least this many diagonal tasks run their GEMM
 // tiles (TRSM and fused update tiles) as a second launch (k_gemm).
 constexpr int kApartDiag = 512;
-
-// Backward solve steps with at most this many row chunks split each chunk
-// into four 16-column tasks (shorter tasks where the step is latency-bound).
-constexpr int kSplitChunks = 256;
 
 // The in-panel update of the large fronts runs every `period` steps with
 // K = period panels (fewer passes over the trailing columns); the TRSM tiles
@@ -96,9 +89,8 @@ constexpr int kWideTile = 128;
 constexpr int kWideMinRows = 0;
 
 // Fronts with at least super_min pivot columns solve forward and backward
-// over 256-column superblocks (k_fwd_super, k_bwd_super: a quarter of the
-// dependent launches of the 64-column steps), with their superblock
-// matrices formed at the end of the factorization; set per handle by
+// through explicit superblock matrices (kFwdTop, kBwdTop: sixteen workgroups
+// a superblock), formed at the end of the factorization; set per handle by
 // mfd_set_solve_block (0: never).  256: on the 64^3 workload the bounds 128,
 // 256, 512 and 1024 gave FP64 steps of 25.08, 25.13, 25.17 and 25.39 ms,
 // and on the 512-system batch 128 was slower than 512 (FP64 step 21.26
@@ -194,27 +186,17 @@ struct mfd_handle {
     std::vector<GemmTask> gemm;
     std::vector<Launch> fseq;
     std::vector<int> level_ptr, level_nodes, child_ptr, child_list;
-    // solve schedule: kinds kFI/kFA/kFS (forward) and kBG/kBS (backward)
-    std::vector<int2> fi, fa, bg;  // (front, first row) tasks of the gathers
-    int2 *d_fi = nullptr, *d_fa = nullptr, *d_bg = nullptr;
-    std::vector<SolveTask> fstep, bstep;
-    std::vector<Launch> fwd_seq, bwd_seq;
-    int64_t part_slots = 0;
-    SolveTask *d_fstep = nullptr, *d_bstep = nullptr;
-    // superblock forward steps (kind kFX), backward top tasks (kind kBX)
-    // and the blocks of the superblock matrices: X by block distance i - j
-    // ([xinv_ptr[d], xinv_ptr[d + 1]), d = 0..3), then W and V
-    // ([xinv_ptr[4], xinv_ptr[5]))
-    std::vector<SuperTask> xstep, xbstep;
-    std::vector<SuperInvTask> xinv;
-    int xinv_ptr[6] = {};
-    int64_t sinv_elems = 0;
-    SuperTask *d_xstep = nullptr, *d_xbstep = nullptr;
+    // the solves: task list (mfd_solve_plan.h) and its device copies
+    SolvePlan sp;
+    SolveTask* d_stasks = nullptr;
+    SolveBundle* d_sbundles = nullptr;
+    int *d_grow = nullptr, *d_gptr = nullptr, *d_gsrc = nullptr;
     SuperInvTask* d_xinv = nullptr;
+    int solve_rc = 0;          // build_solve_plan's result for the current schedule
+    int* solve_err = nullptr;  // pinned: set by a solve whose wait reached its bound
     double* d_sinv64 = nullptr;
     float* d_sinv32 = nullptr;
-    double* d_part = nullptr;
-    int64_t pool_elems = 0, z_per_rhs = 0;
+    int64_t pool_elems = 0;
     int num_levels = 0;
 
     // device copies
@@ -239,7 +221,8 @@ struct mfd_handle {
     int* d_info = nullptr;
     // solve buffers
     int nrhs_cap = 0;
-    double *d_z = nullptr, *d_bin = nullptr, *d_bp = nullptr, *d_xp = nullptr;
+    double *d_z = nullptr, *d_y = nullptr, *d_bin = nullptr, *d_bp = nullptr, *d_xp = nullptr;
+    int* d_sflags = nullptr;  // control words and counters of a solve
     // refinement
     int *d_csr_ptr = nullptr, *d_csr_col = nullptr;
     int64_t* d_csr_src = nullptr;  // index into the caller-order values of each CSR entry
@@ -360,8 +343,9 @@ void free_device(mfd_handle* h)
     h->d_fill = nullptr;
     h->d_gemm = nullptr;
     h->d_level_nodes = h->d_child_ptr = h->d_child_list = nullptr;
-    h->d_fstep = h->d_bstep = nullptr;
-    h->d_xstep = h->d_xbstep = nullptr;
+    h->d_stasks = nullptr;
+    h->d_sbundles = nullptr;
+    h->d_grow = h->d_gptr = h->d_gsrc = nullptr;
     h->d_xinv = nullptr;
     h->d_segs = nullptr;
     h->d_seg_ptr = nullptr;
@@ -369,8 +353,6 @@ void free_device(mfd_handle* h)
     h->d_segpart = nullptr;
     h->d_sinv64 = nullptr;
     h->d_sinv32 = nullptr;
-    h->d_fi = h->d_fa = h->d_bg = nullptr;
-    h->d_part = nullptr;
     h->d_dst = h->d_src = nullptr;
     h->d_scat_rc = nullptr;
     h->d_diag_src = nullptr;
@@ -381,7 +363,8 @@ void free_device(mfd_handle* h)
     h->d_a = nullptr;
     h->d_info = nullptr;
     h->nrhs_cap = 0;
-    h->d_z = h->d_bin = h->d_bp = h->d_xp = nullptr;
+    h->d_z = h->d_y = h->d_bin = h->d_bp = h->d_xp = nullptr;
+    h->d_sflags = nullptr;
     h->d_csr_ptr = h->d_csr_col = nullptr;
     h->d_csr_src = nullptr;
     h->d_csr_val = nullptr;
@@ -392,293 +375,13 @@ void free_device(mfd_handle* h)
 int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 
 // ------------------------------------------------------------- schedule
-enum SolveKind { kFI = 100, kFA, kFS, kBG, kBS, kFX, kBX, kFC, kBC };
-
-// A solve step with at least this many chunk tasks launches them apart from
-// its block tasks (k_fwd_chunk, k_bwd_chunk: more workgroups per CU than the
-// block tasks' two).
-constexpr int kChunkLaunch = 1024;
-
-// Solve schedule.  Forward: one launch setting every front's Z from b,
-// then per level: one launch per child rank adding the children's update
-// parts, then launches t = 0 .. steps: the block task of block t (which
-// first applies block t - 1 to block t) and the row chunks applying block
-// t - 1 to the rows after block t.  Fronts with at least super_min pivot columns step over
-// superblocks of 256 columns instead (kind kFX, launched beside step t's
-// kFS launch): the superblock task of superblock t and the row chunks
-// applying superblock t - 1 to the rows after it.
-// Backward, per level: a gather launch, then launches t = steps .. 0: the
-// block task of block t (for fronts that have it) and the row chunks forming
-// the partial sums block t - 1 needs from the rows after block t (launch
-// t = steps only has chunks).  Partials of block j live in bank j % 2, so a
-// launch never overwrites the partials its block tasks read.  Superblock
-// fronts step 256 columns at a time here too: the top tasks of superblock t
-// (kind kBX, after step t's kBS launch) and, in the kBS launch, chunk tasks
-// forming the partial sums of superblock t - 1's four 64-column blocks from
-// the rows after superblock t; their pivot part of x lives in Z (NodeDev::xz).
-void build_solve_plan(mfd_handle* h)
-{
-    h->fstep.clear();
-    h->bstep.clear();
-    h->fi.clear();
-    h->fa.clear();
-    h->bg.clear();
-    h->fwd_seq.clear();
-    h->bwd_seq.clear();
-    h->part_slots = 0;
-    h->xstep.clear();
-    h->xbstep.clear();
-    h->xinv.clear();
-    h->sinv_elems = 0;
-    auto push = [](std::vector<Launch>& seq, int kind, int64_t first, int64_t end, int step = -1) {
-        if (end > first) {
-            seq.push_back(Launch{kind, first, (int)(end - first)});
-            seq.back().step = step;
-        }
-    };
-    auto super = [&](const NodeDev& d) { return h->super_min > 0 && d.c >= h->super_min; };
-    // steps of a level when superblock fronts step 256 columns at a time
-    // (forward and backward alike)
-    auto fsteps_of = [&](int L) {
-        int steps = 0;
-        for (int k = h->level_ptr[L]; k < h->level_ptr[L + 1]; ++k) {
-            const NodeDev& d = h->nodes[h->level_nodes[k]];
-            steps = std::max(steps, (d.c + (super(d) ? kSuper : 64) - 1) / (super(d) ? kSuper : 64));
-        }
-        return steps;
-    };
-    for (auto& d : h->nodes) d.xz = super(d) ? 1 : 0;
-    // superblock matrices (X, W and V, 3 x 256^2 entries per superblock):
-    // four launches of X blocks by block distance, then one of W and V
-    // blocks
-    const int64_t per_super = kSuperMats;
-    std::vector<int64_t> xoff(h->nodes.size(), -1);
-    for (size_t s = 0; s < h->nodes.size(); ++s)
-        if (super(h->nodes[s])) {
-            xoff[s] = h->sinv_elems;
-            h->sinv_elems += (int64_t)((h->nodes[s].c + kSuper - 1) / kSuper) * per_super;
-        }
-    for (int dist = 0; dist <= 4; ++dist) {
-        h->xinv_ptr[dist] = (int)h->xinv.size();
-        for (size_t s = 0; s < h->nodes.size(); ++s) {
-            if (xoff[s] < 0) continue;
-            const int c = h->nodes[s].c;
-            for (int u = 0; u * kSuper < c; ++u) {
-                const int64_t xo = xoff[s] + u * per_super;
-                if (dist == 4) {
-                    if (u > 0)
-                        for (int i = 0; i < 4; ++i)
-                            for (int j = 0; j < 4; ++j) h->xinv.push_back(SuperInvTask{(int)s, u, i, 4 + j, xo});
-                    if ((u + 1) * kSuper < c)
-                        for (int i = 0; i < 4; ++i)
-                            for (int j = 0; j < 4; ++j) h->xinv.push_back(SuperInvTask{(int)s, u, i, 8 + j, xo});
-                    continue;
-                }
-                for (int i = dist; i < 4; ++i)
-                    if (dist == 0 || u * kSuper + 64 * i < c) h->xinv.push_back(SuperInvTask{(int)s, u, i, i - dist, xo});
-            }
-        }
-    }
-    h->xinv_ptr[5] = (int)h->xinv.size();
-    // every front's Z (pivot part from b, update part zero) in one launch:
-    // the fronts' Z regions are disjoint
-    for (int L = 0; L < h->num_levels; ++L)
-        for (int k = h->level_ptr[L]; k < h->level_ptr[L + 1]; ++k) {
-            const int s = h->level_nodes[k];
-            for (int r0 = 0; r0 < h->nodes[s].n; r0 += 256) h->fi.push_back(make_int2(s, r0));
-        }
-    push(h->fwd_seq, kFI, 0, (int64_t)h->fi.size());
-    for (int L = 0; L < h->num_levels; ++L) {
-        const int b0 = h->level_ptr[L], b1 = h->level_ptr[L + 1];
-        {
-            int64_t f;
-            // children's update parts, one launch per child rank
-            size_t maxch = 0;
-            for (int k = b0; k < b1; ++k) {
-                const int s = h->level_nodes[k];
-                maxch = std::max(maxch, (size_t)(h->child_ptr[s + 1] - h->child_ptr[s]));
-            }
-            for (size_t r = 0; r < maxch; ++r) {
-                f = (int64_t)h->fa.size();
-                for (int k = b0; k < b1; ++k) {
-                    const int s = h->level_nodes[k];
-                    if ((size_t)(h->child_ptr[s + 1] - h->child_ptr[s]) <= r) continue;
-                    const int ch = h->child_list[h->child_ptr[s] + r];
-                    for (int r0 = 0; r0 < h->nodes[ch].w; r0 += 256) h->fa.push_back(make_int2(ch, r0));
-                }
-                push(h->fwd_seq, kFA, f, (int64_t)h->fa.size());
-            }
-        }
-        const int steps = fsteps_of(L);
-        std::vector<SolveTask> chunks;
-        for (int t = 0; t <= steps; ++t) {
-            int64_t f0 = (int64_t)h->fstep.size(), x0 = (int64_t)h->xstep.size();
-            chunks.clear();
-            for (int k = b0; k < b1; ++k) {
-                const int s = h->level_nodes[k];
-                const NodeDev& d = h->nodes[s];
-                if (super(d)) {
-                    const int U = (d.c + kSuper - 1) / kSuper;
-                    const int64_t xo = xoff[s] + t * per_super;
-                    if (t <= U - 1) {
-                        const int sb = std::min(kSuper, d.c - kSuper * t);
-                        for (int r0 = 0; r0 < sb; r0 += 16)
-                            h->xstep.push_back(SuperTask{s, t, r0, sb, t > 0 ? kSuper : 0, 1, 0, 0, xo});
-                    }
-                    if (t >= 1 && t - 1 <= U - 1) {
-                        // superblock t - 1 applied to the rows after superblock t
-                        const int pb = std::min(kSuper, d.c - kSuper * (t - 1));
-                        for (int r0 = std::min(kSuper * (t + 1), d.c); r0 < d.n; r0 += 16)
-                            h->xstep.push_back(SuperTask{s, t, r0, 0, pb, 0, 0, 0, xo});
-                    }
-                    continue;
-                }
-                const int T = (d.c + 63) / 64;
-                // a front of one block with few update rows: one task solves
-                // the block and applies it to those rows
-                const bool whole = T == 1 && d.w <= kWholeRows;
-                if (t <= T - 1) {
-                    const int k0 = 64 * t, kb = std::min(64, d.c - k0);
-                    h->fstep.push_back(SolveTask{s, k0, kb, -1, 0, 0, whole ? 1 : 0, t > 0 ? 64 : 0});
-                }
-                if (!whole && t >= 1 && t - 1 <= T - 1) {
-                    // block t - 1 applied to the rows after block t
-                    const int k0 = 64 * (t - 1), kb = std::min(64, d.c - k0);
-                    for (int r0 = std::min(64 * (t + 1), d.c); r0 < d.n; r0 += 64)
-                        chunks.push_back(SolveTask{s, k0, kb, r0, 0, 0, 0, 0});
-                }
-            }
-            // the step's chunk tasks after its block tasks, in the same
-            // launch, or in a launch of their own when there are many
-            const bool apart = (int)chunks.size() >= kChunkLaunch;
-            if (!apart) h->fstep.insert(h->fstep.end(), chunks.begin(), chunks.end());
-            push(h->fwd_seq, kFS, f0, (int64_t)h->fstep.size(), t);
-            push(h->fwd_seq, kFX, x0, (int64_t)h->xstep.size(), t);
-            if (apart) {
-                const int64_t c0 = (int64_t)h->fstep.size();
-                h->fstep.insert(h->fstep.end(), chunks.begin(), chunks.end());
-                push(h->fwd_seq, kFC, c0, (int64_t)h->fstep.size(), t);
-            }
-        }
-    }
-    // chunks of the partial sums of block j of front s: rows [min(64 (j + 2), c), n)
-    auto chunk_rows = [&](const NodeDev& d, int j) {
-        const int start = std::min(64 * (j + 2), d.c);
-        return std::make_pair(start, (d.n - start + 255) / 256);
-    };
-    // superblock fronts: the partial sums of superblock w, rows
-    // [min(256 (w + 2), c), n), for each of its (at most four) 64-column
-    // blocks
-    auto super_chunk_rows = [&](const NodeDev& d, int w) {
-        const int start = std::min(kSuper * (w + 2), d.c);
-        return std::make_pair(start, (d.n - start + 255) / 256);
-    };
-    auto super_blocks = [&](const NodeDev& d, int w) { return std::min(4, (d.c - kSuper * w + 63) / 64); };
-    auto blocks = [&](const NodeDev& d) { return super(d) ? (d.c + kSuper - 1) / kSuper : (d.c + 63) / 64; };
-    // slots written by the chunk tasks of backward step t of front d
-    auto step_slots = [&](const NodeDev& d, int t) -> int64_t {
-        if (t < 1 || t - 1 >= blocks(d)) return 0;
-        if (super(d)) return (int64_t)super_blocks(d, t - 1) * super_chunk_rows(d, t - 1).second;
-        return std::max(0, chunk_rows(d, t - 1).second);
-    };
-    int64_t bank = 1;  // slots per bank: the most chunks any launch has
-    for (int L = 0; L < h->num_levels; ++L) {
-        const int b0 = h->level_ptr[L], b1 = h->level_ptr[L + 1];
-        for (int t = fsteps_of(L); t >= 1; --t) {
-            int64_t cnt = 0;
-            for (int k = b0; k < b1; ++k) cnt += step_slots(h->nodes[h->level_nodes[k]], t);
-            bank = std::max(bank, cnt);
-        }
-    }
-    std::vector<int> qfirst(h->nodes.size(), 0), qcount(h->nodes.size(), 0);
-    std::vector<SolveTask> bchunks;  // a backward step's chunk tasks
-    for (int L = h->num_levels - 1; L >= 0; --L) {
-        const int b0 = h->level_ptr[L], b1 = h->level_ptr[L + 1];
-        {
-            int64_t f = (int64_t)h->bg.size();
-            for (int k = b0; k < b1; ++k) {
-                const int s = h->level_nodes[k];
-                if (h->nodes[s].parent < 0) continue;
-                for (int r0 = 0; r0 < h->nodes[s].w; r0 += 256) h->bg.push_back(make_int2(s, r0));
-            }
-            push(h->bwd_seq, kBG, f, (int64_t)h->bg.size());
-        }
-        for (int t = fsteps_of(L); t >= 0; --t) {
-            int64_t f0 = (int64_t)h->bstep.size(), x0 = (int64_t)h->xbstep.size();
-            bchunks.clear();
-            int idx = 0;
-            // few chunks (latency-bound steps): four 16-column tasks per
-            // chunk; many: one task per chunk
-            int64_t nch = 0;
-            for (int k = b0; k < b1; ++k) nch += step_slots(h->nodes[h->level_nodes[k]], t);
-            const bool split = nch <= kSplitChunks;
-            for (int k = b0; k < b1; ++k) {
-                const int s = h->level_nodes[k];
-                const NodeDev& d = h->nodes[s];
-                const int T = blocks(d);
-                if (super(d)) {
-                    const int64_t xo = xoff[s] + (int64_t)t * per_super;
-                    if (t <= T - 1) {
-                        // superblock t from the partial sums of the previous
-                        // launch and x of superblock t + 1
-                        const int sb = std::min(kSuper, d.c - kSuper * t);
-                        const int pb = t + 1 <= T - 1 ? std::min(kSuper, d.c - kSuper * (t + 1)) : 0;
-                        for (int r0 = 0; r0 < sb; r0 += 16)
-                            h->xbstep.push_back(SuperTask{s, t, r0, sb, pb, 2, qfirst[s], qcount[s], xo});
-                    }
-                    if (t >= 1 && t - 1 <= T - 1) {
-                        // partial sums of superblock t - 1 over the rows after superblock t
-                        const int w = t - 1;
-                        const auto rc = super_chunk_rows(d, w);
-                        qfirst[s] = (int)((w % 2) * bank + idx);
-                        qcount[s] = rc.second;
-                        for (int j = 0; j < super_blocks(d, w); ++j) {
-                            const int k0 = kSuper * w + 64 * j, kb = std::min(64, d.c - k0);
-                            for (int q = 0; q < rc.second; ++q, ++idx)
-                                for (int cq = 0; cq < (split ? 4 : 1); ++cq)
-                                    bchunks.push_back(SolveTask{s, k0, kb, rc.first + 256 * q,
-                                                                 (int)((w % 2) * bank + idx), 0, split ? cq : -1, 0});
-                        }
-                    }
-                    continue;
-                }
-                if (t <= T - 1) {
-                    const int k0 = 64 * t, kb = std::min(64, d.c - k0);
-                    const int kn = t + 1 <= T - 1 ? std::min(64, d.c - k0 - 64) : 0;
-                    h->bstep.push_back(SolveTask{s, k0, kb, -1, qfirst[s], qcount[s], 0, kn});
-                }
-                if (t >= 1 && t - 1 <= T - 1) {
-                    const int j = t - 1, k0 = 64 * j, kb = std::min(64, d.c - k0);
-                    const auto rc = chunk_rows(d, j);
-                    qfirst[s] = (int)((j % 2) * bank + idx);
-                    qcount[s] = rc.second;
-                    for (int q = 0; q < rc.second; ++q, ++idx)
-                        for (int cq = 0; cq < (split ? 4 : 1); ++cq)
-                            bchunks.push_back(
-                                SolveTask{s, k0, kb, rc.first + 256 * q, (int)((j % 2) * bank + idx), 0, split ? cq : -1, 0});
-                }
-            }
-            const bool apart = (int)bchunks.size() >= kChunkLaunch;
-            if (!apart) h->bstep.insert(h->bstep.end(), bchunks.begin(), bchunks.end());
-            push(h->bwd_seq, kBS, f0, (int64_t)h->bstep.size(), t);
-            push(h->bwd_seq, kBX, x0, (int64_t)h->xbstep.size(), t);
-            if (apart) {
-                const int64_t c0 = (int64_t)h->bstep.size();
-                h->bstep.insert(h->bstep.end(), bchunks.begin(), bchunks.end());
-                push(h->bwd_seq, kBC, c0, (int64_t)h->bstep.size(), t);
-            }
-        }
-    }
-    h->part_slots = 2 * bank;
-}
-
 void build_plan(mfd_handle* h)
 {
     const Structure& S = h->S;
     const int m = S.num_node;
     const int period_set = h->upd_period;
     h->nodes.assign(m, NodeDev{});
-    int64_t off = 0, zoff = 0, inv_blocks = 0;
+    int64_t off = 0, inv_blocks = 0;
     for (int s = 0; s < m; ++s) {
         NodeDev& d = h->nodes[s];
         d.n = S.c[s] + S.w[s];
@@ -686,11 +389,9 @@ void build_plan(mfd_handle* h)
         d.w = S.w[s];
         d.front = off;
         d.lidx = S.li_ptr[s];
-        d.z = zoff;
         d.parent = S.parent[s] - 1;
         d.first = S.first[s] - 1;
         off += align_up((int64_t)d.n * d.n, 32);
-        zoff += d.n + d.c;
         d.inv = inv_blocks;  // rebased below
         inv_blocks += (d.c + kPanel - 1) / kPanel;
     }
@@ -698,7 +399,6 @@ void build_plan(mfd_handle* h)
     for (int s = 0; s < m; ++s) h->nodes[s].inv = off + h->nodes[s].inv * kPanel * kPanel;
     off += inv_blocks * kPanel * kPanel;
     h->pool_elems = off;
-    h->z_per_rhs = zoff;
     // subtrees factored on the host (CPU+GPU hybrid): their fronts get no
     // zeroing, assembly or factorization launch; a host subtree root adds
     // into its parent by the extend-add launch, like a small child
@@ -1061,7 +761,7 @@ void build_plan(mfd_handle* h)
             if (S.parent[r] > 0) jl = std::min(jl, lev[S.parent[r] - 1]);
         h->host_join = jl < h->num_levels ? h->level_launch[jl] : (int)h->fseq.size();
     }
-    build_solve_plan(h);
+    h->solve_rc = build_solve_plan(S, h->nodes, h->level_ptr, h->level_nodes, h->super_min, h->sp);
 }
 
 // Full symmetric CSR (both triangles) of the postordered matrix for the
@@ -1111,6 +811,7 @@ int setup_device(mfd_handle* h)
     const Structure& S = h->S;
     build_plan(h);
     MFD_TRY(h->host_rc);
+    MFD_TRY(h->solve_rc);
     if (h->hplan.stage_elems > 0)
         HIP_TRY(hipHostMalloc((void**)&h->hstage, h->hplan.stage_elems * sizeof(double), hipHostMallocDefault));
     MFD_TRY(upload(h, &h->d_nodes, h->nodes));
@@ -1134,15 +835,13 @@ int setup_device(mfd_handle* h)
     MFD_TRY(upload(h, &h->d_level_nodes, h->level_nodes));
     MFD_TRY(upload(h, &h->d_child_ptr, h->child_ptr));
     MFD_TRY(upload(h, &h->d_child_list, h->child_list));
-    MFD_TRY(upload(h, &h->d_fstep, h->fstep));
-    MFD_TRY(upload(h, &h->d_bstep, h->bstep));
-    MFD_TRY(upload(h, &h->d_xstep, h->xstep));
-    MFD_TRY(upload(h, &h->d_xbstep, h->xbstep));
-    MFD_TRY(upload(h, &h->d_xinv, h->xinv));
-    if (h->sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv64, h->sinv_elems));
-    MFD_TRY(upload(h, &h->d_fi, h->fi));
-    MFD_TRY(upload(h, &h->d_fa, h->fa));
-    MFD_TRY(upload(h, &h->d_bg, h->bg));
+    MFD_TRY(upload(h, &h->d_stasks, h->sp.tasks));
+    MFD_TRY(upload(h, &h->d_sbundles, h->sp.bundles));
+    MFD_TRY(upload(h, &h->d_grow, h->sp.grow));
+    MFD_TRY(upload(h, &h->d_gptr, h->sp.gptr));
+    MFD_TRY(upload(h, &h->d_gsrc, h->sp.gsrc));
+    MFD_TRY(upload(h, &h->d_xinv, h->sp.xinv));
+    if (h->sp.sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv64, h->sp.sinv_elems));
     // assembly map: A entry -> front position (coefficient_setter_m.f90:26-41),
     // the entries in the fill groups' order
     const int64_t nnz = (int64_t)S.snidx.size();
@@ -1199,18 +898,25 @@ int setup_device(mfd_handle* h)
     return MFD_OK;
 }
 
+// Control words and counters of a solve of nrhs right-hand sides.
+int64_t solve_words(const mfd_handle* h, int nrhs)
+{
+    return kSolveCtl + (int64_t)h->sp.nflags * ((nrhs + kRhsGroup - 1) / kRhsGroup);
+}
+
 int ensure_rhs(mfd_handle* h, int nrhs)
 {
     if (nrhs <= h->nrhs_cap) return MFD_OK;
     const int64_t n = h->S.n;
-    MFD_TRY(dalloc(h, &h->d_z, h->z_per_rhs * nrhs));
+    MFD_TRY(dalloc(h, &h->d_z, h->sp.plane * nrhs));
+    MFD_TRY(dalloc(h, &h->d_y, n * nrhs));
+    MFD_TRY(dalloc(h, &h->d_sflags, solve_words(h, nrhs)));
     MFD_TRY(dalloc(h, &h->d_bin, n * nrhs));
     MFD_TRY(dalloc(h, &h->d_bp, n * nrhs));
     MFD_TRY(dalloc(h, &h->d_xp, n * nrhs));
     MFD_TRY(dalloc(h, &h->d_r, n * nrhs));
     MFD_TRY(dalloc(h, &h->d_d, n * nrhs));
     MFD_TRY(dalloc(h, &h->d_norms, 4 * nrhs + 1 + 2 * kSumParts * nrhs));
-    MFD_TRY(dalloc(h, &h->d_part, h->part_slots * 64 * nrhs));
     drop_solve_graphs(h);  // captured solves refer to the old buffers
     h->nrhs_cap = nrhs;
     return MFD_OK;
@@ -1357,8 +1063,8 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
     if (hybrid) ok(host_join(h, st));
     // superblock inverses of the solves, after every front is final
     for (int dist = 0; dist <= 4; ++dist)
-        launch_superinv<T>(pool, sinv_of<T>(h), h->d_nodes, h->d_xinv + h->xinv_ptr[dist],
-                           h->xinv_ptr[dist + 1] - h->xinv_ptr[dist], dist == 4, st);
+        launch_superinv<T>(pool, sinv_of<T>(h), h->d_nodes, h->d_xinv + h->sp.xinv_ptr[dist],
+                           h->sp.xinv_ptr[dist + 1] - h->sp.xinv_ptr[dist], dist == 4, st);
     return err;
 }
 
@@ -1451,7 +1157,7 @@ int factorize_common(mfd_handle* h, int precision)
     int rc = MFD_OK;
     if (precision == MFD_FP16_IR || precision == MFD_BF16_IR) {
         if (!h->d_pool32) MFD_TRY(dalloc(h, &h->d_pool32, h->pool_elems));
-        if (!h->d_sinv32 && h->sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv32, h->sinv_elems));
+        if (!h->d_sinv32 && h->sp.sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv32, h->sp.sinv_elems));
         h->lowp = precision == MFD_FP16_IR ? 1 : 2;
         rc = run_factor<float>(h);
         h->lowp = 0;
@@ -1460,7 +1166,7 @@ int factorize_common(mfd_handle* h, int precision)
     }
     if (precision == MFD_FP32_IR) {
         if (!h->d_pool32) MFD_TRY(dalloc(h, &h->d_pool32, h->pool_elems));
-        if (!h->d_sinv32 && h->sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv32, h->sinv_elems));
+        if (!h->d_sinv32 && h->sp.sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv32, h->sp.sinv_elems));
         rc = run_factor<float>(h);
         // a pivot not positive in FP32: the FP64 refactorization the
         // refinement falls back to when it stalls; only an FP64 failure
@@ -1478,78 +1184,65 @@ int factorize_common(mfd_handle* h, int precision)
 }
 
 // --------------------------------------------------------------- solve
+// Both sweeps, one launch (when profiling, one per sweep).
 template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double* xp, int nrhs)
 {
     hipStream_t st = h->stream;
-    const T* pool = pool_of<T>(h);
-    const int n = h->S.n;
-    const bool profile = (h->flags & MFD_FLAG_PROFILE) != 0;
+    SolveArgs<T> a{};
+    a.pool = pool_of<T>(h);
+    a.sinv = sinv_of<T>(h);
+    a.z = h->d_z;
+    a.b = bp;
+    a.y = h->d_y;
+    a.x = xp;
+    a.grow = h->d_grow;
+    a.gptr = h->d_gptr;
+    a.gsrc = h->d_gsrc;
+    a.tasks = h->d_stasks;
+    a.bundles = h->d_sbundles;
+    a.flags = h->d_sflags;
+    a.err = h->solve_err;
+    a.zs = h->sp.plane;
+    a.n = h->S.n;
+    a.nrhs = nrhs;
+    a.ngroups = (nrhs + kRhsGroup - 1) / kRhsGroup;
+    a.nflags = h->sp.nflags;
+    a.nbundles = (int)h->sp.bundles.size();
+    a.ticket = kSolveTicket;
+    launch_solve_reset(h->d_sflags, solve_words(h, nrhs), st);
+    if ((h->flags & MFD_FLAG_PROFILE) == 0) {
+        launch_solve<T>(a, st);
+        return;
+    }
     hipEvent_t pe[3] = {};
-    if (profile)
-        for (auto& e : pe) (void)hipEventCreate(&e);
-    if (profile) (void)hipEventRecord(pe[0], st);
-    // a step's kFS and kFX launches (kBS and kBX) touch different fronts (the
-    // kBX tasks read the partial-sum bank the kBS tasks do not write): one
-    // launch of both
-    auto paired = [](const std::vector<Launch>& seq, size_t i, int a, int b) {
-        return seq[i].kind == a && i + 1 < seq.size() && seq[i + 1].kind == b && seq[i].step == seq[i + 1].step;
-    };
-    int nfwd = 0, nbwd = 0;  // launches issued
-    for (size_t i = 0; i < h->fwd_seq.size(); ++i, ++nfwd) {
-        const Launch& l = h->fwd_seq[i];
-        if (paired(h->fwd_seq, i, kFS, kFX)) {
-            const Launch& x = h->fwd_seq[++i];
-            launch_fwd_pair<T>(pool, sinv_of<T>(h), h->d_z, nrhs, h->d_nodes, h->d_xstep + x.first, x.count,
-                               h->d_fstep + l.first, l.count, st);
-            continue;
-        }
-        switch (l.kind) {
-        case kFI: launch_fwd_init(h->d_z, bp, n, nrhs, h->d_nodes, h->d_fi + l.first, l.count, st); break;
-        case kFA: launch_fwd_add(h->d_z, nrhs, h->d_nodes, h->d_lidx, h->d_fa + l.first, l.count, st); break;
-        case kFS: launch_fwd_step<T>(pool, h->d_z, nrhs, h->d_nodes, h->d_fstep + l.first, l.count, st); break;
-        case kFC: launch_fwd_chunk<T>(pool, h->d_z, nrhs, h->d_nodes, h->d_fstep + l.first, l.count, st); break;
-        case kFX:
-            launch_fwd_super<T>(pool, sinv_of<T>(h), h->d_z, nrhs, h->d_nodes, h->d_xstep + l.first, l.count, st);
-            break;
-        default: break;
-        }
-    }
-    if (profile) (void)hipEventRecord(pe[1], st);
-    for (size_t i = 0; i < h->bwd_seq.size(); ++i, ++nbwd) {
-        const Launch& l = h->bwd_seq[i];
-        if (paired(h->bwd_seq, i, kBS, kBX)) {
-            const Launch& x = h->bwd_seq[++i];
-            launch_bwd_pair<T>(pool, sinv_of<T>(h), h->d_z, h->d_part, xp, n, nrhs, h->d_nodes, h->d_xbstep + x.first,
-                               x.count, h->d_bstep + l.first, l.count, st);
-            continue;
-        }
-        switch (l.kind) {
-        case kBG: launch_bwd_gather(h->d_z, nrhs, h->d_nodes, h->d_lidx, h->d_bg + l.first, l.count, st); break;
-        case kBS:
-            launch_bwd_step<T>(pool, h->d_z, h->d_part, xp, n, nrhs, h->d_nodes, h->d_bstep + l.first, l.count, st);
-            break;
-        case kBC:
-            launch_bwd_chunk<T>(pool, h->d_z, h->d_part, nrhs, h->d_nodes, h->d_bstep + l.first, l.count, st);
-            break;
-        case kBX:
-            launch_bwd_super<T>(pool, sinv_of<T>(h), h->d_z, h->d_part, xp, n, nrhs, h->d_nodes, h->d_xbstep + l.first,
-                                l.count, st);
-            break;
-        default: break;
-        }
-    }
-    if (profile) {
-        (void)hipEventRecord(pe[2], st);
-        (void)hipEventSynchronize(pe[2]);
-        float a = 0, b = 0;
-        (void)hipEventElapsedTime(&a, pe[0], pe[1]);
-        (void)hipEventElapsedTime(&b, pe[1], pe[2]);
-        h->ktime[MFD_K_SOLVE_FWD] += a;
-        h->kcount[MFD_K_SOLVE_FWD] += nfwd;
-        h->ktime[MFD_K_SOLVE_BWD] += b;
-        h->kcount[MFD_K_SOLVE_BWD] += nbwd;
-        for (auto e : pe) (void)hipEventDestroy(e);
-    }
+    for (auto& e : pe) (void)hipEventCreate(&e);
+    (void)hipEventRecord(pe[0], st);
+    a.nbundles = h->sp.fwd_bundles;
+    launch_solve<T>(a, st);
+    (void)hipEventRecord(pe[1], st);
+    a.bundle0 = h->sp.fwd_bundles;
+    a.nbundles = (int)h->sp.bundles.size() - h->sp.fwd_bundles;
+    a.ticket = kSolveTicketBwd;
+    launch_solve<T>(a, st);
+    (void)hipEventRecord(pe[2], st);
+    (void)hipEventSynchronize(pe[2]);
+    float f = 0, b = 0;
+    (void)hipEventElapsedTime(&f, pe[0], pe[1]);
+    (void)hipEventElapsedTime(&b, pe[1], pe[2]);
+    h->ktime[MFD_K_SOLVE_FWD] += f;
+    h->kcount[MFD_K_SOLVE_FWD] += 1;
+    h->ktime[MFD_K_SOLVE_BWD] += b;
+    h->kcount[MFD_K_SOLVE_BWD] += 1;
+    for (auto e : pe) (void)hipEventDestroy(e);
+}
+
+// After a synchronization: whether a solve's wait reached its bound (the
+// task list is broken; never with a plan that check_solve_plan passes).
+int solve_status(mfd_handle* h)
+{
+    if (*h->solve_err == 0) return MFD_OK;
+    *h->solve_err = 0;
+    return MFD_ERR_INTERNAL;
 }
 
 // One forward + backward sweep, replayed from a captured graph when graphs
@@ -1605,6 +1298,7 @@ int backward_error(mfd_handle* h, const double* bp, const double* xp, double* r,
     std::vector<unsigned long long> v(nm + 2 * parts * nrhs);
     HIP_TRY(hipMemcpyAsync(v.data(), h->d_norms, v.size() * 8, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    MFD_TRY(solve_status(h));
     auto val = [&](int i) {
         double x;
         memcpy(&x, &v[i], 8);
@@ -1748,6 +1442,7 @@ int solve_host(mfd_handle* h, double* b, int nrhs, int ldb, bool permuted, bool 
     HIP_TRY(hipMemcpy2DAsync(b, (size_t)ldb * 8, h->d_bin, (size_t)n * 8, (size_t)n * 8, nrhs, kout, st));
     HIP_TRY(hipStreamSynchronize(st));
     HIP_TRY(hipGetLastError());
+    MFD_TRY(solve_status(h));
     float ms = 0;
     HIP_TRY(hipEventElapsedTime(&ms, h->ev[2], h->ev[3]));
     h->st.solve_ms = ms;
@@ -1791,13 +1486,13 @@ double* scratch_on_current_device()
 }
 
 // Bytes of scratch a solve of nrhs right-hand sides takes (each buffer
-// 256-byte aligned): Z/Y slices, partial sums, permuted b and x and, for
-// the refined forms, residual, correction and norm slots.
+// 256-byte aligned): the planes passed between tasks, counters, y, permuted b
+// and x and, for the refined forms, residual, correction and norm slots.
 int64_t noalloc_bytes(const mfd_handle* h, int nrhs)
 {
     auto al = [](int64_t b) { return (b + 255) & ~int64_t(255); };
     const int64_t n = h->S.n;
-    int64_t b = al(h->z_per_rhs * nrhs * 8) + al(h->part_slots * 64 * nrhs * 8) + 2 * al(n * nrhs * 8);
+    int64_t b = al(h->sp.plane * nrhs * 8) + al(solve_words(h, nrhs) * 4) + 3 * al(n * nrhs * 8);
     if (h->precision != MFD_FP64) b += 2 * al(n * nrhs * 8) + al((4 * nrhs + 1 + 2 * kSumParts * nrhs) * 8);
     return b;
 }
@@ -1806,11 +1501,13 @@ int64_t noalloc_bytes(const mfd_handle* h, int nrhs)
 // point into the scratch array and no_alloc is set; both restored after.
 struct NoAllocScope {
     mfd_handle* h;
-    double *z, *part, *bp, *xp, *r, *d;
+    double *z, *y, *bp, *xp, *r, *d;
+    int* sflags;
     unsigned long long* norms;
     NoAllocScope(mfd_handle* h_, int nrhs) : h(h_)
     {
-        z = h->d_z, part = h->d_part, bp = h->d_bp, xp = h->d_xp, r = h->d_r, d = h->d_d, norms = h->d_norms;
+        z = h->d_z, y = h->d_y, bp = h->d_bp, xp = h->d_xp, r = h->d_r, d = h->d_d, norms = h->d_norms;
+        sflags = h->d_sflags;
         auto al = [](int64_t b) { return (b + 255) & ~int64_t(255); };
         const int64_t n = h->S.n;
         char* p = reinterpret_cast<char*>(h->scratch);
@@ -1819,8 +1516,9 @@ struct NoAllocScope {
             p += al(bytes);
             return q;
         };
-        h->d_z = reinterpret_cast<double*>(take(h->z_per_rhs * nrhs * 8));
-        h->d_part = reinterpret_cast<double*>(take(h->part_slots * 64 * nrhs * 8));
+        h->d_z = reinterpret_cast<double*>(take(h->sp.plane * nrhs * 8));
+        h->d_sflags = reinterpret_cast<int*>(take(solve_words(h, nrhs) * 4));
+        h->d_y = reinterpret_cast<double*>(take(n * nrhs * 8));
         h->d_bp = reinterpret_cast<double*>(take(n * nrhs * 8));
         h->d_xp = reinterpret_cast<double*>(take(n * nrhs * 8));
         if (h->precision != MFD_FP64) {
@@ -1832,7 +1530,7 @@ struct NoAllocScope {
     }
     ~NoAllocScope()
     {
-        h->d_z = z, h->d_part = part, h->d_bp = bp, h->d_xp = xp, h->d_r = r, h->d_d = d, h->d_norms = norms;
+        h->d_z = z, h->d_y = y, h->d_sflags = sflags, h->d_bp = bp, h->d_xp = xp, h->d_r = r, h->d_d = d, h->d_norms = norms;
         h->no_alloc = false;
     }
 };
@@ -2209,6 +1907,10 @@ int mfd_create(mfd_handle** out, int nb, int flags)
             h->device_ok = true;
             h->scratch = scratch_on_current_device();  // set-up of mfd_solve_device_noalloc
             for (auto& e : h->ev) (void)hipEventCreate(&e);
+            if (hipHostMalloc((void**)&h->solve_err, sizeof(int), hipHostMallocDefault) == hipSuccess)
+                *h->solve_err = 0;
+            else
+                h->device_ok = false;
             if (hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking) != hipSuccess) h->side = nullptr;
             if (hipStreamCreateWithFlags(&h->fillst, hipStreamNonBlocking) != hipSuccess) h->fillst = nullptr;
             (void)hipEventCreateWithFlags(&h->fork, hipEventDisableTiming);
@@ -2226,6 +1928,7 @@ void mfd_destroy(mfd_handle* h)
     if (h->device_ok) {
         (void)hipStreamSynchronize(h->stream);
         free_device(h);
+        (void)hipHostFree(h->solve_err);
         for (auto& b : h->spare) (void)hipFree(b.first);
         h->spare.clear();
         h->device_bytes = 0;
@@ -2346,6 +2049,7 @@ int mfd_check_schedule(mfd_handle* h, int variant, int64_t* conflicts, char* rep
     if (!h->device_ok) build_plan(h);  // a handle without a GPU keeps no schedule
     std::string rep;
     *conflicts = check_schedule(h, variant, rep);
+    if (variant == 0) *conflicts += h->solve_rc == MFD_OK ? check_solve_plan(h->sp, rep) : 1;
     if (report && report_len > 0) {
         const size_t n = std::min(rep.size(), (size_t)report_len - 1);
         memcpy(report, rep.data(), n);
@@ -2559,6 +2263,7 @@ int mfd_solve_device_noalloc(mfd_handle* h, double* d_b, int nrhs, int ldb)
         HIP_TRY(hipEventRecord(h->ev[3], st));
         HIP_TRY(hipStreamSynchronize(st));
         HIP_TRY(hipGetLastError());
+        if (rc == MFD_OK) rc = solve_status(h);
     }
     if (rc != MFD_OK) return rc;
     float ms = 0;
@@ -2681,7 +2386,7 @@ int mfd_get_stats(mfd_handle* h, mfd_stats* st)
     h->st.device_bytes = h->device_bytes;
     h->st.num_levels = h->num_levels;
     h->st.num_launches_factor = (int)h->fseq.size() + 3;
-    h->st.num_launches_solve = (int)(h->fwd_seq.size() + h->bwd_seq.size()) + 2;
+    h->st.num_launches_solve = 4;  // permutation, counters, both sweeps, permutation
     *st = h->st;
     return MFD_OK;
 }

@@ -1,0 +1,789 @@
+// The supernodal triangular solves as one dependency-driven launch, written
+// for gfx950 (CDNA4, wave64).
+//
+// Replaces (paths relative to the reference root, src/main/):
+//   seq_forward   (scatter_add, TRSV, GEMV)  seq_solve/seq_forward_m.f90:14-81
+//   seq_backward  (gather, GEMV, TRSV)       seq_solve/seq_backward_m.f90:14-131
+//
+// A sweep is a chain of a few hundred dependent, tiny products: what bounds
+// it is the time from one product's result to the next one's start, not the
+// 2 nnz(L) entries it reads.  One launch per step of the chain cost 8 to 14
+// us a step (the launch itself 1.8, then three dependent reads -- task, front,
+// operands -- before the first multiply).  Here every task of both sweeps is
+// a workgroup's turn in one launch: workgroups take tickets in task order,
+// load the factor entries of their task into registers, wait on a counter in
+// device memory for the vectors they need, and raise a counter when their
+// own result is out; a hop from one workgroup to the next measured 1.4 us
+// with one producer and 3 us with sixteen.
+//
+// No deadlock: a task waits only for tasks earlier in the order
+// (mfd_check_schedule proves it for a built schedule), tickets are handed
+// out in that order by an atomic counter, and a workgroup that holds a
+// ticket is running; so the earliest unfinished task is always running and
+// never waits, whatever the number of resident workgroups and whatever else
+// the GPU runs.  Each wait is bounded all the same (kSpinLimit): a workgroup
+// that reaches the bound raises the stop word, every other wait then ends,
+// and the host reports an internal error.
+//
+// Values passed between tasks (y, x, the update rows Z, partial sums) are
+// written and read by relaxed agent-scope accesses, which meet in memory
+// common to the eight XCDs; a workgroup waits for its stores' completion
+// before it raises its counter.  The factor is read through the caches.
+//
+// Every product runs on FP64 MFMA (FP32 factors are widened as they are
+// read) with 16 right-hand sides as the second operand's columns; all sums
+// have a fixed order, so results do not depend on timing.
+#include <hip/hip_runtime.h>
+
+#include "mfd_kernels.h"
+
+namespace mfd {
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kRhs = kRhsGroup;      // right-hand sides per group: the columns of an MFMA operand
+constexpr int kSpinLimit = 1 << 23;  // polls of one wait (about 6 s)
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// D(16x16) += A(16x4) B(4x16): lane l supplies A[l%16][l/16] and
+// B[l/16][l%16]; element v of lane l is D[l/16 + 4v][l%16].
+__device__ __forceinline__ d4 mma(double a, double b, d4 c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ double ld_agent(const double* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int ld_agent(const int* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(double* p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// *p by scalar loads (uniform address, memory that no launch writes while
+// this one runs).
+template <typename S> __device__ __forceinline__ S ld_scalar(const S* p)
+{
+    typedef const __attribute__((address_space(4))) int* words;
+    static_assert(sizeof(S) % 4 == 0, "copied in words");
+    S v;
+    words w = (words)(const void*)p;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(S) / 4; ++i) reinterpret_cast<int*>(&v)[i] = w[i];
+    return v;
+}
+
+// p[i] for a uniform base and a 32-bit index (one VGPR per address).
+template <typename T> __device__ __forceinline__ T ld_off(const T* p, unsigned i)
+{
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (size_t)(i * (unsigned)sizeof(T)));
+}
+
+// The vector operand of a task's products, rows of 16 right-hand sides, and
+// the four waves' partial products (which take the same place once the
+// operand has been read): four workgroups per CU.
+union SolveLds {
+    double v[kSuper][kRhs + 1];
+    double red[4][16][kRhs + 1];
+};
+
+// What a task knows of its launch, its right-hand-side group and its place
+// in the workgroup.
+template <typename T> struct Ctx {
+    const SolveArgs<T>& A;
+    SolveLds& S;
+    int* flags;  // the group's counters
+    int rb, nr;  // its right-hand sides rb .. rb + nr - 1
+    int tid, lane, wv, li, g;
+};
+
+// Waits until counter f reaches target (all threads; ends with a barrier,
+// after which the values the counter stands for can be read).
+template <typename T> __device__ __forceinline__ void wait_for(const Ctx<T>& C, int f, int target)
+{
+    if (f >= 0 && C.tid == 0) {
+        const int* p = C.flags + f;
+        int* stop = C.A.flags + kSolveStop;
+        for (int spins = 0; ld_agent(p) < target;) {
+            __builtin_amdgcn_s_sleep(1);
+            if ((++spins & 255) == 0 && (ld_agent(stop) != 0 || spins >= kSpinLimit)) {
+                __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(C.A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                break;
+            }
+        }
+    }
+    __syncthreads();
+}
+// Raises counters f and f2 (negative: none) once every store of the
+// workgroup has completed (all threads; holds a barrier).
+template <typename T> __device__ __forceinline__ void signal(const Ctx<T>& C, int f, int f2 = -1)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (C.tid == 0) {
+        if (f >= 0) __hip_atomic_fetch_add(C.flags + f, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (f2 >= 0) __hip_atomic_fetch_add(C.flags + f2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// Counters of a front (SolveTask::flag, fstr): y_u and x_u of superblock u.
+__device__ __forceinline__ int y_flag(const SolveTask& t, int u) { return t.flag + t.fstr * (1 + t.nsup + u); }
+__device__ __forceinline__ int x_flag(const SolveTask& t, int u) { return t.flag + t.fstr * (1 + 4 * t.nsup + u); }
+// Tasks that form superblock u's y (or x).
+__device__ __forceinline__ int yx_target(const SolveTask& t, int u)
+{
+    return t.super ? (min(kSuper, t.c - kSuper * u) + 15) / 16 : 1;
+}
+
+// S.v[k][r] = src[k + (rb + r) ld] for k < cnt, zero for the other k < 256
+// (thread k's row; all loads before the stores of four columns).
+template <typename T>
+__device__ __forceinline__ void stage_rows(const Ctx<T>& C, const double* src, int64_t ld, int cnt)
+{
+    const int k = C.tid;
+    for (int r = 0; r < C.nr; r += 4) {
+        double q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            q[i] = (k < cnt && r + i < C.nr) ? ld_agent(src + k + (int64_t)(C.rb + r + i) * ld) : 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (r + i < C.nr) C.S.v[k][r + i] = q[i];
+    }
+}
+
+// The children's contributions to row i of a front: list entries gptr[goff +
+// i] .. of the children's update rows, in child order (goff < 0: a leaf).
+// The first two are looked up before the wait for the children.
+struct Gather {
+    int k0 = 0, k1 = 0, s0 = 0, s1 = 0;
+};
+template <typename T> __device__ __forceinline__ Gather gather_begin(const Ctx<T>& C, const SolveTask& t, int i)
+{
+    Gather q;
+    if (t.goff < 0) return q;
+    q.k0 = C.A.gptr[t.goff + i];
+    q.k1 = C.A.gptr[t.goff + i + 1];
+    if (q.k0 < q.k1) q.s0 = C.A.gsrc[q.k0];
+    if (q.k0 + 1 < q.k1) q.s1 = C.A.gsrc[q.k0 + 1];
+    return q;
+}
+// Four right-hand-side entries of a front, entry e that of row i[e], column
+// rhs[e] (live[e] false: zero): b on pivot rows, plus the children's
+// contributions (scatter_add, sparse_add_subroutines_m.f90:13-30).  All
+// loads are issued before the first sum.
+template <typename T>
+__device__ __forceinline__ void gather4(const Ctx<T>& C, const SolveTask& t, const Gather (&q)[4], const int (&i)[4],
+                                        const int (&rhs)[4], const bool (&live)[4], double (&z)[4])
+{
+    double bv[4], c0[4], c1[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bv[e] = (live[e] && i[e] < t.c) ? C.A.b[t.first + i[e] + (int64_t)rhs[e] * C.A.n] : 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const double* Z = C.A.z + (int64_t)rhs[e] * C.A.zs;
+        c0[e] = (live[e] && q[e].k0 < q[e].k1) ? ld_agent(Z + q[e].s0) : 0.0;
+        c1[e] = (live[e] && q[e].k0 + 1 < q[e].k1) ? ld_agent(Z + q[e].s1) : 0.0;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        z[e] = bv[e] + c0[e] + c1[e];
+        if (live[e])
+            for (int k = q[e].k0 + 2; k < q[e].k1; ++k)
+                z[e] += ld_agent(C.A.z + (int64_t)rhs[e] * C.A.zs + C.A.gsrc[k]);
+    }
+}
+
+// 64 entries of K for 16 rows of column-major M (uniform address): lane (row
+// `row`, column k0 + 4 j + g), j < 16 -- 16 consecutive rows of four columns
+// per load.  cmax: the last column read.
+template <typename T>
+__device__ __forceinline__ void load_cols(T (&a)[16], const T* M, int row, int ld, int k0, int g, int cmax)
+{
+#pragma unroll
+    for (int j = 0; j < 16; ++j) a[j] = ld_off(M, (unsigned)(row + min(k0 + 4 * j + g, cmax) * ld));
+}
+// acc += a S.v[k0 ..] in load_cols's order.
+template <typename T> __device__ __forceinline__ void mma_cols(d4& acc, const T (&a)[16], const Ctx<T>& C, int k0)
+{
+    const bool ok = C.li < C.nr;
+    const int r = ok ? C.li : 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const double b = C.S.v[k0 + 4 * j + C.g][r];
+        acc = mma((double)a[j], ok ? b : 0.0, acc);
+    }
+}
+
+// 64 entries of K for 16 columns of column-major M (the transposed
+// product): lane (column li) reads 16-byte pieces of its column, the four
+// lanes of a column consecutive ones: rows row_of(j, g).
+template <typename T> struct Piece;
+template <> struct Piece<double> {
+    typedef double vec __attribute__((ext_vector_type(2), aligned(8)));
+    static constexpr int V = 2;
+};
+template <> struct Piece<float> {
+    typedef float vec __attribute__((ext_vector_type(4), aligned(4)));
+    static constexpr int V = 4;
+};
+template <typename T> __device__ __forceinline__ int row_of(int j, int g)
+{
+    constexpr int V = Piece<T>::V;
+    return 4 * V * (j / V) + V * g + j % V;
+}
+// M: uniform address; col: the lane's offset from it at the product's first
+// row; rows past lim give 0 (a piece that crosses lim is read whole: it lies
+// inside the pool, whose stored inverses follow the fronts).
+template <typename T>
+__device__ __forceinline__ void load_rows(T (&a)[16], const T* M, int col, int r0, int g, int lim)
+{
+    constexpr int V = Piece<T>::V;
+    typedef typename Piece<T>::vec vec;
+#pragma unroll
+    for (int j = 0; j < 16; j += V) {
+        const int r = r0 + row_of<T>(j, g);
+        const unsigned at = (unsigned)(col + (r < lim ? r : 0));
+        const vec p = *reinterpret_cast<const vec*>(reinterpret_cast<const char*>(M) + (size_t)(at * (unsigned)sizeof(T)));
+#pragma unroll
+        for (int e = 0; e < V; ++e) a[j + e] = r + e < lim ? p[e] : T(0);
+    }
+}
+template <typename T> __device__ __forceinline__ void mma_rows(d4& acc, const T (&a)[16], const Ctx<T>& C, int k0)
+{
+    const bool ok = C.li < C.nr;
+    const int r = ok ? C.li : 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const double b = C.S.v[k0 + row_of<T>(j, C.g)][r];
+        acc = mma((double)a[j], ok ? b : 0.0, acc);
+    }
+}
+
+// The four waves' partial products added in wave order: thread (row tid /
+// 16, right-hand side tid % 16) returns its entry.
+template <typename T> __device__ __forceinline__ double reduce_waves(const Ctx<T>& C, d4 acc)
+{
+    __syncthreads();  // S.v has been read
+#pragma unroll
+    for (int v = 0; v < 4; ++v) C.S.red[C.wv][C.g + 4 * v][C.li] = acc[v];
+    __syncthreads();
+    const int row = C.tid >> 4, rhs = C.tid & 15;
+    return (C.S.red[0][row][rhs] + C.S.red[1][row][rhs]) + (C.S.red[2][row][rhs] + C.S.red[3][row][rhs]);
+}
+
+// ---------------------------------------------------------------- forward
+// 16 rows of a front (kFwdRows): z = their right-hand side - sum over
+// superblocks v < nv of L[rows, B_v] y_v as the y_v come out, each wave a
+// quarter of B_v's columns.
+template <typename T> __device__ __forceinline__ void fwd_rows(const Ctx<T>& C, const SolveTask& t)
+{
+    const T* F = C.A.pool + t.front;
+    const int nv = t.nslot, lrow = min(t.r0 + C.li, t.n - 1);
+    auto load = [&](T(&a)[16], int v) {
+        load_cols<T>(a, F + (int64_t)kSuper * v * t.n, lrow, t.n, 64 * C.wv, C.g, min(kSuper, t.c - kSuper * v) - 1);
+    };
+    T a[16], an[16];
+    if (nv > 0) load(a, 0);
+    const int row = C.tid >> 4, rhs = C.tid & 15, i = t.r0 + row;
+    const bool live = row < t.nr && rhs < C.nr;
+    const Gather q = gather_begin(C, t, live ? i : t.r0);
+    wait_for(C, t.w0, t.w0t);
+    double z = 0.0;
+    if (live) {
+        const double* Z = C.A.z + (int64_t)(C.rb + rhs) * C.A.zs;
+        const double bv = i < t.c ? C.A.b[t.first + i + (int64_t)(C.rb + rhs) * C.A.n] : 0.0;
+        const double c0 = q.k0 < q.k1 ? ld_agent(Z + q.s0) : 0.0;
+        const double c1 = q.k0 + 1 < q.k1 ? ld_agent(Z + q.s1) : 0.0;
+        z = bv + c0 + c1;
+        for (int k = q.k0 + 2; k < q.k1; ++k) z += ld_agent(Z + C.A.gsrc[k]);
+    }
+    d4 acc = {0, 0, 0, 0};
+    for (int v = 0; v < nv; ++v) {
+        wait_for(C, y_flag(t, v), yx_target(t, v));
+        stage_rows(C, C.A.y + t.first + kSuper * v, C.A.n, min(kSuper, t.c - kSuper * v));
+        __syncthreads();
+        if (v + 1 < nv) load(an, v + 1);
+        mma_cols(acc, a, C, 64 * C.wv);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = an[j];
+    }
+    const double s = reduce_waves(C, acc);
+    if (live) st_agent(C.A.z + (int64_t)(C.rb + rhs) * C.A.zs + t.z + i, z - s);
+    signal(C, t.sig);
+}
+
+// The lane's four entries of a wave's 16 x 16 result over rows r0 + rw ..,
+// nr of them from r0 on: rows, right-hand sides and gather lists.
+template <typename T>
+__device__ __forceinline__ void own_rows(const Ctx<T>& C, const SolveTask& t, int r0, int rw, int nr, Gather (&q)[4],
+                                         int (&at)[4], int (&rhs)[4], bool (&live)[4])
+{
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int i = rw + C.g + 4 * v;
+        live[v] = i < nr && C.li < C.nr;
+        at[v] = r0 + min(i, nr - 1);
+        rhs[v] = C.rb + (C.li < C.nr ? C.li : 0);
+        q[v] = gather_begin(C, t, at[v]);
+    }
+}
+
+// 64 rows of a front (kFwdRows64, where rows are many): each wave 16 of
+// them over all columns.
+template <typename T> __device__ __forceinline__ void fwd_rows64(const Ctx<T>& C, const SolveTask& t)
+{
+    const int rw = 16 * C.wv, nv = t.nslot, lrow = min(t.r0 + rw + C.li, t.n - 1);
+    const T* F = C.A.pool + t.front;
+    auto load = [&](T(&a)[16], int k0) {
+        load_cols<T>(a, F + (int64_t)k0 * t.n, lrow, t.n, 0, C.g, t.c - 1 - k0);
+    };
+    T a[16], an[16];
+    if (nv > 0) load(a, 0);
+    Gather q[4];
+    int at[4], rhs[4];
+    bool live[4];
+    own_rows(C, t, t.r0, rw, t.nr, q, at, rhs, live);
+    wait_for(C, t.w0, t.w0t);
+    double z[4];
+    gather4(C, t, q, at, rhs, live, z);
+    d4 acc = {0, 0, 0, 0};
+    for (int v = 0; v < nv; ++v) {
+        const int pb = min(kSuper, t.c - kSuper * v);
+        wait_for(C, y_flag(t, v), yx_target(t, v));
+        stage_rows(C, C.A.y + t.first + kSuper * v, C.A.n, pb);
+        __syncthreads();
+        for (int k0 = 0; k0 < pb; k0 += 64) {
+            const int kn = kSuper * v + k0 + 64;
+            if (kn < t.c) load(an, kn);
+            mma_cols(acc, a, C, k0);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) a[j] = an[j];
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int i = rw + C.g + 4 * v;
+        if (i < t.nr && C.li < C.nr)
+            st_agent(C.A.z + (int64_t)(C.rb + C.li) * C.A.zs + t.z + t.r0 + i, z[v] - acc[v]);
+    }
+    signal(C, t.sig);
+}
+
+// S.v = the right-hand side of superblock u's rows: gathered (u has no
+// earlier superblock to take off, or only the one the caller takes off) or
+// from Z, where kFwdRows tasks left it.
+template <typename T> __device__ __forceinline__ void stage_z(const Ctx<T>& C, const SolveTask& t, int sb, bool gather)
+{
+    const int k = C.tid, i = kSuper * t.u + k;
+    if (gather) {
+        const Gather q = gather_begin(C, t, k < sb ? i : kSuper * t.u);
+        const Gather qs[4] = {q, q, q, q};
+        const int at[4] = {i, i, i, i};
+        wait_for(C, t.w0, t.w0t);
+        for (int r = 0; r < C.nr; r += 4) {
+            const int rhs[4] = {C.rb + r, C.rb + r + 1, C.rb + r + 2, C.rb + r + 3};
+            const bool live[4] = {k < sb, k < sb && r + 1 < C.nr, k < sb && r + 2 < C.nr, k < sb && r + 3 < C.nr};
+            double z[4];
+            gather4(C, t, qs, at, rhs, live, z);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (r + e < C.nr) C.S.v[k][r + e] = z[e];
+        }
+    } else {
+        wait_for(C, t.w0, t.w0t);
+        stage_rows(C, C.A.z + t.z + kSuper * t.u, C.A.zs, sb);
+    }
+    __syncthreads();
+}
+
+// 16 rows of superblock u through its explicit inverse (kFwdTop): y_u =
+// X z_u - W y_{u-1}, z_u holding every superblock before u - 1.
+template <typename T> __device__ __forceinline__ void fwd_top(const Ctx<T>& C, const SolveTask& t)
+{
+    const T* X = C.A.sinv + t.aux + t.r0;
+    const int sb = min(kSuper, t.c - kSuper * t.u), k0 = 64 * C.wv;
+    T a[16], w[16];
+    load_cols<T>(a, X, C.li, kSuper, k0, C.g, kSuper - 1);
+    // (W of the first superblock is unused storage)
+    load_cols<T>(w, X + kSuper * kSuper, C.li, kSuper, k0, C.g, kSuper - 1);
+    stage_z(C, t, sb, t.u < 2);
+    d4 acc = {0, 0, 0, 0}, accw = {0, 0, 0, 0};
+    if (k0 <= t.r0) mma_cols(acc, a, C, k0);  // X is lower triangular
+    if (t.u > 0) {
+        wait_for(C, y_flag(t, t.u - 1), yx_target(t, t.u - 1));
+        stage_rows(C, C.A.y + t.first + kSuper * (t.u - 1), C.A.n, kSuper);
+        __syncthreads();
+        mma_cols(accw, w, C, k0);
+    }
+    const double y = reduce_waves(C, acc - accw);
+    const int row = C.tid >> 4, rhs = C.tid & 15;
+    if (t.r0 + row < sb && rhs < C.nr)
+        st_agent(C.A.y + t.first + kSuper * t.u + t.r0 + row + (int64_t)(C.rb + rhs) * C.A.n, y);
+    signal(C, y_flag(t, t.u));
+}
+
+// Superblock u by one workgroup (kFwdPiv), 64 columns at a time through the
+// stored inverses of the diagonal blocks: y_b = inv(L_bb) (z_b - sum_{a<b}
+// L_ba y_a).  nr > 0 (fronts of one superblock): then the front's nr update
+// rows as well, Z = right-hand side - L[rows, :] y.
+template <typename T> __device__ __forceinline__ void fwd_piv(const Ctx<T>& C, const SolveTask& t)
+{
+    const int sb = min(kSuper, t.c - kSuper * t.u), nb = (sb + 63) / 64, rw = 16 * C.wv, c0 = kSuper * t.u;
+    const T* F = C.A.pool + t.front + (int64_t)c0 * t.n;  // the superblock's columns
+    const bool ok = C.li < C.nr;
+    stage_z(C, t, sb, t.u == 0);
+    for (int b = 0; b < nb; ++b) {
+        T iv[16], a[16];
+        // inv[r + 64 q] = L^{-1}(q, r): the lane's row q, 16-byte pieces along r
+        load_rows<T>(iv, C.A.pool + t.aux + b * 4096, 64 * (rw + C.li), 0, C.g, 64);
+        if (b > 0) {
+            d4 acc = {0, 0, 0, 0};
+            const int lrow = min(c0 + 64 * b + rw + C.li, t.n - 1);
+            for (int j = 0; j < b; ++j) {
+                load_cols<T>(a, F, lrow, t.n, 64 * j, C.g, sb - 1);
+                mma_cols(acc, a, C, 64 * j);
+            }
+            if (ok) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) C.S.v[64 * b + rw + C.g + 4 * v][C.li] -= acc[v];
+            }
+            __syncthreads();
+        }
+        d4 y = {0, 0, 0, 0};
+        mma_rows(y, iv, C, 64 * b);
+        __syncthreads();
+        if (ok) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int k = 64 * b + rw + C.g + 4 * v;
+                C.S.v[k][C.li] = k < sb ? y[v] : 0.0;
+                if (k < sb) st_agent(C.A.y + t.first + c0 + k + (int64_t)(C.rb + C.li) * C.A.n, y[v]);
+            }
+        }
+        __syncthreads();
+    }
+    for (int r0 = 0; r0 < t.nr; r0 += 64) {
+        const int lrow = min(t.c + r0 + rw + C.li, t.n - 1);
+        T a[16];
+        load_cols<T>(a, F, lrow, t.n, 0, C.g, sb - 1);
+        Gather q[4];
+        int at[4], rhs[4];
+        bool live[4];
+        own_rows(C, t, t.c + r0, rw, t.nr - r0, q, at, rhs, live);
+        double z[4];
+        gather4(C, t, q, at, rhs, live, z);
+        d4 acc = {0, 0, 0, 0};
+        mma_cols(acc, a, C, 0);
+        for (int j = 1; j < nb; ++j) {
+            load_cols<T>(a, F, lrow, t.n, 64 * j, C.g, sb - 1);
+            mma_cols(acc, a, C, 64 * j);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = r0 + rw + C.g + 4 * v;
+            if (ok && i < t.nr)
+                st_agent(C.A.z + (int64_t)(C.rb + C.li) * C.A.zs + t.z + t.c + i, z[v] - acc[v]);
+        }
+    }
+    signal(C, y_flag(t, t.u), t.sig);
+}
+
+// --------------------------------------------------------------- backward
+// S.v = x at the global rows of update rows r0 .. r0 + nr - 1 (gather,
+// sparse_add_subroutines_m.f90:32-49), zero past nr; the rows' positions are
+// read before the wait on counter f.
+template <typename T>
+__device__ __forceinline__ void stage_x(const Ctx<T>& C, const SolveTask& t, int r0, int nr, int f, int target)
+{
+    const int k = C.tid, at = k < nr ? C.A.grow[t.grow + (r0 - t.c) + k] : 0;
+    wait_for(C, f, target);
+    for (int r = 0; r < C.nr; r += 4) {
+        double q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            q[i] = (k < nr && r + i < C.nr) ? ld_agent(C.A.x + at + (int64_t)(C.rb + r + i) * C.A.n) : 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (r + i < C.nr) C.S.v[k][r + i] = q[i];
+    }
+    __syncthreads();
+}
+
+// Partial sums (kBwdPart): L[rows, 64 columns]^T x over at most 256 update
+// rows, each wave 16 of the columns (first column nslot of the front), into
+// 64 entries at slot.
+template <typename T> __device__ __forceinline__ void bwd_part(const Ctx<T>& C, const SolveTask& t)
+{
+    const int cw = 16 * C.wv, col0 = t.nslot;
+    const T* F = C.A.pool + t.front + (int64_t)col0 * t.n + t.r0;
+    const int lcol = min(cw + C.li, t.c - 1 - col0) * t.n;
+    T a[16], an[16];
+    load_rows<T>(a, F, lcol, 0, C.g, t.nr);
+    stage_x(C, t, t.r0, t.nr, t.w0, t.w0t);
+    d4 acc = {0, 0, 0, 0};
+    for (int q = 0; q < t.nr; q += 64) {
+        if (q + 64 < t.nr) load_rows<T>(an, F, lcol, q + 64, C.g, t.nr);
+        mma_rows(acc, a, C, q);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = an[j];
+    }
+    if (C.li < C.nr) {
+        double* P = C.A.z + (int64_t)(C.rb + C.li) * C.A.zs + t.slot + cw;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) st_agent(P + C.g + 4 * v, acc[v]);
+    }
+    signal(C, t.sig);
+}
+
+// y of column k of superblock u, right-hand sides r .. r + 3 (below lim),
+// less its partial sums, in chunk order; 16 loads in flight.
+template <typename T>
+__device__ __forceinline__ void y_less_parts(const Ctx<T>& C, const SolveTask& t, int k, int r, int lim, double (&v)[4])
+{
+    const double* Y = C.A.y + t.first + kSuper * t.u + k;
+    const double* P = C.A.z + t.slot + (int64_t)64 * t.nslot * (k >> 6) + (k & 63);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = r + i < lim ? ld_agent(Y + (int64_t)(r + i) * C.A.n) : 0.0;
+    for (int ch = 0; ch < t.nslot; ch += 4) {
+        double q[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                q[i][e] = (r + i < lim && ch + e < t.nslot) ? ld_agent(P + (int64_t)(r + i) * C.A.zs + 64 * (ch + e)) : 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[i] -= q[i][e];
+    }
+}
+
+// 16 columns of superblock u (kBwdCols): y less the update rows' partial
+// sums and less L[B_v, columns]^T x_v for v = nsup - 1 .. vlo as the x_v come
+// out, each wave a quarter of B_v's rows; the result replaces y.
+template <typename T> __device__ __forceinline__ void bwd_cols(const Ctx<T>& C, const SolveTask& t)
+{
+    const int col0 = kSuper * t.u + t.r0, lcol = min(C.li, t.c - 1 - col0) * t.n;
+    const T* F = C.A.pool + t.front + (int64_t)col0 * t.n;
+    const int vlo = t.grow, r0 = 64 * C.wv;
+    auto load = [&](T(&a)[16], int v) {
+        load_rows<T>(a, F + kSuper * v, lcol, r0, C.g, min(kSuper, t.c - kSuper * v));
+    };
+    T a[16], an[16];
+    load(a, t.nsup - 1);
+    const int col = C.tid >> 4, rhs = C.tid & 15;
+    const bool live = col < t.nr && rhs < C.nr;
+    wait_for(C, t.w0, t.w0t);
+    double y[4] = {0.0, 0.0, 0.0, 0.0};
+    if (live) y_less_parts(C, t, t.r0 + col, C.rb + rhs, C.rb + rhs + 1, y);
+    d4 acc = {0, 0, 0, 0};
+    for (int v = t.nsup - 1; v >= vlo; --v) {
+        wait_for(C, x_flag(t, v), yx_target(t, v));
+        stage_rows(C, C.A.x + t.first + kSuper * v, C.A.n, min(kSuper, t.c - kSuper * v));
+        __syncthreads();
+        if (v > vlo) load(an, v - 1);
+        mma_rows(acc, a, C, r0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = an[j];
+    }
+    const double s = reduce_waves(C, acc);
+    if (live) st_agent(C.A.y + t.first + kSuper * t.u + t.r0 + col + (int64_t)(C.rb + rhs) * C.A.n, y[0] - s);
+    signal(C, t.sig);
+}
+
+// S.v = superblock u's y less everything after it (nslot > 0: less the
+// partial sums still; otherwise kBwdCols tasks have done it all).
+template <typename T> __device__ __forceinline__ void stage_t(const Ctx<T>& C, const SolveTask& t, int sb)
+{
+    wait_for(C, t.w0, t.w0t);
+    const int k = C.tid;
+    if (t.nslot > 0)
+        for (int r = 0; r < C.nr; r += 4) {
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+            if (k < sb) y_less_parts(C, t, k, C.rb + r, C.rb + C.nr, v);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (r + i < C.nr) C.S.v[k][r + i] = v[i];
+        }
+    else
+        stage_rows(C, C.A.y + t.first + kSuper * t.u, C.A.n, sb);
+    __syncthreads();
+}
+
+// 16 rows of superblock u through its explicit inverse (kBwdTop): x_u =
+// X^T t_u - V^T x_{u+1}.
+template <typename T> __device__ __forceinline__ void bwd_top(const Ctx<T>& C, const SolveTask& t)
+{
+    const int sb = min(kSuper, t.c - kSuper * t.u), k0 = 64 * C.wv;
+    const bool next = t.u + 1 < t.nsup;
+    const T* X = C.A.sinv + t.aux + kSuper * t.r0;
+    T a[16], w[16];
+    load_rows<T>(a, X, kSuper * C.li, k0, C.g, kSuper);
+    if (next) load_rows<T>(w, X + 2 * kSuper * kSuper, kSuper * C.li, k0, C.g, kSuper);
+    stage_t(C, t, sb);
+    d4 acc = {0, 0, 0, 0}, accv = {0, 0, 0, 0};
+    if (k0 + 64 > t.r0) mma_rows(acc, a, C, k0);  // X is lower triangular
+    if (next) {
+        wait_for(C, x_flag(t, t.u + 1), yx_target(t, t.u + 1));
+        stage_rows(C, C.A.x + t.first + kSuper * (t.u + 1), C.A.n, min(kSuper, t.c - kSuper * (t.u + 1)));
+        __syncthreads();
+        mma_rows(accv, w, C, k0);
+    }
+    const double x = reduce_waves(C, acc - accv);
+    const int row = C.tid >> 4, rhs = C.tid & 15;
+    if (t.r0 + row < sb && rhs < C.nr)
+        st_agent(C.A.x + t.first + kSuper * t.u + t.r0 + row + (int64_t)(C.rb + rhs) * C.A.n, x);
+    signal(C, x_flag(t, t.u));
+}
+
+// Superblock u by one workgroup (kBwdPiv): x_b = inv(L_bb)^T (t_b -
+// sum_{a>b} L_ab^T x_a).  nr > 0 (fronts of one superblock): the front's nr
+// update rows first, t = y - L[rows, :]^T x.
+template <typename T> __device__ __forceinline__ void bwd_piv(const Ctx<T>& C, const SolveTask& t)
+{
+    const int sb = min(kSuper, t.c - kSuper * t.u), nb = (sb + 63) / 64, cw = 16 * C.wv, c0 = kSuper * t.u;
+    const T* F = C.A.pool + t.front + (int64_t)c0 * t.n;
+    const bool ok = C.li < C.nr;
+    if (t.nr > 0) {
+        d4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+        for (int r0 = 0; r0 < t.nr; r0 += kSuper) {
+            const int nr = min(kSuper, t.nr - r0);
+            stage_x(C, t, t.c + r0, nr, r0 == 0 ? t.w0 : -1, t.w0t);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                if (b >= nb) continue;
+                const int lcol = min(64 * b + cw + C.li, sb - 1) * t.n;
+                for (int q = 0; q < nr; q += 64) {
+                    T a[16];
+                    load_rows<T>(a, F + t.c + r0, lcol, q, C.g, nr);
+                    mma_rows(acc[b], a, C, q);
+                }
+            }
+            __syncthreads();
+        }
+        const double* Y = C.A.y + t.first + (int64_t)(C.rb + (ok ? C.li : 0)) * C.A.n;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            if (b >= nb || !ok) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int k = 64 * b + cw + C.g + 4 * v;
+                C.S.v[k][C.li] = k < sb ? ld_agent(Y + k) - acc[b][v] : 0.0;
+            }
+        }
+        __syncthreads();
+    } else {
+        stage_t(C, t, sb);
+    }
+    for (int b = nb - 1; b >= 0; --b) {
+        T iv[16], a[16];
+        load_cols<T>(iv, C.A.pool + t.aux + b * 4096, cw + C.li, 64, 0, C.g, 63);
+        if (b + 1 < nb) {
+            d4 acc = {0, 0, 0, 0};
+            const int lcol = (64 * b + cw + C.li) * t.n;
+            for (int j = b + 1; j < nb; ++j) {
+                load_rows<T>(a, F + c0, lcol, 64 * j, C.g, sb);
+                mma_rows(acc, a, C, 64 * j);
+            }
+            if (ok) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) C.S.v[64 * b + cw + C.g + 4 * v][C.li] -= acc[v];
+            }
+            __syncthreads();
+        }
+        d4 x = {0, 0, 0, 0};
+        mma_cols(x, iv, C, 64 * b);
+        __syncthreads();
+        if (ok) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int k = 64 * b + cw + C.g + 4 * v;
+                C.S.v[k][C.li] = x[v];
+                if (k < sb) st_agent(C.A.x + t.first + c0 + k + (int64_t)(C.rb + C.li) * C.A.n, x[v]);
+            }
+        }
+        __syncthreads();
+    }
+    signal(C, x_flag(t, t.u));
+}
+
+}  // namespace
+
+template <typename T> __global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 3 : 4) void k_solve(SolveArgs<T> A)
+{
+    __shared__ SolveLds S;
+    __shared__ int ticket;
+    const int tid = threadIdx.x;
+    int* counter = A.flags + A.ticket;
+    const int total = A.nbundles * A.ngroups;
+    if (tid == 0) ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    int k = __builtin_amdgcn_readfirstlane(ticket);
+    while (k < total) {
+        const SolveBundle bd = ld_scalar(A.bundles + A.bundle0 + k / A.ngroups);
+        const int grp = k % A.ngroups;
+        for (int i = bd.first; i < bd.first + bd.count; ++i) {
+            const SolveTask t = ld_scalar(A.tasks + i);
+            // hidden from the compiler, which would otherwise compute every
+            // kind's lane offsets once, before the loop, and spill them
+            int lid = tid;
+            asm volatile("" : "+v"(lid));
+            const Ctx<T> C{A,
+                           S,
+                           A.flags + kSolveCtl + (int64_t)grp * A.nflags,
+                           kRhs * grp,
+                           min(kRhs, A.nrhs - kRhs * grp),
+                           lid,
+                           lid & 63,
+                           __builtin_amdgcn_readfirstlane(lid >> 6),
+                           lid & 15,
+                           (lid >> 4) & 3};
+            switch (t.kind) {
+            case kFwdRows: fwd_rows(C, t); break;
+            case kFwdRows64: fwd_rows64(C, t); break;
+            case kFwdTop: fwd_top(C, t); break;
+            case kFwdPiv: fwd_piv(C, t); break;
+            case kBwdPart: bwd_part(C, t); break;
+            case kBwdCols: bwd_cols(C, t); break;
+            case kBwdTop: bwd_top(C, t); break;
+            default: bwd_piv(C, t); break;
+            }
+        }
+        // every task ends with a barrier after its last use of S and ticket
+        if (tid == 0) ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        k = __builtin_amdgcn_readfirstlane(ticket);
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void k_solve_reset(int* p, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) p[i] = 0;
+}
+
+void launch_solve_reset(int* flags, int64_t n, hipStream_t st)
+{
+    if (n > 0)
+        hipLaunchKernelGGL(k_solve_reset, dim3((unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, 512)),
+                           dim3(kThreads), 0, st, flags, n);
+}
+// As many workgroups as the chip holds (four per CU); fewer tickets, fewer.
+template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st)
+{
+    const int64_t total = (int64_t)A.nbundles * A.ngroups;
+    if (total > 0)
+        hipLaunchKernelGGL(k_solve<T>, dim3((unsigned)std::min<int64_t>(total, 1024)), dim3(kThreads), 0, st, A);
+}
+template void launch_solve<double>(const SolveArgs<double>&, hipStream_t);
+template void launch_solve<float>(const SolveArgs<float>&, hipStream_t);
+
+}  // namespace mfd
