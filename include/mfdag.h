@@ -352,7 +352,8 @@ int mfd_get_host_part(mfd_handle* h, double* ms, int* fronts, double* flops);
    and parent entries.  *conflicts = the number of task pairs that touch a
    common entry, one of them writing, without an order: in one launch, or in
    two launches no path of the DAG orders.  Variant 0 checks the schedule as
-   built; variant 1 a model of a schedule the library does not use (each
+   built, and adds the solves' tasks whose waits the tasks before them would
+   not satisfy exactly; variant 1 a model of a schedule the library does not use (each
    front's Schur tiles on a fourth stream forked after the launch with the
    front's last diagonal task).  report (nullable) receives the first few
    pairs.  Runs on the host; works without a GPU. */

@@ -56,8 +56,8 @@ void launch_gemm_seg(T* pool, const GemmTask* tasks, const SegTask* segs, const 
 template <typename T>
 void launch_superinv(const T* pool, T* sinv, const NodeDev* nodes, const SuperInvTask* tasks, int count, bool wv,
                      hipStream_t st);
-// The solves (mfd_solve.hip): tasks of bundles bundle0 .. bundle0 + nbundles
-// - 1 for every group of 16 right-hand sides, one ticket word per launch.
+// The solves (mfd_solve.hip): tasks task0 .. task0 + ntasks - 1 for every
+// group of 16 right-hand sides, one ticket word per launch.
 // z: planes of zs entries, one per right-hand side; b, y, x: n x nrhs.
 // flags: kSolveCtl control words, then nflags counters per group, all zero
 // at the start (launch_solve_reset); err: set when a wait reached its bound.
@@ -67,12 +67,12 @@ template <typename T> struct SolveArgs {
     double* z;
     const double* b;
     double *y, *x;
-    const int *grow, *gptr, *gsrc;
+    const int2* gat;
+    const int *gsrc, *grow;
     const SolveTask* tasks;
-    const SolveBundle* bundles;
     int *flags, *err;
     int64_t zs;
-    int n, nrhs, ngroups, nflags, bundle0, nbundles, ticket;
+    int n, nrhs, ngroups, nflags, task0, ntasks, ticket;
 };
 constexpr int kRhsGroup = 16;
 void launch_solve_reset(int* flags, int64_t n, hipStream_t st);

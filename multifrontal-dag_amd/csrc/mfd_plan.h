@@ -61,7 +61,7 @@ constexpr int64_t kSuperMats = 3 * (int64_t)kSuper * kSuper;  // entries per sup
 // rows from r0, superblocks v < nslot applied to them, sig raised; kFwdTop,
 // rows r0 .. r0 + 15 of superblock u (super fronts); kFwdPiv, superblock u
 // (other fronts) and then, nr > 0, the front's nr update rows, sig raised.
-// Backward: kBwdPart, partial sums of the 64 columns from column nslot over
+// Backward: kBwdPart, partial sums of the 32 columns from column nslot over
 // nr (<= 256) rows from r0, to plane offset slot, sig raised; kBwdCols, nr
 // (<= 16) columns r0 .. of superblock u, superblocks v >= grow applied to
 // them, sig raised; kBwdTop, columns r0 .. r0 + 15 of superblock u; kBwdPiv,
@@ -76,17 +76,13 @@ struct SolveTask {
     int n, c, first;  // the front; its 0-based first global column
     int z;            // front row i lies at z + i of a right-hand side's plane
     int kind, u, r0, nr;
-    int goff;         // the front's gather list (gptr[goff + i], row i; < 0: no children)
+    int goff;         // the front's gather table (gat[goff + i], row i; < 0: no children)
     int grow;         // its update rows' global rows (backward), or the first superblock of kBwdCols
     int slot, nslot;
     int w0, w0t, sig;
     int flag, fstr;   // the front's counters: asm, then z, y, p, t, x of each superblock, fstr apart
     int nsup, super;  // superblocks; 1: super front
-    int pad;
-};
-// A ticket: tasks [first, first + count) in order.
-struct SolveBundle {
-    int first, count;
+    int per;          // turns the next ticket of the workgroup takes
 };
 // Words before the counters in the solve's control array: the two tickets
 // (whole solve or forward part; backward part), the stop word.

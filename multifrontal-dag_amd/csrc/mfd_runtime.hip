@@ -189,8 +189,8 @@ struct mfd_handle {
     // the solves: task list (mfd_solve_plan.h) and its device copies
     SolvePlan sp;
     SolveTask* d_stasks = nullptr;
-    SolveBundle* d_sbundles = nullptr;
-    int *d_grow = nullptr, *d_gptr = nullptr, *d_gsrc = nullptr;
+    SolvePlan::Gather* d_gat = nullptr;
+    int *d_gsrc = nullptr, *d_grow = nullptr;
     SuperInvTask* d_xinv = nullptr;
     int solve_rc = 0;          // build_solve_plan's result for the current schedule
     int* solve_err = nullptr;  // pinned: set by a solve whose wait reached its bound
@@ -344,8 +344,8 @@ void free_device(mfd_handle* h)
     h->d_gemm = nullptr;
     h->d_level_nodes = h->d_child_ptr = h->d_child_list = nullptr;
     h->d_stasks = nullptr;
-    h->d_sbundles = nullptr;
-    h->d_grow = h->d_gptr = h->d_gsrc = nullptr;
+    h->d_gat = nullptr;
+    h->d_gsrc = h->d_grow = nullptr;
     h->d_xinv = nullptr;
     h->d_segs = nullptr;
     h->d_seg_ptr = nullptr;
@@ -836,9 +836,8 @@ int setup_device(mfd_handle* h)
     MFD_TRY(upload(h, &h->d_child_ptr, h->child_ptr));
     MFD_TRY(upload(h, &h->d_child_list, h->child_list));
     MFD_TRY(upload(h, &h->d_stasks, h->sp.tasks));
-    MFD_TRY(upload(h, &h->d_sbundles, h->sp.bundles));
     MFD_TRY(upload(h, &h->d_grow, h->sp.grow));
-    MFD_TRY(upload(h, &h->d_gptr, h->sp.gptr));
+    MFD_TRY(upload(h, &h->d_gat, h->sp.gat));
     MFD_TRY(upload(h, &h->d_gsrc, h->sp.gsrc));
     MFD_TRY(upload(h, &h->d_xinv, h->sp.xinv));
     if (h->sp.sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv64, h->sp.sinv_elems));
@@ -1195,11 +1194,10 @@ template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double
     a.b = bp;
     a.y = h->d_y;
     a.x = xp;
-    a.grow = h->d_grow;
-    a.gptr = h->d_gptr;
+    a.gat = reinterpret_cast<const int2*>(h->d_gat);
     a.gsrc = h->d_gsrc;
+    a.grow = h->d_grow;
     a.tasks = h->d_stasks;
-    a.bundles = h->d_sbundles;
     a.flags = h->d_sflags;
     a.err = h->solve_err;
     a.zs = h->sp.plane;
@@ -1207,7 +1205,7 @@ template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double
     a.nrhs = nrhs;
     a.ngroups = (nrhs + kRhsGroup - 1) / kRhsGroup;
     a.nflags = h->sp.nflags;
-    a.nbundles = (int)h->sp.bundles.size();
+    a.ntasks = (int)h->sp.tasks.size();
     a.ticket = kSolveTicket;
     launch_solve_reset(h->d_sflags, solve_words(h, nrhs), st);
     if ((h->flags & MFD_FLAG_PROFILE) == 0) {
@@ -1217,11 +1215,11 @@ template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double
     hipEvent_t pe[3] = {};
     for (auto& e : pe) (void)hipEventCreate(&e);
     (void)hipEventRecord(pe[0], st);
-    a.nbundles = h->sp.fwd_bundles;
+    a.ntasks = h->sp.fwd_tasks;
     launch_solve<T>(a, st);
     (void)hipEventRecord(pe[1], st);
-    a.bundle0 = h->sp.fwd_bundles;
-    a.nbundles = (int)h->sp.bundles.size() - h->sp.fwd_bundles;
+    a.task0 = h->sp.fwd_tasks;
+    a.ntasks = (int)h->sp.tasks.size() - h->sp.fwd_tasks;
     a.ticket = kSolveTicketBwd;
     launch_solve<T>(a, st);
     (void)hipEventRecord(pe[2], st);

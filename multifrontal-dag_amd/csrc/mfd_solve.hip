@@ -105,14 +105,20 @@ template <typename T> struct Ctx {
 };
 
 // Waits until counter f reaches target (all threads; ends with a barrier,
-// after which the values the counter stands for can be read).
-template <typename T> __device__ __forceinline__ void wait_for(const Ctx<T>& C, int f, int target)
+// after which the values the counter stands for can be read).  SLOW: polls
+// every 0.4 us at most, for tasks off the chain that many workgroups run (so
+// that their polls do not delay the counter's additions).
+template <typename T, bool SLOW = false>
+__device__ __forceinline__ void wait_for(const Ctx<T>& C, int f, int target)
 {
     if (f >= 0 && C.tid == 0) {
         const int* p = C.flags + f;
         int* stop = C.A.flags + kSolveStop;
         for (int spins = 0; ld_agent(p) < target;) {
-            __builtin_amdgcn_s_sleep(1);
+            if (SLOW)
+                __builtin_amdgcn_s_sleep(12);
+            else
+                __builtin_amdgcn_s_sleep(1);
             if ((++spins & 255) == 0 && (ld_agent(stop) != 0 || spins >= kSpinLimit)) {
                 __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(C.A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -160,45 +166,50 @@ __device__ __forceinline__ void stage_rows(const Ctx<T>& C, const double* src, i
     }
 }
 
-// The children's contributions to row i of a front: list entries gptr[goff +
-// i] .. of the children's update rows, in child order (goff < 0: a leaf).
-// The first two are looked up before the wait for the children.
-struct Gather {
-    int k0 = 0, k1 = 0, s0 = 0, s1 = 0;
-};
-template <typename T> __device__ __forceinline__ Gather gather_begin(const Ctx<T>& C, const SolveTask& t, int i)
+// The children's contributions to row i of a front, in child order: table
+// entry gat[goff + i] holds the plane positions of the first and the second
+// (-1: none), or, where there are more, -2 - k with the list of the second
+// and the others at gsrc[k] (their number, then their positions); goff < 0:
+// a leaf.  Read before the wait for the children.
+template <typename T> __device__ __forceinline__ int2 gather_at(const Ctx<T>& C, const SolveTask& t, int i)
 {
-    Gather q;
-    if (t.goff < 0) return q;
-    q.k0 = C.A.gptr[t.goff + i];
-    q.k1 = C.A.gptr[t.goff + i + 1];
-    if (q.k0 < q.k1) q.s0 = C.A.gsrc[q.k0];
-    if (q.k0 + 1 < q.k1) q.s1 = C.A.gsrc[q.k0 + 1];
-    return q;
+    return t.goff < 0 ? make_int2(-1, -1) : C.A.gat[t.goff + i];
 }
-// Four right-hand-side entries of a front, entry e that of row i[e], column
-// rhs[e] (live[e] false: zero): b on pivot rows, plus the children's
-// contributions (scatter_add, sparse_add_subroutines_m.f90:13-30).  All
-// loads are issued before the first sum.
-template <typename T>
-__device__ __forceinline__ void gather4(const Ctx<T>& C, const SolveTask& t, const Gather (&q)[4], const int (&i)[4],
-                                        const int (&rhs)[4], const bool (&live)[4], double (&z)[4])
+template <typename T> __device__ __forceinline__ double gather_list(const Ctx<T>& C, int y, int rhs, double v)
 {
-    double bv[4], c0[4], c1[4];
+    const int* p = C.A.gsrc + (-2 - y);
+    for (int k = 1; k <= p[0]; ++k) v += ld_agent(C.A.z + (int64_t)rhs * C.A.zs + p[k]);
+    return v;
+}
+// Four right-hand-side entries of a front, entry e that of row i[e] (gather
+// entry q[e]), column rhs[e] (live[e] false: zero): b on pivot rows, plus the
+// children's contributions (scatter_add, sparse_add_subroutines_m.f90:13-30).
+// begin issues the loads, end adds them up.
+struct Gather4 {
+    double b[4], c0[4], c1[4];
+};
+template <typename T>
+__device__ __forceinline__ void gather_begin(const Ctx<T>& C, const SolveTask& t, const int2 (&q)[4], const int (&i)[4],
+                                             const int (&rhs)[4], const bool (&live)[4], Gather4& v)
+{
 #pragma unroll
-    for (int e = 0; e < 4; ++e) bv[e] = (live[e] && i[e] < t.c) ? C.A.b[t.first + i[e] + (int64_t)rhs[e] * C.A.n] : 0.0;
+    for (int e = 0; e < 4; ++e)
+        v.b[e] = (live[e] && i[e] < t.c) ? C.A.b[t.first + i[e] + (int64_t)rhs[e] * C.A.n] : 0.0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const double* Z = C.A.z + (int64_t)rhs[e] * C.A.zs;
-        c0[e] = (live[e] && q[e].k0 < q[e].k1) ? ld_agent(Z + q[e].s0) : 0.0;
-        c1[e] = (live[e] && q[e].k0 + 1 < q[e].k1) ? ld_agent(Z + q[e].s1) : 0.0;
+        v.c0[e] = (live[e] && q[e].x >= 0) ? ld_agent(Z + q[e].x) : 0.0;
+        v.c1[e] = (live[e] && q[e].y >= 0) ? ld_agent(Z + q[e].y) : 0.0;
     }
+}
+template <typename T>
+__device__ __forceinline__ void gather_end(const Ctx<T>& C, const int2 (&q)[4], const int (&rhs)[4],
+                                           const bool (&live)[4], const Gather4& v, double (&z)[4])
+{
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        z[e] = bv[e] + c0[e] + c1[e];
-        if (live[e])
-            for (int k = q[e].k0 + 2; k < q[e].k1; ++k)
-                z[e] += ld_agent(C.A.z + (int64_t)rhs[e] * C.A.zs + C.A.gsrc[k]);
+        z[e] = v.b[e] + v.c0[e] + v.c1[e];
+        if (live[e] && q[e].y < -1) z[e] = gather_list(C, q[e].y, rhs[e], z[e]);
     }
 }
 
@@ -295,20 +306,20 @@ template <typename T> __device__ __forceinline__ void fwd_rows(const Ctx<T>& C, 
     if (nv > 0) load(a, 0);
     const int row = C.tid >> 4, rhs = C.tid & 15, i = t.r0 + row;
     const bool live = row < t.nr && rhs < C.nr;
-    const Gather q = gather_begin(C, t, live ? i : t.r0);
+    const int2 q = gather_at(C, t, live ? i : t.r0);
     wait_for(C, t.w0, t.w0t);
     double z = 0.0;
     if (live) {
         const double* Z = C.A.z + (int64_t)(C.rb + rhs) * C.A.zs;
         const double bv = i < t.c ? C.A.b[t.first + i + (int64_t)(C.rb + rhs) * C.A.n] : 0.0;
-        const double c0 = q.k0 < q.k1 ? ld_agent(Z + q.s0) : 0.0;
-        const double c1 = q.k0 + 1 < q.k1 ? ld_agent(Z + q.s1) : 0.0;
+        const double c0 = q.x >= 0 ? ld_agent(Z + q.x) : 0.0;
+        const double c1 = q.y >= 0 ? ld_agent(Z + q.y) : 0.0;
         z = bv + c0 + c1;
-        for (int k = q.k0 + 2; k < q.k1; ++k) z += ld_agent(Z + C.A.gsrc[k]);
+        if (q.y < -1) z = gather_list(C, q.y, C.rb + rhs, z);
     }
     d4 acc = {0, 0, 0, 0};
     for (int v = 0; v < nv; ++v) {
-        wait_for(C, y_flag(t, v), yx_target(t, v));
+        wait_for<T, true>(C, y_flag(t, v), yx_target(t, v));
         stage_rows(C, C.A.y + t.first + kSuper * v, C.A.n, min(kSuper, t.c - kSuper * v));
         __syncthreads();
         if (v + 1 < nv) load(an, v + 1);
@@ -322,19 +333,25 @@ template <typename T> __device__ __forceinline__ void fwd_rows(const Ctx<T>& C, 
 }
 
 // The lane's four entries of a wave's 16 x 16 result over rows r0 + rw ..,
-// nr of them from r0 on: rows, right-hand sides and gather lists.
+// nr of them from r0 on (nr <= 0: none): rows and right-hand sides.
 template <typename T>
-__device__ __forceinline__ void own_rows(const Ctx<T>& C, const SolveTask& t, int r0, int rw, int nr, Gather (&q)[4],
-                                         int (&at)[4], int (&rhs)[4], bool (&live)[4])
+__device__ __forceinline__ void own_rows(const Ctx<T>& C, const SolveTask& t, int r0, int rw, int nr, int (&at)[4],
+                                         int (&rhs)[4], bool (&live)[4])
 {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         const int i = rw + C.g + 4 * v;
         live[v] = i < nr && C.li < C.nr;
-        at[v] = r0 + min(i, nr - 1);
+        at[v] = live[v] ? r0 + i : 0;
         rhs[v] = C.rb + (C.li < C.nr ? C.li : 0);
-        q[v] = gather_begin(C, t, at[v]);
     }
+}
+template <typename T>
+__device__ __forceinline__ void gather_rows(const Ctx<T>& C, const SolveTask& t, const int (&at)[4],
+                                            const bool (&live)[4], int2 (&q)[4])
+{
+#pragma unroll
+    for (int v = 0; v < 4; ++v) q[v] = live[v] ? gather_at(C, t, at[v]) : make_int2(-1, -1);
 }
 
 // 64 rows of a front (kFwdRows64, where rows are many): each wave 16 of
@@ -348,17 +365,22 @@ template <typename T> __device__ __forceinline__ void fwd_rows64(const Ctx<T>& C
     };
     T a[16], an[16];
     if (nv > 0) load(a, 0);
-    Gather q[4];
+    int2 q[4];
     int at[4], rhs[4];
     bool live[4];
-    own_rows(C, t, t.r0, rw, t.nr, q, at, rhs, live);
+    own_rows(C, t, t.r0, rw, t.nr, at, rhs, live);
+    gather_rows(C, t, at, live, q);
     wait_for(C, t.w0, t.w0t);
     double z[4];
-    gather4(C, t, q, at, rhs, live, z);
+    {
+        Gather4 g4;
+        gather_begin(C, t, q, at, rhs, live, g4);
+        gather_end(C, q, rhs, live, g4, z);
+    }
     d4 acc = {0, 0, 0, 0};
     for (int v = 0; v < nv; ++v) {
         const int pb = min(kSuper, t.c - kSuper * v);
-        wait_for(C, y_flag(t, v), yx_target(t, v));
+        wait_for<T, true>(C, y_flag(t, v), yx_target(t, v));
         stage_rows(C, C.A.y + t.first + kSuper * v, C.A.n, pb);
         __syncthreads();
         for (int k0 = 0; k0 < pb; k0 += 64) {
@@ -385,15 +407,17 @@ template <typename T> __device__ __forceinline__ void stage_z(const Ctx<T>& C, c
 {
     const int k = C.tid, i = kSuper * t.u + k;
     if (gather) {
-        const Gather q = gather_begin(C, t, k < sb ? i : kSuper * t.u);
-        const Gather qs[4] = {q, q, q, q};
+        const int2 q = gather_at(C, t, k < sb ? i : kSuper * t.u);
+        const int2 qs[4] = {q, q, q, q};
         const int at[4] = {i, i, i, i};
         wait_for(C, t.w0, t.w0t);
         for (int r = 0; r < C.nr; r += 4) {
             const int rhs[4] = {C.rb + r, C.rb + r + 1, C.rb + r + 2, C.rb + r + 3};
             const bool live[4] = {k < sb, k < sb && r + 1 < C.nr, k < sb && r + 2 < C.nr, k < sb && r + 3 < C.nr};
             double z[4];
-            gather4(C, t, qs, at, rhs, live, z);
+            Gather4 g4;
+            gather_begin(C, t, qs, at, rhs, live, g4);
+            gather_end(C, qs, rhs, live, g4, z);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (r + e < C.nr) C.S.v[k][r + e] = z[e];
@@ -431,6 +455,13 @@ template <typename T> __device__ __forceinline__ void fwd_top(const Ctx<T>& C, c
     signal(C, y_flag(t, t.u));
 }
 
+// The 64 x 64 tiles a superblock's solve takes up, in order: for each block b
+// its tiles (b, j), j < b, then its inverse (j = b).  Two tiles are in flight
+// ahead of the one in use (their loads wait for no barrier).
+constexpr int kTiles = 10;
+__device__ constexpr int kTileB[kTiles] = {0, 1, 1, 2, 2, 2, 3, 3, 3, 3};
+__device__ constexpr int kTileJ[kTiles] = {0, 0, 1, 0, 1, 2, 0, 1, 2, 3};
+
 // Superblock u by one workgroup (kFwdPiv), 64 columns at a time through the
 // stored inverses of the diagonal blocks: y_b = inv(L_bb) (z_b - sum_{a<b}
 // L_ba y_a).  nr > 0 (fronts of one superblock): then the front's nr update
@@ -440,58 +471,90 @@ template <typename T> __device__ __forceinline__ void fwd_piv(const Ctx<T>& C, c
     const int sb = min(kSuper, t.c - kSuper * t.u), nb = (sb + 63) / 64, rw = 16 * C.wv, c0 = kSuper * t.u;
     const T* F = C.A.pool + t.front + (int64_t)c0 * t.n;  // the superblock's columns
     const bool ok = C.li < C.nr;
-    stage_z(C, t, sb, t.u == 0);
-    for (int b = 0; b < nb; ++b) {
-        T iv[16], a[16];
-        // inv[r + 64 q] = L^{-1}(q, r): the lane's row q, 16-byte pieces along r
-        load_rows<T>(iv, C.A.pool + t.aux + b * 4096, 64 * (rw + C.li), 0, C.g, 64);
-        if (b > 0) {
-            d4 acc = {0, 0, 0, 0};
-            const int lrow = min(c0 + 64 * b + rw + C.li, t.n - 1);
-            for (int j = 0; j < b; ++j) {
-                load_cols<T>(a, F, lrow, t.n, 64 * j, C.g, sb - 1);
-                mma_cols(acc, a, C, 64 * j);
-            }
-            if (ok) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) C.S.v[64 * b + rw + C.g + 4 * v][C.li] -= acc[v];
-            }
-            __syncthreads();
-        }
-        d4 y = {0, 0, 0, 0};
-        mma_rows(y, iv, C, 64 * b);
-        __syncthreads();
-        if (ok) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int k = 64 * b + rw + C.g + 4 * v;
-                C.S.v[k][C.li] = k < sb ? y[v] : 0.0;
-                if (k < sb) st_agent(C.A.y + t.first + c0 + k + (int64_t)(C.rb + C.li) * C.A.n, y[v]);
-            }
-        }
-        __syncthreads();
-    }
-    for (int r0 = 0; r0 < t.nr; r0 += 64) {
-        const int lrow = min(t.c + r0 + rw + C.li, t.n - 1);
-        T a[16];
-        load_cols<T>(a, F, lrow, t.n, 0, C.g, sb - 1);
-        Gather q[4];
+    T buf[3][16];
+    auto fetch = [&](T(&a)[16], int b, int j) {
+        if (j < b)
+            load_cols<T>(a, F, min(c0 + 64 * b + rw + C.li, t.n - 1), t.n, 64 * j, C.g, sb - 1);
+        else  // inv[r + 64 q] = L^{-1}(q, r): the lane's row q, 16-byte pieces along r
+            load_rows<T>(a, C.A.pool + t.aux + b * 4096, 64 * (rw + C.li), 0, C.g, 64);
+    };
+    fetch(buf[0], 0, 0);
+    if (nb > 1) fetch(buf[1], 1, 0);
+    int2 qr[4];  // the first update rows' gather entries
+    {
         int at[4], rhs[4];
         bool live[4];
-        own_rows(C, t, t.c + r0, rw, t.nr - r0, q, at, rhs, live);
-        double z[4];
-        gather4(C, t, q, at, rhs, live, z);
-        d4 acc = {0, 0, 0, 0};
-        mma_cols(acc, a, C, 0);
-        for (int j = 1; j < nb; ++j) {
-            load_cols<T>(a, F, lrow, t.n, 64 * j, C.g, sb - 1);
-            mma_cols(acc, a, C, 64 * j);
-        }
+        own_rows(C, t, t.c, rw, t.nr, at, rhs, live);
+        gather_rows(C, t, at, live, qr);
+    }
+    stage_z(C, t, sb, t.u == 0);
+    d4 acc = {0, 0, 0, 0};
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int i = r0 + rw + C.g + 4 * v;
-            if (ok && i < t.nr)
-                st_agent(C.A.z + (int64_t)(C.rb + C.li) * C.A.zs + t.z + t.c + i, z[v] - acc[v]);
+    for (int q = 0; q < kTiles; ++q) {
+        const int b = kTileB[q], j = kTileJ[q];
+        if (b < nb) {
+            if (q + 2 < kTiles && kTileB[q + 2] < nb) fetch(buf[(q + 2) % 3], kTileB[q + 2], kTileJ[q + 2]);
+            if (j < b) {
+                mma_cols(acc, buf[q % 3], C, 64 * j);
+                if (j == b - 1) {
+                    if (ok) {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) C.S.v[64 * b + rw + C.g + 4 * v][C.li] -= acc[v];
+                    }
+                    acc = d4{0, 0, 0, 0};
+                    __syncthreads();
+                }
+            } else {
+                d4 y = {0, 0, 0, 0};
+                mma_rows(y, buf[q % 3], C, 64 * b);
+                __syncthreads();
+                if (ok) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int k = 64 * b + rw + C.g + 4 * v;
+                        C.S.v[k][C.li] = k < sb ? y[v] : 0.0;
+                        if (k < sb) st_agent(C.A.y + t.first + c0 + k + (int64_t)(C.rb + C.li) * C.A.n, y[v]);
+                    }
+                }
+                __syncthreads();
+            }
+        }
+    }
+    if (t.nr > 0) {
+        // tiles (64 rows, 64 columns) with the next one's entries, and the
+        // next rows' gather entries, in flight
+        auto rows = [&](T(&a)[16], int r0, int j) {
+            load_cols<T>(a, F, min(t.c + r0 + rw + C.li, t.n - 1), t.n, 64 * j, C.g, sb - 1);
+        };
+        int at[4], rhs[4];
+        bool live[4];
+        rows(buf[0], 0, 0);
+        for (int r0 = 0; r0 < t.nr; r0 += 64) {
+            Gather4 g4;
+            own_rows(C, t, t.c + r0, rw, t.nr - r0, at, rhs, live);
+            gather_begin(C, t, qr, at, rhs, live, g4);
+            int2 qn[4];
+            {
+                int atn[4];
+                bool liven[4];
+                own_rows(C, t, t.c + r0 + 64, rw, t.nr - r0 - 64, atn, rhs, liven);
+                gather_rows(C, t, atn, liven, qn);
+            }
+            acc = d4{0, 0, 0, 0};
+            for (int j = 0; j < nb; ++j) {
+                const bool last = j + 1 == nb;
+                if (!last || r0 + 64 < t.nr) rows(buf[1], last ? r0 + 64 : r0, last ? 0 : j + 1);
+                mma_cols(acc, buf[0], C, 64 * j);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) buf[0][e] = buf[1][e];
+            }
+            double z[4];
+            gather_end(C, qr, rhs, live, g4, z);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if (live[v]) st_agent(C.A.z + (int64_t)rhs[v] * C.A.zs + t.z + at[v], z[v] - acc[v]);
+                qr[v] = qn[v];
+            }
         }
     }
     signal(C, y_flag(t, t.u), t.sig);
@@ -518,28 +581,32 @@ __device__ __forceinline__ void stage_x(const Ctx<T>& C, const SolveTask& t, int
     __syncthreads();
 }
 
-// Partial sums (kBwdPart): L[rows, 64 columns]^T x over at most 256 update
-// rows, each wave 16 of the columns (first column nslot of the front), into
-// 64 entries at slot.
+// Partial sums (kBwdPart): L[rows, 32 columns]^T x over at most 256 update
+// rows (first column nslot of the front) into 32 entries at slot; a wave
+// takes 16 of the columns and half the rows, so that all of the task's
+// entries are in registers before the wait for x.
 template <typename T> __device__ __forceinline__ void bwd_part(const Ctx<T>& C, const SolveTask& t)
 {
-    const int cw = 16 * C.wv, col0 = t.nslot;
+    const int cw = 16 * (C.wv & 1), h = 128 * (C.wv >> 1), col0 = t.nslot;
     const T* F = C.A.pool + t.front + (int64_t)col0 * t.n + t.r0;
     const int lcol = min(cw + C.li, t.c - 1 - col0) * t.n;
     T a[16], an[16];
-    load_rows<T>(a, F, lcol, 0, C.g, t.nr);
+    load_rows<T>(a, F, lcol, h, C.g, t.nr);
+    load_rows<T>(an, F, lcol, h + 64, C.g, t.nr);
     stage_x(C, t, t.r0, t.nr, t.w0, t.w0t);
     d4 acc = {0, 0, 0, 0};
-    for (int q = 0; q < t.nr; q += 64) {
-        if (q + 64 < t.nr) load_rows<T>(an, F, lcol, q + 64, C.g, t.nr);
-        mma_rows(acc, a, C, q);
+    mma_rows(acc, a, C, h);
+    mma_rows(acc, an, C, h + 64);
+    __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 16; ++j) a[j] = an[j];
-    }
-    if (C.li < C.nr) {
-        double* P = C.A.z + (int64_t)(C.rb + C.li) * C.A.zs + t.slot + cw;
+    for (int v = 0; v < 4; ++v) C.S.red[C.wv][C.g + 4 * v][C.li] = acc[v];
+    __syncthreads();
 #pragma unroll
-        for (int v = 0; v < 4; ++v) st_agent(P + C.g + 4 * v, acc[v]);
+    for (int e = 0; e < 2; ++e) {
+        const int k = (C.tid & 15) + 16 * e, rhs = C.tid >> 4;
+        if (rhs < C.nr)
+            st_agent(C.A.z + (int64_t)(C.rb + rhs) * C.A.zs + t.slot + k,
+                     C.S.red[e][C.tid & 15][rhs] + C.S.red[e + 2][C.tid & 15][rhs]);
     }
     signal(C, t.sig);
 }
@@ -646,72 +713,101 @@ template <typename T> __device__ __forceinline__ void bwd_top(const Ctx<T>& C, c
 }
 
 // Superblock u by one workgroup (kBwdPiv): x_b = inv(L_bb)^T (t_b -
-// sum_{a>b} L_ab^T x_a).  nr > 0 (fronts of one superblock): the front's nr
-// update rows first, t = y - L[rows, :]^T x.
+// sum_{a>b} L_ab^T x_a), tiles in fwd_piv's order counted from the last
+// block.  nr > 0 (fronts of one superblock): the front's nr update rows
+// first, t = y - L[rows, :]^T x.
 template <typename T> __device__ __forceinline__ void bwd_piv(const Ctx<T>& C, const SolveTask& t)
 {
     const int sb = min(kSuper, t.c - kSuper * t.u), nb = (sb + 63) / 64, cw = 16 * C.wv, c0 = kSuper * t.u;
     const T* F = C.A.pool + t.front + (int64_t)c0 * t.n;
     const bool ok = C.li < C.nr;
+    T buf[3][16];
     if (t.nr > 0) {
         d4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+        auto rows = [&](T(&a)[16], int r, int b) {  // rows r .. r + 63 of the update part, column block b
+            load_rows<T>(a, F + t.c, min(64 * b + cw + C.li, sb - 1) * t.n, r, C.g, t.nr);
+        };
+        rows(buf[0], 0, 0);
         for (int r0 = 0; r0 < t.nr; r0 += kSuper) {
             const int nr = min(kSuper, t.nr - r0);
             stage_x(C, t, t.c + r0, nr, r0 == 0 ? t.w0 : -1, t.w0t);
+            for (int q = 0; q < nr; q += 64) {
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                if (b >= nb) continue;
-                const int lcol = min(64 * b + cw + C.li, sb - 1) * t.n;
-                for (int q = 0; q < nr; q += 64) {
-                    T a[16];
-                    load_rows<T>(a, F + t.c + r0, lcol, q, C.g, nr);
-                    mma_rows(acc[b], a, C, q);
+                for (int b = 0; b < 4; ++b) {
+                    if (b >= nb) continue;
+                    const bool last = b + 1 >= nb;
+                    if (!last || r0 + q + 64 < t.nr) rows(buf[1], r0 + q + (last ? 64 : 0), last ? 0 : b + 1);
+                    mma_rows(acc[b], buf[0], C, q);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) buf[0][e] = buf[1][e];
                 }
             }
             __syncthreads();
         }
         const double* Y = C.A.y + t.first + (int64_t)(C.rb + (ok ? C.li : 0)) * C.A.n;
+        double y[4][4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int k = 64 * b + cw + C.g + 4 * v;
+                y[b][v] = ok && k < sb ? ld_agent(Y + k) : 0.0;
+            }
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             if (b >= nb || !ok) continue;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int k = 64 * b + cw + C.g + 4 * v;
-                C.S.v[k][C.li] = k < sb ? ld_agent(Y + k) - acc[b][v] : 0.0;
+                C.S.v[k][C.li] = k < sb ? y[b][v] - acc[b][v] : 0.0;
             }
         }
-        __syncthreads();
-    } else {
-        stage_t(C, t, sb);
     }
-    for (int b = nb - 1; b >= 0; --b) {
-        T iv[16], a[16];
-        load_cols<T>(iv, C.A.pool + t.aux + b * 4096, cw + C.li, 64, 0, C.g, 63);
-        if (b + 1 < nb) {
-            d4 acc = {0, 0, 0, 0};
-            const int lcol = (64 * b + cw + C.li) * t.n;
-            for (int j = b + 1; j < nb; ++j) {
-                load_rows<T>(a, F + c0, lcol, 64 * j, C.g, sb);
-                mma_rows(acc, a, C, 64 * j);
-            }
-            if (ok) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) C.S.v[64 * b + cw + C.g + 4 * v][C.li] -= acc[v];
-            }
-            __syncthreads();
-        }
-        d4 x = {0, 0, 0, 0};
-        mma_cols(x, iv, C, 64 * b);
+    auto fetch = [&](T(&a)[16], int bq, int jq) {
+        const int b = nb - 1 - bq, j = nb - 1 - jq;
+        if (jq < bq)
+            load_rows<T>(a, F + c0, (64 * b + cw + C.li) * t.n, 64 * j, C.g, sb);
+        else
+            load_cols<T>(a, C.A.pool + t.aux + b * 4096, cw + C.li, 64, 0, C.g, 63);
+    };
+    fetch(buf[0], 0, 0);
+    if (nb > 1) fetch(buf[1], 1, 0);
+    if (t.nr > 0)
         __syncthreads();
-        if (ok) {
+    else
+        stage_t(C, t, sb);
+    d4 acc = {0, 0, 0, 0};
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int k = 64 * b + cw + C.g + 4 * v;
-                C.S.v[k][C.li] = x[v];
-                if (k < sb) st_agent(C.A.x + t.first + c0 + k + (int64_t)(C.rb + C.li) * C.A.n, x[v]);
+    for (int q = 0; q < kTiles; ++q) {
+        const int bq = kTileB[q], jq = kTileJ[q];
+        if (bq < nb) {
+            const int b = nb - 1 - bq, j = nb - 1 - jq;
+            if (q + 2 < kTiles && kTileB[q + 2] < nb) fetch(buf[(q + 2) % 3], kTileB[q + 2], kTileJ[q + 2]);
+            if (jq < bq) {
+                mma_rows(acc, buf[q % 3], C, 64 * j);
+                if (jq == bq - 1) {
+                    if (ok) {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) C.S.v[64 * b + cw + C.g + 4 * v][C.li] -= acc[v];
+                    }
+                    acc = d4{0, 0, 0, 0};
+                    __syncthreads();
+                }
+            } else {
+                d4 x = {0, 0, 0, 0};
+                mma_cols(x, buf[q % 3], C, 64 * b);
+                __syncthreads();
+                if (ok) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int k = 64 * b + cw + C.g + 4 * v;
+                        C.S.v[k][C.li] = x[v];
+                        if (k < sb) st_agent(C.A.x + t.first + c0 + k + (int64_t)(C.rb + C.li) * C.A.n, x[v]);
+                    }
+                }
+                __syncthreads();
             }
         }
-        __syncthreads();
     }
     signal(C, x_flag(t, t.u));
 }
@@ -724,15 +820,21 @@ template <typename T> __global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 3 
     __shared__ int ticket;
     const int tid = threadIdx.x;
     int* counter = A.flags + A.ticket;
-    const int total = A.nbundles * A.ngroups;
-    if (tid == 0) ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    int k = __builtin_amdgcn_readfirstlane(ticket);
-    while (k < total) {
-        const SolveBundle bd = ld_scalar(A.bundles + A.bundle0 + k / A.ngroups);
-        const int grp = k % A.ngroups;
-        for (int i = bd.first; i < bd.first + bd.count; ++i) {
-            const SolveTask t = ld_scalar(A.tasks + i);
+    // a ticket: the next `per` turns (turn k: task k / ngroups for group k %
+    // ngroups); per is the last task's, 1 where a level's tasks are few
+    int per = 1, k0 = 0;
+    for (;;) {
+        if (tid == 0) ticket = __hip_atomic_fetch_add(counter, per, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        k0 = __builtin_amdgcn_readfirstlane(ticket);
+        const int k1 = min(k0 + per, A.ntasks * A.ngroups);
+        if (k0 >= k1) return;
+        SolveTask next = ld_scalar(A.tasks + A.task0 + k0 / A.ngroups);
+        for (int k = k0; k < k1; ++k) {
+            const SolveTask t = next;
+            const int grp = k % A.ngroups;
+            per = t.per;
+            if (k + 1 < k1) next = ld_scalar(A.tasks + A.task0 + (k + 1) / A.ngroups);
             // hidden from the compiler, which would otherwise compute every
             // kind's lane offsets once, before the loop, and spill them
             int lid = tid;
@@ -757,11 +859,8 @@ template <typename T> __global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 3 
             case kBwdTop: bwd_top(C, t); break;
             default: bwd_piv(C, t); break;
             }
+            // (each ends with a barrier after its last use of S and ticket)
         }
-        // every task ends with a barrier after its last use of S and ticket
-        if (tid == 0) ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        k = __builtin_amdgcn_readfirstlane(ticket);
     }
 }
 
@@ -779,7 +878,7 @@ void launch_solve_reset(int* flags, int64_t n, hipStream_t st)
 // As many workgroups as the chip holds (four per CU); fewer tickets, fewer.
 template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st)
 {
-    const int64_t total = (int64_t)A.nbundles * A.ngroups;
+    const int64_t total = (int64_t)A.ntasks * A.ngroups;
     if (total > 0)
         hipLaunchKernelGGL(k_solve<T>, dim3((unsigned)std::min<int64_t>(total, 1024)), dim3(kThreads), 0, st, A);
 }

@@ -19,16 +19,17 @@ namespace {
 
 // A front of one superblock whose update rows its own workgroup takes as
 // well (no hand-over to other workgroups): with at most kWholeRows of them,
-// where a hand-over (about 3 us) costs more than the rows do; or on a level
-// of at least kManyFronts fronts, which fill the chip by themselves.
-constexpr int kWholeRows = 128;
+// where a hand-over (about 3 us) costs more than the rows do; on a level of
+// at least kManyFronts fronts, which fill the chip by themselves, at most
+// kWholeMany.
+constexpr int kWholeRows = 128, kWholeMany = 256;
 constexpr int kManyFronts = 512;
 // Rows per forward task: 16, four waves a quarter of the columns each, until
 // a level has more than kManyRows tasks of them; then 64.
 constexpr int kManyRows = 2048;
-// A level's tasks of one phase beyond kBundleFrom share tickets, at most
-// kBundleMost of them each (one counter hands out about 100 tickets per us).
-constexpr int kBundleFrom = 4096, kBundleMost = 8;
+// A level's tasks of one phase beyond kManyTasks are taken several to a
+// ticket, at most kTicketMost (every ticket is an addition to one counter).
+constexpr int kManyTasks = 4096, kTicketMost = 8;
 constexpr int kFlagLine = 32;  // super fronts keep their counters a cache line apart: many workgroups poll each
 
 }  // namespace
@@ -79,7 +80,7 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
         const bool many = level_ptr[L + 1] - level_ptr[L] >= kManyFronts;
         for (int k = level_ptr[L]; k < level_ptr[L + 1]; ++k) {
             const int s = level_nodes[k];
-            whole[s] = !super(s) && nsup(s) == 1 && nodes[s].w > 0 && (many || nodes[s].w <= kWholeRows);
+            whole[s] = !super(s) && nsup(s) == 1 && nodes[s].w > 0 && nodes[s].w <= (many ? kWholeMany : kWholeRows);
         }
     }
 
@@ -103,10 +104,9 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
             base[s] = P.plane;
             P.plane += std::max(rows[s], slots[s]);
         }
-    // gather lists, children in child order
     int64_t glen = 0, grows = (int64_t)S.l_rows.size();
     for (int s = 0; s < m; ++s)
-        if (!S.children[s].empty()) glen += nodes[s].n + 1;
+        if (!S.children[s].empty()) glen += nodes[s].n;
     // counters
     std::vector<int> flag(m), fstr(m);
     int64_t nflags = 0;
@@ -120,27 +120,42 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     P.nflags = (int)nflags;
     P.grow.resize(grows);
     for (int64_t k = 0; k < grows; ++k) P.grow[k] = S.l_rows[k] - 1;
+    // gather tables, children in child order
     std::vector<int> goff(m, -1);
-    P.gptr.reserve(glen);
-    P.gsrc.reserve(grows);
-    std::vector<int> pos;
+    P.gat.reserve(glen);
+    std::vector<int> more;
     for (int s = 0; s < m; ++s) {
         if (S.children[s].empty()) continue;
-        goff[s] = (int)P.gptr.size();
+        goff[s] = (int)P.gat.size();
         const int n = nodes[s].n;
-        pos.assign(n + 1, 0);
-        for (int ch : S.children[s])
-            for (int k = 0; k < nodes[ch - 1].w; ++k) pos[S.lidx[nodes[ch - 1].lidx + k]]++;
-        const int g0 = (int)P.gsrc.size();
-        pos[0] = g0;
-        for (int i = 0; i < n; ++i) pos[i + 1] += pos[i];
-        P.gptr.insert(P.gptr.end(), pos.begin(), pos.end());
-        P.gsrc.resize(pos[n]);
-        for (int ch : S.children[s]) {
-            const NodeDev& d = nodes[ch - 1];
-            for (int k = 0; k < d.w; ++k)
-                P.gsrc[pos[S.lidx[d.lidx + k] - 1]++] = (int)(base[root[s]] + z[ch - 1] + d.c + k);
-        }
+        P.gat.resize(P.gat.size() + n, SolvePlan::Gather{-1, -1});
+        SolvePlan::Gather* g = P.gat.data() + goff[s];
+        auto each = [&](auto&& f) {
+            for (int ch : S.children[s]) {
+                const NodeDev& d = nodes[ch - 1];
+                for (int k = 0; k < d.w; ++k)
+                    f(S.lidx[d.lidx + k] - 1, (int)(base[root[s]] + z[ch - 1] + d.c + k));
+            }
+        };
+        more.assign(n, 0);
+        int most = 0;
+        each([&](int i, int at) {
+            most = std::max(most, ++more[i]);
+            (more[i] == 1 ? g[i].s0 : g[i].s1) = at;  // a third and later ones replace it below
+        });
+        if (most <= 2) continue;
+        for (int i = 0; i < n; ++i)
+            if (more[i] > 2) {
+                g[i].s1 = -2 - (int)P.gsrc.size();
+                P.gsrc.resize(P.gsrc.size() + more[i], 0);
+            }
+        more.assign(n, 0);
+        each([&](int i, int at) {
+            if (++more[i] >= 2 && g[i].s1 < -1) {
+                int* list = &P.gsrc[-2 - g[i].s1];
+                list[++list[0]] = at;
+            }
+        });
     }
 
     // counter of front s: kind q (0 z, 1 y, 2 p, 3 t, 4 x) of superblock u
@@ -174,11 +189,10 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
         t.w0t = target;
     };
     size_t seg = 0;
-    auto close = [&]() {  // the tasks since the last call become tickets
+    auto close = [&]() {  // ends a phase of a level
         const int cnt = (int)(P.tasks.size() - seg);
-        const int per = cnt > kBundleFrom ? std::min(kBundleMost, cnt / (kBundleFrom / 2)) : 1;
-        for (int i = 0; i < cnt; i += per) P.bundles.push_back(SolveBundle{(int)seg + i, std::min(per, cnt - i)});
-        seg = P.tasks.size();
+        const int per = cnt > kManyTasks ? std::min(kTicketMost, cnt / (kManyTasks / 2)) : 1;
+        for (; seg < P.tasks.size(); ++seg) P.tasks[seg].per = per;
     };
 
     for (int L = 0; L < levels; ++L) {
@@ -240,7 +254,7 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
         }
         close();
     }
-    P.fwd_bundles = (int)P.bundles.size();
+    P.fwd_tasks = (int)P.tasks.size();
     for (int L = levels - 1; L >= 0; --L) {
         const int b0 = level_ptr[L], b1 = level_ptr[L + 1];
         int steps = 0;
@@ -248,12 +262,12 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
             const int s = level_nodes[k], pa = nodes[s].parent;
             steps = std::max(steps, nsup(s));
             if (whole[s] || nodes[s].w == 0) continue;
-            for (int c0 = 0; c0 < nodes[s].c; c0 += 64)
+            for (int c0 = 0; c0 < nodes[s].c; c0 += 32)
                 for (int q = 0; q < chunks(s); ++q) {
                     SolveTask t = task(s, kBwdPart, c0 / kSuper);
                     t.r0 = nodes[s].c + kSuper * q;
                     t.nr = std::min(kSuper, nodes[s].n - t.r0);
-                    t.slot = (int)(base[root[s]] + slot0[s]) + 64 * (c0 / 64 * chunks(s) + q);
+                    t.slot = (int)(base[root[s]] + slot0[s]) + 64 * (c0 / 64 * chunks(s) + q) + c0 % 64;
                     t.nslot = c0;
                     t.sig = counter(s, 2, c0 / kSuper);
                     if (pa >= 0) wait(t, counter(pa, 4, 0), yx_target(pa, 0));
@@ -271,7 +285,7 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
                 // rows, its own forward tasks
                 auto wait_y = [&](SolveTask& t) {
                     if (nslot > 0)
-                        wait(t, counter(s, 2, u), (w + 63) / 64 * nslot);
+                        wait(t, counter(s, 2, u), (w + 31) / 32 * nslot);
                     else
                         wait(t, counter(s, 1, u), yx_target(s, u));
                     t.nslot = nslot;
@@ -303,6 +317,7 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
             close();
         }
     }
+    if (P.tasks.size() > (size_t)INT_MAX) return MFD_ERR_NOMEM;
     return MFD_OK;
 }
 
@@ -318,13 +333,8 @@ int64_t check_solve_plan(const SolvePlan& P, std::string& report)
         if (t.kind != kFwdTop && t.kind != kBwdTop && t.kind != kBwdPiv && t.sig >= 0) f[t.sig]++;
     };
     for (const SolveTask& t : P.tasks) raise(t, total);
-    int64_t bad = 0, next = 0;
+    int64_t bad = 0;
     char line[160];
-    for (const SolveBundle& b : P.bundles) {
-        if (b.first != next || b.count < 1) ++bad;
-        next = b.first + b.count;
-    }
-    if (next != (int64_t)P.tasks.size()) ++bad;
     for (size_t i = 0; i < P.tasks.size(); ++i) {
         const SolveTask& t = P.tasks[i];
         auto need = [&](int f, int want) {

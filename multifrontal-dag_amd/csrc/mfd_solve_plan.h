@@ -12,10 +12,16 @@ namespace mfd {
 
 struct SolvePlan {
     std::vector<SolveTask> tasks;
-    std::vector<SolveBundle> bundles;  // tickets, in task order
-    int fwd_bundles = 0;               // those of the forward sweep (the first ones)
-    std::vector<int> gptr, gsrc;       // gather lists: children's update rows that add into each front row
-    std::vector<int> grow;             // global row (0-based) of every update row
+    int fwd_tasks = 0;          // those of the forward sweep (the first ones)
+    // children's update rows that add into each front row: plane positions
+    // of the first and the second (-1: none), or -2 - k: the second and the
+    // others at gsrc[k] (their number, then their positions)
+    struct Gather {
+        int s0, s1;
+    };
+    std::vector<Gather> gat;
+    std::vector<int> gsrc;
+    std::vector<int> grow;  // global row (0-based) of every update row
     // blocks of the superblock matrices: X by block distance i - j
     // ([xinv_ptr[d], xinv_ptr[d + 1]), d = 0..3), then W and V
     // ([xinv_ptr[4], xinv_ptr[5]))
