@@ -79,9 +79,11 @@ void launch_solve_reset(int* flags, int64_t n, hipStream_t st);
 template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st);
 void launch_set_int(int* p, int v, hipStream_t st);
 void launch_residual(double* r, const double* b, const double* x, int n, int nrhs, const int* ptr, const int* col,
-                     const double* val, hipStream_t st);
-// val[e] = a[src[e]] for e < nnz (the matrix values in CSR order).
-void launch_gather_vals(double* val, const double* a, const int64_t* src, int64_t nnz, hipStream_t st);
+                     const double* val, int64_t nnz, hipStream_t st);
+// val[e] = a[src[e]] (the matrix values in CSR order) and the infinity norm
+// of A into out[0] (zeroed by the caller).
+void launch_gather_vals(unsigned long long* out, double* val, const double* a, const int64_t* src, int n,
+                        const int* ptr, int64_t nnz, hipStream_t st);
 // Partials per column of the sums of squares in launch_err_norms:
 // sumsq_parts(n) <= kSumParts.
 constexpr int kSumParts = 256;
@@ -92,7 +94,6 @@ int sumsq_parts(int64_t n);
 // sumsq_parts(n) nrhs), in one pass.
 void launch_err_norms(unsigned long long* out, double* part, const double* r, const double* x, const double* b,
                       const double* d, int64_t n, int nrhs, hipStream_t st);
-void launch_norm_inf(unsigned long long* out, int n, const int* ptr, const double* val, hipStream_t st);
 void launch_axpy(double* x, const double* d, int64_t n, hipStream_t st);
 void launch_zero_u64(unsigned long long* p, int n, hipStream_t st);
 void launch_gather_rows(double* out, int ld_out, const double* in, int ld_in, const int* perm, int n, int nrhs,

@@ -1444,16 +1444,21 @@ __global__ __launch_bounds__(kThreads) void k_scatter_rows(double* out, int ld_o
 // ------------------------------------------------------ FP64 refinement
 // r = b - A x over the full symmetric matrix in CSR order (val: the values
 // in that order, gathered once per factorization), four right-hand sides per
-// pass over a row; each sum runs over the row's entries in order.
+// pass over a row.  G lanes take a row's entries G apart, so that a wave reads
+// consecutive entries of 64 / G rows, and their sums are added pairwise (a
+// fixed order).  What bounds it is the entries' 12 bytes each, once from
+// memory: one lane per row read every line of them 64 / G times over and
+// took 506 us on the 40^3 three-unknown stencil (15.0M entries).
+template <int G>
 __global__ __launch_bounds__(kThreads) void k_residual(double* r, const double* b, const double* x, int n, int nrhs,
                                                        const int* ptr, const int* col, const double* val)
 {
-    const int row = blockIdx.x * kThreads + threadIdx.x;
-    if (row >= n) return;
-    const int e0 = ptr[row], e1 = ptr[row + 1];
+    const int row = blockIdx.x * (kThreads / G) + (int)threadIdx.x / G, g = threadIdx.x % G;
+    const int at = min(row, n - 1);  // lanes past the last row repeat it and store nothing
+    const int e0 = ptr[at], e1 = ptr[at + 1];
     for (int k0 = 0; k0 < nrhs; k0 += 4) {
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int e = e0; e < e1; ++e) {
+        for (int e = e0 + g; e < e1; e += G) {
             const double v = val[e];
             const double* xc = x + col[e] + (int64_t)k0 * n;
 #pragma unroll
@@ -1461,16 +1466,13 @@ __global__ __launch_bounds__(kThreads) void k_residual(double* r, const double* 
                 if (k0 + q < nrhs) acc[q] += v * xc[(int64_t)q * n];
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (k0 + q < nrhs) r[row + (int64_t)(k0 + q) * n] = b[row + (int64_t)(k0 + q) * n] - acc[q];
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+            for (int off = G / 2; off > 0; off >>= 1) acc[q] += __shfl_xor(acc[q], off);
+            if (g == 0 && row < n && k0 + q < nrhs)
+                r[row + (int64_t)(k0 + q) * n] = b[row + (int64_t)(k0 + q) * n] - acc[q];
+        }
     }
-}
-
-// val[e] = a[src[e]]: the caller's values in CSR order
-__global__ __launch_bounds__(kThreads) void k_gather_vals(double* val, const double* a, const int64_t* src, int64_t nnz)
-{
-    const int64_t e = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (e < nnz) val[e] = a[src[e]];
 }
 
 // Maximum over the workgroup, then one atomic per workgroup (as IEEE bits:
@@ -1535,14 +1537,26 @@ __global__ __launch_bounds__(kThreads) void k_err_norms(unsigned long long* out,
     }
 }
 
-// out[0] = max over rows of sum_e |val[e]|  (the infinity norm of A)
-__global__ __launch_bounds__(kThreads) void k_norm_inf(unsigned long long* out, int n, const int* ptr,
-                                                       const double* val)
+// val[e] = a[src[e]], the caller's values in CSR order, and out[0] = max over
+// rows of sum_e |val[e]|, the infinity norm of A (zeroed by the caller), in
+// one pass over the entries, G lanes per row as in k_residual (apart, and one
+// lane per row for the norm, they took 82 and 78 us on the 40^3 three-unknown
+// stencil).
+template <int G>
+__global__ __launch_bounds__(kThreads) void k_gather_vals(unsigned long long* out, double* val, const double* a,
+                                                          const int64_t* src, int n, const int* ptr)
 {
+    const int g = threadIdx.x % G;
     double m = 0.0;
-    for (int row = blockIdx.x * kThreads + threadIdx.x; row < n; row += gridDim.x * kThreads) {
+    for (int row = blockIdx.x * (kThreads / G) + (int)threadIdx.x / G; row < n; row += gridDim.x * (kThreads / G)) {
         double s = 0.0;
-        for (int e = ptr[row]; e < ptr[row + 1]; ++e) s += fabs(val[e]);
+        for (int e = ptr[row] + g; e < ptr[row + 1]; e += G) {
+            const double v = a[src[e]];
+            val[e] = v;
+            s += fabs(v);
+        }
+#pragma unroll
+        for (int off = G / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
         m = fmax(m, s);
     }
     block_max_to(out, m);
@@ -1559,18 +1573,40 @@ __global__ void k_zero_u64(unsigned long long* p, int n)
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0ull;
 }
 
-void launch_residual(double* r, const double* b, const double* x, int n, int nrhs, const int* ptr, const int* col,
-                     const double* val, hipStream_t st)
+// Lanes per row of the CSR kernels: about a third of a row's entries, so that
+// few lanes idle on the last ones (4 for the 7-point grids, 8 and 32 for the
+// 27-point ones with one and three unknowns).
+static int row_lanes(int n, int64_t nnz)
 {
-    if (n > 0)
-        hipLaunchKernelGGL(k_residual, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, r, b, x, n, nrhs, ptr,
-                           col, val);
+    const int64_t per = nnz / n;
+    return per <= 12 ? 4 : per <= 40 ? 8 : 32;
 }
-void launch_gather_vals(double* val, const double* a, const int64_t* src, int64_t nnz, hipStream_t st)
+void launch_residual(double* r, const double* b, const double* x, int n, int nrhs, const int* ptr, const int* col,
+                     const double* val, int64_t nnz, hipStream_t st)
 {
-    if (nnz > 0)
-        hipLaunchKernelGGL(k_gather_vals, dim3((unsigned)((nnz + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, val, a,
-                           src, nnz);
+    if (n <= 0) return;
+    const int g = row_lanes(n, nnz);
+    const dim3 grid((unsigned)(((int64_t)n * g + kThreads - 1) / kThreads)), block(kThreads);
+    if (g == 4)
+        hipLaunchKernelGGL(k_residual<4>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
+    else if (g == 8)
+        hipLaunchKernelGGL(k_residual<8>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
+    else
+        hipLaunchKernelGGL(k_residual<32>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
+}
+// (at most 2048 workgroups, each one atomic on the norm)
+void launch_gather_vals(unsigned long long* out, double* val, const double* a, const int64_t* src, int n,
+                        const int* ptr, int64_t nnz, hipStream_t st)
+{
+    if (n <= 0) return;
+    const int g = row_lanes(n, nnz);
+    const dim3 grid((unsigned)std::min<int64_t>(((int64_t)n * g + kThreads - 1) / kThreads, 2048)), block(kThreads);
+    if (g == 4)
+        hipLaunchKernelGGL(k_gather_vals<4>, grid, block, 0, st, out, val, a, src, n, ptr);
+    else if (g == 8)
+        hipLaunchKernelGGL(k_gather_vals<8>, grid, block, 0, st, out, val, a, src, n, ptr);
+    else
+        hipLaunchKernelGGL(k_gather_vals<32>, grid, block, 0, st, out, val, a, src, n, ptr);
 }
 // at least 8 entries per thread: few workgroups per column, so few atomics
 // on each maximum and a short read-back of the partial sums
@@ -1580,11 +1616,6 @@ void launch_err_norms(unsigned long long* out, double* part, const double* r, co
 {
     if (n > 0)
         hipLaunchKernelGGL(k_err_norms, dim3(sumsq_parts(n), nrhs), dim3(kThreads), 0, st, out, part, r, x, b, d, n, nrhs);
-}
-void launch_norm_inf(unsigned long long* out, int n, const int* ptr, const double* val, hipStream_t st)
-{
-    const int g = std::min((n + kThreads - 1) / kThreads, 4096);
-    if (n > 0) hipLaunchKernelGGL(k_norm_inf, dim3(g), dim3(kThreads), 0, st, out, n, ptr, val);
 }
 void launch_axpy(double* x, const double* d, int64_t n, hipStream_t st)
 {

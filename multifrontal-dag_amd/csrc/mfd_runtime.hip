@@ -1288,11 +1288,11 @@ int backward_error(mfd_handle* h, const double* bp, const double* xp, double* r,
     // the values in CSR order and ||A||_inf once per factorization (the
     // values do not change in between)
     const bool anorm_known = h->anorm >= 0;
-    if (!anorm_known) launch_gather_vals(h->d_csr_val, h->d_a, h->d_csr_src, h->csr_nnz, st);
-    launch_residual(r, bp, xp, n, nrhs, h->d_csr_ptr, h->d_csr_col, h->d_csr_val, st);
     launch_zero_u64(h->d_norms, nm, st);
+    if (!anorm_known)
+        launch_gather_vals(h->d_norms + 4 * nrhs, h->d_csr_val, h->d_a, h->d_csr_src, n, h->d_csr_ptr, h->csr_nnz, st);
+    launch_residual(r, bp, xp, n, nrhs, h->d_csr_ptr, h->d_csr_col, h->d_csr_val, h->csr_nnz, st);
     launch_err_norms(h->d_norms, sq, r, xp, bp, d, n, nrhs, st);
-    if (!anorm_known) launch_norm_inf(h->d_norms + 4 * nrhs, n, h->d_csr_ptr, h->d_csr_val, st);
     std::vector<unsigned long long> v(nm + 2 * parts * nrhs);
     HIP_TRY(hipMemcpyAsync(v.data(), h->d_norms, v.size() * 8, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
