@@ -72,7 +72,7 @@ typedef struct mfd_handle mfd_handle;
 /* kernel classes reported by mfd_get_kernel_time */
 #define MFD_K_ASSEMBLE 0
 #define MFD_K_EXTEND_ADD 1  /* extend-add of small children (n <= 64) */
-#define MFD_K_SMALL_FRONT 2
+#define MFD_K_SMALL_FRONT 2 /* the bottom of the tree (fronts of order <= 128, in one launch, assembly included) and other fronts of order <= 64 */
 #define MFD_K_POTRF 3       /* per panel step: next diagonal block (its panel updates, Cholesky, inverse), panel TRSM tiles, small updates */
 #define MFD_K_TRSM 4        /* a step's GEMM tiles (panel TRSM, small updates) launched apart from its diagonal tasks (levels with many fronts) */
 #define MFD_K_UPDATE 5      /* in-panel trailing update (GEMM/SYRK, K = panel width) */
@@ -290,9 +290,11 @@ int mfd_get_update_period(mfd_handle* h);
    turn; many such fronts of one level run side by side).
    mfd_set_front_split: fronts with at most cmax pivot columns are medium
    (0, the default: none).  mfd_set_front_kinds: one choice per node
-   (num_node entries, 1-based node order: 1 medium, 0 large, -1 by cmax;
-   NULL clears); fronts of order <= 64 are always factored whole in LDS.
-   Both rebuild the schedule of the current analysis like
+   (num_node entries, 1-based node order: 1 medium, 0 not, -1 by cmax; NULL
+   clears).  A front of order <= 128 whose descendants are all such fronts,
+   none of them chosen medium, is neither: one launch factors the whole
+   bottom of the tree, one workgroup per front (MFD_K_SMALL_FRONT); other
+   fronts of order <= 64 are factored whole in LDS.  Both rebuild the schedule of the current analysis like
    mfd_set_update_period.  mfd_get_front_times: per node, the duration in
    microseconds of its workgroup in the last factorization (in-kernel
    clocks), -1 for fronts that are not medium. */

@@ -74,6 +74,23 @@ template <typename T> struct SolveArgs {
     int64_t zs;
     int n, nrhs, ngroups, nflags, task0, ntasks, ticket;
 };
+// The bottom of the tree (mfd_tree.hip).  a: caller values; entry e of A is
+// a[asrc[e]] at row (apos[e] & 255), panel column (apos[e] >> 8); scale (may
+// be null): the 16-bit forms' diagonal scaling, (row, column) = arc[e].  flags
+// as for the solves, one counter per front; err likewise.
+template <typename T> struct TreeArgs {
+    T* pool;
+    const double* a;
+    const int *apos, *asrc, *aptr;
+    const int2* arc;
+    const double* scale;
+    const int* lidx;
+    const TreeTask* tasks;
+    const TreeChild* children;
+    int *flags, *err, *info;
+    int ntasks;
+};
+template <typename T> void launch_tree(const TreeArgs<T>& A, hipStream_t st);
 constexpr int kRhsGroup = 16;
 void launch_solve_reset(int* flags, int64_t n, hipStream_t st);
 template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st);

@@ -19,33 +19,12 @@
 // The solves are in mfd_solve.hip.
 #include <hip/hip_runtime.h>
 
+#include "mfd_device.h"
 #include "mfd_kernels.h"
 
 namespace mfd {
 
 namespace {
-
-constexpr int kThreads = 256;
-
-// ------------------------------------------------------------ MFMA traits
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-// D(16x16) += A(16x4) B(4x16); lane l supplies A[l%16][l/16] and
-// B[l/16][l%16].  The accumulator layouts differ (measured on gfx950):
-//   f64: element v of lane l is D[l/16 + 4v][l%16]
-//   f32: element v of lane l is D[4(l/16) + v][l%16]
-template <typename T> struct Mfma;
-template <> struct Mfma<double> {
-    typedef d4 acc_t;
-    static __device__ acc_t mma(double a, double b, acc_t c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-    static __device__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
-};
-template <> struct Mfma<float> {
-    typedef f4 acc_t;
-    static __device__ acc_t mma(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-    static __device__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
-};
 
 // 16-bit operands with FP32 accumulation (the FP16_IR / BF16_IR forms):
 // D(16x16) += A(16x16) B(16x16); lane l supplies A[l%16][4(l/16) + i] and
@@ -73,68 +52,6 @@ template <> struct Mfma16<kBF16> {
 };
 
 
-// 1 / sqrt(d): the hardware estimate (v_rsq) refined by Newton-Raphson
-// steps r <- r + (r / 2) (1 - d r^2), each squaring the relative error (two
-// for double, one for float): within a few ulp of the exact value, with a
-// dependent chain of seven steps where a correctly rounded sqrt and
-// division take about twenty.
-__device__ __forceinline__ double rsqrt_nr(double d)
-{
-    double r = __builtin_amdgcn_rsq(d);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const double e = fma(-(d * r), r, 1.0);
-        r = fma(0.5 * r, e, r);
-    }
-    return r;
-}
-__device__ __forceinline__ float rsqrt_nr(float d)
-{
-    const float r = __builtin_amdgcn_rsqf(d);
-    const float e = fmaf(-(d * r), r, 1.0f);
-    return fmaf(0.5f * r, e, r);
-}
-// a / b given rb ~ 1 / b (within a few ulp): q = a rb, then one correction
-// with the exact residual a - q b (Markstein), which returns a / b exactly
-// whenever it is representable and is within an ulp of it otherwise.  Its
-// chain is a multiply and two fmas after rb and b, against the ten
-// dependent steps of a correctly rounded division.
-template <typename T> __device__ __forceinline__ T quot(T a, T b, T rb)
-{
-    const T q = a * rb;
-    return fma(fma(-q, b, a), rb, q);
-}
-
-// p[i] for a uniform base p and a 32-bit unsigned index: the address is
-// base + zero-extended byte offset, which keeps one VGPR per address when
-// many loads are in flight.
-template <typename T> __device__ __forceinline__ T ld_off(const T* p, unsigned i)
-{
-    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (size_t)(i * (unsigned)sizeof(T)));
-}
-
-// Value of v in lane src (uniform src; only its low 6 bits select the lane).
-__device__ __forceinline__ double bcast(double v, int src)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, src);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ float bcast(float v, int src)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
-}
-
-// Orders one wave's LDS accesses (they complete in issue order within a
-// wave) against compiler reordering; no workgroup barrier is involved.
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ------------------------------------------- dense 64 x 64 partial Cholesky
 // A front (or diagonal block) of order n <= 64 in LDS, factored in its first
 // c columns by a blocked right-looking algorithm with 16-column panels:
@@ -159,16 +76,6 @@ template <typename T> struct Front64 {
     T Ts[4][16][17];
     T rs[64];
 };
-
-// sqrt(d) from r ~ 1/sqrt(d) (within a few ulp): s = d r and one Newton
-// step s + (d - s^2) r / 2 with the exact residual (fma); exact whenever
-// sqrt(d) is representable, within an ulp otherwise, in three dependent
-// operations after r.
-template <typename T> __device__ __forceinline__ T sqrt_from_rs(T d, T r)
-{
-    const T s = d * r;
-    return fma(fma(-s, s, d), T(0.5) * r, s);
-}
 
 // Panel b16 .. b16 + cb - 1 (cb <= 16; FULL: cb == 16) by one wave, rows
 // b16 .. 63 on their lanes.  Column k: d = x_k on lane k, L_kk = sqrt(d),

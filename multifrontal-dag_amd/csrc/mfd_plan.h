@@ -98,6 +98,25 @@ struct SuperInvTask {
     int64_t xoff;
 };
 
+// A front of order <= kTreeFront all of whose children are such fronts
+// (mfd_tree.hip): child .. child + nchild its children, aptr the panels'
+// ranges of its entries of A, flag its counter of finished children, sig the
+// parent's (-1: none, or the parent is no such front), per the turns the next
+// ticket of the workgroup takes.
+constexpr int kTreeFront = 128;
+struct TreeTask {
+    int64_t front, inv;  // element offsets in the pool
+    int n, c, first;     // first: 0-based first global column
+    int child, nchild, aptr;
+    int flag, sig;
+    int per, pad;
+};
+struct TreeChild {
+    int64_t u;  // element offset of the child's update matrix
+    int ld, w;
+    int lidx, pad;
+};
+
 // mode 0: C (m x n tile, ldc) -= A (m x k, lda) * B (n x k, ldb)^T;
 // mode 1: C = A B^T with B stored transposed (B[j][k] at b + j * ldb + k);
 // A may be C itself: the panel TRSM X = P L^{-T}, with b the stored L^{-T}

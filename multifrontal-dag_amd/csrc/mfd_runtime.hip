@@ -30,6 +30,7 @@
 #include "mfd_kernels.h"
 #include "mfd_layout.h"
 #include "mfd_solve_plan.h"
+#include "mfd_tree_plan.h"
 #include "mfdag.h"
 
 using namespace mfd;
@@ -186,6 +187,13 @@ struct mfd_handle {
     std::vector<GemmTask> gemm;
     std::vector<Launch> fseq;
     std::vector<int> level_ptr, level_nodes, child_ptr, child_list;
+    // the fronts factored in one launch at the bottom of the tree
+    // (mfd_tree_plan.h) and its device copies
+    TreePlan tp;
+    TreeTask* d_ttasks = nullptr;
+    TreeChild* d_tchildren = nullptr;
+    int *d_tapos = nullptr, *d_tasrc = nullptr, *d_taptr = nullptr, *d_tflags = nullptr;
+    TreePlan::RowCol* d_tarc = nullptr;
     // the solves: task list (mfd_solve_plan.h) and its device copies
     SolvePlan sp;
     SolveTask* d_stasks = nullptr;
@@ -193,7 +201,7 @@ struct mfd_handle {
     int *d_gsrc = nullptr, *d_grow = nullptr;
     SuperInvTask* d_xinv = nullptr;
     int solve_rc = 0;          // build_solve_plan's result for the current schedule
-    int* solve_err = nullptr;  // pinned: set by a solve whose wait reached its bound
+    int* wait_err = nullptr;   // pinned: set by a launch of which a wait reached its bound
     double* d_sinv64 = nullptr;
     float* d_sinv32 = nullptr;
     int64_t pool_elems = 0;
@@ -343,6 +351,10 @@ void free_device(mfd_handle* h)
     h->d_fill = nullptr;
     h->d_gemm = nullptr;
     h->d_level_nodes = h->d_child_ptr = h->d_child_list = nullptr;
+    h->d_ttasks = nullptr;
+    h->d_tchildren = nullptr;
+    h->d_tapos = h->d_tasrc = h->d_taptr = h->d_tflags = nullptr;
+    h->d_tarc = nullptr;
     h->d_stasks = nullptr;
     h->d_gat = nullptr;
     h->d_gsrc = h->d_grow = nullptr;
@@ -406,6 +418,19 @@ void build_plan(mfd_handle* h)
     h->host_rc = h->host_roots.empty() ? MFD_OK : build_host_plan(S, h->nodes, h->host_roots, h->hplan);
     if (h->host_rc != MFD_OK) h->hplan = HostPlan{};
     auto on_host = [&](int s) { return !h->hplan.is_host.empty() && h->hplan.is_host[s]; };
+    // medium fronts by choice (mfd_set_front_kinds, mfd_set_front_split)
+    auto chosen_kind = [&](int s) {
+        const int k = (int)h->front_kind.size() == m ? h->front_kind[s] : -1;
+        return k >= 0 ? k : (int)(h->nodes[s].c <= h->fuse_cmax);
+    };
+    // the bottom of the tree in one launch: fronts of order <= 64, and larger
+    // ones unless they were chosen to be medium
+    {
+        std::vector<char> eligible(m, 0);
+        for (int s = 0; s < m; ++s)
+            eligible[s] = !on_host(s) && (h->nodes[s].n <= kSmallFront || chosen_kind(s) != 1);
+        build_tree_plan(S, h->nodes, eligible, h->tp);
+    }
 
     // Levels.  Rule 1 (the default): a front sits one level below its
     // parent (roots on the top level), so siblings share a level and their
@@ -449,7 +474,7 @@ void build_plan(mfd_handle* h)
         h->fill_gptr.assign(1, 0);
         for (int g = 0; g < G; ++g) {
             for (int s2 = 0; s2 < m; ++s2)
-                if (group[s2] == g && !on_host(s2))
+                if (group[s2] == g && !on_host(s2) && !h->tp.has(s2))
                     for (int j0 = 0; j0 < h->nodes[s2].n; j0 += 64) h->fill.push_back(make_int2(s2, j0));
             h->fill_gptr.push_back((int)h->fill.size());
         }
@@ -472,7 +497,7 @@ void build_plan(mfd_handle* h)
     h->fused_pos.assign(m, -1);
     // front classes: small (n <= 64, whole in LDS), medium (one workgroup
     // per front), large (64-column steps over the chip)
-    enum { kClsSmall = 0, kClsMedium = 1, kClsLarge = 2, kClsHost = 3 };
+    enum { kClsSmall = 0, kClsMedium = 1, kClsLarge = 2, kClsHost = 3, kClsTree = 4 };
     std::vector<int> cls(m, kClsLarge);
     for (int s = 0; s < m; ++s) {
         const NodeDev& d = h->nodes[s];
@@ -480,13 +505,15 @@ void build_plan(mfd_handle* h)
             cls[s] = kClsHost;
             continue;
         }
+        if (h->tp.has(s)) {
+            cls[s] = kClsTree;
+            continue;
+        }
         if (d.n <= kSmallFront) {
             cls[s] = kClsSmall;
             continue;
         }
-        const int k = (int)h->front_kind.size() == m ? h->front_kind[s] : -1;
-        const bool medium = k >= 0 ? k == 1 : d.c <= h->fuse_cmax;
-        cls[s] = medium ? kClsMedium : kClsLarge;
+        cls[s] = chosen_kind(s) == 1 ? kClsMedium : kClsLarge;
     }
     h->diag.clear();
     h->gemm.clear();
@@ -557,7 +584,7 @@ void build_plan(mfd_handle* h)
             int64_t first = (int64_t)h->ext.size();
             for (int k = 0; k < cnt; ++k) {
                 const auto& chs = S.children[lv[k]];
-                if (chs.size() <= r || cls[lv[k]] == kClsHost) continue;
+                if (chs.size() <= r || cls[lv[k]] == kClsHost || cls[lv[k]] == kClsTree) continue;
                 int ch = chs[r] - 1, nt = (S.w[ch] + kTile - 1) / kTile;
                 if (cls[ch] == kClsLarge) continue;
                 for (int ti = 0; ti < nt; ++ti)
@@ -835,6 +862,13 @@ int setup_device(mfd_handle* h)
     MFD_TRY(upload(h, &h->d_level_nodes, h->level_nodes));
     MFD_TRY(upload(h, &h->d_child_ptr, h->child_ptr));
     MFD_TRY(upload(h, &h->d_child_list, h->child_list));
+    MFD_TRY(upload(h, &h->d_ttasks, h->tp.tasks));
+    MFD_TRY(upload(h, &h->d_tchildren, h->tp.children));
+    MFD_TRY(upload(h, &h->d_tapos, h->tp.apos));
+    MFD_TRY(upload(h, &h->d_tasrc, h->tp.asrc));
+    MFD_TRY(upload(h, &h->d_taptr, h->tp.aptr));
+    MFD_TRY(upload(h, &h->d_tarc, h->tp.arc));
+    MFD_TRY(dalloc(h, &h->d_tflags, kSolveCtl + (int64_t)h->tp.tasks.size()));
     MFD_TRY(upload(h, &h->d_stasks, h->sp.tasks));
     MFD_TRY(upload(h, &h->d_grow, h->sp.grow));
     MFD_TRY(upload(h, &h->d_gat, h->sp.gat));
@@ -860,7 +894,7 @@ int setup_device(mfd_handle* h)
                     const int r = S.snidx[p];
                     const int grow = r <= S.c[s] ? S.first[s] + r - 1 : S.l_rows[S.l_ptr[s] + (r - S.c[s] - 1)];
                     if (grow == j) diag_src[j - 1] = S.ccs_perm[p] - 1;
-                    if (host) continue;  // assembled on the host
+                    if (host || h->tp.has(s)) continue;  // assembled on the host, or in its own launch
                     dst[e] = d.front + (S.snidx[p] - 1) + q * d.n;
                     src[e] = S.ccs_perm[p] - 1;
                     rc[e] = make_int2(grow - 1, j - 1);
@@ -870,7 +904,7 @@ int setup_device(mfd_handle* h)
         }
         h->scat_gptr.push_back(e);
     }
-    if (e != nnz - h->hplan.entries) return MFD_ERR_INTERNAL;
+    if (e != nnz - h->hplan.entries - h->tp.entries) return MFD_ERR_INTERNAL;
     dst.resize(e);
     src.resize(e);
     rc.resize(e);
@@ -1000,6 +1034,8 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
         (void)k;
     };
     launch_set_int(h->d_info, INT_MAX, st);
+    const bool tree = !h->tp.tasks.empty();
+    if (tree) launch_solve_reset(h->d_tflags, kSolveCtl + (int64_t)h->tp.tasks.size(), st);
     mark(0);
     // Zeroing and assembly of the fronts: beside the factorization, group by
     // group, when the fill stream and its events exist; otherwise (and when
@@ -1024,6 +1060,28 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
         if (split_fill) ok(hipEventRecord(h->fill_ev[g], fst));
     }
     mark(0);
+    if (tree) {
+        // (in the 16-bit forms behind the fill stream's scaling, which the
+        // first group's event follows)
+        if (scaled && split_fill && G > 0) ok(hipStreamWaitEvent(st, h->fill_ev[0], 0));
+        TreeArgs<T> a{};
+        a.pool = pool;
+        a.a = h->d_a;
+        a.apos = h->d_tapos;
+        a.asrc = h->d_tasrc;
+        a.aptr = h->d_taptr;
+        a.arc = reinterpret_cast<const int2*>(h->d_tarc);
+        a.scale = scaled ? h->d_dscale : nullptr;
+        a.lidx = h->d_lidx;
+        a.tasks = h->d_ttasks;
+        a.children = h->d_tchildren;
+        a.flags = h->d_tflags;
+        a.err = h->wait_err;
+        a.info = h->d_info;
+        a.ntasks = (int)h->tp.tasks.size();
+        launch_tree<T>(a, st);
+        mark(MFD_K_SMALL_FRONT);
+    }
     // Side launches fork from the main stream's current position and run
     // beside it; a step's launches join the side launch they depend on, and
     // any other launch joins every side launch before it.
@@ -1084,6 +1142,16 @@ void collect_profile(mfd_handle* h, const std::vector<int>& kinds)
     h->prof_ev.clear();
 }
 
+// After a synchronization: whether a wait of a launch reached its bound (its
+// task list is broken; never with a plan that check_solve_plan or
+// check_tree_plan passes).
+int wait_status(mfd_handle* h)
+{
+    if (*h->wait_err == 0) return MFD_OK;
+    *h->wait_err = 0;
+    return MFD_ERR_INTERNAL;
+}
+
 template <typename T> int run_factor(mfd_handle* h)
 {
     const bool profile = (h->flags & MFD_FLAG_PROFILE) != 0;
@@ -1128,6 +1196,7 @@ template <typename T> int run_factor(mfd_handle* h)
     HIP_TRY(hipEventSynchronize(h->ev[1]));
     if (profile) {
         std::vector<int> kinds;
+        if (!h->tp.tasks.empty()) kinds.push_back(MFD_K_SMALL_FRONT);
         for (const Launch& l : h->fseq) kinds.push_back(l.kind);
         collect_profile(h, kinds);
     }
@@ -1136,11 +1205,13 @@ template <typename T> int run_factor(mfd_handle* h)
     h->st.factor_ms = ms;
     int info = INT_MAX;
     HIP_TRY(hipMemcpy(&info, h->d_info, sizeof(int), hipMemcpyDeviceToHost));
+    const int waited = wait_status(h);
     if (hybrid) {
         if (h->host_thr.joinable()) h->host_thr.join();
         h->host_factored = true;
         if (h->host_info > 0) info = std::min(info, h->host_info);
     }
+    MFD_TRY(waited);
     return info == INT_MAX ? MFD_OK : info;
 }
 
@@ -1199,7 +1270,7 @@ template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double
     a.grow = h->d_grow;
     a.tasks = h->d_stasks;
     a.flags = h->d_sflags;
-    a.err = h->solve_err;
+    a.err = h->wait_err;
     a.zs = h->sp.plane;
     a.n = h->S.n;
     a.nrhs = nrhs;
@@ -1232,15 +1303,6 @@ template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double
     h->ktime[MFD_K_SOLVE_BWD] += b;
     h->kcount[MFD_K_SOLVE_BWD] += 1;
     for (auto e : pe) (void)hipEventDestroy(e);
-}
-
-// After a synchronization: whether a solve's wait reached its bound (the
-// task list is broken; never with a plan that check_solve_plan passes).
-int solve_status(mfd_handle* h)
-{
-    if (*h->solve_err == 0) return MFD_OK;
-    *h->solve_err = 0;
-    return MFD_ERR_INTERNAL;
 }
 
 // One forward + backward sweep, replayed from a captured graph when graphs
@@ -1296,7 +1358,7 @@ int backward_error(mfd_handle* h, const double* bp, const double* xp, double* r,
     std::vector<unsigned long long> v(nm + 2 * parts * nrhs);
     HIP_TRY(hipMemcpyAsync(v.data(), h->d_norms, v.size() * 8, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    MFD_TRY(solve_status(h));
+    MFD_TRY(wait_status(h));
     auto val = [&](int i) {
         double x;
         memcpy(&x, &v[i], 8);
@@ -1440,7 +1502,7 @@ int solve_host(mfd_handle* h, double* b, int nrhs, int ldb, bool permuted, bool 
     HIP_TRY(hipMemcpy2DAsync(b, (size_t)ldb * 8, h->d_bin, (size_t)n * 8, (size_t)n * 8, nrhs, kout, st));
     HIP_TRY(hipStreamSynchronize(st));
     HIP_TRY(hipGetLastError());
-    MFD_TRY(solve_status(h));
+    MFD_TRY(wait_status(h));
     float ms = 0;
     HIP_TRY(hipEventElapsedTime(&ms, h->ev[2], h->ev[3]));
     h->st.solve_ms = ms;
@@ -1739,7 +1801,30 @@ int64_t check_schedule(mfd_handle* h, int variant, std::string& report)
         fill_node[g] = v;
         C.kind = -1;
         for (int s = 0; s < m; ++s)
-            if (h->front_group[s] == g) C.rect(s, 0, h->nodes[s].n, 0, h->nodes[s].n, v, C.next_task++, true);
+            if (h->front_group[s] == g && !h->tp.has(s))
+                C.rect(s, 0, h->nodes[s].n, 0, h->nodes[s].n, v, C.next_task++, true);
+    }
+    // the bottom of the tree, one node for each height of its fronts: its
+    // tasks wait for their children, which check_tree_plan checks
+    if (!h->tp.tasks.empty()) {
+        C.kind = MFD_K_SMALL_FRONT;
+        std::vector<int> height(m, 0);
+        int last = -1;
+        for (int s : h->tp.node) {
+            for (int ch : h->S.children[s]) height[s] = std::max(height[s], height[ch - 1] + 1);
+            if (height[s] != last) {
+                const int v = C.add_node();
+                C.edge(main_last, v);
+                main_last = v;
+                last = height[s];
+            }
+            const int64_t task = C.next_task++;
+            C.front_all(s, main_last, task);
+            for (int ch : h->S.children[s]) {
+                const NodeDev& d = h->nodes[ch - 1];
+                C.rect(ch - 1, d.c, d.n, d.c, d.n, main_last, task, false);
+            }
+        }
     }
     // variants 1 and 2: per large front, the launch the fourth stream forks
     // after -- the one with its last diagonal task (1), or the last one with
@@ -1905,8 +1990,8 @@ int mfd_create(mfd_handle** out, int nb, int flags)
             h->device_ok = true;
             h->scratch = scratch_on_current_device();  // set-up of mfd_solve_device_noalloc
             for (auto& e : h->ev) (void)hipEventCreate(&e);
-            if (hipHostMalloc((void**)&h->solve_err, sizeof(int), hipHostMallocDefault) == hipSuccess)
-                *h->solve_err = 0;
+            if (hipHostMalloc((void**)&h->wait_err, sizeof(int), hipHostMallocDefault) == hipSuccess)
+                *h->wait_err = 0;
             else
                 h->device_ok = false;
             if (hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking) != hipSuccess) h->side = nullptr;
@@ -1926,7 +2011,7 @@ void mfd_destroy(mfd_handle* h)
     if (h->device_ok) {
         (void)hipStreamSynchronize(h->stream);
         free_device(h);
-        (void)hipHostFree(h->solve_err);
+        (void)hipHostFree(h->wait_err);
         for (auto& b : h->spare) (void)hipFree(b.first);
         h->spare.clear();
         h->device_bytes = 0;
@@ -2047,7 +2132,10 @@ int mfd_check_schedule(mfd_handle* h, int variant, int64_t* conflicts, char* rep
     if (!h->device_ok) build_plan(h);  // a handle without a GPU keeps no schedule
     std::string rep;
     *conflicts = check_schedule(h, variant, rep);
-    if (variant == 0) *conflicts += h->solve_rc == MFD_OK ? check_solve_plan(h->sp, rep) : 1;
+    if (variant == 0) {
+        *conflicts += h->solve_rc == MFD_OK ? check_solve_plan(h->sp, rep) : 1;
+        *conflicts += check_tree_plan(h->tp, rep);
+    }
     if (report && report_len > 0) {
         const size_t n = std::min(rep.size(), (size_t)report_len - 1);
         memcpy(report, rep.data(), n);
@@ -2261,7 +2349,7 @@ int mfd_solve_device_noalloc(mfd_handle* h, double* d_b, int nrhs, int ldb)
         HIP_TRY(hipEventRecord(h->ev[3], st));
         HIP_TRY(hipStreamSynchronize(st));
         HIP_TRY(hipGetLastError());
-        if (rc == MFD_OK) rc = solve_status(h);
+        if (rc == MFD_OK) rc = wait_status(h);
     }
     if (rc != MFD_OK) return rc;
     float ms = 0;
@@ -2443,7 +2531,7 @@ int mfd_get_kernel_work(mfd_handle* h, int k, int s, double* flops, double* byte
     case MFD_K_EXTEND_ADD:  // small and medium children (large ones add in their Schur launch)
         for (size_t q = 0; q < h->nodes.size(); ++q) {
             const NodeDev& d = h->nodes[q];
-            if (d.parent >= 0 && (d.n <= kSmallFront || h->fused_pos[q] >= 0)) {
+            if (d.parent >= 0 && !h->tp.has(d.parent) && (h->tp.has((int)q) || d.n <= kSmallFront || h->fused_pos[q] >= 0)) {
                 double e = tri(d.w);
                 f += e;
                 b += e * 3 * s + 4.0 * d.w;
@@ -2458,6 +2546,15 @@ int mfd_get_kernel_work(mfd_handle* h, int k, int s, double* flops, double* byte
         }
         break;
     case MFD_K_SMALL_FRONT:
+        // the launch at the bottom of the tree: the fronts' lower triangles
+        // written, their children's update matrices read, their entries of A
+        for (int s0 : h->tp.node) {
+            const NodeDev& d = h->nodes[s0];
+            for (int64_t m = d.w + 1; m <= d.n; ++m) f += (double)m * m;
+            b += s * tri(d.n);
+            if (d.parent >= 0 && h->tp.has(d.parent)) f += tri(d.w), b += s * tri(d.w) + 4.0 * d.w;
+        }
+        b += 16.0 * h->tp.entries;
         for (int s0 : h->small) {
             const NodeDev& d = h->nodes[s0];
             for (int64_t m = d.w + 1; m <= d.n; ++m) f += (double)m * m;

@@ -35,56 +35,16 @@
 // have a fixed order, so results do not depend on timing.
 #include <hip/hip_runtime.h>
 
+#include "mfd_device.h"
 #include "mfd_kernels.h"
 
 namespace mfd {
 
 namespace {
 
-constexpr int kThreads = 256;
 constexpr int kRhs = kRhsGroup;      // right-hand sides per group: the columns of an MFMA operand
-constexpr int kSpinLimit = 1 << 23;  // polls of one wait (about 6 s)
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-// D(16x16) += A(16x4) B(4x16): lane l supplies A[l%16][l/16] and
-// B[l/16][l%16]; element v of lane l is D[l/16 + 4v][l%16].
-__device__ __forceinline__ d4 mma(double a, double b, d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ double ld_agent(const double* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ int ld_agent(const int* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(double* p, double v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// *p by scalar loads (uniform address, memory that no launch writes while
-// this one runs).
-template <typename S> __device__ __forceinline__ S ld_scalar(const S* p)
-{
-    typedef const __attribute__((address_space(4))) int* words;
-    static_assert(sizeof(S) % 4 == 0, "copied in words");
-    S v;
-    words w = (words)(const void*)p;
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(S) / 4; ++i) reinterpret_cast<int*>(&v)[i] = w[i];
-    return v;
-}
-
-// p[i] for a uniform base and a 32-bit index (one VGPR per address).
-template <typename T> __device__ __forceinline__ T ld_off(const T* p, unsigned i)
-{
-    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (size_t)(i * (unsigned)sizeof(T)));
-}
+__device__ __forceinline__ d4 mma(double a, double b, d4 c) { return Mfma<double>::mma(a, b, c); }
 
 // The vector operand of a task's products, rows of 16 right-hand sides, and
 // the four waves' partial products (which take the same place once the
@@ -111,32 +71,18 @@ template <typename T> struct Ctx {
 template <typename T, bool SLOW = false>
 __device__ __forceinline__ void wait_for(const Ctx<T>& C, int f, int target)
 {
-    if (f >= 0 && C.tid == 0) {
-        const int* p = C.flags + f;
-        int* stop = C.A.flags + kSolveStop;
-        for (int spins = 0; ld_agent(p) < target;) {
-            if (SLOW)
-                __builtin_amdgcn_s_sleep(12);
-            else
-                __builtin_amdgcn_s_sleep(1);
-            if ((++spins & 255) == 0 && (ld_agent(stop) != 0 || spins >= kSpinLimit)) {
-                __hip_atomic_store(stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(C.A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                break;
-            }
-        }
-    }
+    if (f >= 0 && C.tid == 0) poll<SLOW>(C.flags + f, target, C.A.flags + kSolveStop, C.A.err);
     __syncthreads();
 }
 // Raises counters f and f2 (negative: none) once every store of the
 // workgroup has completed (all threads; holds a barrier).
 template <typename T> __device__ __forceinline__ void signal(const Ctx<T>& C, int f, int f2 = -1)
 {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    stores_done();
     __syncthreads();
     if (C.tid == 0) {
-        if (f >= 0) __hip_atomic_fetch_add(C.flags + f, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (f2 >= 0) __hip_atomic_fetch_add(C.flags + f2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (f >= 0) add_agent(C.flags + f, 1);
+        if (f2 >= 0) add_agent(C.flags + f2, 1);
     }
 }
 
@@ -824,7 +770,7 @@ template <typename T> __global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 3 
     // ngroups); per is the last task's, 1 where a level's tasks are few
     int per = 1, k0 = 0;
     for (;;) {
-        if (tid == 0) ticket = __hip_atomic_fetch_add(counter, per, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) ticket = add_agent(counter, per);
         __syncthreads();
         k0 = __builtin_amdgcn_readfirstlane(ticket);
         const int k1 = min(k0 + per, A.ntasks * A.ngroups);

@@ -1,0 +1,106 @@
+// Builds the bottom-of-the-tree launch; see mfd_tree_plan.h.
+#include "mfd_tree_plan.h"
+
+#include <algorithm>
+#include <climits>
+#include <cstdio>
+
+namespace mfd {
+
+namespace {
+// Fronts of one height beyond kManyTasks are taken several to a ticket, at
+// most kTicketMost (every ticket is an addition to one counter).
+constexpr int kManyTasks = 8192, kTicketMost = 4;
+}  // namespace
+
+void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible,
+                     TreePlan& P)
+{
+    P = TreePlan{};
+    const int m = (int)nodes.size();
+    if (S.snidx.size() > (size_t)INT_MAX) return;  // entry indices are 32-bit here
+    std::vector<char> in(m, 0);
+    std::vector<int> height(m, 0);
+    int count = 0;
+    for (int s = 0; s < m; ++s) {  // children before parents
+        in[s] = eligible[s] && nodes[s].n <= kTreeFront;
+        for (int ch : S.children[s]) {
+            in[s] = in[s] && in[ch - 1];
+            height[s] = std::max(height[s], height[ch - 1] + 1);
+        }
+        count += in[s];
+    }
+    if (count == 0) return;
+    P.in = in;
+    P.node.reserve(count);
+    for (int s = 0; s < m; ++s)
+        if (in[s]) P.node.push_back(s);
+    // by height; the largest of a height first, so that the last to start are short
+    std::stable_sort(P.node.begin(), P.node.end(), [&](int a, int b) {
+        return height[a] != height[b] ? height[a] < height[b] : nodes[a].n > nodes[b].n;
+    });
+    std::vector<int> pos(m, -1);
+    for (int i = 0; i < count; ++i) pos[P.node[i]] = i;
+    P.tasks.reserve(count);
+    for (int i = 0; i < count; ++i) {
+        const int s = P.node[i];
+        const NodeDev& d = nodes[s];
+        TreeTask t{};
+        t.front = d.front;
+        t.inv = d.inv;
+        t.n = d.n;
+        t.c = d.c;
+        t.first = d.first;
+        t.child = (int)P.children.size();
+        t.nchild = (int)S.children[s].size();
+        t.aptr = (int)P.aptr.size();
+        t.flag = i;
+        t.sig = d.parent >= 0 && in[d.parent] ? pos[d.parent] : -1;
+        for (int ch : S.children[s]) {
+            const NodeDev& k = nodes[ch - 1];
+            P.children.push_back(TreeChild{k.front + k.c + (int64_t)k.c * k.n, k.n, k.w, (int)k.lidx, 0});
+        }
+        for (int q = 0; q < d.c; ++q) {
+            if (q % 16 == 0) P.aptr.push_back((int)P.asrc.size());
+            const int j = d.first + q;  // 0-based global column
+            for (int64_t p = S.a_colptr[j]; p < S.a_colptr[j + 1]; ++p) {
+                const int r = S.snidx[p];
+                const int grow = r <= d.c ? d.first + r - 1 : S.l_rows[S.l_ptr[s] + (r - d.c - 1)] - 1;
+                P.apos.push_back((r - 1) | (q % 16) << 8);
+                P.asrc.push_back((int)(S.ccs_perm[p] - 1));
+                P.arc.push_back(TreePlan::RowCol{grow, j});
+            }
+        }
+        P.aptr.push_back((int)P.asrc.size());
+        P.tasks.push_back(t);
+    }
+    P.entries = (int64_t)P.asrc.size();
+    for (int i = 0; i < count;) {
+        int e = i;
+        while (e < count && height[P.node[e]] == height[P.node[i]]) ++e;
+        const int per = e - i > kManyTasks ? std::min(kTicketMost, (e - i) / (kManyTasks / 2)) : 1;
+        for (; i < e; ++i) P.tasks[i].per = per;
+    }
+}
+
+int64_t check_tree_plan(const TreePlan& P, std::string& report)
+{
+    std::vector<int> now(P.tasks.size(), 0), total(P.tasks.size(), 0);
+    for (const TreeTask& t : P.tasks)
+        if (t.sig >= 0) total[t.sig]++;
+    int64_t bad = 0;
+    char line[128];
+    for (size_t i = 0; i < P.tasks.size(); ++i) {
+        const TreeTask& t = P.tasks[i];
+        if (now[t.flag] != t.nchild || total[t.flag] != t.nchild || t.flag != (int)i)
+            if (++bad <= 8) {
+                snprintf(line, sizeof line, "tree task %zu: %d of %d children before it, %d in all\n", i, now[t.flag],
+                         t.nchild, total[t.flag]);
+                report += line;
+            }
+        if (t.sig >= 0) now[t.sig]++;
+    }
+    return bad;
+}
+
+}  // namespace mfd
