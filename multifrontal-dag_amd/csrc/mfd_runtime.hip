@@ -877,9 +877,9 @@ int setup_device(mfd_handle* h)
     if (h->sp.sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv64, h->sp.sinv_elems));
     // assembly map: A entry -> front position (coefficient_setter_m.f90:26-41),
     // the entries in the fill groups' order
-    const int64_t nnz = (int64_t)S.snidx.size();
-    std::vector<int64_t> dst(nnz), src(nnz), diag_src(S.n, 0);
-    std::vector<int2> rc(nnz);
+    const int64_t nscat = (int64_t)S.snidx.size() - h->tp.entries;
+    std::vector<int64_t> dst(nscat), src(nscat), diag_src(S.n, 0);
+    std::vector<int2> rc(nscat);
     h->scat_gptr.assign(1, 0);
     int64_t e = 0;
     for (size_t g = 0; g < h->group_level.size(); ++g) {
@@ -904,7 +904,7 @@ int setup_device(mfd_handle* h)
         }
         h->scat_gptr.push_back(e);
     }
-    if (e != nnz - h->hplan.entries - h->tp.entries) return MFD_ERR_INTERNAL;
+    if (e != nscat - h->hplan.entries) return MFD_ERR_INTERNAL;
     dst.resize(e);
     src.resize(e);
     rc.resize(e);
@@ -916,7 +916,7 @@ int setup_device(mfd_handle* h)
     std::vector<int> perm0(S.n);
     for (int i = 0; i < S.n; ++i) perm0[i] = S.perm[i] - 1;
     MFD_TRY(upload(h, &h->d_perm, perm0));
-    MFD_TRY(dalloc(h, &h->d_a, nnz));
+    MFD_TRY(dalloc(h, &h->d_a, (int64_t)S.snidx.size()));
     MFD_TRY(dalloc(h, &h->d_info, 1));
     MFD_TRY(dalloc(h, &h->d_pool64, h->pool_elems));
     h->front_bytes = h->pool_elems * (int64_t)sizeof(double);

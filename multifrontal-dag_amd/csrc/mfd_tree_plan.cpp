@@ -42,6 +42,16 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     std::vector<int> pos(m, -1);
     for (int i = 0; i < count; ++i) pos[P.node[i]] = i;
     P.tasks.reserve(count);
+    int64_t entries = 0, panels = 0;
+    for (int s : P.node) {
+        const int c0 = nodes[s].first, c1 = c0 + nodes[s].c;
+        entries += S.a_colptr[c1] - S.a_colptr[c0];
+        panels += (nodes[s].c + 15) / 16 + 1;
+    }
+    P.apos.reserve(entries);
+    P.asrc.reserve(entries);
+    P.arc.reserve(entries);
+    P.aptr.reserve(panels);
     for (int i = 0; i < count; ++i) {
         const int s = P.node[i];
         const NodeDev& d = nodes[s];
