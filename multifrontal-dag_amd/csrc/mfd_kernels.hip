@@ -420,19 +420,21 @@ __global__ __launch_bounds__(kThreads) void k_small_front(T* pool, const NodeDev
 }
 
 // ------------------------------------------------------ large fronts
-// LDS staging of one 64 x 64 MFMA tile product.
-template <typename T> struct TileLds {
-    T As[16][kTile + 4];
-    T Bs[16][kTile + 4];
+// LDS staging of one 64 x 64 MFMA tile product: NB chunks of 16 columns.
+template <typename T, int NB = 1> struct TileLds {
+    T As[NB][16][kTile + 4];
+    T Bs[NB][16][kTile + 4];
 };
 
 // sum_kk A[row][kk] B[col][kk] over a 64 x 64 tile (rows past m and columns
 // past n give 0), FP64/FP32 MFMA 16x16x4.  Four waves each own a 32 x 32
 // quarter (2 x 2 MFMA blocks c[i][j]: rows wr + 16 i, columns wc + 16 j).  K
-// is staged through LDS in chunks of 16 with the next chunk's global loads
-// issued before the current chunk's MFMAs.  Every read of A and B happens
-// before the function returns (it ends with a barrier), so the caller may
-// overwrite A afterwards.
+// is staged through LDS in chunks of 16, the global loads two chunks ahead
+// of their MFMAs; with NB = 2 the chunks alternate between two buffers and
+// one barrier a chunk is enough (Schur updates of the 64^3 workload: 8.4 ms
+// with one chunk ahead and two barriers, 8.1 so; the matrix cores were busy
+// 59% of that time).  Every read of A and B happens before the function
+// returns (it ends with a barrier), so the caller may overwrite A afterwards.
 //
 // tb != 0 takes B transposed in memory (B[col][kk] at B + col * ldb + kk);
 // its chunks are then read 16 entries at a time along kk.
@@ -441,9 +443,9 @@ template <typename T> struct TileLds {
 // it leaves LDS and multiplies on the 16-bit MFMA with FP32 accumulation.
 // TB: 0 = B stored like A (B[col + kk * ldb]), 1 = B transposed in memory,
 // -1 = as the runtime flag tb says (the panel TRSM kernel holds both).
-template <typename T, int LP = kNative, int TB = -1>
+template <typename T, int LP = kNative, int TB = -1, int NB = 1>
 __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ldb, bool tb, int m, int n, int k,
-                                         TileLds<T>& L, typename Mfma<T>::acc_t (&c)[2][2], int tid = threadIdx.x)
+                                         TileLds<T, NB>& L, typename Mfma<T>::acc_t (&c)[2][2], int tid = threadIdx.x)
 {
     static_assert(LP == kNative || sizeof(T) == 4, "16-bit operands come from FP32 fronts");
     typedef typename Mfma<T>::acc_t acc_t;
@@ -452,39 +454,42 @@ __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ld
     const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
     const int li = tid & 63, lp = tid >> 6;
     acc_t c00 = {0, 0, 0, 0}, c01 = {0, 0, 0, 0}, c10 = {0, 0, 0, 0}, c11 = {0, 0, 0, 0};
-    T ra[4], rb[4];
+    T ra[2][4], rb[2][4];
     // transposed-B chunk: element e = tid + 256 p is (col e / 16, kk e % 16)
     const int tcol = tid >> 4, tkk = tid & 15;
     // Every load from a clamped in-bounds position (m, n, k >= 1), its value
     // kept raw and masked only as it is stored to LDS: no branch around the
     // loads, which all go out together.
     const int lic = min(li, m - 1), lib = min(li, n - 1);
-    auto load = [&](int k0) {
+    auto load = [&](int k0, T (&xa)[4], T (&xb)[4]) {
+        // uniform bases, 32-bit offsets within the chunk: one VGPR an address
+        const T* Ak = A + (int64_t)k0 * lda;
+        const T* Bk = trb ? B + k0 : B + (int64_t)k0 * ldb;
+        const int kl = k - 1 - k0;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            const int kc = min(k0 + lp + 4 * p, k - 1);
-            ra[p] = A[lic + (int64_t)kc * lda];
+            const int kc = min(lp + 4 * p, kl);
+            xa[p] = ld_off(Ak, (unsigned)(lic + kc * lda));
             if (trb)
-                rb[p] = B[(int64_t)min(tcol + 16 * p, n - 1) * ldb + min(k0 + tkk, k - 1)];
+                xb[p] = ld_off(Bk, (unsigned)(min(tcol + 16 * p, n - 1) * ldb + min(tkk, kl)));
             else
-                rb[p] = B[lib + (int64_t)kc * ldb];
+                xb[p] = ld_off(Bk, (unsigned)(lib + kc * ldb));
         }
     };
-    load(0);
-    for (int k0 = 0; k0 < k; k0 += 16) {
+    auto store = [&](int k0, int buf, const T (&xa)[4], const T (&xb)[4]) {
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             const int kk = k0 + lp + 4 * p;
-            L.As[lp + 4 * p][li] = (li < m && kk < k) ? ra[p] : T(0);
+            L.As[buf][lp + 4 * p][li] = (li < m && kk < k) ? xa[p] : T(0);
             if (trb) {
                 const int col = tcol + 16 * p;
-                L.Bs[tkk][col] = (col < n && k0 + tkk < k) ? rb[p] : T(0);
+                L.Bs[buf][tkk][col] = (col < n && k0 + tkk < k) ? xb[p] : T(0);
             } else {
-                L.Bs[lp + 4 * p][li] = (li < n && kk < k) ? rb[p] : T(0);
+                L.Bs[buf][lp + 4 * p][li] = (li < n && kk < k) ? xb[p] : T(0);
             }
         }
-        __syncthreads();
-        if (k0 + 16 < k) load(k0 + 16);
+    };
+    auto multiply = [&](int buf) {
         if constexpr (LP == kNative) {
             // the operands of the chunk's four k-steps, then its 16 MFMAs (the
             // compiler interleaves the reads with the MFMAs)
@@ -492,10 +497,10 @@ __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ld
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int kr = q * 4 + (lane >> 4);
-                a0[q] = L.As[kr][wr + (lane & 15)];
-                a1[q] = L.As[kr][wr + 16 + (lane & 15)];
-                b0[q] = L.Bs[kr][wc + (lane & 15)];
-                b1[q] = L.Bs[kr][wc + 16 + (lane & 15)];
+                a0[q] = L.As[buf][kr][wr + (lane & 15)];
+                a1[q] = L.As[buf][kr][wr + 16 + (lane & 15)];
+                b0[q] = L.Bs[buf][kr][wc + (lane & 15)];
+                b1[q] = L.Bs[buf][kr][wc + 16 + (lane & 15)];
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -510,17 +515,39 @@ __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ld
             const int kr = 4 * (lane >> 4);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                a0[i] = M16::cvt(L.As[kr + i][wr + (lane & 15)]);
-                a1[i] = M16::cvt(L.As[kr + i][wr + 16 + (lane & 15)]);
-                b0[i] = M16::cvt(L.Bs[kr + i][wc + (lane & 15)]);
-                b1[i] = M16::cvt(L.Bs[kr + i][wc + 16 + (lane & 15)]);
+                a0[i] = M16::cvt(L.As[buf][kr + i][wr + (lane & 15)]);
+                a1[i] = M16::cvt(L.As[buf][kr + i][wr + 16 + (lane & 15)]);
+                b0[i] = M16::cvt(L.Bs[buf][kr + i][wc + (lane & 15)]);
+                b1[i] = M16::cvt(L.Bs[buf][kr + i][wc + 16 + (lane & 15)]);
             }
             c00 = M16::mma(a0, b0, c00);
             c01 = M16::mma(a0, b1, c01);
             c10 = M16::mma(a1, b0, c10);
             c11 = M16::mma(a1, b1, c11);
         }
+    };
+    // chunk k0 is in LDS, chunk k0 + 16 on its way in (xa, xb), chunk k0 + 32
+    // is sent for in (ya, yb); the main loop without conditions, which would
+    // make the wait for (xa, xb) a wait for every load
+    auto step = [&](int k0, int buf, bool inner, T (&xa)[4], T (&xb)[4], T (&ya)[4], T (&yb)[4]) {
+        if (inner || k0 + 32 < k) load(k0 + 32, ya, yb);
+        multiply(NB == 2 ? buf : 0);
+        if (NB == 1) __syncthreads();
+        if (inner || k0 + 16 < k) store(k0 + 16, NB == 2 ? buf ^ 1 : 0, xa, xb);
         __syncthreads();
+    };
+    load(0, ra[0], rb[0]);
+    if (k > 16) load(16, ra[1], rb[1]);
+    store(0, 0, ra[0], rb[0]);
+    __syncthreads();
+    int k0 = 0;
+    for (; k0 + 48 < k; k0 += 32) {
+        step(k0, 0, true, ra[1], rb[1], ra[0], rb[0]);
+        step(k0 + 16, 1, true, ra[0], rb[0], ra[1], rb[1]);
+    }
+    for (; k0 < k; k0 += 32) {
+        step(k0, 0, false, ra[1], rb[1], ra[0], rb[0]);
+        if (k0 + 16 < k) step(k0 + 16, 1, false, ra[0], rb[0], ra[1], rb[1]);
     }
     c[0][0] = c00;
     c[0][1] = c01;
@@ -528,12 +555,12 @@ __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ld
     c[1][1] = c11;
 }
 // The same product staged as Cs[col][row]; ends with a barrier.
-template <typename T, int LP = kNative, int TB = -1>
+template <typename T, int LP = kNative, int TB = -1, int NB = 1>
 __device__ __forceinline__ void tile_product(const T* A, int lda, const T* B, int ldb, bool tb, int m, int n, int k,
-                                             TileLds<T>& L, T (*Cs)[kTile + 1])
+                                             TileLds<T, NB>& L, T (*Cs)[kTile + 1])
 {
     typename Mfma<T>::acc_t c[2][2];
-    tile_mma<T, LP, TB>(A, lda, B, ldb, tb, m, n, k, L, c);
+    tile_mma<T, LP, TB, NB>(A, lda, B, ldb, tb, m, n, k, L, c);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32, q0 = wc + (lane & 15);
 #pragma unroll
@@ -551,9 +578,9 @@ __device__ __forceinline__ void tile_product(const T* A, int lda, const T* B, in
 // Am[kk][row] holds A (k columns, zero from column k up to a multiple of
 // 16), B comes from global memory like tile_mma's B (staged through L.Bs in
 // chunks of 16).  Ends with a barrier.
-template <typename T>
+template <typename T, int NB>
 __device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T* B, int ldb, bool tb, int n, int k,
-                                              TileLds<T>& L, typename Mfma<T>::acc_t (&c)[2][2])
+                                              TileLds<T, NB>& L, typename Mfma<T>::acc_t (&c)[2][2])
 {
     typedef typename Mfma<T>::acc_t acc_t;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -575,10 +602,10 @@ __device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T*
         for (int p = 0; p < 4; ++p) {
             if (tb) {
                 const int col = tcol + 16 * p, kt = k0 + tkk;
-                L.Bs[tkk][col] = (col < n && kt < k) ? rb[p] : T(0);
+                L.Bs[0][tkk][col] = (col < n && kt < k) ? rb[p] : T(0);
             } else {
                 const int kk = k0 + lp + 4 * p;
-                L.Bs[lp + 4 * p][li] = (li < n && kk < k) ? rb[p] : T(0);
+                L.Bs[0][lp + 4 * p][li] = (li < n && kk < k) ? rb[p] : T(0);
             }
         }
         __syncthreads();
@@ -586,7 +613,7 @@ __device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T*
         for (int q = 0; q < 4; ++q) {
             const int kr = q * 4 + (lane >> 4);
             const T a0 = Am[k0 + kr][wr + (lane & 15)], a1 = Am[k0 + kr][wr + 16 + (lane & 15)];
-            const T b0 = L.Bs[kr][wc + (lane & 15)], b1 = L.Bs[kr][wc + 16 + (lane & 15)];
+            const T b0 = L.Bs[0][kr][wc + (lane & 15)], b1 = L.Bs[0][kr][wc + 16 + (lane & 15)];
             c00 = Mfma<T>::mma(a0, b0, c00);
             c01 = Mfma<T>::mma(a0, b1, c01);
             c10 = Mfma<T>::mma(a1, b0, c10);
@@ -651,40 +678,39 @@ __device__ __forceinline__ void stage_acc(const typename Mfma<T>::acc_t (&c)[2][
 // (TRSM, in-panel update, Schur update), so that profiles tell them apart.
 // The result goes through LDS so the write of C is coalesced along columns
 // (written straight from the accumulators it would be 32-byte pieces).
-template <typename T, int LP = kNative, bool PRE = true, int TB = -1>
-__device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T>& L, T (*Cs)[kTile + 1],
+template <typename T, int LP = kNative, bool PRE = true, int TB = -1, int NB = 1>
+__device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T, NB>& L, T (*Cs)[kTile + 1],
                                           const int* lidx = nullptr)
 {
     T* C = pool + t.c;
     const int tid = threadIdx.x, row = tid & 63;
     // the entries of C this thread reads afterwards (row, column tid / 64 +
     // 4 j), loaded before the K loop so that their latency hides behind it
-    // (from clamped positions, masked where used); PRE = false (the Schur
-    // tiles, whose K loop is long) loads them after it
+    // (from clamped positions, masked where used); PRE = false (the update
+    // and Schur tiles, four workgroups per CU, where the registers they would
+    // hold are those of the second chunk in flight) loads them after it
     T cpre[16];
-    if (!PRE && t.mode != 1) {
-        // loaded below, after the product
-    } else if (t.mode != 1) {
+    if (PRE && t.mode != 1) {
         const int rc = min(row, t.m - 1);
 #pragma unroll
         for (int j = 0; j < 16; ++j) cpre[j] = C[rc + (int64_t)min((tid >> 6) + 4 * j, t.n - 1) * t.ldc];
     }
-    // mode 3 in the instances that load C after the K loop (the Schur
-    // tiles): the parent positions of this thread's row and columns
-    // (local_index), loaded before it so that the parent entries can be read
-    // as soon as it ends (the others read them in the epilogue)
+    typename Mfma<T>::acc_t acc[2][2];
+    tile_mma<T, LP, TB, NB>(pool + t.a, t.lda, pool + t.b, t.ldb, t.mode == 1, t.m, t.n, t.k, L, acc);
+    // the parent positions of this thread's row and columns (local_index)
     int lrow = 1, lcol[16];
-    if (!PRE && t.mode == 3) {
+    if (t.mode == 3) {
         lrow = lidx[t.li + min(row, t.m - 1)];
 #pragma unroll
         for (int j = 0; j < 16; ++j) lcol[j] = lidx[t.lj + min((tid >> 6) + 4 * j, t.n - 1)];
     }
-    tile_product<T, LP, TB>(pool + t.a, t.lda, pool + t.b, t.ldb, t.mode == 1, t.m, t.n, t.k, L, Cs);
     if (!PRE && t.mode != 1) {
         const int rc = min(row, t.m - 1);
 #pragma unroll
         for (int j = 0; j < 16; ++j) cpre[j] = C[rc + (int64_t)min((tid >> 6) + 4 * j, t.n - 1) * t.ldc];
     }
+    stage_acc<T>(acc, Cs, false);
+    __syncthreads();
     if (t.mode == 2) {
         // Cs = C - A B^T, then C = Cs D^T (D = L^{-1}, stored transposed)
 #pragma unroll
@@ -694,7 +720,7 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T>
         }
         __syncthreads();
         typename Mfma<T>::acc_t c[2][2];
-        tile_mma_ldsA<T>(Cs, pool + t.d, kPanel, true, t.n, t.kd, L, c);
+        tile_mma_ldsA<T, NB>(Cs, pool + t.d, kPanel, true, t.n, t.kd, L, c);
         stage_acc<T>(c, Cs, false);
         __syncthreads();
         if (row < t.m)
@@ -706,29 +732,30 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T>
         // C -= the product; mode 3 also adds the new entry into the parent
         // (one launch holds at most one child of each parent, and local_index
         // is injective within a child: no two lanes add into one entry).
-        // Four columns at a time, their loads (from clamped columns) all
-        // issued before the stores, which may alias them as far as the
-        // compiler knows.
+        // Their loads (from clamped columns) are all issued before the stores,
+        // which may alias them as far as the compiler knows: sixteen columns
+        // at a time, four where C has been kept since before the K loop.
         const bool ea = t.mode == 3;
-        T* P = ea ? pool + t.p + ((PRE ? lidx[t.li + row] : lrow) - 1) : C;
+        T* P = ea ? pool + t.p + (lrow - 1) : C;
+        constexpr int G = PRE ? 4 : 16;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int c0 = (tid >> 6) + 16 * k;
+        for (int k = 0; k < 16; k += G) {
+            const int c0 = (tid >> 6) + 4 * k;
             if (c0 >= t.n) break;
-            T pv[4];
-            int64_t po[4];
+            T pv[G];
+            T* pp[G];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                po[q] = ea ? (int64_t)((PRE ? lidx[t.lj + min(c0 + 4 * q, t.n - 1)] : lcol[4 * k + q]) - 1) * t.np : 0;
+            for (int q = 0; q < G; ++q) {
+                pp[q] = P + (ea ? (int64_t)(lcol[k + q] - 1) * t.np : 0);
+                pv[q] = ea ? *pp[q] : T(0);
+            }
 #pragma unroll
-            for (int q = 0; q < 4; ++q) pv[q] = ea ? P[po[q]] : T(0);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < G; ++q) {
                 const int col = c0 + 4 * q;
                 if (col < t.n && (!t.tri || row >= col)) {
-                    const T v = cpre[4 * k + q] - Cs[col][row];
+                    const T v = cpre[k + q] - Cs[col][row];
                     C[row + (int64_t)col * t.ldc] = v;
-                    if (ea) P[po[q]] = pv[q] + v;
+                    if (ea) *pp[q] = pv[q] + v;
                 }
             }
         }
@@ -741,13 +768,13 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T>
 // loses R R^T over its lower syrk x syrk part, R = the tile's rows over the
 // pending panels and the panel just solved (contiguous columns, A then C,
 // which this workgroup has just written).
-template <typename T>
-__device__ __forceinline__ void trsm_syrk(T* pool, const GemmTask& t, TileLds<T>& L, T (*Cs)[kTile + 1])
+template <typename T, int NB>
+__device__ __forceinline__ void trsm_syrk(T* pool, const GemmTask& t, TileLds<T, NB>& L, T (*Cs)[kTile + 1])
 {
     __syncthreads();
     const T* R = pool + (t.mode == 2 ? t.a : t.c);
     const int k = t.mode == 2 ? t.k + t.kd : t.k;
-    tile_product<T, kNative, 0>(R, t.lda, R, t.lda, false, t.syrk, t.syrk, k, L, Cs);
+    tile_product<T, kNative, 0, NB>(R, t.lda, R, t.lda, false, t.syrk, t.syrk, k, L, Cs);
     T* D = pool + t.cd;
     const int row = threadIdx.x & 63;
     if (row < t.syrk)
@@ -767,16 +794,16 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 3 : 4) void k_gemm(T* pool, c
         __shared__ T Cs[kTile][kTile + 1];
         const GemmTask t = tasks[blockIdx.x];
         gemm_task<T>(pool, t, L, Cs);
-        if (t.syrk > 0) trsm_syrk<T>(pool, t, L, Cs);
+        if (t.syrk > 0) trsm_syrk<T, 1>(pool, t, L, Cs);
     } else {
         // modes 0 and 3 (B never transposed): the staged result Cs is written
         // after the last read of the operand staging L, so the two share LDS
         // (four workgroups per CU instead of three)
         __shared__ union {
-            TileLds<T> L;
+            TileLds<T, 2> L;
             T Cs[kTile][kTile + 1];
         } u;
-        gemm_task<T, LP, KIND != 2, 0>(pool, tasks[blockIdx.x], u.L, u.Cs, lidx);
+        gemm_task<T, LP, false, 0, 2>(pool, tasks[blockIdx.x], u.L, u.Cs, lidx);
     }
 }
 
@@ -795,13 +822,13 @@ __global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const NodeDev* n
 {
     __shared__ Front64<T> S;
     __shared__ union {
-        TileLds<T> L;         // GEMM tasks
+        TileLds<T, 2> L;      // GEMM tasks
         T B[2][64][kTile + 1];  // diagonal task: staged operands
     } U;
     if ((int)blockIdx.x >= ndiag) {
         const GemmTask g = tiles[blockIdx.x - ndiag];
-        gemm_task<T>(pool, g, U.L, S.A);
-        if (g.syrk > 0) trsm_syrk<T>(pool, g, U.L, S.A);
+        gemm_task<T, kNative, true, -1, 2>(pool, g, U.L, S.A);
+        if (g.syrk > 0) trsm_syrk<T, 2>(pool, g, U.L, S.A);
         return;
     }
     const DiagTask t = diags[blockIdx.x];
@@ -1312,9 +1339,15 @@ __global__ __launch_bounds__(kThreads) void k_superwv(const T* pool, T* sinv, co
         T Cs[kTile][kTile + 1];
     } u;
     T* dst;
+    const int row = threadIdx.x & 63;
     if (t.j >= 8) {
         const int jv = t.j - 8, rv = c0 + kSuper + 64 * i;
-        const int m = max(0, min(64, nd.c - rv));
+        const int m = min(64, nd.c - rv);
+        if (m < 1) {  // past a partial superblock's last row
+            dst = X + 2 * kSuper * kSuper + 64 * i + kSuper * 64 * jv;
+            for (int col = threadIdx.x >> 6; col < 64; col += 4) dst[row + kSuper * col] = T(0);
+            return;
+        }
         tile_product<T, kNative, 1>(F + rv + (int64_t)(c0 + 64 * jv) * n, n, X + kSuper * 64 * jv + 64 * jv, kSuper, true, m, 64,
                         kSuper - 64 * jv, u.L, u.Cs);
         dst = X + 2 * kSuper * kSuper + 64 * i + kSuper * 64 * jv;
@@ -1324,7 +1357,6 @@ __global__ __launch_bounds__(kThreads) void k_superwv(const T* pool, T* sinv, co
                         u.L, u.Cs);
         dst = X + kSuper * kSuper + 64 * i + kSuper * 64 * jw;
     }
-    const int row = threadIdx.x & 63;
     for (int col = threadIdx.x >> 6; col < 64; col += 4) dst[row + kSuper * col] = u.Cs[col][row];
 }
 
