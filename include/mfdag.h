@@ -71,7 +71,7 @@ typedef struct mfd_handle mfd_handle;
 
 /* kernel classes reported by mfd_get_kernel_time */
 #define MFD_K_ASSEMBLE 0
-#define MFD_K_EXTEND_ADD 1  /* extend-add of small children (n <= 64) */
+#define MFD_K_EXTEND_ADD 1  /* extend-add of the children that are not large fronts */
 #define MFD_K_SMALL_FRONT 2 /* the bottom of the tree (fronts of order <= 128, in one launch, assembly included) and other fronts of order <= 64 */
 #define MFD_K_POTRF 3       /* per panel step: next diagonal block (its panel updates, Cholesky, inverse), panel TRSM tiles, small updates */
 #define MFD_K_TRSM 4        /* a step's GEMM tiles (panel TRSM, small updates) launched apart from its diagonal tasks (levels with many fronts) */

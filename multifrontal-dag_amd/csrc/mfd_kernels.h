@@ -10,20 +10,21 @@
 namespace mfd {
 
 template <typename T> void launch_fill(T* p, int64_t n, hipStream_t st);
-template <typename T> void launch_fill_lower(T* pool, const NodeDev* nodes, const int2* tasks, int count, hipStream_t st);
+// Zero fronts with A's entries in place (see k_assemble); scale: the 16-bit
+// forms' diagonal scaling, or null.
 template <typename T>
-void launch_scatter_a(T* pool, const double* a, const int64_t* dst, const int64_t* src, int64_t nnz, hipStream_t st);
+void launch_assemble(T* pool, const NodeDev* nodes, const FillTask* tasks, int count, const double* a,
+                     const int64_t* dst, const int64_t* src, const int2* rc, const double* scale, hipStream_t st);
 // Diagonal scaling of the 16-bit forms (powers of two: S A S is exact):
 // s[j] from A(j,j) = a[diag_src[j]] so that s_j^2 A(j,j) lies in [0.5, 2);
-// the scaled assembly pool[dst[k]] = s[r] s[c] a[src[k]], (r, c) = rc[k];
 // out = diag(s) in per right-hand side.
 void launch_diag_scale(double* s, const double* a, const int64_t* diag_src, int n, hipStream_t st);
-template <typename T>
-void launch_scatter_a_scaled(T* pool, const double* a, const int64_t* dst, const int64_t* src, const int2* rc,
-                             const double* s, int64_t nnz, hipStream_t st);
 void launch_scale_rows(double* out, const double* in, const double* s, int n, int nrhs, hipStream_t st);
 template <typename T>
 void launch_extend_add(T* pool, const int* lidx, const NodeDev* nodes, const ExtTask* tasks, int count, hipStream_t st);
+template <typename T>
+void launch_pull_children(T* pool, const int* lidx, const NodeDev* nodes, const PullTask* tasks, int count,
+                          const int* children, hipStream_t st);
 template <typename T>
 void launch_small_front(T* pool, const NodeDev* nodes, const int* tasks, int count, int* info, hipStream_t st);
 // Medium fronts: the whole partial factorization of one front per

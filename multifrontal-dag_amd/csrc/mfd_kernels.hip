@@ -298,38 +298,48 @@ __global__ __launch_bounds__(kThreads) void k_fill(T* p, int64_t n)
     for (; i < n; i += stride) p[i] = T(0);
 }
 
-// Zeroes the lower part (row >= col) of 64 columns of one front: task
-// (node, first column).  Only the lower triangle of a front is ever read.
+// The lower part (row >= col; the upper part of a front is never read) of
+// kFillCols columns of one front: zero, but for the stored A entries, each of
+// which lands on exactly one front position (coefficient_setter_m.f90:26-50
+// in the front layout): entry k of the task goes to pool[dst[k]], from
+// a[src[k]], with scale != nullptr (the 16-bit forms) times s[r] s[c], (r, c) =
+// rc[k] its global (postordered, 0-based) row and column.  Bound by its
+// stores; a wave takes whole columns, so that columns of a few hundred
+// entries keep its lanes busy.  (Zeroing 64 columns a workgroup and scattering
+// A in a second launch, one pair of launches per level, took 13 + 4 us and
+// two launch gaps for a level of a 23 x 19 x 17 grid.)
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_fill_lower(T* pool, const NodeDev* nodes, const int2* tasks)
+__global__ __launch_bounds__(kThreads) void k_assemble(T* pool, const NodeDev* nodes, const FillTask* tasks,
+                                                       const double* a, const int64_t* dst, const int64_t* src,
+                                                       const int2* rc, const double* scale)
 {
-    const int2 t = tasks[blockIdx.x];
-    const NodeDev nd = nodes[t.x];
-    const int n = nd.n, jend = min(t.y + 64, n);
+    const FillTask t = tasks[blockIdx.x];
+    const NodeDev nd = nodes[t.node];
+    const int n = nd.n, jend = min(t.j0 + kFillCols, n), lane = threadIdx.x & 63;
     constexpr int V = 16 / sizeof(T);  // elements per 16-byte store
     T* g = pool + nd.front;
-    for (int j = t.y; j < jend; ++j) {
+    for (int j = t.j0 + (threadIdx.x >> 6); j < jend; j += kThreads / 64) {
         // rows [j, n) of column j: scalar head up to a 16-byte boundary,
         // 16-byte stores, scalar tail
         T* col = g + (int64_t)j * n;
         const int head = min((int)((V - ((reinterpret_cast<uintptr_t>(col + j) / sizeof(T)) % V)) % V), n - j);
         const int i0 = j + head, nv = (n - i0) / V, tail = i0 + nv * V;
-        if ((int)threadIdx.x < head) col[j + threadIdx.x] = T(0);
+        if (lane < head) col[j + lane] = T(0);
         uint4* v = reinterpret_cast<uint4*>(col + i0);
-        for (int p = threadIdx.x; p < nv; p += kThreads) v[p] = make_uint4(0u, 0u, 0u, 0u);
-        if ((int)threadIdx.x < n - tail) col[tail + threadIdx.x] = T(0);
+        for (int p = lane; p < nv; p += 64) v[p] = make_uint4(0u, 0u, 0u, 0u);
+        if (lane < n - tail) col[tail + lane] = T(0);
     }
-}
-
-// pool[dst[k]] = a[src[k]]: each stored A entry lands on exactly one front
-// position (coefficient_setter_m.f90:45-50 in the front layout).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_scatter_a(T* pool, const double* a, const int64_t* dst, const int64_t* src,
-                                                        int64_t nnz)
-{
-    int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * kThreads;
-    for (; k < nnz; k += stride) pool[dst[k]] = T(a[src[k]]);
+    if (t.e0 == t.e1) return;
+    stores_done();
+    __syncthreads();
+    for (int64_t k = t.e0 + threadIdx.x; k < t.e1; k += kThreads) {
+        double v = a[src[k]];
+        if (scale) {
+            const int2 q = rc[k];
+            v = v * scale[q.x] * scale[q.y];
+        }
+        pool[dst[k]] = (T)v;
+    }
 }
 
 // Diagonal scaling of the 16-bit forms: s[j] = 2^-e with e = floor(E / 2)
@@ -350,19 +360,6 @@ __global__ __launch_bounds__(kThreads) void k_diag_scale(double* s, const double
         v = ldexp(1.0, -e);
     }
     s[j] = v;
-}
-
-// k_scatter_a for the scaled forms: pool[dst[k]] = s[r] s[c] a[src[k]] with
-// (r, c) = rc[k], the entry's global (postordered, 0-based) row and column.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_scatter_a_scaled(T* pool, const double* a, const int64_t* dst,
-                                                               const int64_t* src, const int2* rc, const double* s,
-                                                               int64_t nnz)
-{
-    const int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (k >= nnz) return;
-    const int2 q = rc[k];
-    pool[dst[k]] = (T)(a[src[k]] * s[q.x] * s[q.y]);
 }
 
 // out[i + k n] = s[i] in[i + k n] (out may be in).
@@ -404,6 +401,64 @@ __global__ __launch_bounds__(kThreads) void k_extend_add(T* pool, const int* lid
         int j = j0 + jj;
         if (j >= ch.w || j > i) break;
         dst[colmap[jj]] += src[(int64_t)j * ch.n];
+    }
+}
+
+// The update matrices of children in the bottom of the tree (order <= 128),
+// added into kPullCols columns of their parent, child after child: all of them
+// in one launch after k_tree, where a launch per level and child rank took
+// 8 to 15 us each (44 of them for 512 systems).  A child's columns that fall
+// into the task's are consecutive (local_index ascends), a wave takes every
+// fourth, and the loads of all of them are in flight together.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_pull_children(T* pool, const int* lidx, const NodeDev* nodes,
+                                                            const PullTask* tasks, const int* children)
+{
+    const PullTask t = tasks[blockIdx.x];
+    const NodeDev pa = nodes[t.node];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    T* dst = pool + pa.front;
+    for (int k = 0; k < t.nchild; ++k) {
+        const NodeDev ch = nodes[children[t.child + k]];
+        const int* li = lidx + ch.lidx;
+        // the first update column at or past parent column j0 (lanes 0 .. 63
+        // and 64 .. 127 of the order look at one each)
+        const int l0 = lane < ch.w ? li[lane] - 1 : INT_MAX, l1 = lane + 64 < ch.w ? li[lane + 64] - 1 : INT_MAX;
+        const int q0 = __popcll(__ballot(l0 < t.j0)) + __popcll(__ballot(l1 < t.j0));
+        const int q1 = __popcll(__ballot(l0 < t.j0 + kPullCols)) + __popcll(__ballot(l1 < t.j0 + kPullCols));
+        const T* src = pool + ch.front + ch.c + (int64_t)ch.c * ch.n;
+        constexpr int G = 4;
+        for (int qb = q0 + wv; qb < q1; qb += 4 * G) {
+            T* p[2 * G];
+            T c[2 * G], v[2 * G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int q = min(qb + 4 * g, q1 - 1);
+                T* col = dst + (int64_t)(li[q] - 1) * pa.n;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    // (lanes without an entry read the column's diagonal one)
+                    const int i = lane + 64 * h;
+                    const bool on = i >= q && i < ch.w;
+                    p[2 * g + h] = col + (on ? (h ? l1 : l0) : li[q] - 1);
+                    c[2 * g + h] = src[(on ? i : q) + (int64_t)q * ch.n];
+                    v[2 * g + h] = *p[2 * g + h];
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int q = qb + 4 * g;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int i = lane + 64 * h;
+                    if (q < q1 && i >= q && i < ch.w) *p[2 * g + h] = v[2 * g + h] + c[2 * g + h];
+                }
+            }
+        }
+        if (k + 1 < t.nchild) {
+            stores_done();
+            __syncthreads();
+        }
     }
 }
 
@@ -1577,14 +1632,19 @@ template <typename T> void launch_fill(T* p, int64_t n, hipStream_t st)
     if (n > 0) hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(n)), dim3(kThreads), 0, st, p, n);
 }
 template <typename T>
-void launch_fill_lower(T* pool, const NodeDev* nodes, const int2* tasks, int count, hipStream_t st)
+void launch_assemble(T* pool, const NodeDev* nodes, const FillTask* tasks, int count, const double* a,
+                     const int64_t* dst, const int64_t* src, const int2* rc, const double* scale, hipStream_t st)
 {
-    if (count > 0) hipLaunchKernelGGL(k_fill_lower<T>, dim3(count), dim3(kThreads), 0, st, pool, nodes, tasks);
+    if (count > 0)
+        hipLaunchKernelGGL(k_assemble<T>, dim3(count), dim3(kThreads), 0, st, pool, nodes, tasks, a, dst, src, rc,
+                           scale);
 }
 template <typename T>
-void launch_scatter_a(T* pool, const double* a, const int64_t* dst, const int64_t* src, int64_t nnz, hipStream_t st)
+void launch_pull_children(T* pool, const int* lidx, const NodeDev* nodes, const PullTask* tasks, int count,
+                          const int* children, hipStream_t st)
 {
-    if (nnz > 0) hipLaunchKernelGGL(k_scatter_a<T>, dim3(grid_for(nnz)), dim3(kThreads), 0, st, pool, a, dst, src, nnz);
+    if (count > 0)
+        hipLaunchKernelGGL(k_pull_children<T>, dim3(count), dim3(kThreads), 0, st, pool, lidx, nodes, tasks, children);
 }
 template <typename T>
 void launch_extend_add(T* pool, const int* lidx, const NodeDev* nodes, const ExtTask* tasks, int count, hipStream_t st)
@@ -1658,14 +1718,6 @@ void launch_diag_scale(double* s, const double* a, const int64_t* diag_src, int 
 {
     if (n > 0) hipLaunchKernelGGL(k_diag_scale, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, s, a, diag_src, n);
 }
-template <typename T>
-void launch_scatter_a_scaled(T* pool, const double* a, const int64_t* dst, const int64_t* src, const int2* rc,
-                             const double* s, int64_t nnz, hipStream_t st)
-{
-    if (nnz > 0)
-        hipLaunchKernelGGL(k_scatter_a_scaled<T>, dim3((unsigned)((nnz + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                           st, pool, a, dst, src, rc, s, nnz);
-}
 void launch_scale_rows(double* out, const double* in, const double* s, int n, int nrhs, hipStream_t st)
 {
     const int64_t m = (int64_t)n * nrhs;
@@ -1724,16 +1776,16 @@ void launch_scatter_rows(double* out, int ld_out, const double* in, int ld_in, c
 
 #define MFD_INSTANTIATE(T)                                                                                             \
     template void launch_fill<T>(T*, int64_t, hipStream_t);                                                            \
-    template void launch_fill_lower<T>(T*, const NodeDev*, const int2*, int, hipStream_t);                            \
-    template void launch_scatter_a<T>(T*, const double*, const int64_t*, const int64_t*, int64_t, hipStream_t);        \
+    template void launch_assemble<T>(T*, const NodeDev*, const FillTask*, int, const double*, const int64_t*,          \
+                                     const int64_t*, const int2*, const double*, hipStream_t);                         \
+    template void launch_pull_children<T>(T*, const int*, const NodeDev*, const PullTask*, int, const int*,            \
+                                          hipStream_t);                                                                \
     template void launch_extend_add<T>(T*, const int*, const NodeDev*, const ExtTask*, int, hipStream_t);              \
     template void launch_small_front<T>(T*, const NodeDev*, const int*, int, int*, hipStream_t);                       \
     template void launch_front_wg<T>(T*, const NodeDev*, const int*, int, int*, long long*, hipStream_t, int);           \
     template void launch_diag<T>(T*, const NodeDev*, const DiagTask*, int, int*, hipStream_t);                        \
     template void launch_upd_diag<T>(T*, const NodeDev*, const DiagTask*, int, const GemmTask*, int, int*, hipStream_t); \
     template void launch_gemm<T>(T*, const GemmTask*, int, int, const int*, hipStream_t, int);                         \
-    template void launch_scatter_a_scaled<T>(T*, const double*, const int64_t*, const int64_t*, const int2*,           \
-                                             const double*, int64_t, hipStream_t);                                    \
     template void launch_superinv<T>(const T*, T*, const NodeDev*, const SuperInvTask*, int, bool, hipStream_t);      \
     template void launch_gemm_seg<T>(T*, const GemmTask*, const SegTask*, const int*, int, const FixTask*, int, T*,  \
                                      const int*, hipStream_t, int);

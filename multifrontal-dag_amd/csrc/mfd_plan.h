@@ -25,6 +25,21 @@ struct NodeDev {
     int pad;
 };
 
+// kFillCols columns of a front from j0 on, zeroed, then the assembly entries
+// [e0, e1) of those columns put in place.
+constexpr int kFillCols = 16;
+struct FillTask {
+    int node, j0;
+    int64_t e0, e1;
+};
+
+// The children of `node` in the bottom of the tree, entries [child, child +
+// nchild) of the list of them, added into its columns [j0, j0 + kPullCols).
+constexpr int kPullCols = 32;
+struct PullTask {
+    int node, j0, child, nchild;
+};
+
 // Extend-add of one 64 x 64 tile (ti >= tj) of child's update matrix.
 struct ExtTask {
     int child, ti, tj, pad;

@@ -41,7 +41,7 @@ struct Launch {
     int kind;       // MFD_K_*
     int64_t first;  // first task in the kind's task array
     int count;
-    int wide = 0;   // GEMM launches: 1 = 128 x 128 tiles (k_gemm_seg + k_gemm_fix)
+    int wide = 0;   // GEMM launches: 1 = 128 x 128 tiles (k_gemm_seg + k_gemm_fix); extend-add: 1 = PullTasks
     // wide launches: K chunks over `groups` workgroups, their segments at
     // seg_ptr[sfirst .. sfirst + groups], then nfix split tiles from fix[xfirst]
     int64_t sfirst = 0, xfirst = 0;
@@ -61,7 +61,11 @@ struct Launch {
 
 // A step's update tiles join the step's launch (k_upd_diag, one workgroup
 // per CU at its LDS) up to this many; more run as their own launch.
-constexpr int kFillGroups = 32;  // most level groups the front zeroing is split into
+// The front zeroing is split into at most kFillGroups groups of levels of at
+// least kFillMin entries (32 MB in FP64, about 8 us of stores; a launch of its
+// own costs about as much).
+constexpr int kFillGroups = 32;
+constexpr int64_t kFillMin = 4 << 20;
 constexpr int kFuseTiles = 1024;
 
 // The order of a launch's tiles: a front's tiles in squares of kSquare x
@@ -158,14 +162,12 @@ struct mfd_handle {
     hipEvent_t fork = nullptr, sev[2] = {};
     // Front-pool zeroing and assembly in groups of levels beside the
     // factorization: group g's fronts (fill tasks [fill_gptr[g],
-    // fill_gptr[g+1]), entries [scat_gptr[g], scat_gptr[g+1])) are first
-    // written by a launch of level group_level[g] or later; the main stream
-    // waits for fill_ev[g] before the first launch of that level
-    // (level_launch).
+    // fill_gptr[g+1])) are first written by a launch of level group_level[g]
+    // or later; the main stream waits for fill_ev[g] before the first launch
+    // of that level (level_launch).
     hipStream_t fillst = nullptr;
     std::vector<hipEvent_t> fill_ev;
     std::vector<int> fill_gptr, group_level, level_launch, front_group;
-    std::vector<int64_t> scat_gptr;
     hipError_t last_hip = hipSuccess;
     int64_t mem_limit = 0, device_bytes = 0, front_bytes = 0;
     // Device buffers in use (pointer, bytes) and released ones kept for
@@ -188,11 +190,13 @@ struct mfd_handle {
     // host schedule
     std::vector<NodeDev> nodes;
     std::vector<ExtTask> ext;
+    std::vector<PullTask> pull;  // extend-add of the bottom of the tree's roots
+    std::vector<int> pull_child;
     std::vector<int> small;
     std::vector<int> fused;             // medium fronts factored whole by one workgroup
     std::vector<int> fused_pos;         // node -> position in fused, or -1
     std::vector<DiagTask> diag;         // diagonal-block factorizations of large fronts
-    std::vector<int2> fill;             // (node, first column) blocks of the pool's lower triangles
+    std::vector<FillTask> fill;             // (node, first column) blocks of the pool's lower triangles
     std::vector<GemmTask> gemm;
     std::vector<Launch> fseq;
     std::vector<int> level_ptr, level_nodes, child_ptr, child_list;
@@ -224,7 +228,9 @@ struct mfd_handle {
     int* d_fused = nullptr;
     long long* d_clocks = nullptr;  // start/end clock of each medium front's workgroup, in fused's order
     DiagTask* d_diag = nullptr;
-    int2* d_fill = nullptr;
+    FillTask* d_fill = nullptr;
+    PullTask* d_pull = nullptr;
+    int* d_pull_child = nullptr;
     GemmTask* d_gemm = nullptr;
     int *d_level_nodes = nullptr, *d_child_ptr = nullptr, *d_child_list = nullptr;
     int64_t *d_dst = nullptr, *d_src = nullptr;
@@ -358,6 +364,8 @@ void free_device(mfd_handle* h)
     h->d_clocks = nullptr;
     h->d_diag = nullptr;
     h->d_fill = nullptr;
+    h->d_pull = nullptr;
+    h->d_pull_child = nullptr;
     h->d_gemm = nullptr;
     h->d_level_nodes = h->d_child_ptr = h->d_child_list = nullptr;
     h->d_ttasks = nullptr;
@@ -467,24 +475,42 @@ void build_plan(mfd_handle* h)
         for (int s = 0; s < m; ++s) h->level_nodes[pos[lev[s]]++] = s;
     }
     // fill groups: a front is first written by its own level's launches or,
-    // earlier, by a child's extend-add
+    // earlier, by a child's extend-add (that of the bottom of the tree comes
+    // before the first level).  A group takes levels until it has kFillMin
+    // entries to zero, so that small problems have one launch and large ones
+    // start on their first levels early.
     std::vector<int> group(m, 0);
     {
-        const int G = std::min(h->num_levels, kFillGroups);
-        h->group_level.resize(G);
-        for (int g = 0; g < G; ++g) h->group_level[g] = (int)((int64_t)g * h->num_levels / G);
+        std::vector<int> ready(lev);
+        std::vector<int64_t> entries(h->num_levels + 1, 0);
+        int64_t total = 0;
         for (int s = 0; s < m; ++s) {
-            int ready = lev[s];
-            for (int ch : S.children[s]) ready = std::min(ready, lev[ch - 1]);
-            group[s] = (int)(std::upper_bound(h->group_level.begin(), h->group_level.end(), ready) -
-                             h->group_level.begin()) - 1;
+            for (int ch : S.children[s]) ready[s] = std::min(ready[s], h->tp.has(ch - 1) ? 0 : lev[ch - 1]);
+            if (on_host(s) || h->tp.has(s)) continue;
+            const int64_t n = h->nodes[s].n;
+            entries[ready[s]] += n * (n + 1) / 2;
+            total += n * (n + 1) / 2;
         }
+        const int64_t most = std::max(kFillMin, total / (kFillGroups - 1));
+        h->group_level.clear();
+        int64_t sum = most;
+        for (int L = 0; L < h->num_levels; ++L) {
+            if (sum >= most) {
+                h->group_level.push_back(L);
+                sum = 0;
+            }
+            sum += entries[L];
+        }
+        const int G = (int)h->group_level.size();
+        for (int s = 0; s < m; ++s)
+            group[s] = (int)(std::upper_bound(h->group_level.begin(), h->group_level.end(), ready[s]) -
+                             h->group_level.begin()) - 1;
         h->fill.clear();
         h->fill_gptr.assign(1, 0);
         for (int g = 0; g < G; ++g) {
             for (int s2 = 0; s2 < m; ++s2)
                 if (group[s2] == g && !on_host(s2) && !h->tp.has(s2))
-                    for (int j0 = 0; j0 < h->nodes[s2].n; j0 += 64) h->fill.push_back(make_int2(s2, j0));
+                    for (int j0 = 0; j0 < h->nodes[s2].n; j0 += kFillCols) h->fill.push_back(FillTask{s2, j0, 0, 0});
             h->fill_gptr.push_back((int)h->fill.size());
         }
     }
@@ -501,6 +527,8 @@ void build_plan(mfd_handle* h)
     }
 
     h->ext.clear();
+    h->pull.clear();
+    h->pull_child.clear();
     h->small.clear();
     h->fused.clear();
     h->fused_pos.assign(m, -1);
@@ -609,6 +637,19 @@ void build_plan(mfd_handle* h)
         // extend-add of the small children (a large child adds its update
         // into the parent in its own Schur launch): the r-th child of every
         // parent of this level in one launch
+        // (the bottom of the tree's roots all at once, before the first level)
+        if (L == 0) {
+            for (int s = 0; s < m; ++s) {
+                if (on_host(s) || h->tp.has(s)) continue;
+                const int first = (int)h->pull_child.size();
+                for (int ch : S.children[s])
+                    if (h->tp.has(ch - 1) && S.w[ch - 1] > 0) h->pull_child.push_back(ch - 1);
+                const int nch = (int)h->pull_child.size() - first;
+                for (int j0 = 0; nch > 0 && j0 < h->nodes[s].n; j0 += kPullCols)
+                    h->pull.push_back(PullTask{s, j0, first, nch});
+            }
+            push(MFD_K_EXTEND_ADD, 0, (int64_t)h->pull.size(), 1);
+        }
         size_t maxch = 0;
         for (int k = 0; k < cnt; ++k) maxch = std::max(maxch, S.children[lv[k]].size());
         for (size_t r = 0; r < maxch; ++r) {
@@ -617,7 +658,7 @@ void build_plan(mfd_handle* h)
                 const auto& chs = S.children[lv[k]];
                 if (chs.size() <= r || cls[lv[k]] == kClsHost || cls[lv[k]] == kClsTree) continue;
                 int ch = chs[r] - 1, nt = (S.w[ch] + kTile - 1) / kTile;
-                if (cls[ch] == kClsLarge) continue;
+                if (cls[ch] == kClsLarge || cls[ch] == kClsTree) continue;
                 for (int ti = 0; ti < nt; ++ti)
                     for (int tj = 0; tj <= ti; ++tj) h->ext.push_back(ExtTask{ch, ti, tj, 0});
             }
@@ -880,11 +921,12 @@ int setup_device(mfd_handle* h)
     MFD_TRY(upload(h, &h->d_nodes, h->nodes));
     MFD_TRY(upload(h, &h->d_lidx, S.lidx));
     MFD_TRY(upload(h, &h->d_ext, h->ext));
+    MFD_TRY(upload(h, &h->d_pull, h->pull));
+    MFD_TRY(upload(h, &h->d_pull_child, h->pull_child));
     MFD_TRY(upload(h, &h->d_small, h->small));
     MFD_TRY(upload(h, &h->d_fused, h->fused));
     MFD_TRY(dalloc(h, &h->d_clocks, 2 * (int64_t)h->fused.size()));
     MFD_TRY(upload(h, &h->d_diag, h->diag));
-    MFD_TRY(upload(h, &h->d_fill, h->fill));
     while (h->fill_ev.size() < h->group_level.size()) {
         hipEvent_t ev;
         HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -912,34 +954,38 @@ int setup_device(mfd_handle* h)
     MFD_TRY(upload(h, &h->d_xinv, h->sp.xinv));
     if (h->sp.sinv_elems > 0) MFD_TRY(dalloc(h, &h->d_sinv64, h->sp.sinv_elems));
     // assembly map: A entry -> front position (coefficient_setter_m.f90:26-41),
-    // the entries in the fill groups' order
+    // the entries in the fill tasks' order
     const int64_t nscat = (int64_t)S.snidx.size() - h->tp.entries;
     std::vector<int64_t> dst(nscat), src(nscat), diag_src(S.n, 0);
     std::vector<int2> rc(nscat);
-    h->scat_gptr.assign(1, 0);
     int64_t e = 0;
+    FillTask* task = h->fill.data();
     for (size_t g = 0; g < h->group_level.size(); ++g) {
         for (int s = 0; s < S.num_node; ++s) {
             if (h->front_group[s] != (int)g) continue;
             const NodeDev& d = h->nodes[s];
             const bool host = !h->hplan.is_host.empty() && h->hplan.is_host[s];
+            const bool mine = !host && !h->tp.has(s);  // not assembled on the host or in its own launch
             for (int j = S.first[s]; j < S.first[s + 1]; ++j) {
                 int64_t q = j - S.first[s];
+                if (mine && q % kFillCols == 0) task[q / kFillCols].e0 = e;
                 for (int64_t p = S.a_colptr[j - 1]; p < S.a_colptr[j]; ++p) {
                     // global row: a pivot row of this front or one of its update rows
                     const int r = S.snidx[p];
                     const int grow = r <= S.c[s] ? S.first[s] + r - 1 : S.l_rows[S.l_ptr[s] + (r - S.c[s] - 1)];
                     if (grow == j) diag_src[j - 1] = S.ccs_perm[p] - 1;
-                    if (host || h->tp.has(s)) continue;  // assembled on the host, or in its own launch
+                    if (!mine) continue;
                     dst[e] = d.front + (S.snidx[p] - 1) + q * d.n;
                     src[e] = S.ccs_perm[p] - 1;
                     rc[e] = make_int2(grow - 1, j - 1);
                     ++e;
                 }
+                if (mine) task[q / kFillCols].e1 = e;
             }
+            if (mine) task += (d.n + kFillCols - 1) / kFillCols;
         }
-        h->scat_gptr.push_back(e);
     }
+    MFD_TRY(upload(h, &h->d_fill, h->fill));
     if (e != nscat - h->hplan.entries) return MFD_ERR_INTERNAL;
     dst.resize(e);
     src.resize(e);
@@ -1003,7 +1049,12 @@ template <typename T> void enqueue_launch(mfd_handle* h, const Launch& l, hipStr
 {
     T* pool = pool_of<T>(h);
     switch (l.kind) {
-    case MFD_K_EXTEND_ADD: launch_extend_add<T>(pool, h->d_lidx, h->d_nodes, h->d_ext + l.first, l.count, st); break;
+    case MFD_K_EXTEND_ADD:
+        if (l.wide)
+            launch_pull_children<T>(pool, h->d_lidx, h->d_nodes, h->d_pull + l.first, l.count, h->d_pull_child, st);
+        else
+            launch_extend_add<T>(pool, h->d_lidx, h->d_nodes, h->d_ext + l.first, l.count, st);
+        break;
     case MFD_K_SMALL_FRONT: launch_small_front<T>(pool, h->d_nodes, h->d_small + l.first, l.count, h->d_info, st); break;
     case MFD_K_FRONT:
         launch_front_wg<T>(pool, h->d_nodes, h->d_fused + l.first, l.count, h->d_info, h->d_clocks + 2 * l.first, st,
@@ -1079,27 +1130,22 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
     const int G = (int)h->group_level.size();
     const bool split_fill = !profile && h->fillst && (int)h->fill_ev.size() >= G;
     hipStream_t fst = split_fill ? h->fillst : st;
+    const bool scaled = sizeof(T) == 4 && h->lowp != 0;
+    if (scaled) launch_diag_scale(h->d_dscale, h->d_a, h->d_diag_src, h->S.n, st);
     if (split_fill) {
         ok(hipEventRecord(h->fork, st));
         ok(hipStreamWaitEvent(fst, h->fork, 0));
     }
-    const bool scaled = sizeof(T) == 4 && h->lowp != 0;
-    if (scaled) launch_diag_scale(h->d_dscale, h->d_a, h->d_diag_src, h->S.n, fst);
-    for (int g = 0; g < G; ++g) {
-        launch_fill_lower<T>(pool, h->d_nodes, h->d_fill + h->fill_gptr[g], h->fill_gptr[g + 1] - h->fill_gptr[g], fst);
-        const int64_t e0 = h->scat_gptr[g], ne = h->scat_gptr[g + 1] - h->scat_gptr[g];
-        if (scaled)
-            launch_scatter_a_scaled<T>(pool, h->d_a, h->d_dst + e0, h->d_src + e0, h->d_scat_rc + e0, h->d_dscale, ne,
-                                       fst);
-        else
-            launch_scatter_a<T>(pool, h->d_a, h->d_dst + e0, h->d_src + e0, ne, fst);
-        if (split_fill) ok(hipEventRecord(h->fill_ev[g], fst));
-    }
+    auto assemble = [&]() {
+        for (int g = 0; g < G; ++g) {
+            launch_assemble<T>(pool, h->d_nodes, h->d_fill + h->fill_gptr[g], h->fill_gptr[g + 1] - h->fill_gptr[g],
+                               h->d_a, h->d_dst, h->d_src, h->d_scat_rc, scaled ? h->d_dscale : nullptr, fst);
+            if (split_fill) ok(hipEventRecord(h->fill_ev[g], fst));
+        }
+    };
+    if (!split_fill) assemble();
     mark(0);
     if (tree) {
-        // (in the 16-bit forms behind the fill stream's scaling, which the
-        // first group's event follows)
-        if (scaled && split_fill && G > 0) ok(hipStreamWaitEvent(st, h->fill_ev[0], 0));
         TreeArgs<T> a{};
         a.pool = pool;
         a.a = h->d_a;
@@ -1118,6 +1164,7 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
         launch_tree<T>(a, st);
         mark(MFD_K_SMALL_FRONT);
     }
+    if (split_fill) assemble();
     // Side launches fork from the main stream's current position and run
     // beside it; a step's launches join the side launch they depend on, and
     // any other launch joins every side launch before it.
@@ -1764,7 +1811,17 @@ struct ScheduleCheck {
         kind = l.kind;
         switch (l.kind) {
         case MFD_K_EXTEND_ADD:
-            for (int64_t i = l.first; i < l.first + l.count; ++i) {
+            for (int64_t i = l.first; l.wide && i < l.first + l.count; ++i) {
+                const PullTask& t = h->pull[i];
+                const NodeDev& d = h->nodes[t.node];
+                const int64_t task = next_task++;
+                rect(t.node, t.j0, d.n, t.j0, std::min(d.n, t.j0 + kPullCols), node, task, true);
+                for (int k = 0; k < t.nchild; ++k) {
+                    const int ch = h->pull_child[t.child + k];
+                    rect(ch, h->nodes[ch].c, h->nodes[ch].n, h->nodes[ch].c, h->nodes[ch].n, node, task, false);
+                }
+            }
+            for (int64_t i = l.first; !l.wide && i < l.first + l.count; ++i) {
                 const ExtTask& t = h->ext[i];
                 const NodeDev& d = h->nodes[t.child];
                 const int64_t task = next_task++;

@@ -78,3 +78,44 @@ def test_first_bad_pivot_is_reported(col):
         assert e.value.code == col + 1
         assert s.factorize(p.val, prec) == 0
     s.close()
+
+
+def subsets(c, w, leaves, order, seed):
+    """`leaves` dense blocks of order c, each coupled to w random columns of a
+    dense block of the given order (> 128): children in the bottom-of-the-tree
+    launch whose parent is not, their update rows scattered over its columns."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    n = c * leaves + order
+    A = np.zeros((n, n))
+    for k in range(leaves):
+        s = slice(c * k, c * k + c)
+        A[s, s] = rng.uniform(-1.0, 1.0, (c, c))
+        A[np.ix_(c * leaves + rng.choice(order, w, replace=False), range(s.start, s.stop))] = rng.uniform(-1, 1, (w, c))
+    A[c * leaves:, c * leaves:] = rng.uniform(-1.0, 1.0, (order, order))
+    L = np.tril(A, -1)
+    A = L + L.T
+    np.fill_diagonal(A, np.abs(A).sum(axis=1) + 1.0)
+    i, j = np.nonzero(np.tril(A))
+    cc, rr, vv = P.lower_ccs(n, i, j, A[i, j])
+    return P.Problem(n, cc, rr, vv, None, f"subsets_{c}_{w}_{leaves}_{order}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c,w,leaves,order", [(1, 1, 1, 129), (3, 31, 2, 144), (20, 32, 5, 160), (20, 33, 5, 161),
+                                              (5, 64, 3, 191), (63, 65, 4, 192), (1, 127, 9, 193), (28, 100, 33, 260)],
+                         ids=lambda v: str(v))
+def test_children_added_into_a_larger_parent(c, w, leaves, order):
+    p = subsets(c, w, leaves, order, seed=c + w)
+    s = mfdag.Solver(nb=64)
+    s.analyze(p.ccs_col, p.ccs_row, 0, np.arange(1, p.n + 1, dtype=np.int32))
+    n = s.structure()["supernode_size"] + s.structure()["work_size"]
+    assert n.max() > 128 and n.min() <= 128
+    assert s.check_schedule(0) == (0, "")
+    _, b = P.rhs(p, 2, seed=4)
+    for prec in (mfdag.FP32_IR, mfdag.FP16_IR, mfdag.BF16_IR, mfdag.FP64):
+        assert s.factorize(p.val, prec) == 0
+        assert P.backward_error(p, s.solve(b.copy()), b) <= 1e-14
+    f, st, info = oracle_for(s, p.val)
+    assert info == 0
+    assert front_errors(s, f, st).max() <= 1e-12
+    s.close()
