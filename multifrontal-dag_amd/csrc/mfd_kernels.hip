@@ -1309,69 +1309,76 @@ __global__ __launch_bounds__(kThreads) void k_front_wg(T* pool, const NodeDev* n
 //       the superblock to the previous one, so that y_u = X z_u - W y_{u-1};
 //   V = L[B_{u+1}, B_u] X (j >= 8: block (i, j - 8), rows of superblock
 //       u+1), so that x_u = X^T (y_u - q_u) - V^T x_{u+1}.
-// One task per block, launched by block distance i - j; the W and V blocks
-// follow in one launch of k_superwv.
+// A task forms 16 columns of X from block row j = t.j / 4 down, one row after
+// another (they depend on no other column): the columns so far are in LDS, a
+// wave has 16 rows of the block row in work and takes the blocks of L and the
+// stored inverse straight into MFMA operands, a block ahead.  Bound by the
+// latency of that chain (up to nine products of 64 x 16 x 64).  As a launch
+// per block distance with a whole 64 x 64 block a workgroup, off the matrix
+// cores, the last front's superblocks took 110 us (one superblock) to 185 us
+// (64^3 workload, 122 of them) in FP64 where this takes 18 and 106.  The W and
+// V blocks follow in one launch of k_superwv.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_superinv(const T* pool, T* sinv, const NodeDev* nodes,
                                                        const SuperInvTask* tasks)
 {
+    typedef typename Mfma<T>::acc_t acc_t;
     const SuperInvTask t = tasks[blockIdx.x];
     const NodeDev nd = nodes[t.node];
-    T* X = sinv + t.xoff;
-    const int n = nd.n, c0 = kSuper * t.u, tid = threadIdx.x;
-    const int i = t.i, j = t.j, b0 = c0 + 64 * i;  // first global pivot column of block row i
-    const int kbi = max(0, min(64, nd.c - b0));     // pivot rows of block row i
-    if (i == j) {
-        const bool live = kbi > 0;
-        const T* inv = pool + nd.inv + (int64_t)(live ? b0 / 64 : 0) * 4096;  // inv[r + 64 q] = L^{-1}(q, r)
-        for (int e = tid; e < 4096; e += kThreads) {
-            const int r = e & 63, q = e >> 6;  // block row q, column r
-            X[(64 * i + q) + kSuper * (64 * i + r)] = (r < kbi && q < kbi) ? inv[r + 64 * q] : T(0);
-            for (int jj = 0; jj < 4; ++jj)
-                if (jj > i || (!live && jj < i)) X[(64 * i + q) + kSuper * (64 * jj + r)] = T(0);
-        }
-        return;
+    const int n = nd.n, c0 = kSuper * t.u, sb = min(kSuper, nd.c - c0), j = t.j >> 2, s0 = 16 * (t.j & 3);
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kl = lane >> 4, r0 = 16 * (tid >> 6);
+    T* X = sinv + t.xoff + kSuper * (64 * j + s0);  // the task's columns
+    __shared__ T Xs[4][64][17];  // X, block row, row, column
+    __shared__ T Ss[64][17];     // sum_k L_ik X_kj
+    const T* inv = pool + nd.inv + (int64_t)(c0 / 64) * 4096;  // block i's: inv[4096 i + r + 64 q] = L^{-1}(q, r)
+    const int nblk = (sb + 63) / 64;                           // block rows in use
+    // X_jj from the stored inverse; zero above it and past the superblock
+    for (int e = tid; e < kSuper * 16; e += kThreads) {
+        const int r = e & 255, col = e >> 8, i = r >> 6, kb = min(64, sb - 64 * j);
+        if (i > j && i < nblk) continue;
+        T v = T(0);
+        if (i == j && (r & 63) < kb && s0 + col < kb) v = inv[4096 * j + (s0 + col) + 64 * (r & 63)];
+        if (i == j) Xs[j][r & 63][col] = v;
+        X[r + kSuper * col] = v;
     }
-    __shared__ T As[64][65], Bs[64][65];  // As[m][r] = A(r, m), Bs[col][m] = B(m, col)
-    const int r = tid & 63, cq = tid >> 6;
-    T acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = T(0);
-    for (int k = j; k < i; ++k) {
-        for (int e = tid; e < 4096; e += kThreads) {
-            const int rr = e & 63, m = e >> 6;
-            // A = L_ik, B = X_kj
-            As[m][rr] = rr < kbi ? pool[nd.front + (b0 + rr) + (int64_t)(c0 + 64 * k + m) * n] : T(0);
-            Bs[m][rr] = X[(64 * k + rr) + kSuper * (64 * j + m)];
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int m = 0; m < 64; ++m) {
-            const T a = As[m][r];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[q] += a * Bs[16 * cq + q][m];
-        }
-        __syncthreads();
-    }
-    // X_ij = -X_ii T1: As[m][rr] = X_ii(rr, m), Bs[col][m] = T1(m, col)
-    for (int e = tid; e < 4096; e += kThreads) {
-        const int rr = e & 63, m = e >> 6;
-        As[m][rr] = X[(64 * i + rr) + kSuper * (64 * i + m)];
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) Bs[16 * cq + q][r] = acc[q];
     __syncthreads();
-    T out[16];
+    for (int i = j + 1; i < nblk; ++i) {
+        const int kbi = min(64, sb - 64 * i);
+        // entry (r0 + li, 4 q + kl) of L_ik, rows past kbi masked
+        const T* Lr = pool + nd.front + c0 + 64 * i + min(r0 + li, kbi - 1) + (int64_t)(c0 + kl) * n;
+        T a[16], an[16];
+        auto load = [&](T (&x)[16], int k) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) out[q] = T(0);
-#pragma unroll 4
-    for (int m = 0; m < 64; ++m) {
-        const T a = As[m][r];
+            for (int q = 0; q < 16; ++q) x[q] = Lr[(int64_t)(64 * k + 4 * q) * n];
+        };
+        load(a, j);
+        acc_t acc = {0, 0, 0, 0};
+        for (int k = j; k < i; ++k) {
+            if (k + 1 < i)
+                load(an, k + 1);
+            else
 #pragma unroll
-        for (int q = 0; q < 16; ++q) out[q] += a * Bs[16 * cq + q][m];
+                for (int q = 0; q < 16; ++q) an[q] = inv[4096 * i + 4 * q + kl + 64 * (r0 + li)];
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+                acc = Mfma<T>::mma(r0 + li < kbi ? a[q] : T(0), Xs[k][4 * q + kl][li], acc);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) a[q] = an[q];
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Ss[r0 + Mfma<T>::row(lane, v)][li] = acc[v];
+        __syncthreads();
+        acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc = Mfma<T>::mma(a[q], Ss[4 * q + kl][li], acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = r0 + Mfma<T>::row(lane, v);
+            Xs[i][r][li] = -acc[v];
+            X[64 * i + r + kSuper * li] = -acc[v];
+        }
+        __syncthreads();
     }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) X[(64 * i + r) + kSuper * (64 * j + 16 * cq + q)] = -out[q];
 }
 
 // The W and V blocks of the superblock matrices (tasks with j >= 4, see

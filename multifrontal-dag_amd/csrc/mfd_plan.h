@@ -103,11 +103,9 @@ struct SolveTask {
 // (whole solve or forward part; backward part), the stop word.
 constexpr int kSolveTicket = 0, kSolveTicketBwd = 16, kSolveStop = 32, kSolveCtl = 64;
 
-// One 64 x 64 block (i, j) of superblock u's matrices: j = i copies the
-// stored 64 x 64 inverse (and clears the row's blocks above the diagonal,
-// or the whole row past the superblock's width); j < i forms
-// X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj; 4 <= j < 8 forms block (i, j - 4)
-// of W; j >= 8 block (i, j - 8) of V.
+// Part of superblock u's matrices.  k_superinv: columns [16 j, 16 j + 16) of
+// X (i unused).  k_superwv: 64 x 64 block (i, j - 4) of W, 4 <= j < 8, or
+// block (i, j - 8) of V, j >= 8.
 struct SuperInvTask {
     int node, u, i, j;
     int64_t xoff;

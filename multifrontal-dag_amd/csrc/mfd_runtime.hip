@@ -1202,9 +1202,8 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
     for (; gnext < G; ++gnext) ok(hipStreamWaitEvent(st, h->fill_ev[gnext], 0));
     if (hybrid) ok(host_join(h, st));
     // superblock inverses of the solves, after every front is final
-    for (int dist = 0; dist <= 4; ++dist)
-        launch_superinv<T>(pool, sinv_of<T>(h), h->d_nodes, h->d_xinv + h->sp.xinv_ptr[dist],
-                           h->sp.xinv_ptr[dist + 1] - h->sp.xinv_ptr[dist], dist == 4, st);
+    launch_superinv<T>(pool, sinv_of<T>(h), h->d_nodes, h->d_xinv, h->sp.nx, false, st);
+    launch_superinv<T>(pool, sinv_of<T>(h), h->d_nodes, h->d_xinv + h->sp.nx, (int)h->sp.xinv.size() - h->sp.nx, true, st);
     return err;
 }
 

@@ -51,28 +51,24 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
             xoff[s] = P.sinv_elems;
             P.sinv_elems += nsup(s) * kSuperMats;
         }
-    for (int dist = 0; dist <= 4; ++dist) {
-        P.xinv_ptr[dist] = (int)P.xinv.size();
+    for (int wv = 0; wv < 2; ++wv) {
+        if (wv) P.nx = (int)P.xinv.size();
         for (int s = 0; s < m; ++s) {
             if (xoff[s] < 0) continue;
             const int c = nodes[s].c;
             for (int u = 0; u * kSuper < c; ++u) {
                 const int64_t xo = xoff[s] + u * kSuperMats;
-                if (dist == 4) {
-                    if (u > 0)
-                        for (int i = 0; i < 4; ++i)
-                            for (int j = 0; j < 4; ++j) P.xinv.push_back(SuperInvTask{s, u, i, 4 + j, xo});
-                    if ((u + 1) * kSuper < c)
-                        for (int i = 0; i < 4; ++i)
-                            for (int j = 0; j < 4; ++j) P.xinv.push_back(SuperInvTask{s, u, i, 8 + j, xo});
+                if (!wv) {
+                    for (int j = 0; j < kSuper / 16; ++j) P.xinv.push_back(SuperInvTask{s, u, 0, j, xo});
                     continue;
                 }
-                for (int i = dist; i < 4; ++i)
-                    if (dist == 0 || u * kSuper + 64 * i < c) P.xinv.push_back(SuperInvTask{s, u, i, i - dist, xo});
+                for (int i = 0; u > 0 && i < 4; ++i)
+                    for (int j = 0; j < 4; ++j) P.xinv.push_back(SuperInvTask{s, u, i, 4 + j, xo});
+                for (int i = 0; (u + 1) * kSuper < c && i < 4; ++i)
+                    for (int j = 0; j < 4; ++j) P.xinv.push_back(SuperInvTask{s, u, i, 8 + j, xo});
             }
         }
     }
-    P.xinv_ptr[5] = (int)P.xinv.size();
 
     // whole[s]: the front's update rows go with its pivot block
     std::vector<char> whole(m, 0);

@@ -22,11 +22,9 @@ struct SolvePlan {
     std::vector<Gather> gat;
     std::vector<int> gsrc;
     std::vector<int> grow;  // global row (0-based) of every update row
-    // blocks of the superblock matrices: X by block distance i - j
-    // ([xinv_ptr[d], xinv_ptr[d + 1]), d = 0..3), then W and V
-    // ([xinv_ptr[4], xinv_ptr[5]))
+    // the superblock matrices: X's columns (up to nx), then the blocks of W and V
     std::vector<SuperInvTask> xinv;
-    int xinv_ptr[6] = {};
+    int nx = 0;
     int64_t sinv_elems = 0;
     int64_t plane = 0;  // entries per right-hand side of the plane array
     int nflags = 0;     // counters per group of right-hand sides
