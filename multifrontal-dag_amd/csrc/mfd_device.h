@@ -30,20 +30,15 @@ template <> struct Mfma<float> {
     static __device__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-// 1 / sqrt(d): the hardware estimate (v_rsq) refined by Newton-Raphson
-// steps r <- r + (r / 2) (1 - d r^2), each squaring the relative error (two
-// for double, one for float): within a few ulp of the exact value, with a
-// dependent chain of seven steps where a correctly rounded sqrt and
-// division take about twenty.
+// 1 / sqrt(d): the hardware estimate r (v_rsq, good to about 2^-23) refined
+// with e = 1 - d r^2: in double one third-order step r + r e (1/2 + 3/8 e),
+// whose chain is two operations shorter than two Newton-Raphson steps, in
+// float one Newton-Raphson step: within a few ulp of the exact value, where a
+// correctly rounded sqrt and division take about twenty dependent steps.
 __device__ __forceinline__ double rsqrt_nr(double d)
 {
-    double r = __builtin_amdgcn_rsq(d);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const double e = fma(-(d * r), r, 1.0);
-        r = fma(0.5 * r, e, r);
-    }
-    return r;
+    const double r = __builtin_amdgcn_rsq(d), e = fma(-(d * r), r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
 }
 __device__ __forceinline__ float rsqrt_nr(float d)
 {
@@ -51,6 +46,10 @@ __device__ __forceinline__ float rsqrt_nr(float d)
     const float e = fmaf(-(d * r), r, 1.0f);
     return fmaf(0.5f * r, e, r);
 }
+// Computes v here: left to itself the compiler puts the updates of a chain
+// off until each value is needed and keeps every operand in registers till then.
+template <typename T> __device__ __forceinline__ void pin(T& v) { asm volatile("" : "+v"(v)); }
+
 // a / b given rb ~ 1 / b (within a few ulp): q = a rb, then one correction
 // with the exact residual a - q b (Markstein), which returns a / b exactly
 // whenever it is representable and is within an ulp of it otherwise.  Its

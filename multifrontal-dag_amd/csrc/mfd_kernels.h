@@ -34,9 +34,9 @@ template <typename T>
 void launch_front_wg(T* pool, const NodeDev* nodes, const int* tasks, int count, int* info, long long* clocks,
                      hipStream_t st, int lowp = 0);
 template <typename T>
-void launch_diag(T* pool, const NodeDev* nodes, const DiagTask* tasks, int count, int* info, hipStream_t st);
+void launch_diag(T* pool, const DiagTask* tasks, int count, int* info, hipStream_t st);
 template <typename T>
-void launch_upd_diag(T* pool, const NodeDev* nodes, const DiagTask* diags, int ndiag, const GemmTask* tiles, int ntiles,
+void launch_upd_diag(T* pool, const DiagTask* diags, int ndiag, const GemmTask* tiles, int ntiles,
                      int* info, hipStream_t st);
 // kind 0: panel TRSM tiles; 1: in-panel update; 2: Schur update (mode 3
 // tiles read local_index from lidx).  lowp (FP32 fronts, kinds 1 and 2): 1

@@ -78,44 +78,57 @@ template <typename T> struct Front64 {
 };
 
 // Panel b16 .. b16 + cb - 1 (cb <= 16; FULL: cb == 16) by one wave, rows
-// b16 .. 63 on their lanes.  Column k: d = x_k on lane k, L_kk = sqrt(d),
-// l = x_k / L_kk (quot: exact whenever the quotient is representable); the
-// column goes to LDS at once, its entry for row k+1 is broadcast by readlane
-// and applied to column k+1 (the next pivot needs it), and its entries for
-// rows k+2 .. 15 are read back from LDS (the wave's LDS accesses complete in
-// issue order, so the reads see the column) and applied to those columns in
-// step k+1, beside that step's pivot chain, by when the reads have landed.
-// A partial panel also updates the block's columns past cb (trailing
+// b16 .. 63 on their lanes.  Column k: d = x_k on lane k, rs = 1 / sqrt(d);
+// x_k rs, with row k+1's entry (from its lane by readlane) times rs, updates
+// column k+1 at once (the next pivot needs it); beside that chain L_kk =
+// sqrt(d) and l = x_k / L_kk (quot: exact whenever the quotient is
+// representable) go to LDS, and l's entries for rows k+2 .. 15 are read back
+// (the wave's LDS accesses complete in issue order, so the reads see the
+// column) and applied to those columns in step k+1, by when the reads have
+// landed.  A partial panel also updates the block's columns past cb (trailing
 // columns of the front) by all of its columns, and stores them.  Every x_j
 // receives its updates in column order, as in the plain loop.  The first
-// non-positive pivot is recorded.
+// non-positive pivot is recorded (each pivot stays on its row's lane; one look
+// at all of them at the end).
+// One wave issues at most an instruction every four cycles, so the panel is
+// bound by its instruction count as much as by the chain: 3900 cycles for 16
+// columns in FP64, 3240 in FP32; with the chain through the finished column,
+// a check per pivot and masked stores 4940 and 4050.
 template <typename T, bool FULL>
 __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, int* info, int col0)
 {
     const int r = threadIdx.x & 63, row = b16 + r;
     const bool live = row < n;
-    T x[16], v[16];
+    const int at = live ? row : 64;  // (column slot 64 of a row is not used)
+    T x[16], v[16], piv = T(1);
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         x[j] = (live && (r >= 16 || j <= r)) ? S.A[b16 + j][row] : T(0);
         v[j] = T(0);
     }
-    int bad = 16;
     T lp = T(0);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         if (FULL || k < cb) {  // no early exit: the loop stays unrolled, x and v in registers
-            const T d = bcast(x[k], k);
-            bad = (!(d > T(0)) && bad == 16) ? k : bad;
-            const T rs = rsqrt_nr(d), sd = sqrt_from_rs(d, rs);
-            // column k-1's updates of columns k+1 .. 15 (its entries read in step k-1)
+            const T d = bcast(x[k], k), rs = rsqrt_nr(d);
+            // column k-1's updates of columns k+1 .. 15 (its entries read in
+            // step k-1), with column k's of column k+1
+            if (k + 1 < 16) {
+                const T u = bcast(x[k], k + 1);
+                x[k + 1] -= lp * v[k + 1];
+                if (FULL || k + 1 < cb) x[k + 1] -= (x[k] * rs) * (u * rs);
+                pin(x[k + 1]);
+            }
+            piv = r == k ? d : piv;
+            const T sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs), l = r == k ? sd : q;
+            x[k] = l;
+            S.A[b16 + k][at] = l;
+            S.rs[b16 + k] = rs;
 #pragma unroll
-            for (int j = k + 1; j < 16; ++j) x[j] -= lp * v[j];
-            const T l = quot(x[k], sd, rs);
-            x[k] = r == k ? sd : l;
-            if (live) S.A[b16 + k][row] = x[k];
-            if (r == 0) S.rs[b16 + k] = rs;
-            if (k + 1 < 16 && (FULL || k + 1 < cb)) x[k + 1] -= l * bcast(l, k + 1);
+            for (int j = k + 2; j < 16; ++j) {
+                x[j] -= lp * v[j];
+                pin(x[j]);
+            }
             lp = l;
             __builtin_amdgcn_wave_barrier();  // the reads below stay after the store above
 #pragma unroll
@@ -136,7 +149,8 @@ __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, i
                 if (j >= cb) S.A[b16 + j][row] = x[j];
         }
     }
-    if (bad < 16 && r == 0) atomicMin(info, col0 + b16 + bad + 1);
+    const unsigned long long bad = __ballot(!(piv > T(0)));
+    if (bad && r == 0) atomicMin(info, col0 + b16 + __ffsll(bad));
 }
 
 // Inverse of panel b16's 16 x 16 diagonal block of L (one wave): lane r < 16
@@ -172,17 +186,24 @@ __device__ __forceinline__ void trailing16(Front64<T>& S, int b16, int cb, int I
 {
     typedef typename Mfma<T>::acc_t acc_t;
     const int lane = threadIdx.x & 63, li = lane & 15;
-    acc_t acc = {0, 0, 0, 0};
+    // two chains of products, subtracted at the end: added to A_IJ one by one
+    // they would round at its magnitude each time
+    acc_t acc = {0, 0, 0, 0}, acc2 = {0, 0, 0, 0}, old;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) old[v] = S.A[16 * J + li][16 * I + Mfma<T>::row(lane, v)];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int kk = 4 * q + (lane >> 4);
         const bool ok = kk < cb;
         const T a = ok ? S.A[b16 + kk][16 * I + li] : T(0);
         const T b = ok ? S.A[b16 + kk][16 * J + li] : T(0);
-        acc = Mfma<T>::mma(a, b, acc);
+        if (q & 1)
+            acc2 = Mfma<T>::mma(a, b, acc2);
+        else
+            acc = Mfma<T>::mma(a, b, acc);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) S.A[16 * J + li][16 * I + Mfma<T>::row(lane, v)] -= acc[v];
+    for (int v = 0; v < 4; ++v) S.A[16 * J + li][16 * I + Mfma<T>::row(lane, v)] = old[v] - (acc[v] + acc2[v]);
 }
 
 // X_ij = -inv(L_ii) sum_{k=j}^{i-1} L_ik X_kj (one wave; staging in Ts[w]).
@@ -191,26 +212,34 @@ __device__ __forceinline__ void inverse16(Front64<T>& S, int i, int j, int w)
 {
     typedef typename Mfma<T>::acc_t acc_t;
     const int lane = threadIdx.x & 63, li = lane & 15;
-    acc_t acc = {0, 0, 0, 0};
+    acc_t acc = {0, 0, 0, 0}, acc2 = {0, 0, 0, 0};  // two chains of products
     for (int k = j; k < i; ++k) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int kk = 4 * q + (lane >> 4);
-            acc = Mfma<T>::mma(S.A[16 * k + kk][16 * i + li], S.X[16 * j + li][16 * k + kk], acc);
+            const T a = S.A[16 * k + kk][16 * i + li], b = S.X[16 * j + li][16 * k + kk];
+            if (q & 1)
+                acc2 = Mfma<T>::mma(a, b, acc2);
+            else
+                acc = Mfma<T>::mma(a, b, acc);
         }
     }
     wave_sync();
 #pragma unroll
-    for (int v = 0; v < 4; ++v) S.Ts[w][Mfma<T>::row(lane, v)][li] = acc[v];
+    for (int v = 0; v < 4; ++v) S.Ts[w][Mfma<T>::row(lane, v)][li] = acc[v] + acc2[v];
     wave_sync();
-    acc_t acc2 = {0, 0, 0, 0};
+    acc = acc2 = acc_t{0, 0, 0, 0};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int m = 4 * q + (lane >> 4);
-        acc2 = Mfma<T>::mma(S.X[16 * i + m][16 * i + li], S.Ts[w][m][li], acc2);
+        const T a = S.X[16 * i + m][16 * i + li], b = S.Ts[w][m][li];
+        if (q & 1)
+            acc2 = Mfma<T>::mma(a, b, acc2);
+        else
+            acc = Mfma<T>::mma(a, b, acc);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) S.X[16 * j + li][16 * i + Mfma<T>::row(lane, v)] = -acc2[v];
+    for (int v = 0; v < 4; ++v) S.X[16 * j + li][16 * i + Mfma<T>::row(lane, v)] = -(acc[v] + acc2[v]);
 }
 
 // All 256 threads: loads the lower n x n block at g (leading dimension ld),
@@ -218,8 +247,8 @@ __device__ __forceinline__ void inverse16(Front64<T>& S, int i, int j, int w)
 // stores L^{-T} of the c x c factor column-major at inv (64 x 64,
 // zero-padded: inv[r + 64 q] = L^{-1}[q][r]).  A pivot that is not positive
 // records the global column col0 + k + 1 in *info (smallest wins).
-// Same, with S.A already holding the block (lower part, zero elsewhere)
-// and S.X zeroed, both visible to the workgroup.
+// Same, with S.A already holding the block (lower part, zero past row n)
+// and S.X zero above the diagonal blocks, both visible to the workgroup.
 template <typename T>
 __device__ __forceinline__ void factor_dense64_loaded(Front64<T>& S, T* g, int64_t ld, int n, int c, int* info,
                                                       int col0, T* inv)
@@ -609,6 +638,20 @@ __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ld
     c[1][0] = c10;
     c[1][1] = c11;
 }
+// Cs[col][row] = c, in the layout of tile_mma's result.
+template <typename T>
+__device__ __forceinline__ void stage_acc(const typename Mfma<T>::acc_t (&c)[2][2], T (*Cs)[kTile + 1])
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32, q0 = wc + (lane & 15);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Cs[q0 + 16 * j][wr + 16 * i + Mfma<T>::row(lane, v)] = c[i][j][v];
+}
+
 // The same product staged as Cs[col][row]; ends with a barrier.
 template <typename T, int LP = kNative, int TB = -1, int NB = 1>
 __device__ __forceinline__ void tile_product(const T* A, int lda, const T* B, int ldb, bool tb, int m, int n, int k,
@@ -616,16 +659,7 @@ __device__ __forceinline__ void tile_product(const T* A, int lda, const T* B, in
 {
     typename Mfma<T>::acc_t c[2][2];
     tile_mma<T, LP, TB, NB>(A, lda, B, ldb, tb, m, n, k, L, c);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32, q0 = wc + (lane & 15);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int r = wr + Mfma<T>::row(lane, v);
-        Cs[q0][r] = c[0][0][v];
-        Cs[q0 + 16][r] = c[0][1][v];
-        Cs[q0][r + 16] = c[1][0][v];
-        Cs[q0 + 16][r + 16] = c[1][1][v];
-    }
+    stage_acc<T>(c, Cs);
     __syncthreads();
 }
 
@@ -681,49 +715,6 @@ __device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T*
     c[1][0] = c10;
     c[1][1] = c11;
 }
-// c += sum_kk Am[kk][row] Bm[kk][col] over kk < 64 with both operands in
-// LDS (zero past the product's true K).  Same wave layout as tile_mma;
-// fully unrolled so the accumulators stay in place; no barrier.
-template <typename T>
-__device__ __forceinline__ void lds_mma(const T (*Am)[kTile + 1], const T (*Bm)[kTile + 1],
-                                        typename Mfma<T>::acc_t (&c)[2][2])
-{
-    typedef typename Mfma<T>::acc_t acc_t;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wr = (wv & 1) * 32 + (lane & 15), wc = (wv >> 1) * 32 + (lane & 15), kl = lane >> 4;
-    acc_t c00 = c[0][0], c01 = c[0][1], c10 = c[1][0], c11 = c[1][1];
-#pragma unroll
-    for (int k0 = 0; k0 < kTile; k0 += 4) {
-        const T a0 = Am[k0 + kl][wr], a1 = Am[k0 + kl][wr + 16];
-        const T b0 = Bm[k0 + kl][wc], b1 = Bm[k0 + kl][wc + 16];
-        c00 = Mfma<T>::mma(a0, b0, c00);
-        c01 = Mfma<T>::mma(a0, b1, c01);
-        c10 = Mfma<T>::mma(a1, b0, c10);
-        c11 = Mfma<T>::mma(a1, b1, c11);
-    }
-    c[0][0] = c00;
-    c[0][1] = c01;
-    c[1][0] = c10;
-    c[1][1] = c11;
-}
-// Cs[col][row] = c (sub = false) or -= c (sub = true), in the layout of
-// tile_mma's result.
-template <typename T>
-__device__ __forceinline__ void stage_acc(const typename Mfma<T>::acc_t (&c)[2][2], T (*Cs)[kTile + 1], bool sub)
-{
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32, q0 = wc + (lane & 15);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                T& dst = Cs[q0 + 16 * j][wr + 16 * i + Mfma<T>::row(lane, v)];
-                dst = sub ? dst - c[i][j][v] : c[i][j][v];
-            }
-}
-
 // One GemmTask per workgroup (see mfd_plan.h): C -= A B^T (mode 0: the
 // DSYRK/DGEMM updates) or C = A B^T with B transposed in memory (mode 1: the
 // panel TRSM as a product with the stored L^{-T} of the diagonal block, C
@@ -764,7 +755,7 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T,
 #pragma unroll
         for (int j = 0; j < 16; ++j) cpre[j] = C[rc + (int64_t)min((tid >> 6) + 4 * j, t.n - 1) * t.ldc];
     }
-    stage_acc<T>(acc, Cs, false);
+    stage_acc<T>(acc, Cs);
     __syncthreads();
     if (t.mode == 2) {
         // Cs = C - A B^T, then C = Cs D^T (D = L^{-1}, stored transposed)
@@ -776,7 +767,7 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T,
         __syncthreads();
         typename Mfma<T>::acc_t c[2][2];
         tile_mma_ldsA<T, NB>(Cs, pool + t.d, kPanel, true, t.n, t.kd, L, c);
-        stage_acc<T>(c, Cs, false);
+        stage_acc<T>(c, Cs);
         __syncthreads();
         if (row < t.m)
             for (int col = tid >> 6; col < t.n; col += 4) C[row + (int64_t)col * t.ldc] = Cs[col][row];
@@ -871,14 +862,22 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 3 : 4) void k_gemm(T* pool, c
 // (and storing) its rows' panel-s entries on the way, so no task of the
 // launch reads what another one writes: the chain of diagonal blocks, the
 // critical path, advances one block per launch.
+//
+// The diagonal task sends for all its operands at once and multiplies in
+// strips: a wave has 16 rows of the block, so that its rows go from product
+// to product without a barrier, and L_s^{-T}'s zeros and the block's upper
+// triangle are left out (40 and at most 48 products of 16 x 16 x 4 a wave
+// where whole squares take 64; 64 cycles each in FP64).  A step with nothing
+// beside it takes 28.5 us in FP64 (30.5 with the operands in two batches and
+// whole squares), 20 in FP32 (23).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const NodeDev* nodes, const DiagTask* diags, int ndiag,
-                                                       const GemmTask* tiles, int* info)
+__global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const DiagTask* diags, int ndiag, const GemmTask* tiles,
+                                                       int* info)
 {
     __shared__ Front64<T> S;
     __shared__ union {
         TileLds<T, 2> L;      // GEMM tasks
-        T B[2][64][kTile + 1];  // diagonal task: staged operands
+        T B[2][64][kTile + 1];  // diagonal task: L_s^{-T}; block s's rows in the pending panels
     } U;
     if ((int)blockIdx.x >= ndiag) {
         const GemmTask g = tiles[blockIdx.x - ndiag];
@@ -886,115 +885,130 @@ __global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const NodeDev* n
         if (g.syrk > 0) trsm_syrk<T, 2>(pool, g, U.L, S.A);
         return;
     }
+    typedef typename Mfma<T>::acc_t acc_t;
     const DiagTask t = diags[blockIdx.x];
-    const NodeDev nd = nodes[t.node];
-    const int n = nd.n, kb = t.kb, kp = t.kprev, kpp = t.kpp;
-    T* front = pool + nd.front;
+    const int n = t.n, kb = t.kb, kp = t.kprev, kpp = t.kpp;
+    T* front = pool + t.front;
     const T* C = front + t.k0 + (int64_t)t.k0 * n;                         // block s+1
     T* Pg = front + t.k0 + (int64_t)(t.k0 - kp) * n;                       // its rows in panel s
     const T* Xd = front + t.k0 + (int64_t)(t.k0 - kp - kpp) * n;          // its rows in the pending panels
     const T* Xs = front + (t.k0 - kp) + (int64_t)(t.k0 - kp - kpp) * n;   // block s's rows in them
-    const T* inv = pool + nd.inv + (int64_t)((t.k0 - kp) / kPanel) * kPanel * kPanel;  // L_s^{-T}
+    const T* inv = pool + t.inv - kPanel * kPanel;                         // L_s^{-T}
     const int tid = threadIdx.x, row = tid & 63, c4 = tid >> 6;
-    // Stage every operand with all loads of a batch in flight: entry (row,
-    // c4 + 4 j) of each 64 x 64 block; positions past the block read entry 0
-    // and are masked after the loads.
-    {
-        T r0[16], r1[16];
-        const unsigned ra = row < kb ? row : 0u, rb = row < kp ? row : 0u;
+    const int lane = tid & 63, li = lane & 15, kl = lane >> 4, r0 = 16 * c4;  // the wave's strip of rows
+    // Entry (row, c4 + 4 j) of each 64 x 64 block, and of the strip's rows of
+    // the pending panels the MFMA operands (r0 + li, 4 q + kl); positions past
+    // the block read entry 0 and are masked after the loads.
+    const unsigned ra = row < kb ? row : 0u, rb = row < kp ? row : 0u, rx = r0 + li < kb ? r0 + li : 0u;
+    auto load_pending = [&](int q0, T (&xs)[16], T (&xd)[16]) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int cs = q0 + c4 + 4 * j, cd = q0 + 4 * j + kl;
+            xs[j] = ld_off(Xs, rb + (cs < kpp ? cs : 0u) * (unsigned)n);
+            xd[j] = ld_off(Xd, rx + (cd < kpp ? cd : 0u) * (unsigned)n);
+        }
+    };
+    auto stage_pending = [&](int q0, const T (&xs)[16]) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int col = c4 + 4 * j;
-            const unsigned cd = col < kpp ? col : 0u;
-            r0[j] = ld_off(Xd, ra + cd * (unsigned)n);
-            r1[j] = ld_off(Xs, rb + cd * (unsigned)n);
+            U.B[1][col][row] = (row < kp && q0 + col < kpp) ? xs[j] : T(0);
         }
+    };
+    T xs[16], xd[16], rc[16], rp[16], ri[16];
+    if (kpp > 0) load_pending(0, xs, xd);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int col = c4 + 4 * j;
-            U.B[0][col][row] = (row < kb && col < kpp) ? r0[j] : T(0);
-            U.B[1][col][row] = (row < kp && col < kpp) ? r1[j] : T(0);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int col = c4 + 4 * j;
-            const unsigned ca = col <= row && row < kb ? col : 0u, cp = col < kp ? col : 0u;
-            r0[j] = ld_off(C, ra + ca * (unsigned)n);
-            r1[j] = ld_off((const T*)Pg, ra + cp * (unsigned)n);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int col = c4 + 4 * j;
-            S.A[col][row] = (row < kb && col <= row) ? r0[j] : T(0);
-            S.X[col][row] = (row < kb && col < kp) ? r1[j] : T(0);
-        }
+    for (int j = 0; j < 16; ++j) {
+        const int col = c4 + 4 * j;
+        rp[j] = ld_off((const T*)Pg, ra + (col < kp ? col : 0u) * (unsigned)n);
+        ri[j] = ld_off(inv, (unsigned)(tid + kThreads * j));
+        rc[j] = ld_off(C, ra + (col <= row && row < kb ? col : 0u) * (unsigned)n);
     }
-    // inverse of block s in flight during the first products:
-    // B[k][j] = L_s^{-1}[j][k] = inv[k + 64 j]
-    T rv[16];
+    if (kpp > 0) stage_pending(0, xs);
 #pragma unroll
-    for (int p = 0; p < 16; ++p) rv[p] = ld_off(inv, (unsigned)(tid + kThreads * p));
+    for (int j = 0; j < 16; ++j) {
+        const int col = c4 + 4 * j, e = tid + kThreads * j, k = e & 63, i = e >> 6;
+        S.X[col][row] = (row < kb && col < kp) ? rp[j] : T(0);
+        U.B[0][k][i] = (k < kp && i < kp) ? ri[j] : T(0);  // B[k][j] = L_s^{-1}[j][k] = inv[k + 64 j]
+        S.A[col][row] = (row < kb && col <= row) ? rc[j] : T(0);
+    }
     __syncthreads();
-    typedef typename Mfma<T>::acc_t acc_t;
-    acc_t c[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};
+    // the pending panels (64 columns per round): S.X -= Xd Xs^T (they have
+    // been applied to the block itself by the TRSM tile of its rows)
     if (kpp > 0) {
-        // the pending panels (64 columns per round): S.A -= Xd Xd^T (unless
-        // the previous step's TRSM tile of these rows has applied it),
-        // S.X -= Xd Xs^T
-        acc_t c2[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};
-        for (int q = 0; q < kpp; q += 64) {
-            if (q > 0) {
-                T r0[16], r1[16];
-                const unsigned ra = row < kb ? row : 0u, rb = row < kp ? row : 0u;
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const int col = q + c4 + 4 * j;
-                    const unsigned cd = col < kpp ? col : 0u;
-                    r0[j] = ld_off(Xd, ra + cd * (unsigned)n);
-                    r1[j] = ld_off(Xs, rb + cd * (unsigned)n);
-                }
+        acc_t c[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+        for (int q0 = 0; q0 < kpp; q0 += 64) {
+            if (q0 > 0) {
+                load_pending(q0, xs, xd);
                 __syncthreads();
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const int col = c4 + 4 * j;
-                    U.B[0][col][row] = (row < kb && q + col < kpp) ? r0[j] : T(0);
-                    U.B[1][col][row] = (row < kp && q + col < kpp) ? r1[j] : T(0);
-                }
+                stage_pending(q0, xs);
                 __syncthreads();
             }
-            if (!t.applied) lds_mma<T>(U.B[0], U.B[0], c);
-            lds_mma<T>(U.B[0], U.B[1], c2);
-        }
-        if (!t.applied) stage_acc<T>(c, S.A, true);
-        stage_acc<T>(c2, S.X, true);
-    }
-    __syncthreads();
 #pragma unroll
-    for (int p = 0; p < 16; ++p) {
-        const int e = tid + kThreads * p, k = e & 63, j = e >> 6;
-        U.B[0][k][j] = (k < kp && j < kp) ? rv[p] : T(0);
+            for (int q = 0; q < 16; ++q) {
+                const T a = (r0 + li < kb && q0 + 4 * q + kl < kpp) ? xd[q] : T(0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) c[j] = Mfma<T>::mma(a, U.B[1][4 * q + kl][16 * j + li], c[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S.X[16 * j + li][r0 + Mfma<T>::row(lane, v)] -= c[j][v];
+        wave_sync();
+    }
+    // X = S.X L_s^{-T}, whose column block j has rows up to its own
+    {
+        acc_t c[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const T a = S.X[4 * q + kl][r0 + li];
+#pragma unroll
+            for (int j = q / 4; j < 4; ++j) c[j] = Mfma<T>::mma(a, U.B[0][4 * q + kl][16 * j + li], c[j]);
+        }
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S.X[16 * j + li][r0 + Mfma<T>::row(lane, v)] = c[j][v];
     }
     __syncthreads();
-    // X = S.X L_s^{-T}, stored into the front (these rows are this task's)
-    c[0][0] = c[0][1] = c[1][0] = c[1][1] = acc_t{0, 0, 0, 0};
-    lds_mma<T>(S.X, U.B[0], c);
-    __syncthreads();
-    stage_acc<T>(c, S.X, false);
-    __syncthreads();
+    // stored into the front (these rows are this task's), and S.A -= X X^T, a
+    // wave every fourth of the ten lower 16 x 16 blocks
     for (int col = c4; col < kp; col += 4)
         if (row < kb) Pg[row + (int64_t)col * n] = S.X[col][row];
-    // panel s: S.A -= X X^T
-    c[0][0] = c[0][1] = c[1][0] = c[1][1] = acc_t{0, 0, 0, 0};
-    lds_mma<T>(S.X, S.X, c);
-    stage_acc<T>(c, S.A, true);
-    __syncthreads();
-    for (int col = c4; col < kTile; col += 4) {
-        S.X[col][row] = T(0);
-        if (!(row < kb && col <= row)) S.A[col][row] = T(0);
+    {
+        // block rows and columns of the ten, two bits each
+        constexpr unsigned bi = 0xffa94, bj = 0xe4910;
+        int I[3], J[3];
+        acc_t c[3] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const int b = min(c4 + 4 * p, 9);
+            I[p] = 16 * ((bi >> 2 * b) & 3) + li, J[p] = 16 * ((bj >> 2 * b) & 3) + li;
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const T* x = S.X[4 * q + kl];
+            c[0] = Mfma<T>::mma(x[I[0]], x[J[0]], c[0]);
+            c[1] = Mfma<T>::mma(x[I[1]], x[J[1]], c[1]);
+            if (c4 < 2) c[2] = Mfma<T>::mma(x[I[2]], x[J[2]], c[2]);
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+            if (p < 2 || c4 < 2) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) S.A[J[p]][I[p] - li + Mfma<T>::row(lane, v)] -= c[p][v];
+            }
     }
     __syncthreads();
-    factor_dense64_loaded<T>(S, front + t.k0 + (int64_t)t.k0 * n, n, kb, kb, info, nd.first + t.k0,
-                             pool + nd.inv + (int64_t)(t.k0 / kPanel) * kPanel * kPanel);
+    // the inverse is zero above its diagonal blocks
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int col = c4 + 4 * j;
+        if (row < (col & ~15)) S.X[col][row] = T(0);
+    }
+    factor_dense64_loaded<T>(S, front + t.k0 + (int64_t)t.k0 * n, n, kb, kb, info, t.first + t.k0, pool + t.inv);
 }
 
 // C -= A B^T on 128 x 128 tiles (GemmTask with m, n <= 128, mode 0 or 3):
@@ -1211,13 +1225,12 @@ __global__ __launch_bounds__(kThreads) void k_gemm_fix(T* pool, const GemmTask* 
 // into the front, and the inverse of L stored for the panel TRSM and the
 // solves.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_diag(T* pool, const NodeDev* nodes, const DiagTask* tasks, int* info)
+__global__ __launch_bounds__(kThreads) void k_diag(T* pool, const DiagTask* tasks, int* info)
 {
     const DiagTask t = tasks[blockIdx.x];
-    const NodeDev nd = nodes[t.node];
     __shared__ Front64<T> S;
-    factor_dense64<T>(S, pool + nd.front + t.k0 + (int64_t)t.k0 * nd.n, nd.n, t.kb, t.kb, info, nd.first + t.k0,
-                      pool + nd.inv + (int64_t)(t.k0 / kPanel) * kPanel * kPanel);
+    factor_dense64<T>(S, pool + t.front + t.k0 + (int64_t)t.k0 * t.n, t.n, t.kb, t.kb, info, t.first + t.k0,
+                      pool + t.inv);
 }
 
 // ---------------------------------------------------------- medium fronts
@@ -1682,16 +1695,16 @@ void launch_front_wg(T* pool, const NodeDev* nodes, const int* tasks, int count,
     hipLaunchKernelGGL((k_front_wg<T, kNative>), dim3(count), dim3(kThreads), 0, st, pool, nodes, tasks, info, clocks);
 }
 template <typename T>
-void launch_diag(T* pool, const NodeDev* nodes, const DiagTask* tasks, int count, int* info, hipStream_t st)
+void launch_diag(T* pool, const DiagTask* tasks, int count, int* info, hipStream_t st)
 {
-    if (count > 0) hipLaunchKernelGGL(k_diag<T>, dim3(count), dim3(kThreads), 0, st, pool, nodes, tasks, info);
+    if (count > 0) hipLaunchKernelGGL(k_diag<T>, dim3(count), dim3(kThreads), 0, st, pool, tasks, info);
 }
 template <typename T>
-void launch_upd_diag(T* pool, const NodeDev* nodes, const DiagTask* diags, int ndiag, const GemmTask* tiles, int ntiles,
+void launch_upd_diag(T* pool, const DiagTask* diags, int ndiag, const GemmTask* tiles, int ntiles,
                      int* info, hipStream_t st)
 {
     if (ndiag + ntiles > 0)
-        hipLaunchKernelGGL(k_upd_diag<T>, dim3(ndiag + ntiles), dim3(kThreads), 0, st, pool, nodes, diags, ndiag, tiles,
+        hipLaunchKernelGGL(k_upd_diag<T>, dim3(ndiag + ntiles), dim3(kThreads), 0, st, pool, diags, ndiag, tiles,
                            info);
 }
 template <typename T>
@@ -1790,8 +1803,8 @@ void launch_scatter_rows(double* out, int ld_out, const double* in, int ld_in, c
     template void launch_extend_add<T>(T*, const int*, const NodeDev*, const ExtTask*, int, hipStream_t);              \
     template void launch_small_front<T>(T*, const NodeDev*, const int*, int, int*, hipStream_t);                       \
     template void launch_front_wg<T>(T*, const NodeDev*, const int*, int, int*, long long*, hipStream_t, int);           \
-    template void launch_diag<T>(T*, const NodeDev*, const DiagTask*, int, int*, hipStream_t);                        \
-    template void launch_upd_diag<T>(T*, const NodeDev*, const DiagTask*, int, const GemmTask*, int, int*, hipStream_t); \
+    template void launch_diag<T>(T*, const DiagTask*, int, int*, hipStream_t);                                        \
+    template void launch_upd_diag<T>(T*, const DiagTask*, int, const GemmTask*, int, int*, hipStream_t);                \
     template void launch_gemm<T>(T*, const GemmTask*, int, int, const int*, hipStream_t, int);                         \
     template void launch_superinv<T>(const T*, T*, const NodeDev*, const SuperInvTask*, int, bool, hipStream_t);      \
     template void launch_gemm_seg<T>(T*, const GemmTask*, const SegTask*, const int*, int, const FixTask*, int, T*,  \

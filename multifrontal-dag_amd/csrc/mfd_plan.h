@@ -52,12 +52,14 @@ struct ExtTask {
 // update has applied yet); the factorizing workgroup also forms the
 // panel-s entries of its own rows (their TRSM with block s's inverse) and
 // stores them.
-// applied = 1: the kpp pending columns were already applied to the block
-// itself (by the previous step's TRSM tile of its rows, GemmTask::syrk); the
-// task still applies them to its rows of block s.
+// The kpp pending columns have been applied to the block itself (by the
+// previous step's TRSM tile of its rows, GemmTask::syrk); the task applies
+// them to its rows of block s.  The front's fields are those of its NodeDev
+// (one load less before the operands'), inv the block's own inverse.
 struct DiagTask {
-    int node, k0, kb, kprev;
-    int kpp, applied, pad1, pad2;
+    int64_t front, inv;
+    int node, n, first;
+    int k0, kb, kprev, kpp, pad;
 };
 
 // Superblocks: the solves step over 256-column superblocks u (columns B_u) of

@@ -582,6 +582,11 @@ void build_plan(mfd_handle* h)
                 for (int j = sj; j < std::min(nc, sj + kSquare); ++j)
                     for (int i = std::max(si, j); i < std::min(nr, si + kSquare); ++i) f(i, j);
     };
+    auto diag_task = [&](int s, int k0, int kprev, int kpp) {
+        const NodeDev& d = h->nodes[s];
+        return DiagTask{d.front, d.inv + (int64_t)(k0 / kPanel) * kPanel * kPanel, s, d.n, d.first,
+                        k0, std::min(kPanel, d.c - k0), kprev, kpp, 0};
+    };
     // a wide launch's K chunks (16 columns) divided evenly over at most
     // kSegGroups workgroups (two per CU), no fewer than kSegMin chunks each
     constexpr int kSegGroups = 512, kSegMin = 16;
@@ -698,7 +703,7 @@ void build_plan(mfd_handle* h)
         const int period = period_set > 0 ? period_set : (steps >= kAutoSteps ? 2 : 1);
         {
             int64_t f0 = (int64_t)h->diag.size();
-            for (int s : large) h->diag.push_back(DiagTask{s, 0, std::min(kPanel, h->nodes[s].c), 0, 0, 0, 0, 0});
+            for (int s : large) h->diag.push_back(diag_task(s, 0, 0, 0));
             push(MFD_K_POTRF, f0, (int64_t)h->diag.size());
         }
         int prev_side = -1;
@@ -786,10 +791,7 @@ void build_plan(mfd_handle* h)
             for (int s : large) {
                 const NodeDev& d = h->nodes[s];
                 if (d.c <= k0 + kPanel) continue;
-                // from step 1 on, the previous step's TRSM tile of its rows
-                // has applied the pending panels to the block
-                h->diag.push_back(
-                    DiagTask{s, k0 + kPanel, std::min(kPanel, d.c - k0 - kPanel), kPanel, pend, t >= 1 ? 1 : 0, 0, 0});
+                h->diag.push_back(diag_task(s, k0 + kPanel, kPanel, pend));
             }
             const int64_t ng = (fuse ? f4u : f3) - f1, nd = (int64_t)h->diag.size() - f2;
             // many diagonal tasks (many fronts at this level): the GEMM tiles
@@ -1062,10 +1064,10 @@ template <typename T> void enqueue_launch(mfd_handle* h, const Launch& l, hipStr
         break;
     case MFD_K_POTRF:
         if (l.fused)
-            launch_upd_diag<T>(pool, h->d_nodes, h->d_diag + l.dfirst, l.dcount, h->d_gemm + l.first, l.count, h->d_info,
+            launch_upd_diag<T>(pool, h->d_diag + l.dfirst, l.dcount, h->d_gemm + l.first, l.count, h->d_info,
                                st);
         else
-            launch_diag<T>(pool, h->d_nodes, h->d_diag + l.first, l.count, h->d_info, st);
+            launch_diag<T>(pool, h->d_diag + l.first, l.count, h->d_info, st);
         break;
     case MFD_K_TRSM:
     case MFD_K_UPDATE:
@@ -2661,7 +2663,7 @@ int mfd_get_kernel_work(mfd_handle* h, int k, int s, double* flops, double* byte
             for (int64_t i = d0; i < d0 + dn; ++i) {
                 const DiagTask& t = h->diag[i];
                 const double kb = t.kb, kp = t.kprev, kpp = t.kpp;
-                f += 2.0 * kb * kb * kb / 3.0 + kb * (kb + 1) * (kp + (t.applied ? 0 : kpp)) + 2.0 * kb * kp * kpp +
+                f += 2.0 * kb * kb * kb / 3.0 + kb * (kb + 1) * kp + 2.0 * kb * kp * kpp +
                      kb * kp * kp;
                 b += s * (2.0 * tri(t.kb) + kb * kb + 2.0 * kb * kp + kp * kp + kpp * (kb + kp));
             }

@@ -47,10 +47,6 @@ template <typename T> struct TreeLds {
     int ticket;
 };
 
-// Computes v here: left to itself the compiler puts the updates of a chain
-// off until each value is needed and keeps every operand in registers till then.
-template <typename T> __device__ __forceinline__ void pin(T& v) { asm volatile("" : "+v"(v)); }
-
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // The workgroup's LDS as the out-of-line functions take it.  Out of line, the
@@ -81,24 +77,28 @@ __device__ __attribute__((noinline)) void tree_panel(Lds<T> Sp, int w, int b16, 
         v[j] = T(0);
     }
     __syncthreads();  // every wave has its copy of the diagonal block's rows
-    int bad = 16;
-    T lp = T(0);
+    T lp = T(0), piv = T(1);
+    const int to = live ? row : kTreeFront;  // (past the last row: not used)
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         if (k < cb) {
-            const T d = bcast(x[k], k);
-            bad = (!(d > T(0)) && bad == 16) ? k : bad;
-            const T rs = rsqrt_nr(d), sd = sqrt_from_rs(d, rs);
+            const T d = bcast(x[k], k), rs = rsqrt_nr(d);
+            if (k + 1 < 16) {
+                const T u = bcast(x[k], k + 1);
+                x[k + 1] -= lp * v[k + 1];
+                if (k + 1 < cb) x[k + 1] -= (x[k] * rs) * (u * rs);
+                pin(x[k + 1]);
+            }
+            piv = r == k ? d : piv;
+            const T sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs), l = r == k ? sd : q;
+            x[k] = l;
+            Sp->P[k][to] = l;
+            Sp->rs[k] = rs;
 #pragma unroll
-            for (int j = k + 1; j < 16; ++j) {
+            for (int j = k + 2; j < 16; ++j) {
                 x[j] -= lp * v[j];
                 pin(x[j]);
             }
-            const T l = quot(x[k], sd, rs);
-            x[k] = r == k ? sd : l;
-            if (live) Sp->P[k][row] = x[k];
-            if (w == 0 && r == 0) Sp->rs[k] = rs;
-            if (k + 1 < 16 && k + 1 < cb) x[k + 1] -= l * bcast(l, k + 1);
             lp = l;
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -116,7 +116,8 @@ __device__ __attribute__((noinline)) void tree_panel(Lds<T> Sp, int w, int b16, 
                 if (live) Sp->P[j][row] = x[j];
             }
     }
-    if (w == 0 && bad < 16 && r == 0) atomicMin(info, col0 + b16 + bad + 1);
+    const unsigned long long bad = __ballot(!(piv > T(0)));
+    if (w == 0 && bad && r == 0) atomicMin(info, col0 + b16 + __ffsll(bad));
 }
 
 // Row p of the inverse of panel p's 64-column block, by one wave: the 16 x 16
@@ -347,19 +348,23 @@ template <typename T> __device__ __forceinline__ void tree_front(const TreeArgs<
         // stores, so that no later wait for a load waits for those too)
         pin(val);
         pin(pos);
-        // the panel's product off the tiles to the right, its diagonal tile
+        // the panel's product off the tiles to the right (summed by itself:
+        // accumulated onto the tile it would round at the tile's magnitude
+        // four times instead of once), its diagonal tile
         // to D, and the panel to the front (past the pivots: update columns,
         // which the parent's workgroup reads) by the chain's waves: the
         // inverse's wave reads the front next
 #pragma unroll
         for (int s = 0; s < kOwn; ++s)
             if (tj[s] > b && ti[s] != 255) {
+                typename Mfma<T>::acc_t d = {0, 0, 0, 0};
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int k = 4 * q + g;
                     const T x = S.P[k][16 * ti[s] + li], y = S.P[k][16 * tj[s] + li];
-                    acc[s] = Mfma<T>::mma(k < cb ? -x : T(0), k < cb ? y : T(0), acc[s]);
+                    d = Mfma<T>::mma(k < cb ? x : T(0), k < cb ? y : T(0), d);
                 }
+                acc[s] -= d;
             }
         S.D[tid >> 4][tid & 15] = S.P[tid >> 4][b16 + (tid & 15)];
         if (tid < 16) S.rsd[tid] = S.rs[tid];
