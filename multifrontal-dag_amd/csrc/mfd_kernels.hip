@@ -86,8 +86,12 @@ template <typename T> struct Front64 {
 // (the wave's LDS accesses complete in issue order, so the reads see the
 // column) and applied to those columns in step k+1, by when the reads have
 // landed.  A partial panel also updates the block's columns past cb (trailing
-// columns of the front) by all of its columns, and stores them.  Every x_j
-// receives its updates in column order, as in the plain loop.  The first
+// columns of the front) by all of its columns, and stores them.  After the
+// first panel the 16 lanes past row 63 hold the unit vectors, which the same
+// operations turn into the rows of L_bb^{-T}: the diagonal block's inverse
+// (column id of it to X[b16 + id]; in a partial panel the rows past its cb
+// pivots are not used, and its columns past them are zero in the others).
+// Every x_j receives its updates in column order, as in the plain loop.  The first
 // non-positive pivot is recorded (each pivot stays on its row's lane; one look
 // at all of them at the end).
 // One wave issues at most an instruction every four cycles, so the panel is
@@ -97,13 +101,21 @@ template <typename T> struct Front64 {
 template <typename T, bool FULL>
 __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, int* info, int col0)
 {
-    const int r = threadIdx.x & 63, row = b16 + r;
+    int r = threadIdx.x & 63, diag = 66 * b16;
+    pin(r);  // (the comparisons with it stay here: hoisted, their masks spill)
+    pin(diag);
+    T* const Ad = &S.A[0][0] + diag;  // the panel's diagonal block, by vector address
+    const int row = b16 + r;
     const bool live = row < n;
     const int at = live ? row : 64;  // (column slot 64 of a row is not used)
+    const int id = row - 64;         // the unit vector on this lane
     T x[16], v[16], piv = T(1);
 #pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = S.A[b16 + j][at];
+#pragma unroll
     for (int j = 0; j < 16; ++j) {
-        x[j] = (live && (r >= 16 || j <= r)) ? S.A[b16 + j][row] : T(0);
+        pin(x[j]);  // (read by every lane: no branch around each)
+        x[j] = (live && (r >= 16 || j <= r)) ? x[j] : id == j ? T(1) : T(0);
         v[j] = T(0);
     }
     T lp = T(0);
@@ -120,6 +132,7 @@ __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, i
                 pin(x[k + 1]);
             }
             piv = r == k ? d : piv;
+            pin(piv);
             const T sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs), l = r == k ? sd : q;
             x[k] = l;
             S.A[b16 + k][at] = l;
@@ -132,8 +145,8 @@ __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, i
             lp = l;
             __builtin_amdgcn_wave_barrier();  // the reads below stay after the store above
 #pragma unroll
-            for (int j = k + 2; j < 16; ++j) v[j] = S.A[b16 + k][b16 + j];
-            if (!FULL && k + 1 == cb && k + 1 < 16) v[k + 1] = S.A[b16 + k][b16 + k + 1];
+            for (int j = k + 2; j < 16; ++j) v[j] = Ad[65 * k + j];
+            if (!FULL && k + 1 == cb && k + 1 < 16) v[k + 1] = Ad[65 * k + k + 1];
         }
     }
     if (!FULL) {
@@ -149,11 +162,16 @@ __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, i
                 if (j >= cb) S.A[b16 + j][row] = x[j];
         }
     }
+    if (id >= 0 && id < 16) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) S.X[b16 + id][b16 + j] = x[j];
+    }
     const unsigned long long bad = __ballot(!(piv > T(0)));
     if (bad && r == 0) atomicMin(info, col0 + b16 + __ffsll(bad));
 }
 
-// Inverse of panel b16's 16 x 16 diagonal block of L (one wave): lane r < 16
+// Inverse of panel b16's 16 x 16 diagonal block of L (one wave; the first
+// panel's, whose 64 rows leave panel16 no lanes for it): lane r < 16
 // solves L u = e_r by forward substitution, u = column r of the inverse,
 // stored as X[b16 + r][b16 + k] = u_k.  For a partial panel the rows and
 // columns past its cb pivots are finite stand-ins (rs = 1 there; the
@@ -249,52 +267,68 @@ __device__ __forceinline__ void inverse16(Front64<T>& S, int i, int j, int w)
 // records the global column col0 + k + 1 in *info (smallest wins).
 // Same, with S.A already holding the block (lower part, zero past row n)
 // and S.X zero above the diagonal blocks, both visible to the workgroup.
-template <typename T>
+// pre(w), w = 0 .. 2: what three waves do during the first panel's chain.
+template <typename T, typename Pre>
 __device__ __forceinline__ void factor_dense64_loaded(Front64<T>& S, T* g, int64_t ld, int n, int c, int* info,
-                                                      int col0, T* inv)
+                                                      int col0, T* inv, Pre pre)
 {
-    const int tid = threadIdx.x, wv = tid >> 6;
-    const int nblk = (c + 15) >> 4, nall = (n + 15) >> 4;
-    // Phase b: wave 0 runs panel b's chain; wave 1 inverts panel b-1's
-    // diagonal block; waves 2 and 3 form row b-2 of the inverse's
-    // off-diagonal blocks (it needs the diagonal inverses up to b-2 and the
-    // rows above it).  Then all four waves apply panel b to the trailing
-    // blocks.  The last diagonal inverse and the last two rows follow the
-    // loop.  Only the last panel can be partial.
-    for (int b = 0; b < nblk; ++b) {
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    const int nblk = (c + 15) >> 4, nall = (n + 15) >> 4, last = nblk - 1;
+    // columns 16 jb .. of L (or of the trailing block) and rows 16 ib .. of
+    // the inverse to memory, by wave w of nw
+    auto put_cols = [&](int jb, int w, int nw) {
+#pragma unroll 4
+        for (int q = w; q < 16; q += nw) {
+            const int col = 16 * jb + q;
+            if (lane < n && col <= lane) g[lane + (int64_t)col * ld] = S.A[col][lane];
+        }
+    };
+    auto put_inv = [&](int ib, int w, int nw) {
+#pragma unroll 4
+        for (int q = 16 * ib + w; q < 16 * ib + 16; q += nw)
+            inv[lane + 64 * q] = (lane < c && q < c) ? S.X[lane][q] : T(0);
+    };
+    // Phase b: wave 0 runs panel b's chain, which also inverts its diagonal
+    // block (b > 0); beside it the other waves finish panel b-1's update
+    // (block column b, which the chain needs, came before), form row b-1 of
+    // the inverse's off-diagonal blocks and store what is final: block column
+    // b-1 of L, block row b-2 of the inverse.  Then all waves apply panel b to
+    // block column b+1.  Phase nblk has the last row of the inverse alone.
+    // Only the last panel can be partial.
+    for (int b = 0; b <= nblk; ++b) {
         const int b16 = 16 * b, cb = min(16, c - b16);
-        if (wv == 0) {
+        if (wv == 0 && b < nblk) {
             if (cb == 16)
                 panel16<T, true>(S, b16, 16, n, info, col0);
             else
                 panel16<T, false>(S, b16, cb, n, info, col0);
-        } else if (wv == 1) {
-            if (b >= 1) diaginv16<T>(S, b16 - 16);
-        } else if (wv - 2 < b - 2) {
-            inverse16<T>(S, b - 2, wv - 2, wv);
+        } else if (b == 0) {
+            pre(wv - 1);
+        } else {
+            if (b == 1 && wv == 1) diaginv16<T>(S, 0);
+            const int j = b < nblk ? wv - 2 : wv;
+            if (j >= 0 && j < b - 1) inverse16<T>(S, b - 1, j, wv);
+            int idx = 0;
+            for (int J = b + 1; b < nblk && J < nall; ++J)
+                for (int I = J; I < nall; ++I, ++idx)
+                    if (1 + (idx + b) % 3 == wv) trailing16<T>(S, b16 - 16, 16, I, J);
+            if (wv == (b == 3 && b < nblk ? 1 : 3)) {
+                for (int jb = b - 1; jb < (b < nblk ? b : nall); ++jb) put_cols(jb, 0, 1);
+                if (b >= 2) put_inv(b - 2, 0, 1);
+            }
         }
+        if (b == nblk) break;
         __syncthreads();
-        int idx = 0;
-        for (int J = b + 1; J < nall; ++J)
-            for (int I = J; I < nall; ++I, ++idx)
-                if ((idx & 3) == wv) trailing16<T>(S, b16, cb, I, J);
-        __syncthreads();
-    }
-    const int last = nblk - 1;
-    if (last >= 0) {
-        if (wv == 1)
-            diaginv16<T>(S, 16 * last);
-        else if (wv >= 2 && wv - 2 < last - 1)
-            inverse16<T>(S, last - 1, wv - 2, wv);
-        __syncthreads();
-        if (wv < last) inverse16<T>(S, last, wv, wv);
+        if (b + 1 < nall) {
+            int idx = 0;
+            for (int J = b + 1; J < (b < last ? b + 2 : nall); ++J)
+                for (int I = J; I < nall; ++I, ++idx)
+                    if ((idx & 3) == wv) trailing16<T>(S, b16, cb, I, J);
+            __syncthreads();
+        }
     }
     __syncthreads();
-    for (int e = tid; e < 64 * 64; e += kThreads) {
-        const int row = e & 63, col = e >> 6;
-        if (row < n && col <= row) g[row + (int64_t)col * ld] = S.A[col][row];
-        inv[e] = (row < c && col < c) ? S.X[row][col] : T(0);
-    }
+    for (int ib = max(last, 0); ib < 4; ++ib) put_inv(ib, wv, 4);
 }
 template <typename T>
 __device__ __forceinline__ void factor_dense64(Front64<T>& S, T* g, int64_t ld, int n, int c, int* info, int col0,
@@ -313,7 +347,7 @@ __device__ __forceinline__ void factor_dense64(Front64<T>& S, T* g, int64_t ld, 
         S.X[col][row] = T(0);
     }
     __syncthreads();
-    factor_dense64_loaded<T>(S, g, ld, n, c, info, col0, inv);
+    factor_dense64_loaded<T>(S, g, ld, n, c, info, col0, inv, [](int) {});
 }
 
 }  // namespace
@@ -527,9 +561,12 @@ template <typename T, int NB = 1> struct TileLds {
 // it leaves LDS and multiplies on the 16-bit MFMA with FP32 accumulation.
 // TB: 0 = B stored like A (B[col + kk * ldb]), 1 = B transposed in memory,
 // -1 = as the runtime flag tb says (the panel TRSM kernel holds both).
-template <typename T, int LP = kNative, int TB = -1, int NB = 1>
+// OWN: also the rows' product with themselves, own[i][j] += sum_kk A[row][kk]
+// A[col][kk] (the block at wr = 0, wc = 32 above the diagonal left out).
+template <typename T, int LP = kNative, int TB = -1, int NB = 1, bool OWN = false>
 __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ldb, bool tb, int m, int n, int k,
-                                         TileLds<T, NB>& L, typename Mfma<T>::acc_t (&c)[2][2], int tid = threadIdx.x)
+                                         TileLds<T, NB>& L, typename Mfma<T>::acc_t (&c)[2][2],
+                                         typename Mfma<T>::acc_t (&own)[2][2], int tid = threadIdx.x)
 {
     static_assert(LP == kNative || sizeof(T) == 4, "16-bit operands come from FP32 fronts");
     typedef typename Mfma<T>::acc_t acc_t;
@@ -592,6 +629,17 @@ __device__ __forceinline__ void tile_mma(const T* A, int lda, const T* B, int ld
                 c01 = Mfma<T>::mma(a0[q], b1[q], c01);
                 c10 = Mfma<T>::mma(a1[q], b0[q], c10);
                 c11 = Mfma<T>::mma(a1[q], b1[q], c11);
+            }
+            if (OWN && wc <= wr) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int kr = q * 4 + (lane >> 4);
+                    const T w0 = L.As[buf][kr][wc + (lane & 15)], w1 = L.As[buf][kr][wc + 16 + (lane & 15)];
+                    own[0][0] = Mfma<T>::mma(a0[q], w0, own[0][0]);
+                    own[0][1] = Mfma<T>::mma(a0[q], w1, own[0][1]);
+                    own[1][0] = Mfma<T>::mma(a1[q], w0, own[1][0]);
+                    own[1][1] = Mfma<T>::mma(a1[q], w1, own[1][1]);
+                }
             }
         } else {
             typedef Mfma16<LP> M16;
@@ -658,63 +706,59 @@ __device__ __forceinline__ void tile_product(const T* A, int lda, const T* B, in
                                              TileLds<T, NB>& L, T (*Cs)[kTile + 1])
 {
     typename Mfma<T>::acc_t c[2][2];
-    tile_mma<T, LP, TB, NB>(A, lda, B, ldb, tb, m, n, k, L, c);
+    tile_mma<T, LP, TB, NB>(A, lda, B, ldb, tb, m, n, k, L, c, c);
     stage_acc<T>(c, Cs);
     __syncthreads();
 }
 
-// Products with operands already in LDS, same wave layout as tile_mma.
-// Am[kk][row] holds A (k columns, zero from column k up to a multiple of
-// 16), B comes from global memory like tile_mma's B (staged through L.Bs in
-// chunks of 16).  Ends with a barrier.
+// The same wave layout with A in LDS (Am[kk][row], zero past row m and column
+// k) and B (transposed in memory) in registers: rb[4 i + p] is entry (column
+// tid / 16 + 16 p, kk 16 i + tid % 16), staged through L.Bs in chunks of 16.
+// Ends with a barrier.
+template <typename T>
+__device__ __forceinline__ void load_tb(const T* B, int ldb, int n, int k, T (&rb)[16])
+{
+    const int tcol = threadIdx.x >> 4, tkk = threadIdx.x & 15;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+            rb[4 * i + p] = ld_off(B, (unsigned)(min(tcol + 16 * p, n - 1) * ldb + min(16 * i + tkk, k - 1)));
+}
 template <typename T, int NB>
-__device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T* B, int ldb, bool tb, int n, int k,
+__device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T (&rb)[16], int n, int k,
                                               TileLds<T, NB>& L, typename Mfma<T>::acc_t (&c)[2][2])
 {
-    typedef typename Mfma<T>::acc_t acc_t;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
-    const int li = tid & 63, lp = tid >> 6, tcol = tid >> 4, tkk = tid & 15;
-    acc_t c00 = {0, 0, 0, 0}, c01 = {0, 0, 0, 0}, c10 = {0, 0, 0, 0}, c11 = {0, 0, 0, 0};
-    for (int k0 = 0; k0 < k; k0 += 16) {
-        // loads from clamped in-bounds positions, all issued before the
-        // masked stores (no branch around each load)
-        T rb[4];
+    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32, tcol = tid >> 4, tkk = tid & 15;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            if (tb)
-                rb[p] = B[(int64_t)min(tcol + 16 * p, n - 1) * ldb + min(k0 + tkk, k - 1)];
-            else
-                rb[p] = B[min(li, n - 1) + (int64_t)min(k0 + lp + 4 * p, k - 1) * ldb];
-        }
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            if (tb) {
-                const int col = tcol + 16 * p, kt = k0 + tkk;
-                L.Bs[0][tkk][col] = (col < n && kt < k) ? rb[p] : T(0);
-            } else {
-                const int kk = k0 + lp + 4 * p;
-                L.Bs[0][lp + 4 * p][li] = (li < n && kk < k) ? rb[p] : T(0);
+        for (int j = 0; j < 2; ++j) c[i][j] = typename Mfma<T>::acc_t{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (16 * i < k) {
+            const int buf = NB == 2 ? i & 1 : 0;
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                L.Bs[buf][tkk][tcol + 16 * p] = (tcol + 16 * p < n && 16 * i + tkk < k) ? rb[4 * i + p] : T(0);
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int kr = q * 4 + (lane >> 4);
+                const T a0 = Am[16 * i + kr][wr + (lane & 15)], a1 = Am[16 * i + kr][wr + 16 + (lane & 15)];
+                const T b0 = L.Bs[buf][kr][wc + (lane & 15)], b1 = L.Bs[buf][kr][wc + 16 + (lane & 15)];
+                c[0][0] = Mfma<T>::mma(a0, b0, c[0][0]);
+                c[0][1] = Mfma<T>::mma(a0, b1, c[0][1]);
+                c[1][0] = Mfma<T>::mma(a1, b0, c[1][0]);
+                c[1][1] = Mfma<T>::mma(a1, b1, c[1][1]);
             }
+            if (NB == 1) __syncthreads();
         }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int kr = q * 4 + (lane >> 4);
-            const T a0 = Am[k0 + kr][wr + (lane & 15)], a1 = Am[k0 + kr][wr + 16 + (lane & 15)];
-            const T b0 = L.Bs[0][kr][wc + (lane & 15)], b1 = L.Bs[0][kr][wc + 16 + (lane & 15)];
-            c00 = Mfma<T>::mma(a0, b0, c00);
-            c01 = Mfma<T>::mma(a0, b1, c01);
-            c10 = Mfma<T>::mma(a1, b0, c10);
-            c11 = Mfma<T>::mma(a1, b1, c11);
-        }
-        __syncthreads();
     }
-    c[0][0] = c00;
-    c[0][1] = c01;
-    c[1][0] = c10;
-    c[1][1] = c11;
+    if (NB == 2) __syncthreads();
 }
+
 // One GemmTask per workgroup (see mfd_plan.h): C -= A B^T (mode 0: the
 // DSYRK/DGEMM updates) or C = A B^T with B transposed in memory (mode 1: the
 // panel TRSM as a product with the stored L^{-T} of the diagonal block, C
@@ -724,7 +768,7 @@ __device__ __forceinline__ void tile_mma_ldsA(const T (*Am)[kTile + 1], const T*
 // (TRSM, in-panel update, Schur update), so that profiles tell them apart.
 // The result goes through LDS so the write of C is coalesced along columns
 // (written straight from the accumulators it would be 32-byte pieces).
-template <typename T, int LP = kNative, bool PRE = true, int TB = -1, int NB = 1>
+template <typename T, int LP = kNative, bool PRE = true, int TB = -1, int NB = 1, bool SYRK = false>
 __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T, NB>& L, T (*Cs)[kTile + 1],
                                           const int* lidx = nullptr)
 {
@@ -741,8 +785,21 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T,
 #pragma unroll
         for (int j = 0; j < 16; ++j) cpre[j] = C[rc + (int64_t)min((tid >> 6) + 4 * j, t.n - 1) * t.ldc];
     }
-    typename Mfma<T>::acc_t acc[2][2];
-    tile_mma<T, LP, TB, NB>(pool + t.a, t.lda, pool + t.b, t.ldb, t.mode == 1, t.m, t.n, t.k, L, acc);
+    // the stored inverse of the second product (mode 2), early where
+    // registers are plenty
+    constexpr bool kEarly = PRE && NB == 2, kTrsm = TB != 0;
+    T rb[16];
+    if (kEarly && kTrsm && t.mode == 2) load_tb(pool + t.d, kPanel, t.n, t.kd, rb);
+    typename Mfma<T>::acc_t acc[2][2], own[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};
+    T dpre[16];
+    auto load_d = [&]() {
+        const int rd = min(row, t.syrk - 1);
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            dpre[j] = ld_off((const T*)pool + t.cd, (unsigned)(rd + min((tid >> 6) + 4 * j, rd) * t.ldc));
+    };
+    if constexpr (SYRK && kEarly) load_d();
+    tile_mma<T, LP, TB, NB, SYRK>(pool + t.a, t.lda, pool + t.b, t.ldb, t.mode == 1, t.m, t.n, t.k, L, acc, own);
     // the parent positions of this thread's row and columns (local_index)
     int lrow = 1, lcol[16];
     if (t.mode == 3) {
@@ -757,7 +814,7 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T,
     }
     stage_acc<T>(acc, Cs);
     __syncthreads();
-    if (t.mode == 2) {
+    if (kTrsm && t.mode == 2) {
         // Cs = C - A B^T, then C = Cs D^T (D = L^{-1}, stored transposed)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
@@ -765,12 +822,46 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T,
             Cs[col][row] = (row < t.m && col < t.n) ? cpre[j] - Cs[col][row] : T(0);
         }
         __syncthreads();
-        typename Mfma<T>::acc_t c[2][2];
-        tile_mma_ldsA<T, NB>(Cs, pool + t.d, kPanel, true, t.n, t.kd, L, c);
-        stage_acc<T>(c, Cs);
+        if (!kEarly) load_tb(pool + t.d, kPanel, t.n, t.kd, rb);
+        tile_mma_ldsA<T, NB>(Cs, rb, t.n, t.kd, L, acc);
+        stage_acc<T>(acc, Cs);
         __syncthreads();
-        if (row < t.m)
-            for (int col = tid >> 6; col < t.n; col += 4) C[row + (int64_t)col * t.ldc] = Cs[col][row];
+    }
+    if constexpr (SYRK) {
+        // the diagonal block at cd loses R R^T over its lower syrk x syrk part,
+        // R = the tile's rows over the pending panels (own, formed as they
+        // passed through LDS) and the panel just solved (Cs, zero past the
+        // tile's rows and columns)
+        const int lane = tid & 63, wr = ((tid >> 6) & 1) * 32 + (lane & 15), wc = (tid >> 7) * 32 + (lane & 15);
+        if (!kEarly) load_d();
+        if (t.mode == 1)  // no pending panels: A was the panel itself, unsolved
+#pragma unroll
+            for (int i = 0; i < 2; ++i) own[i][0] = own[i][1] = typename Mfma<T>::acc_t{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int col = (tid >> 6) + 4 * j;
+            if (row < t.m && col < t.n) C[row + (int64_t)col * t.ldc] = Cs[col][row];
+        }
+        if (wc <= wr) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const T* r = Cs[4 * q + (lane >> 4)];
+                const T a0 = r[wr], a1 = r[wr + 16], b0 = r[wc], b1 = r[wc + 16];
+                own[0][0] = Mfma<T>::mma(a0, b0, own[0][0]);
+                own[0][1] = Mfma<T>::mma(a0, b1, own[0][1]);
+                own[1][0] = Mfma<T>::mma(a1, b0, own[1][0]);
+                own[1][1] = Mfma<T>::mma(a1, b1, own[1][1]);
+            }
+        }
+        __syncthreads();
+        stage_acc<T>(own, Cs);
+        __syncthreads();
+        T* D = pool + t.cd;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int col = (tid >> 6) + 4 * j;
+            if (row < t.syrk && col <= row) D[row + (int64_t)col * t.ldc] = dpre[j] - Cs[col][row];
+        }
         return;
     }
     if (row >= t.m) return;
@@ -810,23 +901,6 @@ __device__ __forceinline__ void gemm_task(T* pool, const GemmTask& t, TileLds<T,
     }
 }
 
-// A TRSM tile with syrk > 0, after gemm_task: the diagonal block at cd
-// loses R R^T over its lower syrk x syrk part, R = the tile's rows over the
-// pending panels and the panel just solved (contiguous columns, A then C,
-// which this workgroup has just written).
-template <typename T, int NB>
-__device__ __forceinline__ void trsm_syrk(T* pool, const GemmTask& t, TileLds<T, NB>& L, T (*Cs)[kTile + 1])
-{
-    __syncthreads();
-    const T* R = pool + (t.mode == 2 ? t.a : t.c);
-    const int k = t.mode == 2 ? t.k + t.kd : t.k;
-    tile_product<T, kNative, 0, NB>(R, t.lda, R, t.lda, false, t.syrk, t.syrk, k, L, Cs);
-    T* D = pool + t.cd;
-    const int row = threadIdx.x & 63;
-    if (row < t.syrk)
-        for (int col = threadIdx.x >> 6; col <= row; col += 4) D[row + (int64_t)col * t.ldc] -= Cs[col][row];
-}
-
 // LP != kNative: the update and Schur tiles (KIND 1, 2) of the FP16_IR /
 // BF16_IR forms multiply 16-bit operands.
 template <typename T, int KIND, int LP = kNative>
@@ -839,8 +913,10 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 3 : 4) void k_gemm(T* pool, c
         __shared__ TileLds<T> L;
         __shared__ T Cs[kTile][kTile + 1];
         const GemmTask t = tasks[blockIdx.x];
-        gemm_task<T>(pool, t, L, Cs);
-        if (t.syrk > 0) trsm_syrk<T, 1>(pool, t, L, Cs);
+        if (t.syrk > 0)
+            gemm_task<T, kNative, false, -1, 1, true>(pool, t, L, Cs);
+        else
+            gemm_task<T>(pool, t, L, Cs);
     } else {
         // modes 0 and 3 (B never transposed): the staged result Cs is written
         // after the last read of the operand staging L, so the two share LDS
@@ -868,8 +944,8 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 3 : 4) void k_gemm(T* pool, c
 // to product without a barrier, and L_s^{-T}'s zeros and the block's upper
 // triangle are left out (40 and at most 48 products of 16 x 16 x 4 a wave
 // where whole squares take 64; 64 cycles each in FP64).  A step with nothing
-// beside it takes 28.5 us in FP64 (30.5 with the operands in two batches and
-// whole squares), 20 in FP32 (23).
+// beside it takes 25 us in FP64 (30.5 with the operands in two batches, whole
+// squares and every store at the end), 19 in FP32 (23).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const DiagTask* diags, int ndiag, const GemmTask* tiles,
                                                        int* info)
@@ -881,8 +957,10 @@ __global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const DiagTask* 
     } U;
     if ((int)blockIdx.x >= ndiag) {
         const GemmTask g = tiles[blockIdx.x - ndiag];
-        gemm_task<T, kNative, true, -1, 2>(pool, g, U.L, S.A);
-        if (g.syrk > 0) trsm_syrk<T, 2>(pool, g, U.L, S.A);
+        if (g.syrk > 0)
+            gemm_task<T, kNative, true, -1, 2, true>(pool, g, U.L, S.A);
+        else
+            gemm_task<T, kNative, true, -1, 2>(pool, g, U.L, S.A);
         return;
     }
     typedef typename Mfma<T>::acc_t acc_t;
@@ -973,42 +1051,39 @@ __global__ __launch_bounds__(kThreads) void k_upd_diag(T* pool, const DiagTask* 
             for (int v = 0; v < 4; ++v) S.X[16 * j + li][r0 + Mfma<T>::row(lane, v)] = c[j][v];
     }
     __syncthreads();
-    // stored into the front (these rows are this task's), and S.A -= X X^T, a
-    // wave every fourth of the ten lower 16 x 16 blocks
-    for (int col = c4; col < kp; col += 4)
-        if (row < kb) Pg[row + (int64_t)col * n] = S.X[col][row];
+    // S.A -= X X^T: the ten lower 16 x 16 blocks from three block rows of X a
+    // wave, (o0, o1), (o0, o2) and (o2, o2) of (3, 0, 1), (3, 3, 2), (2, 0, 1),
+    // (1, 0, 0)
     {
-        // block rows and columns of the ten, two bits each
-        constexpr unsigned bi = 0xffa94, bj = 0xe4910;
-        int I[3], J[3];
+        const int o0 = 16 * (0x1233 >> 4 * c4 & 3), o1 = 16 * (0x0030 >> 4 * c4 & 3), o2 = 16 * (0x0121 >> 4 * c4 & 3);
         acc_t c[3] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
-        for (int p = 0; p < 3; ++p) {
-            const int b = min(c4 + 4 * p, 9);
-            I[p] = 16 * ((bi >> 2 * b) & 3) + li, J[p] = 16 * ((bj >> 2 * b) & 3) + li;
-        }
-#pragma unroll
         for (int q = 0; q < 16; ++q) {
-            const T* x = S.X[4 * q + kl];
-            c[0] = Mfma<T>::mma(x[I[0]], x[J[0]], c[0]);
-            c[1] = Mfma<T>::mma(x[I[1]], x[J[1]], c[1]);
-            if (c4 < 2) c[2] = Mfma<T>::mma(x[I[2]], x[J[2]], c[2]);
+            const T* x = S.X[4 * q + kl] + li;
+            const T x0 = x[o0], x1 = x[o1], x2 = x[o2];
+            c[0] = Mfma<T>::mma(x0, x1, c[0]);
+            if (c4 != 3) c[1] = Mfma<T>::mma(x0, x2, c[1]);
+            if (c4 != 2) c[2] = Mfma<T>::mma(x2, x2, c[2]);
         }
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
-            if (p < 2 || c4 < 2) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) S.A[J[p]][I[p] - li + Mfma<T>::row(lane, v)] -= c[p][v];
-            }
+        for (int v = 0; v < 4; ++v) {
+            const int r = Mfma<T>::row(lane, v);
+            S.A[o1 + li][o0 + r] -= c[0][v];
+            if (c4 != 3) S.A[o2 + li][o0 + r] -= c[1][v];
+            if (c4 != 2) S.A[o2 + li][o2 + r] -= c[2][v];
+        }
     }
     __syncthreads();
-    // the inverse is zero above its diagonal blocks
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int col = c4 + 4 * j;
-        if (row < (col & ~15)) S.X[col][row] = T(0);
-    }
-    factor_dense64_loaded<T>(S, front + t.k0 + (int64_t)t.k0 * n, n, kb, kb, info, t.first + t.k0, pool + t.inv);
+    // during the first panel's chain: X into the front (these rows are this
+    // task's), then zero where the inverse is, above its diagonal blocks
+    auto put_x = [&](int w) {
+#pragma unroll 4
+        for (int col = w; col < 64; col += 3) {
+            if (row < kb && col < kp) Pg[row + (int64_t)col * n] = S.X[col][row];
+            if (row < (col & ~15)) S.X[col][row] = T(0);
+        }
+    };
+    factor_dense64_loaded<T>(S, front + t.k0 + (int64_t)t.k0 * n, n, kb, kb, info, t.first + t.k0, pool + t.inv, put_x);
 }
 
 // C -= A B^T on 128 x 128 tiles (GemmTask with m, n <= 128, mode 0 or 3):

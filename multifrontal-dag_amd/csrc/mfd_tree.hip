@@ -90,6 +90,7 @@ __device__ __attribute__((noinline)) void tree_panel(Lds<T> Sp, int w, int b16, 
                 pin(x[k + 1]);
             }
             piv = r == k ? d : piv;
+            pin(piv);
             const T sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs), l = r == k ? sd : q;
             x[k] = l;
             Sp->P[k][to] = l;
