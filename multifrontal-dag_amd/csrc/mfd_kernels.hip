@@ -7,16 +7,15 @@
 //
 // Reference operations these kernels replace (paths relative to the
 // reference root, src/main/):
-//   k_fill_lower,   set_zero + set_coefficient        zero_setter_m.f90:12-31, coefficient_setter_m.f90:15-50
-//   k_scatter_a
-//   k_extend_add    extend_add_tri / extend_add_rect  seq_factorize/kernel/extend_add_kernel_m.f90:6-34
-//                   (small children; k_gemm mode 3 for the others)
+//   k_assemble      set_zero + set_coefficient        zero_setter_m.f90:12-31, coefficient_setter_m.f90:15-50
+//   k_extend_add,   extend_add_tri / extend_add_rect  seq_factorize/kernel/extend_add_kernel_m.f90:6-34
+//   k_pull_children (children that are not large; k_gemm mode 3 for the others)
 //   k_small_front   the per-front tile loop           seq_factorize_m.f90:31-79
 //   k_diag,         DPOTRF("U") of a diagonal block,  seq_factorize/kernel/factorize_kernel_m.f90:4-16,
 //   k_upd_diag      with its panel's DTRSM tiles      border_kernel_m.f90:9-30
 //   k_gemm          DTRSM (modes 1, 2), DSYRK / DGEMM factorize_kernel_m.f90:11-33, border_kernel_m.f90:21-30,
 //                   updates (modes 0, 3)              border_subroutines_m.f90:41-73
-// The solves are in mfd_solve.hip.
+// The solves are in mfd_solve.hip, the bottom of the tree in mfd_tree.hip.
 #include <hip/hip_runtime.h>
 
 #include "mfd_device.h"
