@@ -77,11 +77,13 @@ template <typename T> struct Front64 {
 };
 
 // Panel b16 .. b16 + cb - 1 (cb <= 16; FULL: cb == 16) by one wave, rows
-// b16 .. 63 on their lanes.  Column k: d = x_k on lane k, rs = 1 / sqrt(d);
-// x_k rs, with row k+1's entry (from its lane by readlane) times rs, updates
-// column k+1 at once (the next pivot needs it); beside that chain L_kk =
-// sqrt(d) and l = x_k / L_kk (quot: exact whenever the quotient is
-// representable) go to LDS, and l's entries for rows k+2 .. 15 are read back
+// b16 .. 63 on their lanes.  Column k: d = x_k on lane k, rs = 1 / sqrt(d),
+// L_kk = sqrt(d), l = x_k / L_kk (quot: exact whenever the quotient is
+// representable).  Every lane forms row k+1's quotient too, from the entry its
+// lane had before (by readlane, beside the chain), and updates column k+1 at
+// once (the next pivot needs it): by the finished entries, so that where the
+// factor is representable the pivots are exact, and zero where they are zero.
+// The column goes to LDS, and its entries for rows k+2 .. 15 are read back
 // (the wave's LDS accesses complete in issue order, so the reads see the
 // column) and applied to those columns in step k+1, by when the reads have
 // landed.  A partial panel also updates the block's columns past cb (trailing
@@ -94,9 +96,10 @@ template <typename T> struct Front64 {
 // non-positive pivot is recorded (each pivot stays on its row's lane; one look
 // at all of them at the end).
 // One wave issues at most an instruction every four cycles, so the panel is
-// bound by its instruction count as much as by the chain: 3900 cycles for 16
-// columns in FP64, 3240 in FP32; with the chain through the finished column,
-// a check per pivot and masked stores 4940 and 4050.
+// bound by its instruction count as much as by the chain: 3960 cycles for 16
+// columns in FP64, 3320 in FP32; with a check per pivot and masked stores
+// 4810 and 4020.  (Updating column k+1 by x_k rs times its entry's, not yet
+// corrected, takes 3760 and 3070 and lets singular matrices pass.)
 template <typename T, bool FULL>
 __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, int* info, int col0)
 {
@@ -121,18 +124,18 @@ __device__ __forceinline__ void panel16(Front64<T>& S, int b16, int cb, int n, i
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         if (FULL || k < cb) {  // no early exit: the loop stays unrolled, x and v in registers
-            const T d = bcast(x[k], k), rs = rsqrt_nr(d);
+            const T d = bcast(x[k], k), rs = rsqrt_nr(d), sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs);
             // column k-1's updates of columns k+1 .. 15 (its entries read in
             // step k-1), with column k's of column k+1
             if (k + 1 < 16) {
-                const T u = bcast(x[k], k + 1);
+                const T u = quot(bcast(x[k], k + 1), sd, rs);
                 x[k + 1] -= lp * v[k + 1];
-                if (FULL || k + 1 < cb) x[k + 1] -= (x[k] * rs) * (u * rs);
+                if (FULL || k + 1 < cb) x[k + 1] -= q * u;
                 pin(x[k + 1]);
             }
             piv = r == k ? d : piv;
             pin(piv);
-            const T sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs), l = r == k ? sd : q;
+            const T l = r == k ? sd : q;
             x[k] = l;
             S.A[b16 + k][at] = l;
             S.rs[b16 + k] = rs;

@@ -82,16 +82,16 @@ __device__ __attribute__((noinline)) void tree_panel(Lds<T> Sp, int w, int b16, 
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
         if (k < cb) {
-            const T d = bcast(x[k], k), rs = rsqrt_nr(d);
+            const T d = bcast(x[k], k), rs = rsqrt_nr(d), sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs);
             if (k + 1 < 16) {
-                const T u = bcast(x[k], k + 1);
+                const T u = quot(bcast(x[k], k + 1), sd, rs);
                 x[k + 1] -= lp * v[k + 1];
-                if (k + 1 < cb) x[k + 1] -= (x[k] * rs) * (u * rs);
+                if (k + 1 < cb) x[k + 1] -= q * u;
                 pin(x[k + 1]);
             }
             piv = r == k ? d : piv;
             pin(piv);
-            const T sd = sqrt_from_rs(d, rs), q = quot(x[k], sd, rs), l = r == k ? sd : q;
+            const T l = r == k ? sd : q;
             x[k] = l;
             Sp->P[k][to] = l;
             Sp->rs[k] = rs;
