@@ -530,9 +530,10 @@ __global__ __launch_bounds__(kThreads) void k_pull_children(T* pool, const int* 
 // -------------------------------------------------------- small fronts
 // Whole partial factorization of a front with n <= 64 in one workgroup: L in
 // the first c columns, the Schur complement in the trailing block, and the
-// inverse of the c x c diagonal block for the solves.
+// inverse of the c x c diagonal block for the solves.  As many workgroups per
+// CU as k_diag.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_small_front(T* pool, const NodeDev* nodes, const int* tasks, int* info)
+__global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 2 : 4) void k_small_front(T* pool, const NodeDev* nodes, const int* tasks, int* info)
 {
     const NodeDev nd = nodes[tasks[blockIdx.x]];
     __shared__ Front64<T> S;
@@ -1300,9 +1301,10 @@ __global__ __launch_bounds__(kThreads) void k_gemm_fix(T* pool, const GemmTask* 
 // Diagonal block [k0, k0+kb) of a large front, already updated by every
 // earlier panel (DPOTRF("U"), factorize_kernel_m.f90:4-9): L written back
 // into the front, and the inverse of L stored for the panel TRSM and the
-// solves.
+// solves.  As many workgroups per CU as its LDS allows: two in FP64, four in
+// FP32.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_diag(T* pool, const DiagTask* tasks, int* info)
+__global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 2 : 4) void k_diag(T* pool, const DiagTask* tasks, int* info)
 {
     const DiagTask t = tasks[blockIdx.x];
     __shared__ Front64<T> S;
@@ -1327,28 +1329,39 @@ __global__ __launch_bounds__(kThreads) void k_diag(T* pool, const DiagTask* task
 // update tiles' operands to 16 bits (the FP16_IR / BF16_IR forms).  With
 // clocks != nullptr, task i's start and end (wall_clock64, 100 MHz) go to
 // clocks[2 i], clocks[2 i + 1]: the per-front timings of the schedule tuner.
+template <typename T> union FrontLds {
+    Front64<T> D;
+    struct {
+        TileLds<T, 2> L;
+        T Cs[kTile][kTile + 1];
+    } G;
+};
 // One tile of k_front_wg, kept out of line: the medium-front kernel's
-// registers are then those of its diagonal phase (two waves per SIMD, the
-// call's saved registers on the stack) instead of the sum of both phases.
+// registers are then those of its diagonal phase (the call's saved registers
+// on the stack) instead of the sum of both phases.  The LDS comes by its own
+// address space: through generic pointers each access to it would count as a
+// memory access and wait for the loads of the next chunks.  In FP64 the tile's
+// entries of C come before its K loop (24^3 grid, one front after another:
+// 10.6 ms against 11.3 after it); in FP32, where the loop is shorter than the
+// loads, after it (9.1 against 9.3).
 template <typename T, int LP>
-__device__ __attribute__((noinline)) void front_tile(T* pool, GemmTask g, TileLds<T>& L, T (*Cs)[kTile + 1])
+__device__ __attribute__((noinline)) void front_tile(T* pool, GemmTask g, __attribute__((address_space(3))) FrontLds<T>* U)
 {
-    gemm_task<T, LP, false>(pool, g, L, Cs);
+    FrontLds<T>* u = (FrontLds<T>*)U;
+    gemm_task<T, LP, sizeof(T) == 8, -1, 2>(pool, g, u->G.L, u->G.Cs);
 }
+// Two workgroups per CU, in both types: left to itself the compiler takes
+// registers for one, with which 256 systems of a batch, all their fronts
+// medium, take 9.2 ms in FP64 and 7.4 in FP32 instead of 7.25 and 5.4.
 template <typename T, int LP>
-__global__ __launch_bounds__(kThreads) void k_front_wg(T* pool, const NodeDev* nodes, const int* tasks, int* info,
+__global__ __launch_bounds__(kThreads, 2) void k_front_wg(T* pool, const NodeDev* nodes, const int* tasks, int* info,
                                                        long long* clocks)
 {
     long long t_start = 0;
     if (clocks) t_start = wall_clock64();
     const NodeDev nd = nodes[tasks[blockIdx.x]];
-    __shared__ union {
-        Front64<T> D;
-        struct {
-            TileLds<T> L;
-            T Cs[kTile][kTile + 1];
-        } G;
-    } U;
+    __shared__ FrontLds<T> U;
+    auto* lds = (__attribute__((address_space(3))) FrontLds<T>*)&U;
     const int n = nd.n, c = nd.c;
     for (int k0 = 0; k0 < c; k0 += kPanel) {
         const int kb = min(kPanel, c - k0);
@@ -1364,7 +1377,7 @@ __global__ __launch_bounds__(kThreads) void k_front_wg(T* pool, const NodeDev* n
             g.m = min(kTile, n - r0);
             g.n = g.k = kb;
             g.mode = 1;
-            front_tile<T, kNative>(pool, g, U.G.L, U.G.Cs);
+            front_tile<T, kNative>(pool, g, lds);
             __syncthreads();
         }
         for (int c0 = k0 + kb; c0 < n; c0 += kTile)
@@ -1378,7 +1391,7 @@ __global__ __launch_bounds__(kThreads) void k_front_wg(T* pool, const NodeDev* n
                 g.n = min(kTile, n - c0);
                 g.k = kb;
                 g.tri = r0 == c0;
-                front_tile<T, LP>(pool, g, U.G.L, U.G.Cs);
+                front_tile<T, LP>(pool, g, lds);
                 __syncthreads();
             }
     }
