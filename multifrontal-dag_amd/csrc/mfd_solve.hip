@@ -168,16 +168,36 @@ __device__ __forceinline__ void load_cols(T (&a)[16], const T* M, int row, int l
 #pragma unroll
     for (int j = 0; j < 16; ++j) a[j] = ld_off(M, (unsigned)(row + min(k0 + 4 * j + g, cmax) * ld));
 }
+// acc += sum over j < 16 of a[j] b(j), four entries of K each, in N chains
+// added pairwise and then to acc.  In one chain through all of a task's entries
+// (up to 256) every product rounds at the whole sum's magnitude: over 240
+// systems the backward error of an FP64 solve was 7% larger than with sums of
+// 16 to 64 entries (16% on a 12^3 27-point stencil), and is 2% larger with
+// these.  Four chains in the tasks that run on 16 rows or columns; two in the
+// block tasks (kFwdPiv, kBwdPiv), whose three tiles in flight leave no
+// registers for more (solves 5 to 15% slower at four).
+template <int N, typename T, typename B> __device__ __forceinline__ void mma_chains(d4& acc, const T (&a)[16], B b)
+{
+    static_assert(N == 2 || N == 4, "added pairwise");
+    d4 p[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) p[j] = d4{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 16; ++j) p[j % N] = mma((double)a[j], b(j), p[j % N]);
+    if constexpr (N == 4)
+        acc += (p[0] + p[1]) + (p[2] + p[3]);
+    else
+        acc += p[0] + p[1];
+}
 // acc += a S.v[k0 ..] in load_cols's order.
-template <typename T> __device__ __forceinline__ void mma_cols(d4& acc, const T (&a)[16], const Ctx<T>& C, int k0)
+template <int N = 4, typename T> __device__ __forceinline__ void mma_cols(d4& acc, const T (&a)[16], const Ctx<T>& C, int k0)
 {
     const bool ok = C.li < C.nr;
     const int r = ok ? C.li : 0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
+    mma_chains<N>(acc, a, [&](int j) {
         const double b = C.S.v[k0 + 4 * j + C.g][r];
-        acc = mma((double)a[j], ok ? b : 0.0, acc);
-    }
+        return ok ? b : 0.0;
+    });
 }
 
 // 64 entries of K for 16 columns of column-major M (the transposed
@@ -214,15 +234,14 @@ __device__ __forceinline__ void load_rows(T (&a)[16], const T* M, int col, int r
         for (int e = 0; e < V; ++e) a[j + e] = r + e < lim ? p[e] : T(0);
     }
 }
-template <typename T> __device__ __forceinline__ void mma_rows(d4& acc, const T (&a)[16], const Ctx<T>& C, int k0)
+template <int N = 4, typename T> __device__ __forceinline__ void mma_rows(d4& acc, const T (&a)[16], const Ctx<T>& C, int k0)
 {
     const bool ok = C.li < C.nr;
     const int r = ok ? C.li : 0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
+    mma_chains<N>(acc, a, [&](int j) {
         const double b = C.S.v[k0 + row_of<T>(j, C.g)][r];
-        acc = mma((double)a[j], ok ? b : 0.0, acc);
-    }
+        return ok ? b : 0.0;
+    });
 }
 
 // The four waves' partial products added in wave order: thread (row tid /
@@ -441,7 +460,7 @@ template <typename T> __device__ __forceinline__ void fwd_piv(const Ctx<T>& C, c
         if (b < nb) {
             if (q + 2 < kTiles && kTileB[q + 2] < nb) fetch(buf[(q + 2) % 3], kTileB[q + 2], kTileJ[q + 2]);
             if (j < b) {
-                mma_cols(acc, buf[q % 3], C, 64 * j);
+                mma_cols<2>(acc, buf[q % 3], C, 64 * j);
                 if (j == b - 1) {
                     if (ok) {
 #pragma unroll
@@ -452,7 +471,7 @@ template <typename T> __device__ __forceinline__ void fwd_piv(const Ctx<T>& C, c
                 }
             } else {
                 d4 y = {0, 0, 0, 0};
-                mma_rows(y, buf[q % 3], C, 64 * b);
+                mma_rows<2>(y, buf[q % 3], C, 64 * b);
                 __syncthreads();
                 if (ok) {
 #pragma unroll
@@ -490,7 +509,7 @@ template <typename T> __device__ __forceinline__ void fwd_piv(const Ctx<T>& C, c
             for (int j = 0; j < nb; ++j) {
                 const bool last = j + 1 == nb;
                 if (!last || r0 + 64 < t.nr) rows(buf[1], last ? r0 + 64 : r0, last ? 0 : j + 1);
-                mma_cols(acc, buf[0], C, 64 * j);
+                mma_cols<2>(acc, buf[0], C, 64 * j);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) buf[0][e] = buf[1][e];
             }
@@ -683,7 +702,7 @@ template <typename T> __device__ __forceinline__ void bwd_piv(const Ctx<T>& C, c
                     if (b >= nb) continue;
                     const bool last = b + 1 >= nb;
                     if (!last || r0 + q + 64 < t.nr) rows(buf[1], r0 + q + (last ? 64 : 0), last ? 0 : b + 1);
-                    mma_rows(acc[b], buf[0], C, q);
+                    mma_rows<2>(acc[b], buf[0], C, q);
 #pragma unroll
                     for (int e = 0; e < 16; ++e) buf[0][e] = buf[1][e];
                 }
@@ -730,7 +749,7 @@ template <typename T> __device__ __forceinline__ void bwd_piv(const Ctx<T>& C, c
             const int b = nb - 1 - bq, j = nb - 1 - jq;
             if (q + 2 < kTiles && kTileB[q + 2] < nb) fetch(buf[(q + 2) % 3], kTileB[q + 2], kTileJ[q + 2]);
             if (jq < bq) {
-                mma_rows(acc, buf[q % 3], C, 64 * j);
+                mma_rows<2>(acc, buf[q % 3], C, 64 * j);
                 if (jq == bq - 1) {
                     if (ok) {
 #pragma unroll
@@ -741,7 +760,7 @@ template <typename T> __device__ __forceinline__ void bwd_piv(const Ctx<T>& C, c
                 }
             } else {
                 d4 x = {0, 0, 0, 0};
-                mma_cols(x, buf[q % 3], C, 64 * b);
+                mma_cols<2>(x, buf[q % 3], C, 64 * b);
                 __syncthreads();
                 if (ok) {
 #pragma unroll
