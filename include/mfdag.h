@@ -290,11 +290,12 @@ int mfd_get_update_period(mfd_handle* h);
    turn; many such fronts of one level run side by side).
    mfd_set_front_split: fronts with at most cmax pivot columns are medium
    (0, the default: none).  mfd_set_front_kinds: one choice per node
-   (num_node entries, 1-based node order: 1 medium, 0 not, -1 by cmax; NULL
-   clears).  A front of order <= 128 whose descendants are all such fronts,
-   none of them chosen medium, is neither: one launch factors the whole
-   bottom of the tree, one workgroup per front (MFD_K_SMALL_FRONT); other
-   fronts of order <= 64 are factored whole in LDS.  Both rebuild the schedule of the current analysis like
+   (num_node entries, 1-based node order: 1 medium, 0 large, -1 left to cmax
+   and the library; NULL clears).  A front of order <= 128 that neither makes
+   medium or large, whose descendants are all such fronts or of order <= 64,
+   is neither: one launch factors the whole bottom of the tree, one workgroup
+   per front (MFD_K_SMALL_FRONT); other fronts of order <= 64 are factored
+   whole in LDS.  Both rebuild the schedule of the current analysis like
    mfd_set_update_period.  mfd_get_front_times: per node, the duration in
    microseconds of its workgroup in the last factorization (in-kernel
    clocks), -1 for fronts that are not medium. */

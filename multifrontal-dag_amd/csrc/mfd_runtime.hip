@@ -435,17 +435,16 @@ void build_plan(mfd_handle* h)
     h->host_rc = h->host_roots.empty() ? MFD_OK : build_host_plan(S, h->nodes, h->host_roots, h->hplan);
     if (h->host_rc != MFD_OK) h->hplan = HostPlan{};
     auto on_host = [&](int s) { return !h->hplan.is_host.empty() && h->hplan.is_host[s]; };
-    // medium fronts by choice (mfd_set_front_kinds, mfd_set_front_split)
-    auto chosen_kind = [&](int s) {
-        const int k = (int)h->front_kind.size() == m ? h->front_kind[s] : -1;
-        return k >= 0 ? k : (int)(h->nodes[s].c <= h->fuse_cmax);
-    };
+    // kinds by choice (mfd_set_front_kinds), and medium fronts by
+    // mfd_set_front_split where there is none
+    auto given_kind = [&](int s) { return (int)h->front_kind.size() == m ? h->front_kind[s] : -1; };
+    auto medium = [&](int s) { return given_kind(s) >= 0 ? given_kind(s) == 1 : h->nodes[s].c <= h->fuse_cmax; };
     // the bottom of the tree in one launch: fronts of order <= 64, and larger
-    // ones unless they were chosen to be medium
+    // ones unless a kind was chosen for them
     {
         std::vector<char> eligible(m, 0);
         for (int s = 0; s < m; ++s)
-            eligible[s] = !on_host(s) && (h->nodes[s].n <= kSmallFront || chosen_kind(s) != 1);
+            eligible[s] = !on_host(s) && (h->nodes[s].n <= kSmallFront || (given_kind(s) < 0 && !medium(s)));
         build_tree_plan(S, h->nodes, eligible, h->tp);
     }
 
@@ -550,7 +549,7 @@ void build_plan(mfd_handle* h)
             cls[s] = kClsSmall;
             continue;
         }
-        cls[s] = chosen_kind(s) == 1 ? kClsMedium : kClsLarge;
+        cls[s] = medium(s) ? kClsMedium : kClsLarge;
     }
     h->diag.clear();
     h->gemm.clear();

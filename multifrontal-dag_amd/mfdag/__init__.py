@@ -320,9 +320,9 @@ class Solver:
         self._check(lib().mfd_set_front_split(self.h, int(cmax)), "mfd_set_front_split")
 
     def set_front_kinds(self, kinds):
-        """Per node (0-based order): 1 one workgroup, 0 64-column steps (or
-        the launch for the bottom of the tree, fronts of order <= 128),
-        -1 by the split; None clears."""
+        """Per node (0-based order): 1 one workgroup, 0 64-column steps, -1 by
+        the split (and, if that takes none of them, the launch for the bottom
+        of the tree, fronts of order <= 128); None clears."""
         if kinds is None:
             self._check(lib().mfd_set_front_kinds(self.h, None), "mfd_set_front_kinds")
             return

@@ -354,7 +354,7 @@ def chain_constants(records):
 
 def bottom_of_tree(n, parent, order=128):
     """Per node: whether it and all its descendants are of order <= `order`,
-    the fronts that one launch factors unless they are chosen medium."""
+    the fronts that one launch factors unless a kind is chosen for them."""
     low = np.asarray(n) <= order
     for k in range(len(low)):  # children precede parents
         if not low[k] and parent[k] > 0:
@@ -364,21 +364,22 @@ def bottom_of_tree(n, parent, order=128):
 
 def choose_kinds(structure, model, tau, schur_us, rate, elem_bytes, max_order, slots=2 * CUS, margin=0.1,
                  level_rule=1):
-    """Per node: 1 (medium) or 0 (large), level by level, the k largest
+    """Per node: 1 (medium), 0 (large) or, for the fronts that are left to the
+    launch for the bottom of the tree, -1; level by level, the k largest
     fronts (by pivots) large for the k that minimises the predicted level
     time: medium part max(longest front, sum / slots) by the model, large
     part (rounds of diagonal tasks) * tau + Schur launches (one per child
     rank) * schur_us + Schur flops / rate.  Fronts of order above max_order
     (outside the model's training data) stay large, and a level keeps all
     its fronts large unless the best split is predicted faster by more than
-    margin (the predictions' error is of that order).  Fronts that the
-    solver factors in its launch for the bottom of the tree are left to it
-    (kind 0).  level_rule: the solver's (mfd_set_level_rule)."""
+    margin (the predictions' error is of that order).  level_rule: the
+    solver's (mfd_set_level_rule)."""
     c, w, par = structure["supernode_size"], structure["work_size"], structure["parent"]
     n = c + w
     lev = level_of(par, level_rule)
-    kinds = np.zeros(len(c), dtype=np.int32)
-    big = (n > 64) & ~bottom_of_tree(n, par)
+    low = bottom_of_tree(n, par)
+    kinds = np.where(low, -1, 0).astype(np.int32)
+    big = (n > 64) & ~low
     pred = np.zeros(len(c))
     if big.any():
         pred[big] = model.predict_us(n[big], c[big], w[big], elem_bytes)
