@@ -294,8 +294,9 @@ int mfd_get_update_period(mfd_handle* h);
    and the library; NULL clears).  A front of order <= 128 that neither makes
    medium or large, whose descendants are all such fronts or of order <= 64,
    is neither: one launch factors the whole bottom of the tree, one workgroup
-   per front (MFD_K_SMALL_FRONT); other fronts of order <= 64 are factored
-   whole in LDS.  Both rebuild the schedule of the current analysis like
+   per front (MFD_K_SMALL_FRONT), or only its fronts of order <= 64, or none,
+   where they follow one another in few chains, which levels take faster;
+   other fronts of order <= 64 are factored whole in LDS.  Both rebuild the schedule of the current analysis like
    mfd_set_update_period.  mfd_get_front_times: per node, the duration in
    microseconds of its workgroup in the last factorization (in-kernel
    clocks), -1 for fronts that are not medium. */

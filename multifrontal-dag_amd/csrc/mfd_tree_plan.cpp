@@ -11,6 +11,76 @@ namespace {
 // Fronts of one height beyond kManyTasks are taken several to a ticket, at
 // most kTicketMost (every ticket is an addition to one counter).
 constexpr int kManyTasks = 8192, kTicketMost = 4;
+
+// Microseconds of a factorization (FP64) whose eligible fronts of order <=
+// `order` are in the launch, the others in the level schedule, as far as the
+// choice of `order` changes it.  In the launch a front takes 3 us per panel of
+// 16 pivot columns and 0.06 us per row, 0.0625 per row and panel, and waits
+// only for its children; a level takes 10 us and 0.1 per row for fronts of
+// order <= 64, 12 us, 0.28 per column of a block and 17 per further block for
+// larger ones, whatever their number; where fronts are many, one costs 0.012
+// us and its time over 800 in the launch, 0.02 us and 7.5e-6 n^2 outside it.
+// Fitted to forests of 1 to 1024 chains of equal fronts of order 16 to 128
+// (errors up to 30%).
+double predicted_us(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible, int order)
+{
+    const int m = (int)nodes.size();
+    std::vector<char> in(m, 0);
+    std::vector<int> depth(m, 0);
+    std::vector<double> path(m, 0.0), small, large;
+    double longest = 0.0, many = 0.0;
+    bool any = false;
+    for (int s = 0; s < m; ++s) {  // children before parents
+        const double n = nodes[s].n, panels = (nodes[s].c + 15) / 16, us = 0.06 * n + panels * (3.0 + 0.0625 * n);
+        in[s] = eligible[s] && nodes[s].n <= order;
+        for (int ch : S.children[s]) {
+            in[s] = in[s] && in[ch - 1];
+            path[s] = std::max(path[s], path[ch - 1]);
+        }
+        if (in[s]) {
+            any = true;
+            path[s] += us;
+            longest = std::max(longest, path[s]);
+        }
+        many += in[s] ? 0.012 + us / 800.0 : 0.02 + 7.5e-6 * n * n;
+    }
+    for (int s = m - 1; s >= 0; --s) {  // parents before children
+        const int pa = nodes[s].parent, n = nodes[s].n, c = nodes[s].c;
+        if (pa >= 0) depth[s] = depth[pa] + 1;
+        if (in[s]) continue;
+        auto& level = n <= kTile ? small : large;
+        if ((int)level.size() <= depth[s]) level.resize(depth[s] + 1, 0.0);
+        const double us = n <= kTile ? 10.0 + 0.1 * n : 12.0 + 0.28 * std::min(c, kPanel) + 17.0 * ((c - 1) / kPanel);
+        level[depth[s]] = std::max(level[depth[s]], us);
+    }
+    double t = (any ? 10.0 + longest : 0.0) + many;
+    for (double us : small) t += us;
+    for (double us : large) t += us;
+    return t;
+}
+
+// The largest order of the launch's fronts: kTreeFront, unless the launch is
+// predicted to lose clearly by it.  It wins where the tree branches (512
+// systems of a batch: 9.1 ms against 11.4 in either other way; a 100^2 grid
+// 0.48 against 0.53 with fronts of order <= 64 only, 0.76 without it), and
+// loses where a few fronts follow one another, of which it takes one at a time
+// by one workgroup: 64 x 64 blocks in a chain of 12 took 699 us in it and 387
+// in the level schedule, 60 x 60 blocks by themselves 55 and 34.  The bound of
+// 3/4 keeps every tree that branches where it measured faster; a forest
+// without branches, where the prediction is good to a few percent, needs no
+// such margin.
+int largest_order(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible)
+{
+    bool branches = false;
+    for (const auto& ch : S.children) branches = branches || ch.size() > 1;
+    double best = predicted_us(S, nodes, eligible, kTreeFront) * (branches ? 0.75 : 0.9);
+    int order = kTreeFront;
+    for (int o : {kTile, 0}) {
+        const double us = predicted_us(S, nodes, eligible, o);
+        if (us < best) best = us, order = o;
+    }
+    return order;
+}
 }  // namespace
 
 void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible,
@@ -22,8 +92,9 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     std::vector<char> in(m, 0);
     std::vector<int> height(m, 0);
     int count = 0;
+    const int order = largest_order(S, nodes, eligible);
     for (int s = 0; s < m; ++s) {  // children before parents
-        in[s] = eligible[s] && nodes[s].n <= kTreeFront;
+        in[s] = eligible[s] && nodes[s].n <= order;
         for (int ch : S.children[s]) {
             in[s] = in[s] && in[ch - 1];
             height[s] = std::max(height[s], height[ch - 1] + 1);

@@ -24,8 +24,9 @@ struct TreePlan {
     bool has(int s) const { return !in.empty() && in[s]; }
 };
 
-// eligible: per node, whether the front may be in the plan; it is if its
-// order is at most kTreeFront and all its children are.
+// eligible: per node, whether the front may be in the plan; it is if all its
+// children are and its order is at most kTreeFront, or less where the launch
+// would lose by the larger ones (none: the plan is empty).
 void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible,
                      TreePlan& P);
 
