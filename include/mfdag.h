@@ -146,10 +146,12 @@ int mfd_solve_device(mfd_handle* h, double* d_b, int nrhs, int ldb);
 /* No counterpart in the reference.  For callers that cannot allocate device
    memory (serving loops that solve with one factor many times, harnesses
    that forbid allocation after set-up): mfd_solve_device on a factored
-   handle, the same kernels and results, with every solve buffer (Z/Y slices,
-   partial sums, permuted b and x, and for the refined forms residual,
-   correction and norm slots) taken from one fixed 128 MiB device array of
-   the library instead of the handle's allocations.  It calls no hipMalloc
+   handle, the same kernels and results, with every solve buffer (the vectors
+   passed between fronts, y, permuted b and x, and for the refined forms
+   residual, correction and norm slots) taken from one fixed 128 MiB device
+   array of the library instead of the handle's allocations: about 8 nrhs
+   (sum of work sizes + 4 n) bytes at most, 16 n nrhs more for the refined forms, and
+   a few KB.  It calls no hipMalloc
    or hipFree and captures no graph (launches are eager).  Each GPU holds
    its own copy of the array from the library's load until the process
    ends.  Returns MFD_ERR_SCRATCH when a solve of this size (n, fronts, nrhs)

@@ -79,7 +79,7 @@ constexpr int64_t kSuperMats = 3 * (int64_t)kSuper * kSuper;  // entries per sup
 // rows r0 .. r0 + 15 of superblock u (super fronts); kFwdPiv, superblock u
 // (other fronts) and then, nr > 0, the front's nr update rows, sig raised.
 // Backward: kBwdPart, partial sums of the 32 columns from column nslot over
-// nr (<= 256) rows from r0, to plane offset slot, sig raised; kBwdCols, nr
+// nr rows from r0, to plane offset slot, sig raised; kBwdCols, nr
 // (<= 16) columns r0 .. of superblock u, superblocks v >= grow applied to
 // them, sig raised; kBwdTop, columns r0 .. r0 + 15 of superblock u; kBwdPiv,
 // superblock u, before it (nr > 0) the front's nr update rows.  In kBwdCols,
@@ -97,7 +97,7 @@ struct SolveTask {
     int grow;         // its update rows' global rows (backward), or the first superblock of kBwdCols
     int slot, nslot;
     int w0, w0t, sig;
-    int flag, fstr;   // the front's counters: asm, then z, y, p, t, x of each superblock, fstr apart
+    int flag, fstr;   // the front's counters: asm, then z, y, p, t, x of each superblock, fstr apart; 0: one for all
     int nsup, super;  // superblocks; 1: super front
     int per;          // turns the next ticket of the workgroup takes
 };

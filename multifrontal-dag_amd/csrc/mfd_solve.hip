@@ -86,7 +86,8 @@ template <typename T> __device__ __forceinline__ void signal(const Ctx<T>& C, in
     }
 }
 
-// Counters of a front (SolveTask::flag, fstr): y_u and x_u of superblock u.
+// Counters of a front (SolveTask::flag, fstr): y_u and x_u of superblock u; of
+// a front that has one for all (fstr 0), that one.
 __device__ __forceinline__ int y_flag(const SolveTask& t, int u) { return t.flag + t.fstr * (1 + t.nsup + u); }
 __device__ __forceinline__ int x_flag(const SolveTask& t, int u) { return t.flag + t.fstr * (1 + 4 * t.nsup + u); }
 // Tasks that form superblock u's y (or x).
@@ -94,6 +95,9 @@ __device__ __forceinline__ int yx_target(const SolveTask& t, int u)
 {
     return t.super ? (min(kSuper, t.c - kSuper * u) + 15) / 16 : 1;
 }
+// What the y counter has reached before those tasks: where it counts the
+// children's signals too, w0t, which a task on the front's rows waits for.
+__device__ __forceinline__ int before_y(const SolveTask& t) { return t.fstr == 0 ? t.w0t : 0; }
 
 // S.v[k][r] = src[k + (rb + r) ld] for k < cnt, zero for the other k < 256
 // (thread k's row; all loads before the stores of four columns).
@@ -284,7 +288,7 @@ template <typename T> __device__ __forceinline__ void fwd_rows(const Ctx<T>& C, 
     }
     d4 acc = {0, 0, 0, 0};
     for (int v = 0; v < nv; ++v) {
-        wait_for<T, true>(C, y_flag(t, v), yx_target(t, v));
+        wait_for<T, true>(C, y_flag(t, v), before_y(t) + yx_target(t, v));
         stage_rows(C, C.A.y + t.first + kSuper * v, C.A.n, min(kSuper, t.c - kSuper * v));
         __syncthreads();
         if (v + 1 < nv) load(an, v + 1);
@@ -345,7 +349,7 @@ template <typename T> __device__ __forceinline__ void fwd_rows64(const Ctx<T>& C
     d4 acc = {0, 0, 0, 0};
     for (int v = 0; v < nv; ++v) {
         const int pb = min(kSuper, t.c - kSuper * v);
-        wait_for<T, true>(C, y_flag(t, v), yx_target(t, v));
+        wait_for<T, true>(C, y_flag(t, v), before_y(t) + yx_target(t, v));
         stage_rows(C, C.A.y + t.first + kSuper * v, C.A.n, pb);
         __syncthreads();
         for (int k0 = 0; k0 < pb; k0 += 64) {
@@ -546,22 +550,25 @@ __device__ __forceinline__ void stage_x(const Ctx<T>& C, const SolveTask& t, int
     __syncthreads();
 }
 
-// Partial sums (kBwdPart): L[rows, 32 columns]^T x over at most 256 update
-// rows (first column nslot of the front) into 32 entries at slot; a wave
-// takes 16 of the columns and half the rows, so that all of the task's
-// entries are in registers before the wait for x.
+// Partial sums (kBwdPart): L[rows, 32 columns]^T x over the task's update rows
+// (first column nslot of the front) into 32 entries at slot, 256 rows at a
+// time (few tasks have more); a wave takes 16 of the columns and half the
+// rows, so that all entries of the first 256 rows are in registers before the
+// wait for x.
 template <typename T> __device__ __forceinline__ void bwd_part(const Ctx<T>& C, const SolveTask& t)
 {
     const int cw = 16 * (C.wv & 1), h = 128 * (C.wv >> 1), col0 = t.nslot;
     const T* F = C.A.pool + t.front + (int64_t)col0 * t.n + t.r0;
     const int lcol = min(cw + C.li, t.c - 1 - col0) * t.n;
     T a[16], an[16];
-    load_rows<T>(a, F, lcol, h, C.g, t.nr);
-    load_rows<T>(an, F, lcol, h + 64, C.g, t.nr);
-    stage_x(C, t, t.r0, t.nr, t.w0, t.w0t);
     d4 acc = {0, 0, 0, 0};
-    mma_rows(acc, a, C, h);
-    mma_rows(acc, an, C, h + 64);
+    for (int r = 0; r < t.nr; r += kSuper) {
+        load_rows<T>(a, F, lcol, r + h, C.g, t.nr);
+        load_rows<T>(an, F, lcol, r + h + 64, C.g, t.nr);
+        stage_x(C, t, t.r0 + r, min(kSuper, t.nr - r), r == 0 ? t.w0 : -1, t.w0t);
+        mma_rows(acc, a, C, h);
+        mma_rows(acc, an, C, h + 64);
+    }
     __syncthreads();
 #pragma unroll
     for (int v = 0; v < 4; ++v) C.S.red[C.wv][C.g + 4 * v][C.li] = acc[v];

@@ -8,6 +8,7 @@
 #include "mfd_solve_plan.h"
 
 #include <algorithm>
+#include <array>
 #include <climits>
 #include <cstdio>
 
@@ -30,7 +31,7 @@ constexpr int kManyRows = 2048;
 // A level's tasks of one phase beyond kManyTasks are taken several to a
 // ticket, at most kTicketMost (every ticket is an addition to one counter).
 constexpr int kManyTasks = 4096, kTicketMost = 8;
-constexpr int kFlagLine = 32;  // super fronts keep their counters a cache line apart: many workgroups poll each
+constexpr int kFlagLine = 32;  // super fronts keep their counters up to a cache line apart: many workgroups poll each
 
 }  // namespace
 
@@ -42,7 +43,8 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     auto super = [&](int s) { return super_min > 0 && nodes[s].c >= super_min; };
     auto nsup = [&](int s) { return (nodes[s].c + kSuper - 1) / kSuper; };
     auto width = [&](int s, int u) { return std::min(kSuper, nodes[s].c - kSuper * u); };
-    auto chunks = [&](int s) { return (nodes[s].w + kSuper - 1) / kSuper; };
+    std::vector<int> part_rows(m, kSuper);  // update rows of a kBwdPart task
+    auto chunks = [&](int s) { return (nodes[s].w + part_rows[s] - 1) / part_rows[s]; };
 
     // superblock matrices
     std::vector<int64_t> xoff(m, -1);
@@ -80,36 +82,71 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
         }
     }
 
-    // Planes: a front's update rows (with its pivot rows, where tasks pass
-    // them on) in the forward sweep, its partial sums in the backward one.
-    // The partial sums of a tree take the place of that tree's rows: its
-    // backward sweep starts when its forward sweep has ended.
+    // Planes: a front's update rows (and the pivot rows that tasks pass on,
+    // those of superblock first_kept and later ones) in the forward sweep, its
+    // partial sums in the backward one.  The partial sums of a tree take the
+    // place of that tree's rows: its backward sweep starts when its forward
+    // sweep has ended.  Those of a front's children, written when the front's
+    // x is complete, take the place of its own.
     std::vector<int> root(m);
     for (int s = m - 1; s >= 0; --s) root[s] = nodes[s].parent < 0 ? s : root[nodes[s].parent];
-    std::vector<int64_t> rows(m, 0), slots(m, 0), base(m, 0);  // per root
-    std::vector<int64_t> z(m), slot0(m);
+    std::vector<int64_t> rows(m, 0), base(m, 0), most(m, 0);  // per root
+    std::vector<int64_t> z(m), slots(m), slot0(m, 0);
+    auto first_kept = [&](int s) { return super(s) ? 2 : 1; };
     for (int s = 0; s < m; ++s) {
-        const bool keep = nsup(s) > (super(s) ? 2 : 1);
-        z[s] = rows[root[s]] - (keep ? 0 : nodes[s].c);
-        rows[root[s]] += keep ? nodes[s].n : nodes[s].w;
-        slot0[s] = slots[root[s]];
-        if (!whole[s] && nodes[s].w > 0) slots[root[s]] += (int64_t)64 * ((nodes[s].c + 63) / 64) * chunks(s);
+        const int from = std::min(kSuper * first_kept(s), nodes[s].c);  // the first row kept
+        z[s] = rows[root[s]] - from;
+        rows[root[s]] += nodes[s].n - from;
+        most[root[s]] += nodes[s].w + nodes[s].c * 3LL / 4;
+    }
+    // A tree whose partial sums would take more than its rows do, and than its
+    // update rows and three quarters of an entry per unknown (few, large
+    // fronts), forms them over more rows at a time: with y, b and x a solve
+    // then takes at most the update rows and four vectors, however the fronts
+    // are shaped.
+    for (bool again = true; again;) {
+        again = false;
+        std::vector<int64_t> below(m, 0);
+        for (int s = 0; s < m; ++s) {  // of the subtree: its own, or its children's
+            const int64_t own = !whole[s] && nodes[s].w > 0 ? (int64_t)64 * ((nodes[s].c + 63) / 64) * chunks(s) : 0;
+            slots[s] = std::max(own, below[s]);
+            if (nodes[s].parent >= 0) below[nodes[s].parent] += slots[s];
+        }
+        for (int s = m - 1; s >= 0; --s) {  // roots before their fronts
+            const int r = root[s];
+            if (slots[r] <= std::max(rows[r], most[r]) || part_rows[s] >= nodes[s].w) continue;
+            part_rows[s] *= 2;
+            again = true;
+        }
     }
     for (int s = 0; s < m; ++s)
         if (root[s] == s) {
             base[s] = P.plane;
             P.plane += std::max(rows[s], slots[s]);
         }
+    for (int s = m - 1; s >= 0; --s) {  // parents before children
+        int64_t at = slot0[s];
+        for (int ch : S.children[s]) {
+            slot0[ch - 1] = at;
+            at += slots[ch - 1];
+        }
+    }
     int64_t glen = 0, grows = (int64_t)S.l_rows.size();
     for (int s = 0; s < m; ++s)
         if (!S.children[s].empty()) glen += nodes[s].n;
-    // counters
+    // counters: asm, and z, y, p, t and x of every superblock, or (fstr 0) one
+    // for all of a front of one superblock that is no super front, whose
+    // phases follow one another: asm, y, p, x.  Six words of memory each (two
+    // and four for fronts of one and two columns, so that counters never take
+    // more than an entry per unknown): a word each, 32 fronts polled and raised
+    // in one cache line, makes a solve 2 to 4% slower.
     std::vector<int> flag(m), fstr(m);
     int64_t nflags = 0;
     for (int s = 0; s < m; ++s) {
-        fstr[s] = super(s) ? kFlagLine : 1;
+        const int c = nodes[s].c;
+        fstr[s] = super(s) ? std::max(1, std::min(kFlagLine, c / 3)) : nsup(s) == 1 ? 0 : 1;
         flag[s] = (int)nflags;
-        nflags += (int64_t)fstr[s] * (1 + 5 * nsup(s));
+        nflags += fstr[s] == 0 ? std::min(6, 2 * c) : (int64_t)fstr[s] * (1 + 5 * nsup(s));
         if (nflags > INT_MAX / 2) return MFD_ERR_NOMEM;
     }
     if (P.plane > INT_MAX || glen > INT_MAX || grows > INT_MAX) return MFD_ERR_NOMEM;
@@ -157,8 +194,13 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     // counter of front s: kind q (0 z, 1 y, 2 p, 3 t, 4 x) of superblock u
     auto asm_flag = [&](int s) { return flag[s]; };
     auto counter = [&](int s, int q, int u) { return flag[s] + fstr[s] * (1 + q * nsup(s) + u); };
-    auto yx_target = [&](int s, int u) { return super(s) ? (width(s, u) + 15) / 16 : 1; };
     std::vector<int> arrivals(m, 0);  // signals to each front's asm counter
+    auto before_y = [&](int s) { return fstr[s] == 0 ? arrivals[s] : 0; };
+    auto parts = [&](int s, int u) { return whole[s] || nodes[s].w == 0 ? 0 : (width(s, u) + 31) / 32 * chunks(s); };
+    auto yx_count = [&](int s, int u) { return super(s) ? (width(s, u) + 15) / 16 : 1; };
+    auto y_target = [&](int s, int u) { return before_y(s) + yx_count(s, u); };
+    auto p_target = [&](int s, int u) { return (fstr[s] == 0 ? y_target(s, u) : 0) + parts(s, u); };
+    auto x_target = [&](int s, int u) { return (fstr[s] == 0 ? p_target(s, u) : 0) + yx_count(s, u); };
     auto task = [&](int s, int kind, int u) {
         const NodeDev& d = nodes[s];
         SolveTask t{};
@@ -219,14 +261,14 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
             for (int k = b0; k < b1; ++k) {
                 const int s = level_nodes[k];
                 if (u >= nsup(s)) continue;
-                const int w = width(s, u), first_kept = super(s) ? 2 : 1;
+                const int w = width(s, u);
                 int zt = 0;
-                if (u >= first_kept)
+                if (u >= first_kept(s))
                     zt = add_rows(s, kSuper * u, kSuper * u + w, super(s) ? u - 1 : u, u, counter(s, 0, u));
                 for (int r = 0; r < (super(s) ? w : 1); r += 16) {
                     SolveTask t = task(s, super(s) ? kFwdTop : kFwdPiv, u);
                     t.r0 = r;
-                    if (u >= first_kept)
+                    if (u >= first_kept(s))
                         wait(t, counter(s, 0, u), zt);
                     else
                         wait(t, asm_flag(s), arrivals[s]);
@@ -261,12 +303,12 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
             for (int c0 = 0; c0 < nodes[s].c; c0 += 32)
                 for (int q = 0; q < chunks(s); ++q) {
                     SolveTask t = task(s, kBwdPart, c0 / kSuper);
-                    t.r0 = nodes[s].c + kSuper * q;
-                    t.nr = std::min(kSuper, nodes[s].n - t.r0);
+                    t.r0 = nodes[s].c + part_rows[s] * q;
+                    t.nr = std::min(part_rows[s], nodes[s].n - t.r0);
                     t.slot = (int)(base[root[s]] + slot0[s]) + 64 * (c0 / 64 * chunks(s) + q) + c0 % 64;
                     t.nslot = c0;
                     t.sig = counter(s, 2, c0 / kSuper);
-                    if (pa >= 0) wait(t, counter(pa, 4, 0), yx_target(pa, 0));
+                    if (pa >= 0) wait(t, counter(pa, 4, 0), x_target(pa, 0));
                     P.tasks.push_back(t);
                 }
         }
@@ -281,9 +323,9 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
                 // rows, its own forward tasks
                 auto wait_y = [&](SolveTask& t) {
                     if (nslot > 0)
-                        wait(t, counter(s, 2, u), (w + 31) / 32 * nslot);
+                        wait(t, counter(s, 2, u), p_target(s, u));
                     else
-                        wait(t, counter(s, 1, u), yx_target(s, u));
+                        wait(t, counter(s, 1, u), y_target(s, u));
                     t.nslot = nslot;
                 };
                 const bool cols = vlo < nsup(s);
@@ -303,7 +345,7 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
                         wait(t, counter(s, 3, u), (w + 15) / 16);
                     } else if (whole[s] && pa >= 0) {
                         t.nr = nodes[s].w;
-                        wait(t, counter(pa, 4, 0), yx_target(pa, 0));
+                        wait(t, counter(pa, 4, 0), x_target(pa, 0));
                     } else {
                         wait_y(t);
                     }
@@ -319,36 +361,67 @@ int build_solve_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
 
 int64_t check_solve_plan(const SolvePlan& P, std::string& report)
 {
-    std::vector<int> now(P.nflags, 0), total(P.nflags, 0);
     auto counter = [](const SolveTask& t, int q, int u) { return t.flag + t.fstr * (1 + q * t.nsup + u); };
-    auto target = [](const SolveTask& t, int u) { return t.super ? (std::min(kSuper, t.c - kSuper * u) + 15) / 16 : 1; };
-    // the counters a task raises, as its kernel function does
-    auto raise = [&](const SolveTask& t, std::vector<int>& f) {
-        if (t.kind == kFwdTop || t.kind == kFwdPiv) f[counter(t, 1, t.u)]++;
-        if (t.kind == kBwdTop || t.kind == kBwdPiv) f[counter(t, 4, t.u)]++;
-        if (t.kind != kFwdTop && t.kind != kBwdTop && t.kind != kBwdPiv && t.sig >= 0) f[t.sig]++;
+    auto count = [](const SolveTask& t, int u) { return t.super ? (std::min(kSuper, t.c - kSuper * u) + 15) / 16 : 1; };
+    // the counters a task raises, as its kernel function does; which of its
+    // phases a shared counter (fstr 0) is in: 0 asm, 1 y, 2 p, 3 x
+    auto raise = [&](const SolveTask& t, auto&& f) {
+        if (t.kind == kFwdTop || t.kind == kFwdPiv) f(counter(t, 1, t.u), 1);
+        if (t.kind == kBwdTop || t.kind == kBwdPiv) f(counter(t, 4, t.u), 3);
+        if (t.kind != kFwdTop && t.kind != kBwdTop && t.kind != kBwdPiv && t.sig >= 0)
+            f(t.sig, t.kind == kBwdPart ? 2 : 0);
     };
-    for (const SolveTask& t : P.tasks) raise(t, total);
     int64_t bad = 0;
     char line[160];
+    auto fault = [&](size_t i, const char* what, int f, int now, int want) {
+        if (++bad > 8) return;
+        snprintf(line, sizeof line, "solve task %zu (kind %d, superblock %d): %s, counter %d at %d, wants %d\n", i,
+                 P.tasks[i].kind, P.tasks[i].u, what, f, now, want);
+        report += line;
+    };
+    // signals of each counter up to the end of each phase (separate counters
+    // have one phase, whatever its number)
+    std::vector<int> now(P.nflags, 0);
+    std::vector<std::array<int, 4>> upto(P.nflags, std::array<int, 4>{0, 0, 0, 0});
+    std::vector<char> shared(P.nflags, 0);
+    for (const SolveTask& t : P.tasks)
+        if (t.fstr == 0) shared[t.flag] = 1;
+    for (const SolveTask& t : P.tasks)
+        raise(t, [&](int f, int ph) {
+            for (int q = shared[f] ? ph : 0; q < 4; ++q) upto[f][q]++;
+        });
     for (size_t i = 0; i < P.tasks.size(); ++i) {
         const SolveTask& t = P.tasks[i];
         auto need = [&](int f, int want) {
-            if (f < 0 || (now[f] >= want && total[f] == want)) return;
-            if (++bad <= 8) {
-                snprintf(line, sizeof line, "solve task %zu (kind %d, superblock %d): counter %d at %d of %d, wants %d\n", i,
-                         t.kind, t.u, f, now[f], total[f], want);
-                report += line;
-            }
+            if (f < 0) return;
+            const auto& e = upto[f];
+            if (now[f] < want)
+                fault(i, "waits for later tasks", f, now[f], want);
+            else if (std::find(e.begin(), e.end(), want) == e.end())
+                fault(i, "waits for part of a phase", f, now[f], want);
         };
         need(t.w0, t.w0t);
+        const int y0 = t.fstr == 0 ? t.w0t : 0;  // as fwd_rows and fwd_rows64 wait
         if (t.kind == kFwdRows || t.kind == kFwdRows64)
-            for (int v = 0; v < t.nslot; ++v) need(counter(t, 1, v), target(t, v));
-        if (t.kind == kFwdTop && t.u > 0) need(counter(t, 1, t.u - 1), target(t, t.u - 1));
+            for (int v = 0; v < t.nslot; ++v) need(counter(t, 1, v), y0 + count(t, v));
+        if (t.kind == kFwdTop && t.u > 0) need(counter(t, 1, t.u - 1), count(t, t.u - 1));
         if (t.kind == kBwdCols)
-            for (int v = t.nsup - 1; v >= t.grow; --v) need(counter(t, 4, v), target(t, v));
-        if (t.kind == kBwdTop && t.u + 1 < t.nsup) need(counter(t, 4, t.u + 1), target(t, t.u + 1));
-        raise(t, now);
+            for (int v = t.nsup - 1; v >= t.grow; --v) need(counter(t, 4, v), count(t, v));
+        if (t.kind == kBwdTop && t.u + 1 < t.nsup) need(counter(t, 4, t.u + 1), count(t, t.u + 1));
+        raise(t, [&](int f, int ph) {
+            // a shared counter's phase starts when the one before has ended: y
+            // after a wait for asm; p, and x without partial sums, after one
+            // for the parent's x, which follows this front's y; x after one
+            // for p, or, in a root, for y
+            if (shared[f] && ph > 0) {
+                if (now[f] < upto[f][ph - 1]) fault(i, "raises a phase early", f, now[f], upto[f][ph - 1]);
+                const int after = upto[f][ph - 1];
+                const bool own = t.w0 == f && t.w0t == after, none = after == 0;
+                const bool parent = t.w0 >= 0 && t.w0 != f && (ph == 2 || upto[f][2] == upto[f][1]);
+                if (!own && !(ph == 1 && none) && !(ph >= 2 && parent)) fault(i, "raises a phase unordered", f, now[f], after);
+            }
+            now[f]++;
+        });
     }
     return bad;
 }
