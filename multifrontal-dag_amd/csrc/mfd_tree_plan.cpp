@@ -123,6 +123,7 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     P.asrc.reserve(entries);
     P.arc.reserve(entries);
     P.aptr.reserve(panels);
+    std::vector<int64_t> last;
     for (int i = 0; i < count; ++i) {
         const int s = P.node[i];
         const NodeDev& d = nodes[s];
@@ -144,13 +145,13 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
         for (int q = 0; q < d.c; ++q) {
             if (q % 16 == 0) P.aptr.push_back((int)P.asrc.size());
             const int j = d.first + q;  // 0-based global column
-            for (int64_t p = S.a_colptr[j]; p < S.a_colptr[j + 1]; ++p) {
+            each_assembled(S, j, last, [&](int64_t p) {
                 const int r = S.snidx[p];
                 const int grow = r <= d.c ? d.first + r - 1 : S.l_rows[S.l_ptr[s] + (r - d.c - 1)] - 1;
                 P.apos.push_back((r - 1) | (q % 16) << 8);
                 P.asrc.push_back((int)(S.ccs_perm[p] - 1));
                 P.arc.push_back(TreePlan::RowCol{grow, j});
-            }
+            });
         }
         P.aptr.push_back((int)P.asrc.size());
         P.tasks.push_back(t);
