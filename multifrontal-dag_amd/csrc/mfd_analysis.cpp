@@ -278,6 +278,23 @@ struct Lists {
     }
 };
 
+// S.superseded from S.snidx and S.a_colptr.
+void find_superseded(Structure& S)
+{
+    std::vector<int64_t> last;  // per row, the last entry with it
+    for (int j = 0; j < S.n; ++j) {
+        const int64_t p0 = S.a_colptr[j];
+        for (int64_t p = p0; p < S.a_colptr[j + 1]; ++p) {
+            const int r = S.snidx[p];
+            if (r >= (int)last.size()) last.resize(r + 1, -1);
+            if (last[r] >= p0) {
+                if (S.superseded.empty()) S.superseded.assign(S.snidx.size(), 0);
+                S.superseded[last[r]] = 1;
+            }
+            last[r] = p;
+        }
+    }
+}
 }  // namespace
 
 int analyze(int n, const int* ccs_col, const int* ccs_row, int max_zero, const int* perm_in, Structure& S)
@@ -487,6 +504,7 @@ int analyze(int n, const int* ccs_col, const int* ccs_row, int max_zero, const i
         for (int j = f; j < f + c; ++j)
             for (int64_t p = AS.ptr[j - 1]; p < AS.ptr[j]; ++p) S.snidx[p] = pos[AS.val[p]];
     }
+    find_superseded(S);
     // create_local_index (create_local_index_m.f90:10-45)
     S.li_ptr = L.ptr;
     S.lidx.assign(L.val.size(), 0);
@@ -561,6 +579,7 @@ int structure_from_parts(int num_node, const int* c, const int* w, const int* pa
                     if (r < j - S.first[s] + 1 || r > n) return MFD_ERR_ARG;  // lower part of the front
                 }
         }
+        find_superseded(S);
     }
     return MFD_OK;
 }
@@ -597,10 +616,15 @@ int analyze_batch(int nsys, const int* n, const int* const* ccs_col, const int* 
         }
         for (int v : S.l_rows) out.l_rows.push_back(v + col_off);
         out.lidx.insert(out.lidx.end(), S.lidx.begin(), S.lidx.end());
+        if (!S.superseded.empty()) {
+            out.superseded.resize(a_off, 0);
+            out.superseded.insert(out.superseded.end(), S.superseded.begin(), S.superseded.end());
+        }
         out.n += S.n;
         out.num_node += S.num_node;
         entries += (int64_t)ccs_col[k][n[k]] - 1;
     }
+    if (!out.superseded.empty()) out.superseded.resize(out.snidx.size(), 0);
     out.a_colptr.push_back((int64_t)out.snidx.size());
     out.first.push_back(out.n + 1);
     out.l_ptr.push_back((int64_t)out.l_rows.size());

@@ -16,6 +16,7 @@ struct Structure {
     std::vector<int64_t> ccs_perm;   // a_structure entry -> caller entry (1-based), length nnz
     std::vector<int64_t> a_colptr;   // postordered lower CCS column pointers (0-based), n + 1
     std::vector<int> snidx;          // supernodal_index: front-relative row (1-based) per entry
+    std::vector<char> superseded;    // entry -> a later one of its column has its row (empty: none has)
     std::vector<int> c, w, parent;   // per node: pivot columns, update rows, parent (1-based, 0 root)
     std::vector<int> first;          // first global column (1-based) per node, num_node + 1
     std::vector<int64_t> l_ptr;      // row list (l_structure) pointers, num_node + 1
@@ -44,22 +45,10 @@ int analyze_batch(int nsys, const int* n, const int* const* ccs_col, const int* 
 int structure_from_parts(int num_node, const int* c, const int* w, const int* parent, const int* lidx,
                          const int64_t* a_colptr, const int* snidx, Structure& out);
 
-// Calls f(p) for the entries of A that the fronts' column j (0-based) is
-// assembled from, in order: all of them, but of those with the same row only
-// the last (the reference stores them one after another,
-// coefficient_setter_m.f90:26-41).  last: working space.
-template <typename F> void each_assembled(const Structure& S, int j, std::vector<int64_t>& last, F&& f)
-{
-    const int64_t p0 = S.a_colptr[j], p1 = S.a_colptr[j + 1];
-    bool ascending = true;
-    for (int64_t p = p0 + 1; p < p1; ++p) ascending = ascending && S.snidx[p] > S.snidx[p - 1];
-    for (int64_t p = p0; !ascending && p < p1; ++p) {
-        if ((int)last.size() <= S.snidx[p]) last.resize(S.snidx[p] + 1);
-        last[S.snidx[p]] = p;
-    }
-    for (int64_t p = p0; p < p1; ++p)
-        if (ascending || last[S.snidx[p]] == p) f(p);
-}
+// Whether entry p of A is assembled: of several with one row and column the
+// last is (the reference stores them one after another,
+// coefficient_setter_m.f90:26-41).
+inline bool assembled(const Structure& S, int64_t p) { return S.superseded.empty() || !S.superseded[p]; }
 
 int64_t cost(const Structure& s);      // cost_calculator_m.f90:9-20
 int64_t nonzero(const Structure& s);   // cost_calculator_m.f90:22-33

@@ -887,20 +887,21 @@ void build_csr(const Structure& S, std::vector<int>& ptr, std::vector<int>& col,
         int c = S.c[s];
         return r <= c ? S.first[s] + r - 1 : S.l_rows[S.l_ptr[s] + (r - c - 1)];
     };
-    std::vector<int64_t> last;
     for (int j = 1; j <= n; ++j)
-        each_assembled(S, j - 1, last, [&](int64_t p) {
+        for (int64_t p = S.a_colptr[j - 1]; p < S.a_colptr[j]; ++p) {
+            if (!assembled(S, p)) continue;
             int r = global_row(j, p);
             cnt[r]++;
             if (r != j) cnt[j]++;
-        });
+        }
     ptr.assign(n + 1, 0);
     for (int i = 0; i < n; ++i) ptr[i + 1] = ptr[i] + cnt[i + 1];
     col.assign(ptr[n], 0);
     src.assign(ptr[n], 0);
     std::vector<int> pos(ptr.begin(), ptr.end() - 1);
     for (int j = 1; j <= n; ++j)
-        each_assembled(S, j - 1, last, [&](int64_t p) {
+        for (int64_t p = S.a_colptr[j - 1]; p < S.a_colptr[j]; ++p) {
+            if (!assembled(S, p)) continue;
             int r = global_row(j, p);
             int64_t v = S.ccs_perm[p] - 1;
             col[pos[r - 1]] = j - 1;
@@ -909,7 +910,7 @@ void build_csr(const Structure& S, std::vector<int>& ptr, std::vector<int>& col,
                 col[pos[j - 1]] = r - 1;
                 src[pos[j - 1]++] = v;
             }
-        });
+        }
 }
 
 int setup_device(mfd_handle* h)
@@ -959,35 +960,37 @@ int setup_device(mfd_handle* h)
     // assembly map: A entry -> front position (coefficient_setter_m.f90:26-41),
     // the entries in the fill tasks' order
     const int64_t nscat = (int64_t)S.snidx.size() - h->tp.entries;  // at least those
-    std::vector<int64_t> dst(nscat), src(nscat), diag_src(S.n, 0), last;
+    std::vector<int64_t> dst(nscat), src(nscat), diag_src(S.n, 0);
     std::vector<int2> rc(nscat);
     int64_t e = 0;
     FillTask* task = h->fill.data();
     for (size_t g = 0; g < h->group_level.size(); ++g) {
         for (int s = 0; s < S.num_node; ++s) {
-            if (h->front_group[s] != (int)g) continue;
+            if (h->front_group[s] != (int)g || h->tp.has(s)) continue;  // (assembled in their own launch)
             const NodeDev& d = h->nodes[s];
-            const bool host = !h->hplan.is_host.empty() && h->hplan.is_host[s];
-            const bool mine = !host && !h->tp.has(s);  // not assembled on the host or in its own launch
+            const bool mine = h->hplan.is_host.empty() || !h->hplan.is_host[s];  // not assembled on the host
             for (int j = S.first[s]; j < S.first[s + 1]; ++j) {
                 int64_t q = j - S.first[s];
                 if (mine && q % kFillCols == 0) task[q / kFillCols].e0 = e;
-                each_assembled(S, j - 1, last, [&](int64_t p) {
+                for (int64_t p = S.a_colptr[j - 1]; p < S.a_colptr[j]; ++p) {
+                    if (!assembled(S, p)) continue;
                     // global row: a pivot row of this front or one of its update rows
                     const int r = S.snidx[p];
                     const int grow = r <= S.c[s] ? S.first[s] + r - 1 : S.l_rows[S.l_ptr[s] + (r - S.c[s] - 1)];
                     if (grow == j) diag_src[j - 1] = S.ccs_perm[p] - 1;
-                    if (!mine) return;
+                    if (!mine) continue;
                     dst[e] = d.front + (S.snidx[p] - 1) + q * d.n;
                     src[e] = S.ccs_perm[p] - 1;
                     rc[e] = make_int2(grow - 1, j - 1);
                     ++e;
-                });
+                }
                 if (mine) task[q / kFillCols].e1 = e;
             }
             if (mine) task += (d.n + kFillCols - 1) / kFillCols;
         }
     }
+    for (size_t k = 0; k < h->tp.arc.size(); ++k)
+        if (h->tp.arc[k].row == h->tp.arc[k].col) diag_src[h->tp.arc[k].col] = h->tp.asrc[k];
     MFD_TRY(upload(h, &h->d_fill, h->fill));
     if (e > nscat - h->hplan.entries) return MFD_ERR_INTERNAL;
     dst.resize(e);

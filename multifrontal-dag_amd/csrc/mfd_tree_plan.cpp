@@ -112,7 +112,7 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     });
     std::vector<int> pos(m, -1);
     for (int i = 0; i < count; ++i) pos[P.node[i]] = i;
-    P.tasks.reserve(count);
+    P.tasks.resize(count);
     int64_t entries = 0, panels = 0;
     for (int s : P.node) {
         const int c0 = nodes[s].first, c1 = c0 + nodes[s].c;
@@ -123,9 +123,9 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
     P.asrc.reserve(entries);
     P.arc.reserve(entries);
     P.aptr.reserve(panels);
-    std::vector<int64_t> last;
-    for (int i = 0; i < count; ++i) {
-        const int s = P.node[i];
+    for (int s = 0; s < m; ++s) {  // (the lists in the order of the nodes, as the structure has them)
+        if (!in[s]) continue;
+        const int i = pos[s];
         const NodeDev& d = nodes[s];
         TreeTask t{};
         t.front = d.front;
@@ -145,16 +145,17 @@ void build_tree_plan(const Structure& S, const std::vector<NodeDev>& nodes, cons
         for (int q = 0; q < d.c; ++q) {
             if (q % 16 == 0) P.aptr.push_back((int)P.asrc.size());
             const int j = d.first + q;  // 0-based global column
-            each_assembled(S, j, last, [&](int64_t p) {
+            for (int64_t p = S.a_colptr[j]; p < S.a_colptr[j + 1]; ++p) {
+                if (!assembled(S, p)) continue;
                 const int r = S.snidx[p];
                 const int grow = r <= d.c ? d.first + r - 1 : S.l_rows[S.l_ptr[s] + (r - d.c - 1)] - 1;
                 P.apos.push_back((r - 1) | (q % 16) << 8);
                 P.asrc.push_back((int)(S.ccs_perm[p] - 1));
                 P.arc.push_back(TreePlan::RowCol{grow, j});
-            });
+            }
         }
         P.aptr.push_back((int)P.asrc.size());
-        P.tasks.push_back(t);
+        P.tasks[i] = t;
     }
     P.entries = (int64_t)P.asrc.size();
     for (int i = 0; i < count;) {
