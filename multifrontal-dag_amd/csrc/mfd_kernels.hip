@@ -1679,11 +1679,13 @@ __global__ void k_zero_u64(unsigned long long* p, int n)
 
 // Lanes per row of the CSR kernels: about a third of a row's entries, so that
 // few lanes idle on the last ones (4 for the 7-point grids, 8 and 32 for the
-// 27-point ones with one and three unknowns).
+// 27-point ones with one and three unknowns, 16 with two).  A band of 150,000
+// rows, four right-hand sides: 45 entries a row 63 us with 32 lanes, 43 with
+// 16; 59 entries 66 and 53; 41 entries 42 with 8.
 static int row_lanes(int n, int64_t nnz)
 {
     const int64_t per = nnz / n;
-    return per <= 12 ? 4 : per <= 40 ? 8 : 32;
+    return per <= 12 ? 4 : per <= 40 ? 8 : per <= 72 ? 16 : 32;
 }
 void launch_residual(double* r, const double* b, const double* x, int n, int nrhs, const int* ptr, const int* col,
                      const double* val, int64_t nnz, hipStream_t st)
@@ -1695,6 +1697,8 @@ void launch_residual(double* r, const double* b, const double* x, int n, int nrh
         hipLaunchKernelGGL(k_residual<4>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
     else if (g == 8)
         hipLaunchKernelGGL(k_residual<8>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
+    else if (g == 16)
+        hipLaunchKernelGGL(k_residual<16>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
     else
         hipLaunchKernelGGL(k_residual<32>, grid, block, 0, st, r, b, x, n, nrhs, ptr, col, val);
 }
@@ -1709,6 +1713,8 @@ void launch_gather_vals(unsigned long long* out, double* val, const double* a, c
         hipLaunchKernelGGL(k_gather_vals<4>, grid, block, 0, st, out, val, a, src, n, ptr);
     else if (g == 8)
         hipLaunchKernelGGL(k_gather_vals<8>, grid, block, 0, st, out, val, a, src, n, ptr);
+    else if (g == 16)
+        hipLaunchKernelGGL(k_gather_vals<16>, grid, block, 0, st, out, val, a, src, n, ptr);
     else
         hipLaunchKernelGGL(k_gather_vals<32>, grid, block, 0, st, out, val, a, src, n, ptr);
 }
