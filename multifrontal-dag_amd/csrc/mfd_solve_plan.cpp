@@ -20,16 +20,22 @@ namespace {
 
 // A front of one superblock whose update rows its own workgroup takes as
 // well (no hand-over to other workgroups): with at most kWholeRows of them,
-// where a hand-over (about 3 us) costs more than the rows do; on a level of
-// at least kManyFronts fronts, which fill the chip by themselves, at most
-// kWholeMany.
+// where a hand-over (about 3 us) costs more than the rows do (solves of a
+// 37 x 29 x 23 grid, 33 right-hand sides, and of a 250^2 grid with fronts of
+// its own columns only: 547 and 1619 us; with 64 rows 588 and 1619, with 256
+// 542 and 1728); on a level of at least kManyFronts fronts, which fill the chip
+// by themselves, at most kWholeMany (512 systems 3.82 ms, 3.85 with 128).
 constexpr int kWholeRows = 128, kWholeMany = 256;
 constexpr int kManyFronts = 512;
 // Rows per forward task: 16, four waves a quarter of the columns each, until
-// a level has more than kManyRows tasks of them; then 64.
-constexpr int kManyRows = 2048;
+// a level has more than kManyRows tasks of them; then 64 (48^3 solves 747 us
+// from 2048 tasks on, 729 from 1024, 714 from 512, 729 from 256; 64^3 with four
+// right-hand sides 1.570 ms, 1.556, 1.551, 1.550; with 16 rows throughout 800
+// and 1.765).
+constexpr int kManyRows = 512;
 // A level's tasks of one phase beyond kManyTasks are taken several to a
-// ticket, at most kTicketMost (every ticket is an addition to one counter).
+// ticket, at most kTicketMost (every ticket is an addition to one counter):
+// 512 systems 3.82 ms, 3.86 with one each.
 constexpr int kManyTasks = 4096, kTicketMost = 8;
 constexpr int kFlagLine = 32;  // super fronts keep their counters up to a cache line apart: many workgroups poll each
 

@@ -9,7 +9,8 @@ namespace mfd {
 
 namespace {
 // Fronts of one height beyond kManyTasks are taken several to a ticket, at
-// most kTicketMost (every ticket is an addition to one counter).
+// most kTicketMost (every ticket is an addition to one counter; 512 systems
+// 9.13 ms, 9.15 with one each, 9.11 with 16).
 constexpr int kManyTasks = 8192, kTicketMost = 4;
 
 // Microseconds of a factorization (FP64) whose eligible fronts of order <=
