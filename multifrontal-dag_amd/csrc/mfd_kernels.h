@@ -9,7 +9,6 @@
 
 namespace mfd {
 
-template <typename T> void launch_fill(T* p, int64_t n, hipStream_t st);
 // Zero fronts with A's entries in place (see k_assemble); scale: the 16-bit
 // forms' diagonal scaling, or null.
 template <typename T>
@@ -52,8 +51,8 @@ void launch_gemm(T* pool, const GemmTask* tasks, int count, int kind, const int*
 template <typename T>
 void launch_gemm_seg(T* pool, const GemmTask* tasks, const SegTask* segs, const int* seg_ptr, int groups,
                      const FixTask* fixes, int nfix, T* part, const int* lidx, hipStream_t st, int lowp = 0);
-// 64 x 64 blocks of the superblock matrices: X by block distance (wv =
-// false), then the W and V blocks (wv = true, MFMA tile products)
+// The superblock matrices: columns of X (wv = false), then the 64 x 64 blocks
+// of W and V (wv = true, MFMA tile products).
 template <typename T>
 void launch_superinv(const T* pool, T* sinv, const NodeDev* nodes, const SuperInvTask* tasks, int count, bool wv,
                      hipStream_t st);

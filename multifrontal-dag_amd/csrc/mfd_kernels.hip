@@ -355,14 +355,6 @@ __device__ __forceinline__ void factor_dense64(Front64<T>& S, T* g, int64_t ld, 
 }  // namespace
 
 // ---------------------------------------------------------------- assembly
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_fill(T* p, int64_t n)
-{
-    int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    int64_t stride = (int64_t)gridDim.x * kThreads;
-    for (; i < n; i += stride) p[i] = T(0);
-}
-
 // The lower part (row >= col; the upper part of a front is never read) of
 // kFillCols columns of one front: zero, but for the stored A entries, each of
 // which lands on exactly one front position (coefficient_setter_m.f90:26-50
@@ -1739,14 +1731,8 @@ void launch_zero_u64(unsigned long long* p, int n, hipStream_t st)
 __global__ void k_set_int(int* p, int v) { *p = v; }
 
 // ------------------------------------------------------------- launchers
-static inline int grid_for(int64_t n) { return (int)std::min<int64_t>((n + kThreads - 1) / kThreads, 65536); }
-
 void launch_set_int(int* p, int v, hipStream_t st) { hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, st, p, v); }
 
-template <typename T> void launch_fill(T* p, int64_t n, hipStream_t st)
-{
-    if (n > 0) hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(n)), dim3(kThreads), 0, st, p, n);
-}
 template <typename T>
 void launch_assemble(T* pool, const NodeDev* nodes, const FillTask* tasks, int count, const double* a,
                      const int64_t* dst, const int64_t* src, const int2* rc, const double* scale, hipStream_t st)
@@ -1891,7 +1877,6 @@ void launch_scatter_rows(double* out, int ld_out, const double* in, int ld_in, c
 }
 
 #define MFD_INSTANTIATE(T)                                                                                             \
-    template void launch_fill<T>(T*, int64_t, hipStream_t);                                                            \
     template void launch_assemble<T>(T*, const NodeDev*, const FillTask*, int, const double*, const int64_t*,          \
                                      const int64_t*, const int2*, const double*, hipStream_t);                         \
     template void launch_pull_children<T>(T*, const int*, const NodeDev*, const PullTask*, int, const int*,            \

@@ -59,13 +59,15 @@ struct Launch {
     int side = 0, side_id = -1, wait_id = -1;
 };
 
-// A step's update tiles join the step's launch (k_upd_diag, one workgroup
-// per CU at its LDS) up to this many; more run as their own launch.
 // The front zeroing is split into at most kFillGroups groups of levels of at
 // least kFillMin entries (32 MB in FP64, about 8 us of stores; a launch of its
 // own costs about as much).
 constexpr int kFillGroups = 32;
 constexpr int64_t kFillMin = 4 << 20;
+
+// A step's update tiles join the step's launch (k_upd_diag, one workgroup
+// per CU at its LDS) up to this many; more run as their own launch.  64^3
+// FP64 step 18.95 ms; up to 512 18.98, up to 256 19.10.
 constexpr int kFuseTiles = 1024;
 
 // The order of a launch's tiles: a front's tiles in squares of kSquare x
@@ -78,7 +80,8 @@ constexpr int kFuseTiles = 1024;
 constexpr int kXcds = 8, kXcdGroup = 64, kSquare = 8;
 
 // Step launches with at least this many diagonal tasks run their GEMM
-// tiles (TRSM and fused update tiles) as a second launch (k_gemm).
+// tiles (TRSM and fused update tiles) as a second launch (k_gemm).  Factoring
+// 512 systems takes 9.13 ms so, 9.14 with 256 or 1024, 9.23 in one launch.
 constexpr int kApartDiag = 512;
 
 // The in-panel update of the large fronts runs every `period` steps with
@@ -105,10 +108,11 @@ constexpr int kWideMinRows = 0;
 // Fronts with at least super_min pivot columns solve forward and backward
 // through explicit superblock matrices (kFwdTop, kBwdTop: sixteen workgroups
 // a superblock), formed at the end of the factorization; set per handle by
-// mfd_set_solve_block (0: never).  256: on the 64^3 workload the bounds 128,
-// 256, 512 and 1024 gave FP64 steps of 25.08, 25.13, 25.17 and 25.39 ms,
-// and on the 512-system batch 128 was slower than 512 (FP64 step 21.26
-// against 20.90 ms: its fronts of one partial superblock gain nothing).
+// mfd_set_solve_block (0: never).  256: factoring and solving in FP64 with the
+// bounds 128, 256, 512, 1024 and none took 19.13, 19.23, 19.30, 19.79 and 20.78
+// ms on the 64^3 workload (four right-hand sides), a 48^3 solve 0.67, 0.75,
+// 0.83, 0.99 and 1.58, but 512 systems 13.27 with 128 and 12.96 with 256 or
+// more (their fronts of half a superblock gain nothing).
 constexpr int kSuperMin = 256;
 
 double now_ms()

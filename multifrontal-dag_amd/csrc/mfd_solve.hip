@@ -48,7 +48,8 @@ __device__ __forceinline__ d4 mma(double a, double b, d4 c) { return Mfma<double
 
 // The vector operand of a task's products, rows of 16 right-hand sides, and
 // the four waves' partial products (which take the same place once the
-// operand has been read): four workgroups per CU.
+// operand has been read): four workgroups per CU, of which the registers allow
+// three in FP64.
 union SolveLds {
     double v[kSuper][kRhs + 1];
     double red[4][16][kRhs + 1];
@@ -847,7 +848,8 @@ void launch_solve_reset(int* flags, int64_t n, hipStream_t st)
         hipLaunchKernelGGL(k_solve_reset, dim3((unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, 512)),
                            dim3(kThreads), 0, st, flags, n);
 }
-// As many workgroups as the chip holds (four per CU); fewer tickets, fewer.
+// Four workgroups per CU (in FP64, where the chip holds three, the last quarter
+// finds the tickets gone); fewer tickets, fewer.
 template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st)
 {
     const int64_t total = (int64_t)A.ntasks * A.ngroups;
