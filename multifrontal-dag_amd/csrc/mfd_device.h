@@ -119,11 +119,10 @@ __device__ __forceinline__ int add_agent(int* p, int v)
 }
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// One thread: polls counter p until it reaches target.  After kSpinLimit
-// polls (about 6 s), or once another workgroup has done so, gives up: raises
-// stop and *err (host memory), so that every wait of the launch ends.  SLOW:
-// polls every 0.4 us at most.
-constexpr int kSpinLimit = 1 << 23;
+// One thread: polls counter p until it reaches target.  After as many polls as
+// the word after stop says (kWaitPolls: about 6 s), or once another workgroup
+// has done so, gives up: raises stop and *err (host memory), so that every
+// wait of the launch ends.  SLOW: polls every 0.4 us at most.
 template <bool SLOW = false> __device__ __forceinline__ void poll(const int* p, int target, int* stop, int* err)
 {
     for (int spins = 0; ld_agent(p) < target;) {
@@ -131,7 +130,7 @@ template <bool SLOW = false> __device__ __forceinline__ void poll(const int* p, 
             __builtin_amdgcn_s_sleep(12);
         else
             __builtin_amdgcn_s_sleep(1);
-        if ((++spins & 255) == 0 && (ld_agent(stop) != 0 || spins >= kSpinLimit)) {
+        if ((++spins & 255) == 0 && (ld_agent(stop) != 0 || spins >= ld_agent(stop + 1))) {
             st_agent(stop, 1);
             __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             break;

@@ -92,7 +92,9 @@ template <typename T> struct TreeArgs {
 };
 template <typename T> void launch_tree(const TreeArgs<T>& A, hipStream_t st);
 constexpr int kRhsGroup = 16;
-void launch_solve_reset(int* flags, int64_t n, hipStream_t st);
+// Zeroes n words; polls: the bound of a wait (kWaitPolls by default).
+constexpr int kWaitPolls = 1 << 23;
+void launch_solve_reset(int* flags, int64_t n, int polls, hipStream_t st);
 template <typename T> void launch_solve(const SolveArgs<T>& A, hipStream_t st);
 void launch_set_int(int* p, int v, hipStream_t st);
 void launch_residual(double* r, const double* b, const double* x, int n, int nrhs, const int* ptr, const int* col,

@@ -102,7 +102,8 @@ struct SolveTask {
     int per;          // turns the next ticket of the workgroup takes
 };
 // Words before the counters in the solve's control array: the two tickets
-// (whole solve or forward part; backward part), the stop word.
+// (whole solve or forward part; backward part), the stop word, after it the
+// bound of a wait.
 constexpr int kSolveTicket = 0, kSolveTicketBwd = 16, kSolveStop = 32, kSolveCtl = 64;
 
 // Part of superblock u's matrices.  k_superinv: columns [16 j, 16 j + 16) of

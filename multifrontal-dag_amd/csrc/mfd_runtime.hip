@@ -219,6 +219,7 @@ struct mfd_handle {
     SuperInvTask* d_xinv = nullptr;
     int solve_rc = 0;          // build_solve_plan's result for the current schedule
     int* wait_err = nullptr;   // pinned: set by a launch of which a wait reached its bound
+    int wait_polls = kWaitPolls;  // that bound
     double* d_sinv64 = nullptr;
     float* d_sinv32 = nullptr;
     int64_t pool_elems = 0;
@@ -1132,7 +1133,7 @@ template <typename T> hipError_t enqueue_factor(mfd_handle* h, bool profile)
     };
     launch_set_int(h->d_info, INT_MAX, st);
     const bool tree = !h->tp.tasks.empty();
-    if (tree) launch_solve_reset(h->d_tflags, kSolveCtl + (int64_t)h->tp.tasks.size(), st);
+    if (tree) launch_solve_reset(h->d_tflags, kSolveCtl + (int64_t)h->tp.tasks.size(), h->wait_polls, st);
     mark(0);
     // Zeroing and assembly of the fronts: beside the factorization, group by
     // group, when the fill stream and its events exist; otherwise (and when
@@ -1370,7 +1371,7 @@ template <typename T> void enqueue_solve(mfd_handle* h, const double* bp, double
     a.nflags = h->sp.nflags;
     a.ntasks = (int)h->sp.tasks.size();
     a.ticket = kSolveTicket;
-    launch_solve_reset(h->d_sflags, solve_words(h, nrhs), st);
+    launch_solve_reset(h->d_sflags, solve_words(h, nrhs), h->wait_polls, st);
     if ((h->flags & MFD_FLAG_PROFILE) == 0) {
         launch_solve<T>(a, st);
         return;
@@ -2084,6 +2085,7 @@ int mfd_create(mfd_handle** out, int nb, int flags)
     h->nb = nb;
     h->flags = flags;
     if (const char* lim = getenv("MFD_DEVICE_MEM_LIMIT")) h->mem_limit = atoll(lim);
+    if (const char* lim = getenv("MFD_WAIT_POLLS")) h->wait_polls = std::max(1, atoi(lim));
     int count = 0;
     if (hipGetDeviceCount(&count) == hipSuccess && count > 0) {
         hipDeviceProp_t prop;

@@ -21,7 +21,7 @@
 // out in that order by an atomic counter, and a workgroup that holds a
 // ticket is running; so the earliest unfinished task is always running and
 // never waits, whatever the number of resident workgroups and whatever else
-// the GPU runs.  Each wait is bounded all the same (kSpinLimit): a workgroup
+// the GPU runs.  Each wait is bounded all the same (kWaitPolls): a workgroup
 // that reaches the bound raises the stop word, every other wait then ends,
 // and the host reports an internal error.
 //
@@ -837,16 +837,17 @@ template <typename T> __global__ __launch_bounds__(kThreads, sizeof(T) == 8 ? 3 
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_solve_reset(int* p, int64_t n)
+__global__ __launch_bounds__(kThreads) void k_solve_reset(int* p, int64_t n, int polls)
 {
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) p[i] = 0;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
+        p[i] = i == kSolveStop + 1 ? polls : 0;
 }
 
-void launch_solve_reset(int* flags, int64_t n, hipStream_t st)
+void launch_solve_reset(int* flags, int64_t n, int polls, hipStream_t st)
 {
     if (n > 0)
         hipLaunchKernelGGL(k_solve_reset, dim3((unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, 512)),
-                           dim3(kThreads), 0, st, flags, n);
+                           dim3(kThreads), 0, st, flags, n, polls);
 }
 // Four workgroups per CU (in FP64, where the chip holds three, the last quarter
 // finds the tickets gone); fewer tickets, fewer.
