@@ -180,10 +180,17 @@ __device__ __forceinline__ void load_cols(T (&a)[16], const T* M, int row, int l
 // 16 to 64 entries (16% on a 12^3 27-point stencil), and is 2% larger with
 // these.  Four chains in the tasks that run on 16 rows or columns; two in the
 // block tasks (kFwdPiv, kBwdPiv), whose three tiles in flight leave no
-// registers for more (solves 5 to 15% slower at four).
-template <int N, typename T, typename B> __device__ __forceinline__ void mma_chains(d4& acc, const T (&a)[16], B b)
+// registers for more (solves 5 to 15% slower at four).  One with an FP32
+// factor, whose own rounding is 2^29 times that of these sums.
+template <int N64, typename T, typename B> __device__ __forceinline__ void mma_chains(d4& acc, const T (&a)[16], B b)
 {
-    static_assert(N == 2 || N == 4, "added pairwise");
+    constexpr int N = sizeof(T) == 8 ? N64 : 1;
+    static_assert(N == 1 || N == 2 || N == 4, "added pairwise");
+    if constexpr (N == 1) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc = mma((double)a[j], b(j), acc);
+        return;
+    }
     d4 p[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) p[j] = d4{0, 0, 0, 0};
