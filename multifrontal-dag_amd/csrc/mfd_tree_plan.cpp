@@ -19,16 +19,18 @@ constexpr int kManyTasks = 8192, kTicketMost = 4;
 // 16 pivot columns and 0.06 us per row, 0.0625 per row and panel, and waits
 // only for its children; a level takes 10 us and 0.1 per row for fronts of
 // order <= 64, 12 us, 0.28 per column of a block and 17 per further block for
-// larger ones, whatever their number; where fronts are many, one costs 0.012
-// us and its time over 800 in the launch, 0.02 us and 7.5e-6 n^2 outside it.
-// Fitted to forests of 1 to 1024 chains of equal fronts of order 16 to 128
-// (errors up to 30%).
+// larger ones, whatever their number, and 8 us for every child outside the
+// launch that one of its fronts has beyond the first (a launch per rank);
+// where fronts are many, one costs 0.012 us and its time over 800 in the
+// launch, 0.02 us and 7.5e-6 n^2 outside it.  Fitted to forests of 1 to 1024
+// chains of equal fronts of order 16 to 128 (errors up to 30%).
 double predicted_us(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible, int order)
 {
     const int m = (int)nodes.size();
     std::vector<char> in(m, 0);
     std::vector<int> depth(m, 0);
     std::vector<double> path(m, 0.0), small, large;
+    std::vector<int> ranks;
     double longest = 0.0, many = 0.0;
     bool any = false;
     for (int s = 0; s < m; ++s) {  // children before parents
@@ -53,8 +55,13 @@ double predicted_us(const Structure& S, const std::vector<NodeDev>& nodes, const
         if ((int)level.size() <= depth[s]) level.resize(depth[s] + 1, 0.0);
         const double us = n <= kTile ? 10.0 + 0.1 * n : 12.0 + 0.28 * std::min(c, kPanel) + 17.0 * ((c - 1) / kPanel);
         level[depth[s]] = std::max(level[depth[s]], us);
+        int outside = 0;
+        for (int ch : S.children[s]) outside += !in[ch - 1];
+        if ((int)ranks.size() <= depth[s]) ranks.resize(depth[s] + 1, 1);
+        ranks[depth[s]] = std::max(ranks[depth[s]], outside);
     }
     double t = (any ? 10.0 + longest : 0.0) + many;
+    for (int r : ranks) t += 8.0 * (r - 1);
     for (double us : small) t += us;
     for (double us : large) t += us;
     return t;
@@ -67,14 +74,14 @@ double predicted_us(const Structure& S, const std::vector<NodeDev>& nodes, const
 // loses where a few fronts follow one another, of which it takes one at a time
 // by one workgroup: 64 x 64 blocks in a chain of 12 took 699 us in it and 387
 // in the level schedule, 60 x 60 blocks by themselves 55 and 34.  The bound of
-// 3/4 keeps every tree that branches where it measured faster; a forest
-// without branches, where the prediction is good to a few percent, needs no
-// such margin.
+// 0.85 keeps every tree that branches where it measured faster; a forest
+// without branches, where the prediction is good to a few percent, needs less
+// of a margin.
 int largest_order(const Structure& S, const std::vector<NodeDev>& nodes, const std::vector<char>& eligible)
 {
     bool branches = false;
     for (const auto& ch : S.children) branches = branches || ch.size() > 1;
-    double best = predicted_us(S, nodes, eligible, kTreeFront) * (branches ? 0.75 : 0.9);
+    double best = predicted_us(S, nodes, eligible, kTreeFront) * (branches ? 0.85 : 0.9);
     int order = kTreeFront;
     for (int o : {kTile, 0}) {
         const double us = predicted_us(S, nodes, eligible, o);

@@ -79,6 +79,7 @@ def check_fronts(s, val):
     ("dense_30", lambda: arrow(30, 0, 1, 1), 0), ("dense_64", lambda: arrow(64, 0, 1, 1), 0),
     ("dense_128", lambda: arrow(128, 0, 1, 1), 0), ("chain_8", lambda: chain(8, 16), 128),
     ("chain_64", lambda: chain(64, 12), 0), ("grid_60", lambda: P.laplacian_2d(60), 128),
+    ("star_100", lambda: arrow(100, 28, 40, 1), 128), ("star_60", lambda: arrow(60, 3, 100, 1), 128),
 ], ids=lambda v: v if isinstance(v, str) else "")
 def test_chains_of_large_fronts_are_left_to_the_levels(name, make, order):
     p = make()
